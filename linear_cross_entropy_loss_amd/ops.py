@@ -586,6 +586,13 @@ def linear_cross_entropy(
     """
     _check_inputs(x, y, At)
     if not torch.compiler.is_compiling():
+        if not (torch.is_grad_enabled() and (x.requires_grad or At.requires_grad)):
+            # Nobody can ask for a gradient.  (Inside the Function this would not show: there
+            # `ctx.needs_input_grad` says what the inputs are, not whether grad mode is on, so that a parameter
+            # under no_grad would have its gradient computed along with the loss.)
+            out5 = _forward_impl(_autocast_x(x, At), y, At, int(ignore_index), float(z_regularization),
+                                 float(logit_scale), int(N_chunk_size), bool(monitoring), _pack_mode())[0]
+            return out5.unbind(0)
         loss, z_reg, logit_max, logit_ent, logit_norm = LinearXentImplementation.apply(
             x, y, At, int(ignore_index), float(z_regularization), float(logit_scale), int(N_chunk_size),
             bool(monitoring))
