@@ -381,6 +381,7 @@ class LinearXentImplementation(torch.autograd.Function):
         ctx.x_shape = x_in.shape
         loss, z_reg, logit_max, logit_ent, logit_norm = out5.unbind(0)
         ctx.mark_non_differentiable(z_reg, logit_max, logit_ent, logit_norm)
+        ctx.set_materialize_grads(False)  # (else autograd fills a zero for each of those four, a launch each)
         return loss, z_reg, logit_max, logit_ent, logit_norm
 
     @staticmethod
@@ -388,6 +389,8 @@ class LinearXentImplementation(torch.autograd.Function):
     def backward(ctx, grad_output, void0=None, void1=None, void2=None, void3=None):
         x, y1, w, lse, n_valid = ctx.saved_tensors
         ignore_index, z_regularization, logit_scale, N_chunk_size, pack, layout = ctx.lce_cfg
+        if grad_output is None:
+            return None, None, None, None, None, None, None, None
         grads, ctx.lce_grads = ctx.lce_grads, None
         if grads is not None:
             # computed in the forward for an upstream gradient of 1 (ops.py:810 does the same multiplication); a
