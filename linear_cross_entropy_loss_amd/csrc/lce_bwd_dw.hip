@@ -569,7 +569,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dw_persistent_kernel(const BwdAr
   // (a chunk without a kept row adds nothing to the sums of the earlier chunks)
   if ((ACC == 2 || ACC == 4 || ACC == 7) && prob.rows == 0) return;
   Pipe3<T, E, false, E, false, DwProblem<T, WVH, MODE, ACC>> pipe(prob);
-  pipe.run(prob.ldx, a.vs / kBK, prob.plan.kt, lds);
+  pipe.run(prob.ldx, a.vs / kBK, prob.plan.kt, lds, (int)blockIdx.x);
 }
 
 // Second step for the tail tiles: kTailParts workgroups share tail tile b (16 of its rows each) -- they sum

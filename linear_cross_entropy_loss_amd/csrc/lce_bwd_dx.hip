@@ -229,7 +229,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dx_persistent_kernel(const BwdAr
   typedef typename elem_of<T>::type E;
   DxProblem<T, KMASK, WVH, MODE> prob(a);
   Pipe3<T, E, !WVH, E, true, DxProblem<T, KMASK, WVH, MODE>> pipe(prob);
-  pipe.run(a.ldw, a.vs / kBK, MODE == kDxTails ? prob.plan.kseg : (int)(a.vs / kBK), lds);
+  pipe.run(a.ldw, a.vs / kBK, MODE == kDxTails ? prob.plan.kseg : (int)(a.vs / kBK), lds, (int)blockIdx.x);
 }
 
 // Second step for the tail tiles: kTailParts workgroups share tail tile b (16 rows each) -- they sum its

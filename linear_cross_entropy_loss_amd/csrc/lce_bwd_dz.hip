@@ -363,18 +363,32 @@ template <class T, bool ZREG, bool VTAIL, bool KMASK, bool SPLIT, bool WVH, bool
   }
 };
 
-template <class T, bool ZREG, bool VTAIL, bool KMASK, bool SPLIT, bool WVH, bool FUSE>
+// TAIL: the tile columns that the launch covers, as in the forward (fwd_tiles_persistent_kernel).
+template <class T, bool ZREG, int TAIL, bool KMASK, bool SPLIT, bool WVH, bool FUSE>
 __global__ __launch_bounds__(kThreads) void bwd_dz_persistent_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
-  DzProblem<T, ZREG, VTAIL, KMASK, SPLIT, WVH, FUSE> prob(a);
-  Pipe3<T, E, WVH, E, true, DzProblem<T, ZREG, VTAIL, KMASK, SPLIT, WVH, FUSE>> pipe(prob);
-  pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds);
+  int first = (int)blockIdx.x;
+  if constexpr (TAIL != kTailOnly) {
+    typedef DzProblem<T, ZREG, false, KMASK, SPLIT, WVH, FUSE> Full;
+    Full prob(a);
+    Pipe3<T, E, WVH, E, true, Full> pipe(prob);
+    if (TAIL == kNoTail || first < prob.num_tiles()) pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+    if (TAIL == kWithTail) first = first_tail_tile(first, (int)gridDim.x, prob.num_tiles());
+  }
+  if constexpr (TAIL != kNoTail) {
+    typedef DzProblem<T, ZREG, true, true, SPLIT, WVH, FUSE> Tail;
+    Tail prob(a);
+    if (first >= prob.num_tiles()) return;
+    __syncthreads();  // (every wave is done with the main loop's LDS stages)
+    Pipe3<T, E, WVH, E, true, Tail> pipe(prob);
+    pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+  }
 }
 
-template <class T, bool ZREG, bool VTAIL, bool KMASK, bool SPLIT, bool WVH, bool FUSE = false>
+template <class T, bool ZREG, int TAIL, bool KMASK, bool SPLIT, bool WVH, bool FUSE = false>
 hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
-  auto kern = bwd_dz_persistent_kernel<T, ZREG, VTAIL, KMASK, SPLIT, WVH, FUSE>;
+  auto kern = bwd_dz_persistent_kernel<T, ZREG, TAIL, KMASK, SPLIT, WVH, FUSE>;
   static LdsOptIn optin;
   hipError_t e = optin.ensure(reinterpret_cast<const void*>(kern), kLdsBytes);
   if (e != hipSuccess) return e;
@@ -383,30 +397,29 @@ hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
   return hipGetLastError();
 }
 
-// All full tile columns of the slab, then the column that straddles the end of the vocabulary.
+// All tile columns of the slab in one launch.
 template <class T, bool ZREG, bool SPLIT, bool WVH, bool FUSE = false>
 hipError_t launch_persistent_z(const BwdArgs& a, hipStream_t s) {
   const int64_t tq = a.Np / kTile, full = a.vw / kTile, tail = a.vs / kTile - full;
   const bool exact_k = padded_k(a.H) == a.H;  // the K tiles cover H exactly: no K mask needed
-  if (full > 0) {
-    hipError_t e;
-    if constexpr (FUSE && ZREG) {
-      // (the monitoring sums on top of the K mask do not fit the registers in the kernel for full columns: a hidden
-      // size that is not a multiple of 128 sends every column through the kernel for the last one, which has both)
-      if (!exact_k) {
-        BwdArgs all = a;
-        all.vtail_all = 1;
-        return launch_one<T, ZREG, true, true, SPLIT, WVH, FUSE>(all, (a.vs / kTile) * tq, s);
-      }
-      e = launch_one<T, ZREG, false, false, SPLIT, WVH, FUSE>(a, full * tq, s);
-    } else {
-      e = exact_k ? launch_one<T, ZREG, false, false, SPLIT, WVH, FUSE>(a, full * tq, s)
-                  : launch_one<T, ZREG, false, true, SPLIT, WVH, FUSE>(a, full * tq, s);
+  if (full == 0) return launch_one<T, ZREG, kTailOnly, true, SPLIT, WVH, FUSE>(a, tail * tq, s);
+  if constexpr (FUSE && ZREG) {
+    // (the monitoring sums on top of the K mask do not fit the registers in the kernel for full columns: a hidden
+    // size that is not a multiple of 128 sends every column through the kernel for the last one, which has both)
+    if (!exact_k) {
+      BwdArgs all = a;
+      all.vtail_all = 1;
+      return launch_one<T, ZREG, kTailOnly, true, SPLIT, WVH, FUSE>(all, (a.vs / kTile) * tq, s);
     }
-    if (e != hipSuccess) return e;
+    return tail > 0 ? launch_one<T, ZREG, kWithTail, false, SPLIT, WVH, FUSE>(a, (full + tail) * tq, s)
+                    : launch_one<T, ZREG, kNoTail, false, SPLIT, WVH, FUSE>(a, full * tq, s);
+  } else {
+    if (tail > 0)
+      return exact_k ? launch_one<T, ZREG, kWithTail, false, SPLIT, WVH, FUSE>(a, (full + tail) * tq, s)
+                     : launch_one<T, ZREG, kWithTail, true, SPLIT, WVH, FUSE>(a, (full + tail) * tq, s);
+    return exact_k ? launch_one<T, ZREG, kNoTail, false, SPLIT, WVH, FUSE>(a, full * tq, s)
+                   : launch_one<T, ZREG, kNoTail, true, SPLIT, WVH, FUSE>(a, full * tq, s);
   }
-  if (tail > 0) return launch_one<T, ZREG, true, true, SPLIT, WVH, FUSE>(a, tail * tq, s);
-  return hipSuccess;
 }
 
 template <class T, bool SPLIT, bool WVH> hipError_t launch_persistent(const BwdArgs& a, hipStream_t s) {

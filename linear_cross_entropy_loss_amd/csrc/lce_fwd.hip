@@ -374,13 +374,30 @@ template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON> struct FwdProblem
   }
 };
 
-template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON>
+// TAIL: which tile columns the launch covers: the full ones (kNoTail), the one that straddles V (kTailOnly), or both
+// (kWithTail): the tail tiles are then dealt to the workgroups after those that take part in the last round of full
+// tiles.  A launch of its own for them is one tile's time long whatever their number, on ceil(rows / 256) of the
+// compute units (N=16384, H=1024, V=1000: 36 + 34 us in two launches).
+template <class T, int TAIL, bool KMASK, bool WVH, bool MON>
 __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
-  FwdProblem<T, VTAIL, KMASK, WVH, MON> prob(a);
-  Pipe3<T, E, WVH, E, true, FwdProblem<T, VTAIL, KMASK, WVH, MON>> pipe(prob);
-  pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds);
+  int first = (int)blockIdx.x;
+  if constexpr (TAIL != kTailOnly) {
+    typedef FwdProblem<T, false, KMASK, WVH, MON> Full;
+    Full prob(a);
+    Pipe3<T, E, WVH, E, true, Full> pipe(prob);
+    if (TAIL == kNoTail || first < prob.num_tiles()) pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+    if (TAIL == kWithTail) first = first_tail_tile(first, (int)gridDim.x, prob.num_tiles());
+  }
+  if constexpr (TAIL != kNoTail) {
+    typedef FwdProblem<T, true, true, WVH, MON> Tail;
+    Tail prob(a);
+    if (first >= prob.num_tiles()) return;
+    __syncthreads();  // (every wave is done with the main loop's LDS stages)
+    Pipe3<T, E, WVH, E, true, Tail> pipe(prob);
+    pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+  }
 }
 
 // One workgroup = 64 tokens x 4 strided groups of slices.
@@ -537,9 +554,9 @@ __global__ __launch_bounds__(256) void fwd_final_kernel(const FwdArgs a) {
   }
 }
 
-template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON>
+template <class T, int TAIL, bool KMASK, bool WVH, bool MON>
 hipError_t launch_one(const FwdArgs& a, int64_t tiles, hipStream_t s) {
-  auto kern = fwd_tiles_persistent_kernel<T, VTAIL, KMASK, WVH, MON>;
+  auto kern = fwd_tiles_persistent_kernel<T, TAIL, KMASK, WVH, MON>;
   static LdsOptIn optin;
   hipError_t e = optin.ensure(reinterpret_cast<const void*>(kern), kMainloopLds);
   if (e != hipSuccess) return e;
@@ -548,18 +565,17 @@ hipError_t launch_one(const FwdArgs& a, int64_t tiles, hipStream_t s) {
   return hipGetLastError();
 }
 
-// All full tile columns of the vocabulary, then the column that straddles V.
+// All tile columns of the vocabulary in one launch.
 template <class T, bool WVH, bool MON> hipError_t launch_persistent(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;  // token tiles of this chunk at most
   const int64_t tq = (left < a.nc ? left : a.nc) / kTile, full = a.vw / kTile;
   const bool exact_k = padded_k(a.H) == a.H;  // the K tiles cover H exactly: no K mask needed
-  if (full > 0) {
-    hipError_t e = exact_k ? launch_one<T, false, false, WVH, MON>(a, full * tq, s)
-                           : launch_one<T, false, true, WVH, MON>(a, full * tq, s);
-    if (e != hipSuccess) return e;
-  }
-  if (a.vw % kTile) return launch_one<T, true, true, WVH, MON>(a, tq, s);
-  return hipSuccess;
+  const bool tail = a.vw % kTile != 0;        // a column that straddles V
+  if (full == 0) return launch_one<T, kTailOnly, true, WVH, MON>(a, tq, s);
+  if (tail)
+    return exact_k ? launch_one<T, kWithTail, false, WVH, MON>(a, (full + 1) * tq, s)
+                   : launch_one<T, kWithTail, true, WVH, MON>(a, (full + 1) * tq, s);
+  return exact_k ? launch_one<T, kNoTail, false, WVH, MON>(a, full * tq, s) : launch_one<T, kNoTail, true, WVH, MON>(a, full * tq, s);
 }
 
 template <class T, bool WVH> hipError_t launch_layout(const FwdArgs& a, hipStream_t s) {

@@ -132,6 +132,14 @@ LCE_DEV void tile_coords(int bid, int nblocks, int tiles_p, int tiles_q, int ban
   tp = p0 + (within - tq * width);
 }
 
+// Persistent workgroups that work through `full` tiles of one kind and then through tiles of another: the first tile of
+// the second kind for workgroup `wg` of `grid`, so that these go first to the workgroups that the last round of the first
+// kind leaves idle.
+LCE_DEV int first_tail_tile(int wg, int grid, int full) {
+  const int busy = full % grid;
+  return wg >= busy ? wg - busy : wg - busy + grid;
+}
+
 // ---------------------------------------------------------------------------
 // Fragment readers: per-lane LDS offsets for the four 32-wide blocks of this
 // wave's 128-wide slice of an operand tile.

@@ -428,7 +428,8 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
     prob.epilogue_end(tile, acc, lds + kMainloopLds);
   }
 
-  LCE_DEV void run(int64_t ldp, int64_t ldq, int ktiles_, char* lds_) {
+  // `first`: this workgroup's first output tile (the next ones follow at the distance of the grid).
+  LCE_DEV void run(int64_t ldp, int64_t ldq, int ktiles_, char* lds_, int first) {
     lds = lds_;
     ktiles = ktiles_;
     const int wave = threadIdx.x >> 6;
@@ -446,7 +447,7 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
 
     PRegs sp;
     QRegs sq;
-    stream_begin((int)blockIdx.x);
+    stream_begin(first);
     load_chunks(sp, sq, 0, 16);
     stream_advance();
     store_chunks(sp, sq, lds, 0, 16);
@@ -455,7 +456,7 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
     __syncthreads();
 
     f32x16_t acc[kNB][kNB];
-    for (int tile = (int)blockIdx.x; tile < prob.num_tiles(); tile += (int)gridDim.x) {
+    for (int tile = first; tile < prob.num_tiles(); tile += (int)gridDim.x) {
       if constexpr (Problem::kVarK) ktiles = prob.item_ktiles(tile);
       read_frags(0, lds, 0);
       step<0, true, false, false>(acc, sp, sq);

@@ -43,6 +43,10 @@ constexpr int64_t padded_hidden(int64_t H) { return pad_to(H, 256); }   // hidde
 // K extent of the logit contraction: an even number of 64-wide K tiles, at least four
 constexpr int64_t padded_k(int64_t H) { return pad_to(H, 128) < 256 ? 256 : pad_to(H, 128); }
 
+// Which tile columns of the vocabulary a logit kernel covers: full ones, the one(s) from the column that straddles the end of
+// the vocabulary on, or both.
+enum { kNoTail = 0, kTailOnly = 1, kWithTail = 2 };
+
 struct FwdArgs {
   const void* x;
   const void* w;

@@ -36,3 +36,29 @@ def test_loss_without_gradients_allocates_no_gradients(mode, dtype):
     assert torch.allclose(mod.latest_metrics["logit_max"], want_max, rtol=1e-6, atol=0)
     if dtype == torch.bfloat16:
         assert torch.cuda.max_memory_allocated() - before < H * V * 2
+
+
+# full tile columns and the one that straddles the vocabulary's end in one launch: tile counts around multiples of the 256
+# compute units (a last round of full tiles that is empty, full but one, all but empty; more tail tiles than workgroups)
+@pytest.mark.parametrize("route", [False, "always"])
+@pytest.mark.parametrize("N,V", [(100, 256 * 256 + 8), (100, 255 * 256 + 1), (300, 128 * 256 + 255), (300, 129 * 256 + 8), (66000, 264)])
+def test_tail_column_in_the_launch_of_the_full_ones(N, V, route):
+    from linear_cross_entropy_loss_amd import linear_cross_entropy, ops
+    from oracle import lce_forward_backward_fp64
+
+    H = 72
+    x, y, w = make_inputs(N, H, V, torch.bfloat16, 5, ignore_frac=0.05, device="cuda")
+    x.requires_grad_()
+    w.requires_grad_()
+    token = ops.one_pass.set(route)
+    try:
+        loss = linear_cross_entropy(x, y, w, -1, 1e-3, 1.0, 4096)[0]
+        gx, gw = torch.autograd.grad(loss, (x, w))
+    finally:
+        ops.one_pass.reset(token)
+    ref = lce_forward_backward_fp64(x.detach(), y, w.detach(), -1, 1e-3, 1.0, chunk=4096)
+    assert abs(loss.item() - ref.loss.item()) <= 1e-5 * ref.loss.item()
+    # (bf16: dz, dx and dW are rounded to 8 bits of mantissa, at most 2^-8 relative to the largest entry each)
+    for got, want in ((gx, ref.dx), (gw, ref.dw)):
+        emax, el2 = rel_errors(got, want)
+        assert emax < 2e-2 and el2 < 5e-3
