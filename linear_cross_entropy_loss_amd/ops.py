@@ -366,13 +366,17 @@ class LinearXentImplementation(torch.autograd.Function):
         logit_scale: float = 1.0,
         N_chunk_size: int = 4096,
         monitoring: bool = True,
+        grad_mode: bool = True,
     ):
+        # `grad_mode`: whether gradients were enabled where the Function was applied (in here they never are, and
+        # `ctx.needs_input_grad` says what the inputs are, not whether grad mode is on: a parameter under no_grad would have
+        # its gradient computed along with the loss).
         # Under autocast the activations take the weight's 16-bit type or the autocast dtype; a float32 weight
         # is NOT copied: the library rounds the fp32 master weight one vocabulary slab at a time, inside its
         # workspace.
         x_in = _autocast_x(x_in, At)
         pack = _pack_mode()
-        need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[2]
+        need_dx, need_dw = grad_mode and ctx.needs_input_grad[0], grad_mode and ctx.needs_input_grad[2]
         done = None
         if (need_dx or need_dw) and one_pass.get():
             done = _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack,
@@ -398,7 +402,7 @@ class LinearXentImplementation(torch.autograd.Function):
         x, y1, w, lse, n_valid = ctx.saved_tensors
         ignore_index, z_regularization, logit_scale, N_chunk_size, pack, layout = ctx.lce_cfg
         if grad_output is None:
-            return None, None, None, None, None, None, None, None
+            return (None,) * 9
         grads, ctx.lce_grads = ctx.lce_grads, None
         if grads is not None:
             # computed in the forward for an upstream gradient of 1 (ops.py:810 does the same multiplication); a
@@ -413,7 +417,7 @@ class LinearXentImplementation(torch.autograd.Function):
                                     N_chunk_size, ctx.needs_input_grad[0], ctx.needs_input_grad[2], pack, layout)
         if dx is not None:
             dx = dx.view(ctx.x_shape)
-        return dx, None, dw, None, None, None, None, None
+        return dx, None, dw, None, None, None, None, None, None
 
 
 # ---------------------------------------------------------------------------------------------------------
@@ -597,16 +601,9 @@ def linear_cross_entropy(
     """
     _check_inputs(x, y, At)
     if not torch.compiler.is_compiling():
-        if not (torch.is_grad_enabled() and (x.requires_grad or At.requires_grad)):
-            # Nobody can ask for a gradient.  (Inside the Function this would not show: there
-            # `ctx.needs_input_grad` says what the inputs are, not whether grad mode is on, so that a parameter
-            # under no_grad would have its gradient computed along with the loss.)
-            out5 = _forward_impl(_autocast_x(x, At), y, At, int(ignore_index), float(z_regularization),
-                                 float(logit_scale), int(N_chunk_size), bool(monitoring), _pack_mode())[0]
-            return out5.unbind(0)
         loss, z_reg, logit_max, logit_ent, logit_norm = LinearXentImplementation.apply(
             x, y, At, int(ignore_index), float(z_regularization), float(logit_scale), int(N_chunk_size),
-            bool(monitoring))
+            bool(monitoring), torch.is_grad_enabled())
         return loss, z_reg, logit_max, logit_ent, logit_norm
     x = _autocast_x(x, At)
     route = _route_mode()

@@ -38,6 +38,21 @@ def test_loss_without_gradients_allocates_no_gradients(mode, dtype):
         assert torch.cuda.max_memory_allocated() - before < H * V * 2
 
 
+@pytest.mark.parametrize("transform", ["forward_ad", "vmap"])
+def test_loss_without_gradients_refuses_transforms(transform):
+    """Also where no input needs a gradient: a tangent is not dropped and a batch dimension not misread, the call is refused as
+    the autograd Function refuses it."""
+    from linear_cross_entropy_loss_amd import linear_cross_entropy
+
+    x, y, w = make_inputs(64, 64, 256, torch.bfloat16, 3, device="cuda")
+    with torch.no_grad(), pytest.raises(Exception):
+        if transform == "vmap":
+            torch.func.vmap(lambda xx: linear_cross_entropy(xx, y, w)[0])(x[None])
+        else:
+            with torch.autograd.forward_ad.dual_level():
+                linear_cross_entropy(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), y, w)
+
+
 # full tile columns and the one that straddles the vocabulary's end in one launch: tile counts around multiples of the 256
 # compute units (a last round of full tiles that is empty, full but one, all but empty; more tail tiles than workgroups)
 @pytest.mark.parametrize("route", [False, "always"])
