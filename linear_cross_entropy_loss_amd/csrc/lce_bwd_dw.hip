@@ -377,38 +377,45 @@ LCE_DEV void dw_plane_split_final(const BwdArgs& a, const char* hi, int hi_strid
 }
 
 // fp32 dW summed over chunks of token rows in the caller's buffer itself (BwdArgs::dw_acc 3 / 4): the tile's sum times
-// the final factor is stored (first chunk) or added to what is there (ADD), in the 16-byte quads a lane holds -- rows
-// of the stored matrix along the lanes, as in dw_epilogue; the four quads of an accumulator block are fetched
-// together before any is used.
+// the final factor is stored (first chunk) or added to what is there (ADD).  Bound by the memory traffic of the sums, with the
+// matrix pipe idle: 256 KiB written per tile, and as much read for ADD.  A register quad of a wave is 32 bytes of each of 32
+// rows, pieces that the memory channels serve badly, so a wave takes the 32 rows x 128 columns of one accumulator block row at
+// a time through its own 16 KiB slice of `scratch` (main-loop stage 1, idle during an epilogue) and moves them as 512-byte
+// rows, two per instruction; the old sums of a block row are all in flight before the first is used.  Staging rows have their
+// 16-byte piece index XOR-ed by row & 7.  (Forward + backward with quads stored straight from the registers against this: N=8192,
+// H=2048, V=65536 in bf16 5.91 -> 5.58 ms; N=32768, H=4096, V=262144 in fp16, 3 chunks, 168.6 -> 165.9 ms.)
 template <bool WVH, bool ADD>
-LCE_DEV void dw_epilogue_f32_sum(const BwdArgs& a, f32x16_t (&acc)[kNB][kNB], int tp, int tq) {
+LCE_DEV void dw_epilogue_f32_sum(const BwdArgs& a, f32x16_t (&acc)[kNB][kNB], int tp, int tq, char* scratch) {
+  static_assert(kBlk * kWaveTile * 4 <= kDwSliceBytes, "a block row of sums fits a wave's slice");
   const DwTileGeom<WVH> g(a, tp, tq);
   const int tid = opaque_tid();
   const int lane = tid & 63, wave = tid >> 6;
   const int wp = wave & 1, wq = wave >> 1;
   const int w_row = WVH ? wq : wp, w_col = WVH ? wp : wq;
-  const int half = lane >> 5;
+  const int half = lane >> 5, l31 = lane & 31;
   const float coef = final_factor_of(a);
+  char* mine = scratch + wave * kDwSliceBytes;
+  char* mine_w = mine + l31 * 512;              // this lane's row when it writes its quads
+  // when rows are moved: lane l takes piece l % 32 (four columns) of row 2 * it + l / 32
+  const int64_t col = g.col0 + w_col * kWaveTile + 4 * l31;
+  // pieces that start at or past the last column are left alone; one that it cuts through is written whole, into the stride
+  // padding of its row
+  const bool col_ok = col < g.col_limit;
+  const int64_t first_row = g.row0 + w_row * kWaveTile + half;
+  float* at = reinterpret_cast<float*>(a.dw) + first_row * a.lddw + col;
 #pragma unroll
   for (int rb = 0; rb < kNB; ++rb) {
-    const int64_t row = g.row0 + w_row * kWaveTile + rb * kBlk + (lane & 31);
-    const bool row_exists = row < g.row_limit;
-    const int64_t c0 = g.col0 + w_col * kWaveTile + 4 * half;  // this lane's first column
-    float* prow = reinterpret_cast<float*>(a.dw) + row * a.lddw + c0;
+    f32x4_t old[16];
+    if (ADD) {
+#pragma unroll
+      for (int it = 0; it < 16; ++it) {
+        const int r = rb * kBlk + 2 * it;
+        const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+        old[it] = col_ok && first_row + r < g.row_limit ? *reinterpret_cast<const f32x4_t*>(at + r * a.lddw) : zero;
+      }
+    }
 #pragma unroll
     for (int cbk = 0; cbk < kNB; ++cbk) {
-      f32x4_t old[4];
-      bool ok[4];
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        // quads that start at or past the last column are left alone; one that it cuts through is written whole,
-        // into the stride padding of its row
-        ok[rq] = row_exists && c0 + cbk * kBlk + 8 * rq < g.col_limit;
-        if (ADD) {
-          const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-          old[rq] = ok[rq] ? *reinterpret_cast<const f32x4_t*>(prow + cbk * kBlk + 8 * rq) : zero;
-        }
-      }
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
         f32x4_t v;
@@ -418,14 +425,24 @@ LCE_DEV void dw_epilogue_f32_sum(const BwdArgs& a, f32x16_t (&acc)[kNB][kNB], in
           float t;
           if (WVH) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(t) : "a"(acc[cbk][rb][rq * 4 + j]));
           else asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(t) : "a"(acc[rb][cbk][rq * 4 + j]));
-          v[j] = t * coef;
+          v[j] = t;
         }
-        if (ADD) v += old[rq];
-        if (ok[rq]) *reinterpret_cast<f32x4_t*>(prow + cbk * kBlk + 8 * rq) = v;
+        *reinterpret_cast<f32x4_t*>(mine_w + (((cbk * 8 + rq * 2 + half) ^ (l31 & 7)) << 4)) = v;
       }
-      __builtin_amdgcn_sched_barrier(0);  // (one block in registers at a time: an operand tile is in flight)
     }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int it = 0; it < 16; ++it) {
+      const int lr = 2 * it + half, r = rb * kBlk + 2 * it;
+      f32x4_t v = *reinterpret_cast<const f32x4_t*>(mine + lr * 512 + ((l31 ^ (lr & 7)) << 4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = ADD ? fmaf(v[j], coef, old[it][j]) : v[j] * coef;
+      if (col_ok && first_row + r < g.row_limit) *reinterpret_cast<f32x4_t*>(at + r * a.lddw) = v;
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_sched_barrier(0);  // (one block row in registers at a time: an operand tile is in flight)
   }
+  __syncthreads();  // scratch is handed back to the main loop
 }
 
 // How one launch divides its work: as for dx (lce_bwd_dx.hip).  The T = (vs/256) x (Hp/256) output tiles
@@ -541,7 +558,7 @@ template <class T, bool WVH, int MODE, int ACC = 0> struct DwProblem {
     int item, tp, tq, seg;
     decode(local, item, tp, tq, seg);
     if constexpr (ACC == 3 || ACC == 4) {
-      dw_epilogue_f32_sum<WVH, ACC == 4>(a, acc, tp, tq);
+      dw_epilogue_f32_sum<WVH, ACC == 4>(a, acc, tp, tq, scratch);
       return;
     } else if constexpr (ACC != 0) {
       int stride;
