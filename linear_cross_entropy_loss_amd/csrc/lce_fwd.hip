@@ -8,10 +8,10 @@
 // reference kernel, linear_cross_entropy/ops.py:190-236, computes the same
 // per-tile lse but also stores the fp32 logits, ops.py:216.)
 //
-// fwd_rows_kernel merges the slice partials of each token into its lse and
-// forms the per-token loss terms (ops.py:753-761); fwd_final_kernel sums them
-// in a fixed order into the five scalars of ops.py:802 and the valid-label
-// count of ops.py:705.  All reductions are order-deterministic.
+// fwd_rows_kernel merges the slice partials of each token into its lse, forms
+// the per-token loss terms (ops.py:753-761) and sums them in a fixed order
+// into the five scalars of ops.py:802 and the valid-label count of
+// ops.py:705.  All reductions are order-deterministic.
 #include "lce_gemm3.h"
 #include "lce_internal.h"
 
@@ -383,6 +383,7 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
   int first = (int)blockIdx.x;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && a.row0 == 0) *a.done = 0;  // (for the row merge of the first chunk)
   if constexpr (TAIL != kTailOnly) {
     typedef FwdProblem<T, false, KMASK, WVH, MON> Full;
     Full prob(a);
@@ -400,11 +401,29 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
   }
 }
 
-// One workgroup = 64 tokens x 4 strided groups of slices.
-__global__ __launch_bounds__(256) void fwd_rows_kernel(const FwdArgs a) {
-  __shared__ float sh_m[4][kMergeRows], sh_s[4][kMergeRows], sh_lse[kMergeRows];
-  __shared__ float sh_pz[4][kMergeRows], sh_sq[4][kMergeRows], sh_mx[4][kMergeRows];
-  __shared__ double sh_red[7][kMergeRows];
+// Sum (or, IS_MAX, largest) of a double over the 64 lanes of a wave, the same in every lane and in a fixed order.
+template <bool IS_MAX> LCE_DEV double wave_reduce(double v) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    const double o = __shfl_xor(v, d);
+    v = IS_MAX ? fmax(v, o) : v + o;
+  }
+  return v;
+}
+
+// Row merge: one workgroup = 64 tokens (lanes) x kMergeGroups strided groups of slices (waves).  Bound by latency: a few
+// workgroups (64 for a chunk of 4096 rows), each a chain of batches of 8 loads in flight, so a token's slices go to 16 waves
+// rather than to 4, and the sums over the workgroup's tokens are butterflies over a wave's lanes (394 slices: 12 us a launch with 4 waves
+// and serial sums).
+//   The workgroup that is done last (a count behind the block sums, cleared by the tile kernel before) adds up the block
+// sums of all of them in the order of their numbers and writes the five scalars: no launch of its own for that (4 to 5 us
+// at the end of every step).
+constexpr int kMergeGroups = 16;
+__global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdArgs a) {
+  constexpr int G = kMergeGroups;
+  __shared__ float sh_m[G][kMergeRows], sh_s[G][kMergeRows], sh_lse[kMergeRows];
+  __shared__ float sh_pz[G][kMergeRows], sh_sq[G][kMergeRows], sh_mx[G][kMergeRows];
+  __shared__ int sh_last;
   const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
   const int64_t tokl = (int64_t)blockIdx.x * kMergeRows + r;  // row inside the chunk of this launch
   const int64_t tok = a.row0 + tokl;  // < Np; rows that do not exist only keep the block sums aligned
@@ -419,11 +438,11 @@ __global__ __launch_bounds__(256) void fwd_rows_kernel(const FwdArgs a) {
   // batch are in flight together (a slice without a single valid column holds -inf and
   // contributes exp2(-inf) = 0).
   float M = -INFINITY, S = 0.f;
-  for (int c0 = g; c0 < nslices; c0 += 32) {
+  for (int c0 = g; c0 < nslices; c0 += 8 * G) {
     float l[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int c = c0 + 4 * u;
+      const int c = c0 + G * u;
       l[u] = c < nslices ? a.part_lse[(int64_t)c * a.nc + tokl] : -INFINITY;
     }
     float mb = l[0];
@@ -441,10 +460,11 @@ __global__ __launch_bounds__(256) void fwd_rows_kernel(const FwdArgs a) {
   sh_s[g][r] = S;
   __syncthreads();
   if (g == 0) {
-    float Mt = fmaxf(fmaxf(sh_m[0][r], sh_m[1][r]), fmaxf(sh_m[2][r], sh_m[3][r]));
-    float St = 0.f;
+    float Mt = sh_m[0][r], St = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 1; i < G; ++i) Mt = fmaxf(Mt, sh_m[i][r]);
+#pragma unroll
+    for (int i = 0; i < G; ++i)
       if (sh_s[i][r] != 0.f) St += sh_s[i][r] * fast_exp2((sh_m[i][r] - Mt) * kLog2e);
     const float lse = Mt + fast_log(St);
     sh_lse[r] = lse;
@@ -454,15 +474,15 @@ __global__ __launch_bounds__(256) void fwd_rows_kernel(const FwdArgs a) {
     // and the backward never looks at the lse of such a token.)
     if (exists) a.lse[a.perm != nullptr ? packed_token(a.perm, tok, a.N) : tok] = a.y[tok] != a.ignore_index ? lse : 0.f;
   }
-  __syncthreads();
-  const float lse = sh_lse[r];
   if (a.monitoring) {
+    __syncthreads();
+    const float lse = sh_lse[r];
     float pz = 0.f, sq = 0.f, mx = -INFINITY;
-    for (int c0 = g; c0 < nslices; c0 += 32) {
+    for (int c0 = g; c0 < nslices; c0 += 8 * G) {
       float pl[8], pp[8], ps[8], pm[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int c = c0 + 4 * u;
+        const int c = c0 + G * u;
         const bool in = c < nslices;
         const int64_t o = (int64_t)(in ? c : 0) * a.nc + tokl;
         pl[u] = in ? a.part_lse[o] : -INFINITY;
@@ -480,45 +500,59 @@ __global__ __launch_bounds__(256) void fwd_rows_kernel(const FwdArgs a) {
     sh_pz[g][r] = pz;
     sh_sq[g][r] = sq;
     sh_mx[g][r] = mx;
+    __syncthreads();
   }
-  __syncthreads();
+  double* blk = reinterpret_cast<double*>(a.blk);
+  const int nblk = (int)(a.Np / kMergeRows);  // over all chunks
   if (g == 0) {
     const bool valid = exists && a.y[tok] != a.ignore_index;
-    const double l = (double)lse;
+    const double l = (double)sh_lse[r];
     double ent = 0.0, nrm = 0.0, mx = -INFINITY;
     if (a.monitoring && exists) {
-      const float pz = (sh_pz[0][r] + sh_pz[1][r]) + (sh_pz[2][r] + sh_pz[3][r]);
-      const float sq = (sh_sq[0][r] + sh_sq[1][r]) + (sh_sq[2][r] + sh_sq[3][r]);
-      mx = (double)fmaxf(fmaxf(sh_mx[0][r], sh_mx[1][r]), fmaxf(sh_mx[2][r], sh_mx[3][r]));
-      ent = valid ? (double)(lse - pz) : 0.0;
+      float pz = 0.f, sq = 0.f, m = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        pz += sh_pz[i][r];
+        sq += sh_sq[i][r];
+        m = fmaxf(m, sh_mx[i][r]);
+      }
+      mx = (double)m;
+      ent = valid ? (double)(sh_lse[r] - pz) : 0.0;
       nrm = (double)sqrtf(sq);
     }
     // tgt[tok] is written by the one tile that holds the target column; it is only read for a valid
     // label (for a valid label outside [0, V) nothing wrote it -- and the loss is NaN anyway)
-    sh_red[0][r] = valid ? l - (double)a.tgt[tok] : 0.0;
-    sh_red[1][r] = valid ? l * l : 0.0;
-    sh_red[2][r] = ent;
-    sh_red[3][r] = nrm;
-    sh_red[4][r] = mx;
-    sh_red[5][r] = valid ? 1.0 : 0.0;
-    // a label that is neither ignore_index nor a column of W: poisons the loss (see fwd_final_kernel)
-    sh_red[6][r] = (valid && (a.y[tok] < 0 || a.y[tok] >= a.V)) ? 1.0 : 0.0;
+    double v[7] = {valid ? l - (double)a.tgt[tok] : 0.0,
+                   valid ? l * l : 0.0,
+                   ent,
+                   nrm,
+                   mx,
+                   valid ? 1.0 : 0.0,
+                   // a label that is neither ignore_index nor a column of W: poisons the loss (below)
+                   (valid && (a.y[tok] < 0 || a.y[tok] >= a.V)) ? 1.0 : 0.0};
+    double mine = 0.0;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+      const double t = q == 4 ? wave_reduce<true>(v[q]) : wave_reduce<false>(v[q]);
+      if (r == q) mine = t;
+    }
+    if (r < 7) blk[(a.row0 / kMergeRows + (int64_t)blockIdx.x) * 8 + r] = mine;
+    __threadfence();  // this block's sums are there for every compute unit before it is counted
+    if (r == 0) {
+      const unsigned before = __hip_atomic_fetch_add(a.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sh_last = before == (unsigned)(nblk - 1) ? 1 : 0;
+      // (a call restricted to this phase finds the count as the tile kernel left it)
+      if (before == (unsigned)(nblk - 1)) __hip_atomic_store(a.done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   __syncthreads();
-  if (threadIdx.x < 7) {
-    const int q = threadIdx.x;
-    double acc = sh_red[q][0];
-    for (int i = 1; i < kMergeRows; ++i) acc = (q == 4) ? fmax(acc, sh_red[q][i]) : acc + sh_red[q][i];
-    reinterpret_cast<double*>(a.blk)[(a.row0 / kMergeRows + (int64_t)blockIdx.x) * 8 + q] = acc;
-  }
-}
+  if (!sh_last) return;
+  __threadfence();  // and the sums of all the others are read from where they put them
 
-__global__ __launch_bounds__(256) void fwd_final_kernel(const FwdArgs a) {
-  __shared__ double sh[7][256];
-  const int nblk = (int)(a.Np / kMergeRows);
-  const double* blk = reinterpret_cast<const double*>(a.blk);
+  // final sums, in a fixed order whichever workgroup forms them
+  __shared__ double sh_fin[G][7];
   double v[7] = {0, 0, 0, 0, -INFINITY, 0, 0};
-  for (int b = threadIdx.x; b < nblk; b += 256) {
+  for (int b = threadIdx.x; b < nblk; b += 64 * G) {
 #pragma unroll
     for (int q = 0; q < 7; ++q) {
       const double t = blk[(int64_t)b * 8 + q];
@@ -526,30 +560,29 @@ __global__ __launch_bounds__(256) void fwd_final_kernel(const FwdArgs a) {
     }
   }
 #pragma unroll
-  for (int q = 0; q < 7; ++q) sh[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) {
-#pragma unroll
-      for (int q = 0; q < 7; ++q) {
-        const double t = sh[q][threadIdx.x + w];
-        sh[q][threadIdx.x] = (q == 4) ? fmax(sh[q][threadIdx.x], t) : sh[q][threadIdx.x] + t;
-      }
-    }
-    __syncthreads();
+  for (int q = 0; q < 7; ++q) {
+    const double t = q == 4 ? wave_reduce<true>(v[q]) : wave_reduce<false>(v[q]);
+    if (r == 0) sh_fin[g][q] = t;
   }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const double R = sh[5][0];  // 0 valid labels -> 0/0 = NaN, as F.cross_entropy gives
-    const double ce = sh[0][0] / R, zr = sh[1][0] / R;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+      double t = sh_fin[0][q];
+      for (int i = 1; i < G; ++i) t = (q == 4) ? fmax(t, sh_fin[i][q]) : t + sh_fin[i][q];
+      v[q] = t;
+    }
+    const double R = v[5];  // 0 valid labels -> 0/0 = NaN, as F.cross_entropy gives
+    const double ce = v[0] / R, zr = v[1] / R;
     // Labels outside [0, V) that are not ignore_index have no column to match; the reference lets
     // them contribute lse alone, silently.  Here they turn the loss into NaN (F.cross_entropy
     // raises a device-side assert for them) -- visible to the caller, no synchronisation needed.
-    const bool bad_labels = sh[6][0] != 0.0;
+    const bool bad_labels = v[6] != 0.0;
     a.out5[0] = bad_labels ? __builtin_nanf("") : (float)(ce + (double)a.z_reg * zr);
     a.out5[1] = (float)zr;
-    a.out5[2] = a.monitoring ? (float)sh[4][0] : 0.f;
-    a.out5[3] = a.monitoring ? (float)(sh[2][0] / R) : 0.f;
-    a.out5[4] = a.monitoring ? (float)(sh[3][0] / (double)a.N) : 0.f;
+    a.out5[2] = a.monitoring ? (float)v[4] : 0.f;
+    a.out5[3] = a.monitoring ? (float)(v[2] / R) : 0.f;
+    a.out5[4] = a.monitoring ? (float)(v[3] / (double)a.N) : 0.f;
     a.n_valid[0] = (int64_t)R;
   }
 }
@@ -595,12 +628,7 @@ hipError_t launch_fwd_tiles(const FwdArgs& a, hipStream_t s) {
 
 hipError_t launch_fwd_rows(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;
-  hipLaunchKernelGGL(fwd_rows_kernel, dim3((unsigned)((left < a.nc ? left : a.nc) / kMergeRows)), dim3(256), 0, s, a);
-  return hipGetLastError();
-}
-
-hipError_t launch_fwd_final(const FwdArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(fwd_final_kernel, dim3(1), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(fwd_rows_kernel, dim3((unsigned)((left < a.nc ? left : a.nc) / kMergeRows)), dim3(64 * kMergeGroups), 0, s, a);
   return hipGetLastError();
 }
 
