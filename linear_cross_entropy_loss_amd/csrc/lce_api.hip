@@ -657,12 +657,9 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   // the count of valid labels comes first (the gradients' factor needs it), with it the packing
   hipError_t e = hipSuccess;
   if (ph & LCE_PHASE_PACK) {
-    e = lce::launch_compact_labels(y, p->N, p->ignore_index, (int*)(base + k.cnt), n_rows, perm, yc, s);
+    e = lce::launch_compact_labels(y, p->N, p->ignore_index, (int*)(base + k.cnt), n_rows, perm, yc, s, f.nc,
+                                   f.pack ? f.chunks : 0, chunk_rows);
     if (e != hipSuccess) return hip_fail(e, "compact_labels");
-  }
-  if (f.pack && (ph & LCE_PHASE_PACK)) {
-    e = lce::launch_chunk_rows(n_rows, p->N, f.nc, f.chunks, chunk_rows, s);
-    if (e != hipSuccess) return hip_fail(e, "chunk_rows");
   }
   // an fp32 master weight: one 16-bit copy of all of it, which the three tile kernels of every chunk read
   const void* wk = w;

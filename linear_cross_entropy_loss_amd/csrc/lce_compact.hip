@@ -97,6 +97,59 @@ __global__ __launch_bounds__(256) void pack_kept_kernel(const int64_t* y, int64_
   }
 }
 
+// Rows of the chunks (lce_internal.h): out[c] among `kept` packed rows, out[1024 + c] among all N.
+LCE_DEV void store_chunk_rows(int c, int64_t kept, int64_t N, int64_t nc, int64_t* out) {
+  const int64_t left = kept - (int64_t)c * nc;
+  out[c] = left < 0 ? 0 : (left > nc ? nc : left);
+  const int64_t all = N - (int64_t)c * nc;  // the chunk's rows when the dropped tokens follow the kept ones
+  out[1024 + c] = all < 0 ? 0 : (all > nc ? nc : all);
+}
+
+__global__ __launch_bounds__(1024) void chunk_rows_kernel(const int64_t* n_rows, int64_t N, int64_t nc, int chunks, int64_t* out) {
+  if ((int)threadIdx.x < chunks) store_chunk_rows((int)threadIdx.x, packed_rows(n_rows, N), N, nc, out);
+}
+
+// All of it in one launch, for N <= 1024 * ITER: one workgroup of 16 waves, each on ITER * 64 consecutive tokens that it
+// holds in registers, counted and numbered by ballots.  Bound by latency, as the four kernels are that do it for any N (counts,
+// their scan, packing, the chunks' rows: one launch of about 5 us each, whatever N).
+template <int ITER>
+__global__ __launch_bounds__(1024) void compact_labels_kernel(const int64_t* y, int N, int64_t ignore_index, int64_t* n_rows,
+                                                              int* perm, int64_t* yc, int64_t nc, int chunks,
+                                                              int64_t* chunk_rows) {
+  __shared__ int sh[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int base = wave * (ITER * 64) + lane;
+  int64_t lab[ITER];
+#pragma unroll
+  for (int it = 0; it < ITER; ++it) lab[it] = base + it * 64 < N ? y[base + it * 64] : ignore_index;
+  int mine = 0;
+#pragma unroll
+  for (int it = 0; it < ITER; ++it) mine += __popcll(__ballot(lab[it] != ignore_index));
+  if (lane == 0) sh[wave] = mine;
+  __syncthreads();
+  int j = 0, kept = 0;  // kept tokens before this wave's, and of all
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    if (w < wave) j += sh[w];
+    kept += sh[w];
+  }
+#pragma unroll
+  for (int it = 0; it < ITER; ++it) {
+    const int i = base + it * 64;
+    const bool keep = lab[it] != ignore_index;
+    const unsigned long long mask = __ballot(keep);
+    const int before = j + __popcll(mask & ((1ull << lane) - 1));
+    if (i < N) {
+      const int at = keep ? before : kept + (i - before);  // a dropped token is number i - before among the dropped
+      perm[at] = i;
+      yc[at] = lab[it];
+    }
+    j += __popcll(mask);
+  }
+  if (threadIdx.x == 0) n_rows[0] = kept;
+  if ((int)threadIdx.x < chunks) store_chunk_rows((int)threadIdx.x, kept, N, nc, chunk_rows);
+}
+
 // One workgroup per packed row (grid-stride).  Rows are moved in 16-byte pieces; `chunks` pieces per row.
 // The last row of x may end with its last element (a caller's matrix need not own the stride padding of its
 // last row): of that row only the whole pieces are moved as such, the rest 16 bits at a time, zero-filled.
@@ -204,11 +257,18 @@ unsigned row_grid(int64_t N, int num_cus) {
 int64_t compact_segments(int64_t N) { return (N + kSegTokens - 1) / kSegTokens; }
 
 hipError_t launch_compact_labels(const int64_t* y, int64_t N, int64_t ignore_index, int* cnt, int64_t* n_rows,
-                                 int* perm, int64_t* yc, hipStream_t s) {
+                                 int* perm, int64_t* yc, hipStream_t s, int64_t nc, int chunks, int64_t* chunk_rows) {
+  if (chunks < 0 || chunks > 1024) return hipErrorInvalidValue;
+  if (N <= 32 * 1024) {
+    auto kern = N <= 4 * 1024 ? compact_labels_kernel<4> : N <= 16 * 1024 ? compact_labels_kernel<16> : compact_labels_kernel<32>;
+    hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, s, y, (int)N, ignore_index, n_rows, perm, yc, nc, chunks, chunk_rows);
+    return hipGetLastError();
+  }
   const int64_t nseg = compact_segments(N);
   hipLaunchKernelGGL(count_kept_kernel, dim3((unsigned)nseg), dim3(256), 0, s, y, N, ignore_index, cnt);
   hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(256), 0, s, cnt, nseg, n_rows);
   hipLaunchKernelGGL(pack_kept_kernel, dim3((unsigned)nseg), dim3(256), 0, s, y, N, ignore_index, cnt, n_rows, perm, yc);
+  if (chunks > 0) hipLaunchKernelGGL(chunk_rows_kernel, dim3(1), dim3(1024), 0, s, n_rows, N, nc, chunks, chunk_rows);
   return hipGetLastError();
 }
 

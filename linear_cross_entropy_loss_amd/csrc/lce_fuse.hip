@@ -86,15 +86,6 @@ __global__ __launch_bounds__(256) void stage_scale_kernel(const BwdArgs a) {
   }
 }
 
-__global__ void chunk_rows_kernel(const int64_t* n_rows, int64_t N, int64_t nc, int chunks, int64_t* out) {
-  const int c = threadIdx.x;
-  if (c >= chunks) return;
-  const int64_t left = packed_rows(n_rows, N) - (int64_t)c * nc;
-  out[c] = left < 0 ? 0 : (left > nc ? nc : left);
-  const int64_t all = N - (int64_t)c * nc;  // the chunk's rows when the dropped tokens follow the kept ones
-  out[1024 + c] = all < 0 ? 0 : (all > nc ? nc : all);
-}
-
 // t[r][c] *= g[0] for r < rows, c < cols (row stride ld, rows on 16-byte boundaries), the product formed in fp32;
 // nothing is read or written when g[0] is 1.  Pieces of 16 bytes, the last piece of a row element by element.
 // v * f rounded to fp32 before anything else happens to it (the compiler may otherwise fold the product into
@@ -153,12 +144,6 @@ hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s) {
   if (a.x_dtype == DT_BF16) hipLaunchKernelGGL(stage_scale_kernel<BF16>, grid, dim3(256), 0, s, a);
   else if (a.x_dtype == DT_F16) hipLaunchKernelGGL(stage_scale_kernel<F16>, grid, dim3(256), 0, s, a);
   else return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-hipError_t launch_chunk_rows(const int64_t* n_rows, int64_t N, int64_t nc, int chunks, int64_t* out, hipStream_t s) {
-  if (chunks < 1 || chunks > 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(chunk_rows_kernel, dim3(1), dim3(1024), 0, s, n_rows, N, nc, chunks, out);
   return hipGetLastError();
 }
 

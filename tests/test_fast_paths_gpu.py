@@ -77,3 +77,36 @@ def test_tail_column_in_the_launch_of_the_full_ones(N, V, route):
     for got, want in ((gx, ref.dx), (gw, ref.dw)):
         emax, el2 = rel_errors(got, want)
         assert emax < 2e-2 and el2 < 5e-3
+
+
+# packing in one launch: token counts around a wave, the sizes its three variants end at, and the first one that takes four launches
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 255, 4096, 4097, 16384, 16385, 32768, 32769])
+@pytest.mark.parametrize("ignored", [0.0, 0.3, 1.0])
+def test_packing_counts_and_order(N, ignored):
+    """Rows packed or not: the same loss, lse order and dx; dropped tokens get zeros."""
+    from linear_cross_entropy_loss_amd import _lib, linear_cross_entropy, ops
+
+    H, V = 64, 512
+    x, y, w = make_inputs(N, H, V, torch.bfloat16, 7, ignore_frac=ignored, device="cuda")
+    if ignored == 1.0:
+        y = torch.full_like(y, -1)
+    got = {}
+    for mode in (_lib.PACK_ALWAYS, _lib.PACK_NEVER):
+        token, route = ops.pack_rows.set(mode), ops.one_pass.set("always")
+        try:
+            x.grad = None
+            xx = x.detach().requires_grad_()
+            loss = linear_cross_entropy(xx, y, w, -1, 0.0, 1.0, 65536)[0]
+            got[mode] = (loss.detach(), torch.autograd.grad(loss, xx)[0])
+        finally:
+            ops.pack_rows.reset(token)
+            ops.one_pass.reset(route)
+    (la, da), (lb, db) = got[_lib.PACK_ALWAYS], got[_lib.PACK_NEVER]
+    if ignored == 1.0:
+        assert torch.isnan(la) and torch.isnan(lb) and not da.any() and not db.any()
+        return
+    # (the same logits; sums of N terms in fp64, rounded once to fp32)
+    assert abs(la.item() - lb.item()) <= 1e-6 * abs(lb.item())
+    assert torch.equal(da[y == -1], torch.zeros_like(da[y == -1]))
+    # (each row's K sums are the same, cut into segments at other places: one bf16 rounding apart)
+    assert torch.allclose(da.float(), db.float(), rtol=2.0 ** -7, atol=1e-7)
