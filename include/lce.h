@@ -346,6 +346,14 @@ int lce_forward_backward(const lce_problem* p, const void* x, const void* w, con
  */
 int lce_scale(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* factor, void* stream);
 
+/*
+ * *out (1 float, device) = the largest power of two that is not above the
+ * number of labels in y[0 .. N) that are not ignore_index (1 if there is none):
+ * the grad_out to give lce_forward_backward for fp16 gradients whose upstream
+ * gradient arrives later.  1 <= N <= 2^30.
+ */
+int lce_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

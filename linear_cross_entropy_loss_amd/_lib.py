@@ -33,6 +33,7 @@ EXPORTS = (
     "lce_forward_backward_plan",
     "lce_forward_backward",
     "lce_scale",
+    "lce_stand_in",
 )
 
 _DTYPES = {torch.bfloat16: LCE_BF16, torch.float16: LCE_F16, torch.float32: LCE_F32}
@@ -109,6 +110,8 @@ def load():
     lib.lce_forward_backward.argtypes = [P, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
     lib.lce_scale.restype = ctypes.c_int
     lib.lce_scale.argtypes = [vp, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, vp, vp]
+    lib.lce_stand_in.restype = ctypes.c_int
+    lib.lce_stand_in.argtypes = [vp, ctypes.c_int64, ctypes.c_int64, vp, vp]
     _lib = lib
     return lib
 

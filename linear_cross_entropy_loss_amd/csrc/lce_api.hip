@@ -1017,6 +1017,13 @@ int lce_scale(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const 
   return LCE_OK;
 }
 
+int lce_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, void* stream) {
+  if (!y || !out || N < 1 || N > ((int64_t)1 << 30)) return LCE_EINVAL_ARG;
+  hipError_t e = lce::launch_stand_in(y, N, ignore_index, out, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "stand_in");
+  return LCE_OK;
+}
+
 int lce_forward_backward_workspace_bytes(const lce_problem* p, size_t* bytes) {
   int rc = check(p, true);
   if (rc != LCE_OK) return rc;

@@ -232,6 +232,9 @@ __device__ __forceinline__ int64_t packed_token(const int* perm, int64_t j, int6
   return t < 0 ? 0 : (t >= N ? N - 1 : t);
 }
 
+// *out = the largest power of two not above the number of labels that are not ignore_index (lce_compact.hip).
+hipError_t launch_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, hipStream_t s);
+
 // Packing of the tokens whose label is not ignore_index (lce_compact.hip).  `cnt` holds one int per
 // compact_segments(N); perm and yc hold N entries each: the kept tokens first (*n_rows of them), then the dropped ones.
 // chunks > 0 (at most 1024), with `nc` rows each: chunk_rows[c] = rows of chunk c among the packed rows, min(max(*n_rows - c * nc, 0), nc);

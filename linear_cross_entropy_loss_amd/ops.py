@@ -224,7 +224,12 @@ def _stand_in_gradient(x, y1, ignore_index):
     save them): they are formed for the largest power of two that is not above the number of valid labels -- entries
     of the order of the per-token gradient -- and divided by it again when the real one is multiplied in."""
     if x.dtype == torch.float16:
-        return torch.exp2(torch.floor(torch.log2((y1 != ignore_index).sum().clamp(min=1).to(torch.float32)))).reshape(1)
+        pre = torch.empty(1, dtype=torch.float32, device=x.device)
+        stream = torch.cuda.current_stream(x.device).cuda_stream
+        with torch.cuda.device(x.device):
+            rc = _lib.load().lce_stand_in(_ptr(y1), y1.numel(), int(ignore_index), _ptr(pre), ctypes.c_void_p(stream))
+        _lib.raise_for_status(rc, "lce_stand_in")
+        return pre
     return torch.ones(1, dtype=torch.float32, device=x.device)
 
 

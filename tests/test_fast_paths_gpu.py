@@ -110,3 +110,17 @@ def test_packing_counts_and_order(N, ignored):
     assert torch.equal(da[y == -1], torch.zeros_like(da[y == -1]))
     # (each row's K sums are the same, cut into segments at other places: one bf16 rounding apart)
     assert torch.allclose(da.float(), db.float(), rtol=2.0 ** -7, atol=1e-7)
+
+
+# around a wave, a workgroup and the 8192 labels of one trip; powers of two and their neighbours
+@pytest.mark.parametrize("N", [1, 64, 1023, 1024, 1025, 8191, 8192, 8193, 65536, 100003])
+def test_stand_in_gradient_is_the_power_of_two_below_the_count(N):
+    from linear_cross_entropy_loss_amd import ops
+
+    x = torch.empty((1, 8), dtype=torch.float16, device="cuda")
+    for kept in sorted({0, 1, N // 3, N - 1, N}):
+        y = torch.arange(N, device="cuda")
+        y[kept:] = -1
+        y = y.flip(0).contiguous()
+        want = 2.0 ** (max(kept, 1).bit_length() - 1)
+        assert ops._stand_in_gradient(x, y, -1).tolist() == [want]
