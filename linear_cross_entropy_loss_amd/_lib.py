@@ -34,6 +34,7 @@ EXPORTS = (
     "lce_forward_backward",
     "lce_scale",
     "lce_stand_in",
+    "lce_pad_rows",
 )
 
 _DTYPES = {torch.bfloat16: LCE_BF16, torch.float16: LCE_F16, torch.float32: LCE_F32}
@@ -112,6 +113,8 @@ def load():
     lib.lce_scale.argtypes = [vp, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, vp, vp]
     lib.lce_stand_in.restype = ctypes.c_int
     lib.lce_stand_in.argtypes = [vp, ctypes.c_int64, ctypes.c_int64, vp, vp]
+    lib.lce_pad_rows.restype = ctypes.c_int
+    lib.lce_pad_rows.argtypes = [vp, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, vp, ctypes.c_int64, vp]
     _lib = lib
     return lib
 

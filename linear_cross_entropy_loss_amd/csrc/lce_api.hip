@@ -1024,6 +1024,18 @@ int lce_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, 
   return LCE_OK;
 }
 
+int lce_pad_rows(const void* src, int dtype, int64_t rows, int64_t cols, int64_t ld, void* dst, int64_t dst_ld,
+                 void* stream) {
+  if (dtype != LCE_BF16 && dtype != LCE_F16 && dtype != LCE_F32) return LCE_EINVAL_DTYPE;
+  const int64_t es = dtype == LCE_F32 ? 4 : 2, most = (int64_t)1 << 40;
+  if (!src || !dst || misaligned(dst) || (uintptr_t)src % (uintptr_t)es != 0 || rows < 1 || cols < 1 || ld < 0 || ld > most ||
+      dst_ld < cols || dst_ld > most || dst_ld * es % 16 != 0)
+    return LCE_EINVAL_ARG;
+  hipError_t e = lce::launch_pad_rows(src, ld * es, rows, cols * es, dst, dst_ld * es, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "pad_rows");
+  return LCE_OK;
+}
+
 int lce_forward_backward_workspace_bytes(const lce_problem* p, size_t* bytes) {
   int rc = check(p, true);
   if (rc != LCE_OK) return rc;

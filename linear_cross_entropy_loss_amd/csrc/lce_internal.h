@@ -232,6 +232,10 @@ __device__ __forceinline__ int64_t packed_token(const int* perm, int64_t j, int6
   return t < 0 ? 0 : (t >= N ? N - 1 : t);
 }
 
+// dst row r = row_bytes bytes at src + r * src_ld (2-byte units, any 2-byte address), then zeros to dst_ld (lce_convert.hip).
+hipError_t launch_pad_rows(const void* src, int64_t src_ld, int64_t rows, int64_t row_bytes, void* dst, int64_t dst_ld,
+                           hipStream_t s);
+
 // *out = the largest power of two not above the number of labels that are not ignore_index (lce_compact.hip).
 hipError_t launch_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, hipStream_t s);
 

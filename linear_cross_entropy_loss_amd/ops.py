@@ -120,8 +120,14 @@ def _aligned_rows(t, what=None):
                                  f"multiples of {m} elements")
     rows, cols = t.shape
     padded = torch.empty((rows, _padded_cols(cols)), dtype=t.dtype, device=t.device)
-    padded[:, :cols] = t
-    padded[:, cols:] = 0  # (read, so it has to be finite)
+    if t.stride(1) == 1 and rows > 0 and cols > 0 and padded.is_cuda and t.data_ptr() % t.element_size() == 0:
+        with torch.cuda.device(t.device):
+            rc = _lib.load().lce_pad_rows(_ptr(t), _lib.dtype_code(t.dtype), rows, cols, t.stride(0), _ptr(padded),
+                                          padded.stride(0), ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream))
+        _lib.raise_for_status(rc, "lce_pad_rows")
+    else:  # (columns apart from each other)
+        padded[:, :cols] = t
+        padded[:, cols:] = 0  # (read, so it has to be finite)
     return padded[:, :cols]
 
 

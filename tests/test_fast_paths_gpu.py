@@ -124,3 +124,19 @@ def test_stand_in_gradient_is_the_power_of_two_below_the_count(N):
         y = y.flip(0).contiguous()
         want = 2.0 ** (max(kept, 1).bit_length() - 1)
         assert ops._stand_in_gradient(x, y, -1).tolist() == [want]
+
+
+# row lengths around a 16-byte piece, the threads of a row and their four pieces each; sources at odd addresses
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows, cols", [(1, 1), (3, 7), (5, 257), (33, 511), (257, 1021), (2, 8191), (9, 50257)])
+@pytest.mark.parametrize("offset, extra", [(0, 0), (1, 0), (3, 2)])
+def test_padded_copy_of_rows(dtype, rows, cols, offset, extra):
+    from linear_cross_entropy_loss_amd import ops
+
+    flat = torch.randn(offset + rows * (cols + extra), device="cuda").to(dtype)
+    t = flat[offset:].view(rows, cols + extra)[:, :cols]
+    out = ops._aligned_rows(t)
+    assert out.data_ptr() % 16 == 0 and out.stride(0) * out.element_size() % 16 == 0 and torch.equal(out, t)
+    if out.data_ptr() != t.data_ptr():
+        whole = torch.as_strided(out, (rows, out.stride(0)), (out.stride(0), 1))
+        assert not whole[:, cols:].any()
