@@ -538,7 +538,6 @@ int forward_impl(const lce_problem* p, const void* x, const void* w, const int64
   a.part_sq = (float*)(base + f.part_sq);
   a.tgt = (float*)(base + f.tgt);
   a.blk = (float*)(base + f.blk);
-  a.done = (unsigned*)(base + f.blk) + 14;
   rc = current_num_cus(&a.num_cus, p->max_workgroups);
   if (rc != LCE_OK) return rc;
   a.live = lce::live_bands(lce::padded_k(splits(p) ? 3 * p->H : p->H) * 2);
@@ -607,6 +606,10 @@ int forward_impl(const lce_problem* p, const void* x, const void* w, const int64
       if (e != hipSuccess) return hip_fail(e, "fwd_rows");
     }
   }
+  if (ph & LCE_PHASE_FWD_REDUCE) {
+    e = lce::launch_fwd_final(a, s);
+    if (e != hipSuccess) return hip_fail(e, "fwd_final");
+  }
   return LCE_OK;
 }
 
@@ -643,7 +646,6 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   fa.part_sq = (float*)(base + f.part_sq);
   fa.tgt = (float*)(base + f.tgt);
   fa.blk = (float*)(base + f.blk);
-  fa.done = (unsigned*)(base + f.blk) + 14;
   fa.lse_rows = (float*)(base + f.lse_rows);
   fa.num_cus = num_cus;
   fa.nc = f.nc;
@@ -738,7 +740,6 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
     if (ph & LCE_PHASE_FWD_TILES) {
       lce::BwdArgs af = a;
       if (all_rows) af.n_rows = chunk_rows + 1024 + c;
-      af.done = c == 0 ? fa.done : nullptr;
       e = lce::launch_fwd_stage(af, s);
       if (e != hipSuccess) return hip_fail(e, "fwd_stage");
     }
@@ -760,6 +761,10 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
       e = lce::launch_bwd_dw(a, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_dw");
     }
+  }
+  if (ph & LCE_PHASE_FWD_REDUCE) {
+    e = lce::launch_fwd_final(fa, s);
+    if (e != hipSuccess) return hip_fail(e, "fwd_final");
   }
   if (f.pack && dx && (ph & LCE_PHASE_BWD_DX)) {
     // tokens that were dropped get exact zeros (nothing to do if none was)

@@ -369,7 +369,6 @@ __global__ __launch_bounds__(kThreads) void bwd_dz_persistent_kernel(const BwdAr
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
   int first = (int)blockIdx.x;
-  if (FUSE && blockIdx.x == 0 && threadIdx.x == 0 && a.done != nullptr) *a.done = 0;
   if constexpr (TAIL != kTailOnly) {
     typedef DzProblem<T, ZREG, false, KMASK, SPLIT, WVH, FUSE> Full;
     Full prob(a);

@@ -8,10 +8,10 @@
 // reference kernel, linear_cross_entropy/ops.py:190-236, computes the same
 // per-tile lse but also stores the fp32 logits, ops.py:216.)
 //
-// fwd_rows_kernel merges the slice partials of each token into its lse, forms
-// the per-token loss terms (ops.py:753-761) and sums them in a fixed order
-// into the five scalars of ops.py:802 and the valid-label count of
-// ops.py:705.  All reductions are order-deterministic.
+// fwd_rows_kernel merges the slice partials of each token into its lse and
+// forms the per-token loss terms (ops.py:753-761); fwd_final_kernel sums them
+// in a fixed order into the five scalars of ops.py:802 and the valid-label
+// count of ops.py:705.  All reductions are order-deterministic.
 #include "lce_gemm3.h"
 #include "lce_internal.h"
 
@@ -383,7 +383,6 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
   int first = (int)blockIdx.x;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && a.row0 == 0) *a.done = 0;  // (for the row merge of the first chunk)
   if constexpr (TAIL != kTailOnly) {
     typedef FwdProblem<T, false, KMASK, WVH, MON> Full;
     Full prob(a);
@@ -401,29 +400,35 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
   }
 }
 
-// Sum (or, IS_MAX, largest) of a double over the 64 lanes of a wave, the same in every lane and in a fixed order.
-template <bool IS_MAX> LCE_DEV double wave_reduce(double v) {
+// The seven quantities that the row merge sums over tokens (the fifth is a maximum) are laid out [..][8] in doubles and summed
+// with one quantity to a lane: lane l of a wave takes quantity l % 8 of every eighth row from l / 8 on, so that a thread
+// holds one double and not seven.
+constexpr int kMaxAt = 4, kSums = 7;
+LCE_DEV double join_sums(int q, double v, double o) { return q == kMaxAt ? fmax(v, o) : v + o; }
+LCE_DEV double no_sum(int q) { return q == kMaxAt ? -INFINITY : 0.0; }
+// Over the eight lanes of a wave that hold the same quantity, in a fixed order; the same in all of them.
+LCE_DEV double wave_join(int q, double v) {
 #pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    const double o = __shfl_xor(v, d);
-    v = IS_MAX ? fmax(v, o) : v + o;
-  }
+  for (int d = 8; d < 64; d <<= 1) v = join_sums(q, v, __shfl_xor(v, d));
   return v;
 }
 
 // Row merge: one workgroup = 64 tokens (lanes) x kMergeGroups strided groups of slices (waves).  Bound by latency: a few
-// workgroups (64 for a chunk of 4096 rows), each a chain of batches of 8 loads in flight, so a token's slices go to 16 waves
-// rather than to 4, and the sums over the workgroup's tokens are butterflies over a wave's lanes (394 slices: 12 us a launch with 4 waves
-// and serial sums).
-//   The workgroup that is done last (a count behind the block sums, cleared by the tile kernel before) adds up the block
-// sums of all of them in the order of their numbers and writes the five scalars: no launch of its own for that (4 to 5 us
-// at the end of every step).
+// workgroups (64 for a chunk of 4096 rows), each a chain of batches of 8 loads in flight, so a token's slices go to 16 waves.
+// Against 4 waves, us a launch: 394 slices 9 / 13 (64 workgroups) and 6.7 / 10.4 (4), 512 slices 10 / 17 (64), 1002 slices
+// with monitoring 46 / 80 (128), 32 slices 5.0 / 4.0 (4), 8 slices 5.1 / 4.7 (256): what 16 cost at few slices is less than a
+// second variant would be worth.
+//   No more than half of the registers that 16 waves leave a thread are used (52 of 128): loops over the groups' results in
+// LDS are unrolled by four, and the seven sums go one to a lane.  (Unrolled whole, with seven doubles in every lane, the
+// kernel spilled 16 of them to memory.)
+//   The block sums are added up by a launch of its own (below).  Folded into the last workgroup to be done -- a fence, a count
+// in memory, a second fence -- they cost 4.5 us on 4 workgroups, 6.5 on 64 and 10 on 256, against 2.3 to 5 for the launch.
 constexpr int kMergeGroups = 16;
 __global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdArgs a) {
   constexpr int G = kMergeGroups;
   __shared__ float sh_m[G][kMergeRows], sh_s[G][kMergeRows], sh_lse[kMergeRows];
   __shared__ float sh_pz[G][kMergeRows], sh_sq[G][kMergeRows], sh_mx[G][kMergeRows];
-  __shared__ int sh_last;
+  __shared__ double sh_q[kMergeRows][kSums + 2];  // (rows of 9: those of 8 lanes that write together are in different banks)
   const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
   const int64_t tokl = (int64_t)blockIdx.x * kMergeRows + r;  // row inside the chunk of this launch
   const int64_t tok = a.row0 + tokl;  // < Np; rows that do not exist only keep the block sums aligned
@@ -461,9 +466,9 @@ __global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdAr
   __syncthreads();
   if (g == 0) {
     float Mt = sh_m[0][r], St = 0.f;
-#pragma unroll
+#pragma unroll 4
     for (int i = 1; i < G; ++i) Mt = fmaxf(Mt, sh_m[i][r]);
-#pragma unroll
+#pragma unroll 4
     for (int i = 0; i < G; ++i)
       if (sh_s[i][r] != 0.f) St += sh_s[i][r] * fast_exp2((sh_m[i][r] - Mt) * kLog2e);
     const float lse = Mt + fast_log(St);
@@ -502,15 +507,13 @@ __global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdAr
     sh_mx[g][r] = mx;
     __syncthreads();
   }
-  double* blk = reinterpret_cast<double*>(a.blk);
-  const int nblk = (int)(a.Np / kMergeRows);  // over all chunks
   if (g == 0) {
     const bool valid = exists && a.y[tok] != a.ignore_index;
     const double l = (double)sh_lse[r];
     double ent = 0.0, nrm = 0.0, mx = -INFINITY;
     if (a.monitoring && exists) {
       float pz = 0.f, sq = 0.f, m = -INFINITY;
-#pragma unroll
+#pragma unroll 4
       for (int i = 0; i < G; ++i) {
         pz += sh_pz[i][r];
         sq += sh_sq[i][r];
@@ -522,67 +525,62 @@ __global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdAr
     }
     // tgt[tok] is written by the one tile that holds the target column; it is only read for a valid
     // label (for a valid label outside [0, V) nothing wrote it -- and the loss is NaN anyway)
-    double v[7] = {valid ? l - (double)a.tgt[tok] : 0.0,
-                   valid ? l * l : 0.0,
-                   ent,
-                   nrm,
-                   mx,
-                   valid ? 1.0 : 0.0,
-                   // a label that is neither ignore_index nor a column of W: poisons the loss (below)
-                   (valid && (a.y[tok] < 0 || a.y[tok] >= a.V)) ? 1.0 : 0.0};
-    double mine = 0.0;
+    sh_q[r][0] = valid ? l - (double)a.tgt[tok] : 0.0;
+    sh_q[r][1] = valid ? l * l : 0.0;
+    sh_q[r][2] = ent;
+    sh_q[r][3] = nrm;
+    sh_q[r][kMaxAt] = mx;
+    sh_q[r][5] = valid ? 1.0 : 0.0;
+    // a label that is neither ignore_index nor a column of W: poisons the loss (below)
+    sh_q[r][6] = (valid && (a.y[tok] < 0 || a.y[tok] >= a.V)) ? 1.0 : 0.0;
+    sh_q[r][kSums] = 0.0;
+    __threadfence_block();  // (written and read by this wave alone)
+    __builtin_amdgcn_wave_barrier();
+    const int q = r & 7;
+    double v = no_sum(q);
 #pragma unroll
-    for (int q = 0; q < 7; ++q) {
-      const double t = q == 4 ? wave_reduce<true>(v[q]) : wave_reduce<false>(v[q]);
-      if (r == q) mine = t;
-    }
-    if (r < 7) blk[(a.row0 / kMergeRows + (int64_t)blockIdx.x) * 8 + r] = mine;
-    __threadfence();  // this block's sums are there for every compute unit before it is counted
-    if (r == 0) {
-      const unsigned before = __hip_atomic_fetch_add(a.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sh_last = before == (unsigned)(nblk - 1) ? 1 : 0;
-      // (a call restricted to this phase finds the count as the tile kernel left it)
-      if (before == (unsigned)(nblk - 1)) __hip_atomic_store(a.done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    for (int i = 0; i < kMergeRows / 8; ++i) v = join_sums(q, v, sh_q[i * 8 + (r >> 3)][q]);
+    v = wave_join(q, v);
+    if (r < kSums) reinterpret_cast<double*>(a.blk)[(a.row0 / kMergeRows + (int64_t)blockIdx.x) * 8 + r] = v;
   }
-  __syncthreads();
-  if (!sh_last) return;
-  __threadfence();  // and the sums of all the others are read from where they put them
+}
 
-  // final sums, in a fixed order whichever workgroup forms them
-  __shared__ double sh_fin[G][7];
-  double v[7] = {0, 0, 0, 0, -INFINITY, 0, 0};
-  for (int b = threadIdx.x; b < nblk; b += 64 * G) {
-#pragma unroll
-    for (int q = 0; q < 7; ++q) {
-      const double t = blk[(int64_t)b * 8 + q];
-      v[q] = (q == 4) ? fmax(v[q], t) : v[q] + t;
-    }
+// The block sums of all chunks into the five scalars, in a fixed order.  Bound by latency: one workgroup, a quantity to a lane
+// as above, eight workgroups' sums in one 512-byte load of a wave.
+__global__ __launch_bounds__(64 * kMergeGroups) void fwd_final_kernel(const FwdArgs a) {
+  constexpr int G = kMergeGroups;
+  const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const double* blk = reinterpret_cast<const double*>(a.blk);
+  const int64_t nblk = a.Np / kMergeRows;
+  __shared__ double sh_fin[G][8];
+  const int q = r & 7;
+  double v = no_sum(q);
+  if (q < kSums) {
+#pragma unroll 4
+    for (int64_t b = threadIdx.x >> 3; b < nblk; b += 8 * G) v = join_sums(q, v, blk[b * 8 + q]);
   }
-#pragma unroll
-  for (int q = 0; q < 7; ++q) {
-    const double t = q == 4 ? wave_reduce<true>(v[q]) : wave_reduce<false>(v[q]);
-    if (r == 0) sh_fin[g][q] = t;
-  }
+  v = wave_join(q, v);
+  if (r < 8) sh_fin[g][r] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (g != 0) return;
+  v = no_sum(q);
 #pragma unroll
-    for (int q = 0; q < 7; ++q) {
-      double t = sh_fin[0][q];
-      for (int i = 1; i < G; ++i) t = (q == 4) ? fmax(t, sh_fin[i][q]) : t + sh_fin[i][q];
-      v[q] = t;
-    }
-    const double R = v[5];  // 0 valid labels -> 0/0 = NaN, as F.cross_entropy gives
-    const double ce = v[0] / R, zr = v[1] / R;
-    // Labels outside [0, V) that are not ignore_index have no column to match; the reference lets
-    // them contribute lse alone, silently.  Here they turn the loss into NaN (F.cross_entropy
-    // raises a device-side assert for them) -- visible to the caller, no synchronisation needed.
-    const bool bad_labels = v[6] != 0.0;
+  for (int i = 0; i < G / 8; ++i) v = join_sums(q, v, sh_fin[i * 8 + (r >> 3)][q]);
+  v = wave_join(q, v);
+  // lane 0 .. 6: the total of each quantity
+  const double ce_sum = __shfl(v, 0), zr_sum = __shfl(v, 1), ent_sum = __shfl(v, 2), nrm_sum = __shfl(v, 3);
+  const double z_max = __shfl(v, kMaxAt), R = __shfl(v, 5);  // 0 valid labels -> 0/0 = NaN, as F.cross_entropy gives
+  // Labels outside [0, V) that are not ignore_index have no column to match; the reference lets
+  // them contribute lse alone, silently.  Here they turn the loss into NaN (F.cross_entropy
+  // raises a device-side assert for them) -- visible to the caller, no synchronisation needed.
+  const bool bad_labels = __shfl(v, 6) != 0.0;
+  if (r == 0) {
+    const double ce = ce_sum / R, zr = zr_sum / R;
     a.out5[0] = bad_labels ? __builtin_nanf("") : (float)(ce + (double)a.z_reg * zr);
     a.out5[1] = (float)zr;
-    a.out5[2] = a.monitoring ? (float)v[4] : 0.f;
-    a.out5[3] = a.monitoring ? (float)(v[2] / R) : 0.f;
-    a.out5[4] = a.monitoring ? (float)(v[3] / (double)a.N) : 0.f;
+    a.out5[2] = a.monitoring ? (float)z_max : 0.f;
+    a.out5[3] = a.monitoring ? (float)(ent_sum / R) : 0.f;
+    a.out5[4] = a.monitoring ? (float)(nrm_sum / (double)a.N) : 0.f;
     a.n_valid[0] = (int64_t)R;
   }
 }
@@ -629,6 +627,11 @@ hipError_t launch_fwd_tiles(const FwdArgs& a, hipStream_t s) {
 hipError_t launch_fwd_rows(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;
   hipLaunchKernelGGL(fwd_rows_kernel, dim3((unsigned)((left < a.nc ? left : a.nc) / kMergeRows)), dim3(64 * kMergeGroups), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_fwd_final(const FwdArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(fwd_final_kernel, dim3(1), dim3(64 * kMergeGroups), 0, s, a);
   return hipGetLastError();
 }
 

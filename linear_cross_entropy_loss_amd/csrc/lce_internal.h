@@ -87,7 +87,6 @@ struct FwdArgs {
   float* part_sq;    // [Vp/128][nc]  per-slice sum z^2        (monitoring)
   float* tgt;        // [Np]          target logit (written for tokens whose label is a column of W)
   float* blk;        // [Np/64][8]    per-merge-block partial sums (doubles, seven of a block's eight)
-  unsigned* done;    // merge blocks that are done, over all chunks (in the eighth place of the first block); the tile kernel clears it
   float* lse_rows;   // [Np] or null  lse of every row in the order the tile kernels see them (packed rows), whatever its label
 };
 
@@ -166,7 +165,6 @@ struct BwdArgs {
   float* part_sq;
   float* tgt;
   int64_t nc;
-  unsigned* done;  // null, or the row merge's count of finished blocks, which the logit kernel clears (FwdArgs; first chunk)
   // rows of dx always go to the tokens perm[] names (the rows of a chunk can be all there and still not be the
   // tokens of the same numbers)
   int perm_always;
@@ -200,8 +198,9 @@ __device__ __forceinline__ float final_factor_of(const BwdArgs& a) {
 }
 
 hipError_t launch_fwd_tiles(const FwdArgs& a, hipStream_t s);
-// Row merge of the current chunk (lse, per-block sums) and, in the launch of the last chunk, the final reduction.
+// Row merge of the current chunk (lse, per-block sums), and -- once, after the last chunk -- the final reduction.
 hipError_t launch_fwd_rows(const FwdArgs& a, hipStream_t s);
+hipError_t launch_fwd_final(const FwdArgs& a, hipStream_t s);
 hipError_t launch_bwd_dz(const BwdArgs& a, hipStream_t s);
 // The logit kernel of lce_forward_backward and the pass that follows the row merge (see BwdArgs).
 hipError_t launch_fwd_stage(const BwdArgs& a, hipStream_t s);

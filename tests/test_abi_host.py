@@ -586,3 +586,44 @@ def test_plans_of_the_benchmark_configurations(lib):
     (chunks, rows), ws = plan(65536, 8192, 262144, 8192, fh, f32)
     assert chunks == 10 and ws <= 8192 * 262144 * 4
     assert plan(2048, 2048, 16384, 4096, f32, f32)[0] == (0, 0)
+
+
+def _kernel_notes(path, tmp_path):
+    """(name, bytes of private memory per lane, spilled vector registers) of every gfx950 kernel in a library built here."""
+    import struct
+    import subprocess
+    from pathlib import Path
+
+    data = Path(path).read_bytes()
+    magic, found, at = b"__CLANG_OFFLOAD_BUNDLE__", [], 0
+    while (at := data.find(magic, at)) >= 0:
+        pos = at + len(magic)
+        (count,) = struct.unpack_from("<Q", data, pos)
+        pos += 8
+        for _ in range(count if count < 16 else 0):
+            off, size, idlen = struct.unpack_from("<QQQ", data, pos)
+            target = data[pos + 24:pos + 24 + idlen]
+            pos += 24 + idlen
+            if b"gfx950" not in target or size == 0:
+                continue
+            obj = tmp_path / f"{len(found)}_{at}.co"
+            obj.write_bytes(data[at + off:at + off + size])
+            text = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", str(obj)], capture_output=True, text=True,
+                                  check=True).stdout
+            names = re.findall(r"^ {4}\.name: +(\S+)$", text, flags=re.M)
+            private = re.findall(r"^ {4}\.private_segment_fixed_size: +(\d+)$", text, flags=re.M)
+            spilled = re.findall(r"^ {4}\.vgpr_spill_count: +(\d+)$", text, flags=re.M)
+            assert len(names) == len(private) == len(spilled)
+            found += zip(names, map(int, private), map(int, spilled))
+        at += len(magic)
+    return found
+
+
+def test_no_kernel_keeps_registers_in_memory(lib, tmp_path):
+    """Every kernel's registers fit: none has private memory for spilled ones, which would put memory round trips into
+    loops whose loads are counted."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    kernels = _kernel_notes(_lib.LIB_PATH, tmp_path)
+    assert any("fwd_rows_kernel" in name for name, _, _ in kernels) and len(kernels) > 100
+    assert [k for k in kernels if k[1] or k[2]] == []

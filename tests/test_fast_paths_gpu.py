@@ -140,3 +140,31 @@ def test_padded_copy_of_rows(dtype, rows, cols, offset, extra):
     if out.data_ptr() != t.data_ptr():
         whole = torch.as_strided(out, (rows, out.stride(0)), (out.stride(0), 1))
         assert not whole[:, cols:].any()
+
+
+# row merge and final sums: one token, a workgroup's 64 and their neighbours, more blocks than one trip of the final sums takes;
+# one slice of 128 columns, less and more than the 16 groups, and than the 128 slices of one trip
+@pytest.mark.parametrize("N,V", [(1, 1), (63, 129), (64, 2048), (65, 2049), (257, 16384), (300, 16385), (130, 40000), (9000, 1000), (70000, 300)])
+@pytest.mark.parametrize("route", [False, "always"])
+def test_row_merge_and_final_sums(N, V, route):
+    from linear_cross_entropy_loss_amd import linear_cross_entropy, ops
+
+    H = 64
+    x, y, w = make_inputs(N, H, V, torch.bfloat16, 11, ignore_frac=0.1 if N > 1 else 0.0, device="cuda")
+    token = ops.one_pass.set(route)
+    try:
+        got = linear_cross_entropy(x.clone().requires_grad_(), y, w, -1, 1e-3, 1.0, 65536, True)
+    finally:
+        ops.one_pass.reset(token)
+    z = x.double() @ w.double()
+    lse = torch.logsumexp(z, 1)
+    kept = y != -1
+    zr = (lse[kept] ** 2).mean()
+    loss = (lse[kept] - z[kept].gather(1, y[kept, None])[:, 0]).mean() + 1e-3 * zr
+    ent = lse - (torch.exp(z - lse[:, None]) * z).sum(1)
+    want = (loss, zr, z.max(), ent[kept].mean(), z.norm(dim=1).mean())
+    # (logits are fp32 sums of 64 exact products, each sum over columns one of fp32 terms: 2^-24 times the number of additions
+    # in a chain, some tens, of the size of lse; the totals over tokens are formed in fp64)
+    scale = max(1.0, lse.abs().max().item())
+    for a, b in zip(got, want):
+        assert abs(a.item() - b.item()) <= 1e-5 * max(scale, abs(b.item()))
