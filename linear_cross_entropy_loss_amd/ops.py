@@ -406,8 +406,8 @@ class LinearXentImplementation(torch.autograd.Function):
     def backward(ctx, grad_output, void0=None, void1=None, void2=None, void3=None):
         x, y1, w, lse, n_valid = ctx.saved_tensors
         ignore_index, z_regularization, logit_scale, N_chunk_size, pack, layout = ctx.lce_cfg
-        if grad_output is None:
-            return (None,) * 9
+        if grad_output is None:  # (not materialised, see forward; a consumer of the loss passed no gradient on: zeros)
+            grad_output = torch.zeros((), dtype=torch.float32, device=x.device)
         grads, ctx.lce_grads = ctx.lce_grads, None
         if grads is not None:
             # computed in the forward for an upstream gradient of 1 (ops.py:810 does the same multiplication); a

@@ -168,3 +168,30 @@ def test_row_merge_and_final_sums(N, V, route):
     scale = max(1.0, lse.abs().max().item())
     for a, b in zip(got, want):
         assert abs(a.item() - b.item()) <= 1e-5 * max(scale, abs(b.item()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("route", [False, "always"])
+def test_consumer_that_passes_no_gradient_gives_zeros(route, dtype):
+    """A loss whose consumer returns None for its gradient has gradients of zero, not none."""
+    from linear_cross_entropy_loss_amd import linear_cross_entropy, ops
+
+    class Drop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    x, y, w = make_inputs(70, 72, 300, dtype, 3, device="cuda")
+    x.requires_grad_()
+    w.requires_grad_()
+    token = ops.one_pass.set(route)
+    try:
+        loss = linear_cross_entropy(x, y, w)[0]
+        gx, gw = torch.autograd.grad(Drop.apply(loss), (x, w))
+    finally:
+        ops.one_pass.reset(token)
+    assert gx.shape == x.shape and gw.shape == w.shape and not gx.any() and not gw.any()
