@@ -246,15 +246,12 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(const char* dxc, int6
   }
 }
 
-// The upstream gradient that fp16 gradients are formed for before the real one is known (lce.h).  Bound by the latency of
-// its loads: one workgroup, whose 1024 threads have 8 labels each in flight, reads 64 KiB at a time and needs no second
-// launch to add up partial counts.  It stands for a chain of eight
-// elementwise and reduction launches (fp16 forward + backward, N=1024, H=1024, V=32000: 333 -> 307 us; N=4096: 862 -> 835 us).
-__global__ __launch_bounds__(1024) void stand_in_kernel(const int64_t* y, int64_t N, int64_t ignore_index, float* out) {
-  __shared__ unsigned sh[16];
+// The upstream gradient that fp16 gradients are formed for before the real one is known (lce.h): the labels are counted by
+// workgroups whose 1024 threads have 8 labels each in flight, 64 KiB at a time.
+LCE_DEV unsigned count_valid(const int64_t* y, int64_t N, int64_t ignore_index, unsigned* sh) {  // (thread 0 has the sum)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned mine = 0;
-  for (int64_t base = threadIdx.x; base < N; base += 8 * 1024) {
+  for (int64_t base = (int64_t)blockIdx.x * 8 * 1024 + threadIdx.x; base < N; base += (int64_t)gridDim.x * 8 * 1024) {
     int64_t lab[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) lab[u] = base + u * 1024 < N ? y[base + u * 1024] : ignore_index;
@@ -265,13 +262,36 @@ __global__ __launch_bounds__(1024) void stand_in_kernel(const int64_t* y, int64_
   for (int d = 32; d > 0; d >>= 1) mine += (unsigned)__shfl_xor((int)mine, d);
   if (lane == 0) sh[wave] = mine;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned n = 0;
+  unsigned n = 0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) n += sh[w];
-    out[0] = __builtin_bit_cast(float, (unsigned)(127 + 31 - __builtin_clz(n > 0 ? n : 1)) << 23);
-  }
+  for (int w = 0; w < 16; ++w) n += sh[w];
+  return n;
 }
+
+LCE_DEV float power_of_two_below(unsigned n) {
+  return __builtin_bit_cast(float, (unsigned)(127 + 31 - __builtin_clz(n > 0 ? n : 1)) << 23);
+}
+
+// Up to kStandInOne labels: one launch, bound by the latency of one workgroup's loads.  (It stands for a chain of eight
+// elementwise and reduction launches: fp16 forward + backward, N=1024, H=1024, V=32000 333 -> 307 us; N=4096 862 -> 835 us.)
+__global__ __launch_bounds__(1024) void stand_in_kernel(const int64_t* y, int64_t N, int64_t ignore_index, float* out) {
+  __shared__ unsigned sh[16];
+  const unsigned n = count_valid(y, N, ignore_index, sh);
+  if (threadIdx.x == 0) out[0] = power_of_two_below(n);
+}
+
+// More labels than that: one compute unit reads them at 30 to 60 GB/s, so the counts of up to 256 workgroups are added up in
+// *out itself, as a whole number, which the launch before cleared and the one after turns into the power of two.  (With the
+// call's host time, us, one workgroup / three launches / the eight of torch: 2^16 labels 12 / - / 45, 2^17 19 / - / 48, 2^18
+// 35 / 18 / 48, 2^20 291 / 18 / 47, 2^24 4633 / 28 / 94.)
+constexpr int64_t kStandInOne = (int64_t)1 << 17;
+__global__ void stand_in_clear_kernel(float* out) { reinterpret_cast<unsigned*>(out)[0] = 0; }
+__global__ __launch_bounds__(1024) void stand_in_count_kernel(const int64_t* y, int64_t N, int64_t ignore_index, float* out) {
+  __shared__ unsigned sh[16];
+  const unsigned n = count_valid(y, N, ignore_index, sh);
+  if (threadIdx.x == 0) atomicAdd(reinterpret_cast<unsigned*>(out), n);
+}
+__global__ void stand_in_finish_kernel(float* out) { out[0] = power_of_two_below(reinterpret_cast<const unsigned*>(out)[0]); }
 
 unsigned row_grid(int64_t N, int num_cus) {
   int64_t g = (int64_t)num_cus * 8;
@@ -300,7 +320,14 @@ hipError_t launch_compact_labels(const int64_t* y, int64_t N, int64_t ignore_ind
 }
 
 hipError_t launch_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(stand_in_kernel, dim3(1), dim3(1024), 0, s, y, N, ignore_index, out);
+  if (N <= kStandInOne) {
+    hipLaunchKernelGGL(stand_in_kernel, dim3(1), dim3(1024), 0, s, y, N, ignore_index, out);
+    return hipGetLastError();
+  }
+  const int64_t trips = (N + 8191) / 8192;
+  hipLaunchKernelGGL(stand_in_clear_kernel, dim3(1), dim3(1), 0, s, out);
+  hipLaunchKernelGGL(stand_in_count_kernel, dim3((unsigned)(trips < 256 ? trips : 256)), dim3(1024), 0, s, y, N, ignore_index, out);
+  hipLaunchKernelGGL(stand_in_finish_kernel, dim3(1), dim3(1), 0, s, out);
   return hipGetLastError();
 }
 

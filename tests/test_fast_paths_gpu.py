@@ -112,8 +112,9 @@ def test_packing_counts_and_order(N, ignored):
     assert torch.allclose(da.float(), db.float(), rtol=2.0 ** -7, atol=1e-7)
 
 
-# around a wave, a workgroup and the 8192 labels of one trip; powers of two and their neighbours
-@pytest.mark.parametrize("N", [1, 64, 1023, 1024, 1025, 8191, 8192, 8193, 65536, 100003])
+# around a wave, a workgroup and the 8192 labels of one trip; powers of two and their neighbours; the last size of one workgroup
+# and the first of several, and of more than one trip of theirs
+@pytest.mark.parametrize("N", [1, 64, 1023, 1024, 1025, 8191, 8192, 8193, 65536, 100003, 131072, 131073, 2097153])
 def test_stand_in_gradient_is_the_power_of_two_below_the_count(N):
     from linear_cross_entropy_loss_amd import ops
 
@@ -124,6 +125,24 @@ def test_stand_in_gradient_is_the_power_of_two_below_the_count(N):
         y = y.flip(0).contiguous()
         want = 2.0 ** (max(kept, 1).bit_length() - 1)
         assert ops._stand_in_gradient(x, y, -1).tolist() == [want]
+
+
+def test_stand_in_gradient_of_many_labels_takes_the_whole_chip():
+    """2^24 labels are 128 MiB: 4.6 ms through one compute unit, 0.1 ms through all of them and their launches."""
+    from linear_cross_entropy_loss_amd import ops
+
+    x = torch.empty((1, 8), dtype=torch.float16, device="cuda")
+    y = torch.zeros(1 << 24, dtype=torch.int64, device="cuda")
+    times = []
+    for _ in range(5):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        pre = ops._stand_in_gradient(x, y, -1)
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end))
+    assert pre.item() == 2.0 ** 24
+    assert min(times) < 1.0  # ms: ten times the one, a quarter of the other
 
 
 # row lengths around a 16-byte piece, the threads of a row and their four pieces each; sources at odd addresses
