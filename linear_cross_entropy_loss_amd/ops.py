@@ -97,12 +97,22 @@ def _warn_copy_once(what, t, why):
     )
 
 
-def _padded_cols(cols):
+def _padded_cols(cols, dtype):
     """Row stride of a matrix this module lays out itself: `cols` where that keeps rows on 16-byte boundaries (then the
     matrix is dense), else whole cache lines of 128 bytes -- the kernels fetch 128 bytes of a row at a time, which on
-    rows that start anywhere are two lines (N=8192, H=768, V=50257 in bf16: dx 373 us a chunk with a stride of 50264
-    elements)."""
-    return cols if cols % 8 == 0 else -(-cols // 64) * 64
+    rows that start anywhere are two lines -- unless that would more than double a short row, which then ends with its
+    last 16 bytes.
+
+    Rows of whole lines against rows of 16-byte multiples, bf16 forward + backward, us: N=32768, H=257, V=2003 909 / 920;
+    N=16384, H=500, V=4100 793 / 810; N=8192, H=2049, V=16385 2037 / 2062; H=63, 65, 100, 129 (V=512 ... 1001) equal; N=65536,
+    H=7, V=512 317 / 325, the one that the limit to twice the length gives up: its copy of x and its dx have 16 bytes a row
+    and not 128."""
+    m = _row_multiple(dtype)
+    if cols % m == 0:
+        return cols
+    line = 8 * m  # 128 bytes
+    m = line if 2 * cols >= line else m
+    return -(-cols // m) * m
 
 
 def _aligned_rows(t, what=None):
@@ -119,7 +129,7 @@ def _aligned_rows(t, what=None):
         _warn_copy_once(what, t, f"rows must be contiguous and start on 16-byte boundaries: row strides that are "
                                  f"multiples of {m} elements")
     rows, cols = t.shape
-    padded = torch.empty((rows, _padded_cols(cols)), dtype=t.dtype, device=t.device)
+    padded = torch.empty((rows, _padded_cols(cols, t.dtype)), dtype=t.dtype, device=t.device)
     if t.stride(1) == 1 and rows > 0 and cols > 0 and padded.is_cuda and t.data_ptr() % t.element_size() == 0:
         with torch.cuda.device(t.device):
             rc = _lib.load().lce_pad_rows(_ptr(t), _lib.dtype_code(t.dtype), rows, cols, t.stride(0), _ptr(padded),
@@ -159,7 +169,7 @@ def _weight_rows(At, layout):
 
 def _empty_rows(rows, cols, dtype, device):
     """Uninitialised (rows, cols) matrix whose row stride satisfies the kernels' alignment rule."""
-    return torch.empty((rows, _padded_cols(cols)), dtype=dtype, device=device)[:, :cols]
+    return torch.empty((rows, _padded_cols(cols, dtype)), dtype=dtype, device=device)[:, :cols]
 
 
 def _autocast_x(x, At):
@@ -216,9 +226,9 @@ def _alloc_grads(x, w, layout, N, H, V, need_dx, need_dw):
 
 def _finish_grads(dx, dw, layout):
     if dx is not None and not dx.is_contiguous():
-        dx = dx.contiguous()  # H not a multiple of 8
+        dx = dx.contiguous()  # rows padded: H not a multiple of 8 (fp32: of 4)
     if dw is not None and not dw.is_contiguous():
-        dw = dw.contiguous()  # V not a multiple of 8
+        dw = dw.contiguous()  # the same of V
     if dw is not None and layout == _lib.W_VH:
         dw = dw.t()
     return dx, dw
@@ -255,8 +265,8 @@ def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_c
         vh = layout == _lib.W_VH
         w_cols = H if vh else V
         prob = _lib.make_problem(
-            N, H, V, x.stride(0), w.stride(0), _padded_cols(H), _padded_cols(w_cols), x.dtype, w.dtype, x.dtype, w.dtype,
-            ignore_index, logit_scale, z_regularization, N_chunk_size, monitoring, 0, pack, 0, layout,
+            N, H, V, x.stride(0), w.stride(0), _padded_cols(H, x.dtype), _padded_cols(w_cols, w.dtype), x.dtype, w.dtype,
+            x.dtype, w.dtype, ignore_index, logit_scale, z_regularization, N_chunk_size, monitoring, 0, pack, 0, layout,
             (_lib.ROUTE_ONE_PASS if always else _lib.ROUTE_AUTO) | (_lib.ROUTE_EXACT_SUMS if exact_dw_sums.get() else 0),
         )
         lib = _lib.load()
@@ -299,9 +309,9 @@ def _forward_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_ch
     _check_inputs(x_in, y, At)
     with torch.cuda.device(x_in.device):
         x, y1, w, layout, N, H, V = _problem_views(x_in, y, At) if views is None else views
-        lddw = (H if layout == _lib.W_VH else _padded_cols(V))  # (not used by the forward)
+        lddw = (H if layout == _lib.W_VH else _padded_cols(V, w.dtype))  # (not used by the forward)
         prob = _lib.make_problem(
-            N, H, V, x.stride(0), w.stride(0), _padded_cols(H), lddw, x.dtype, w.dtype, x.dtype, w.dtype,
+            N, H, V, x.stride(0), w.stride(0), _padded_cols(H, x.dtype), lddw, x.dtype, w.dtype, x.dtype, w.dtype,
             ignore_index, logit_scale, z_regularization, N_chunk_size, monitoring, 0, pack, 0, layout,
         )
         lib = _lib.load()
@@ -334,8 +344,8 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
         dw = (_empty_rows(V, H, w.dtype, dev) if vh else _empty_rows(H, V, w.dtype, dev)) if need_dw else None
         if need_dx or need_dw:
             prob = _lib.make_problem(
-                N, H, V, x.stride(0), w.stride(0), dx.stride(0) if need_dx else _padded_cols(H),
-                dw.stride(0) if need_dw else _padded_cols(w_cols), x.dtype, w.dtype, x.dtype, w.dtype,
+                N, H, V, x.stride(0), w.stride(0), dx.stride(0) if need_dx else _padded_cols(H, x.dtype),
+                dw.stride(0) if need_dw else _padded_cols(w_cols, w.dtype), x.dtype, w.dtype, x.dtype, w.dtype,
                 ignore_index, logit_scale, z_regularization, N_chunk_size, False, 0, pack, 0, layout,
             )
             lib = _lib.load()
@@ -348,9 +358,9 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
             _lib.raise_for_status(rc, "lce_backward")
             del ws
     if dx is not None and not dx.is_contiguous():
-        dx = dx.contiguous()  # H not a multiple of 8
+        dx = dx.contiguous()  # rows padded: H not a multiple of 8 (fp32: of 4)
     if dw is not None and not dw.is_contiguous():
-        dw = dw.contiguous()  # V not a multiple of 8
+        dw = dw.contiguous()  # the same of V
     if dw is not None and vh:
         dw = dw.t()
     return dx, dw

@@ -627,3 +627,21 @@ def test_no_kernel_keeps_registers_in_memory(lib, tmp_path):
     kernels = _kernel_notes(_lib.LIB_PATH, tmp_path)
     assert any("fwd_rows_kernel" in name for name, _, _ in kernels) and len(kernels) > 100
     assert [k for k in kernels if k[1] or k[2]] == []
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_row_stride_of_own_matrices(dtype):
+    """Rows on 16-byte boundaries; dense where they are that by themselves (every fourth length in fp32, every eighth
+    in 16 bits); otherwise no more than twice as long, and whole cache lines where that allows it."""
+    from linear_cross_entropy_loss_amd import ops
+
+    es = torch.empty((), dtype=dtype).element_size()
+    for cols in [*range(1, 300), 1000, 1004, 1023, 4097, 50257, 128255]:
+        row, used = ops._padded_cols(cols, dtype) * es, cols * es
+        assert row >= used and row % 16 == 0
+        if used % 16 == 0:
+            assert row == used
+        elif row - used >= 16:
+            assert row <= 2 * used and row % 128 == 0
+        else:
+            assert row % 128 == 0 or 2 * used < 128

@@ -214,3 +214,29 @@ def test_consumer_that_passes_no_gradient_gives_zeros(route, dtype):
     finally:
         ops.one_pass.reset(token)
     assert gx.shape == x.shape and gw.shape == w.shape and not gx.any() and not gw.any()
+
+
+# fp32 rows of an odd number of 16-byte pieces, whose gradients are dense: one column piece, the edge of a tile and beyond, with
+# chunks whose sums are added in the gradient itself (master weight) and without
+@pytest.mark.parametrize("N,H,V,n_chunk", [(70, 4, 12, 4096), (300, 260, 1004, 4096), (1500, 252, 2052, 512), (600, 516, 508, 256)])
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("route", [False, "always"])
+def test_dense_fp32_gradients(N, H, V, n_chunk, x_dtype, route):
+    from linear_cross_entropy_loss_amd import linear_cross_entropy, ops
+    from oracle import lce_forward_backward_fp64
+
+    x, y, w = make_inputs(N, H, V, x_dtype, 5, ignore_frac=0.05, w_dtype=torch.float32, device="cuda")
+    x.requires_grad_()
+    w.requires_grad_()
+    token = ops.one_pass.set(route)
+    try:
+        loss = linear_cross_entropy(x, y, w, -1, 0.0, 1.0, n_chunk)[0]
+        gx, gw = torch.autograd.grad(loss, (x, w))
+    finally:
+        ops.one_pass.reset(token)
+    assert gw.stride() == (V, 1) and (x_dtype != torch.float32 or gx.stride() == (H, 1))
+    w_used = w.detach() if x_dtype == torch.float32 else w.detach().to(x_dtype)  # (rounded once under 16-bit activations)
+    ref = lce_forward_backward_fp64(x.detach(), y, w_used, -1, 0.0, 1.0, chunk=n_chunk)
+    # (fp32: products of bf16 pairs, 2^-16 relative to each operand, so some 2^-15 of the 2-norm; bf16: as above)
+    for got, want in ((gx, ref.dx), (gw, ref.dw)):
+        assert rel_errors(got, want)[1] < (3e-5 if x_dtype == torch.float32 else 5e-3)
