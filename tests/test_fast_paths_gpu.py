@@ -10,42 +10,51 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("mode", ["no_grad", "inference", "detached"])
 def test_loss_without_gradients_allocates_no_gradients(mode, dtype):
-    """A parameter under no_grad needs no gradient: the call computes the loss alone (the same bits) and takes less
-    memory than a weight gradient would."""
-    from linear_cross_entropy_loss_amd import LinearCrossEntropyLoss
+    """A parameter under no_grad needs no gradient: the call computes the loss alone and takes less memory than a weight
+    gradient would, also where a call that needs gradients computes them along with the loss."""
+    from linear_cross_entropy_loss_amd import LinearCrossEntropyLoss, _lib, ops
 
     N, H, V = 300, 256, 8192
     x, y, w = make_inputs(N, H, V, dtype, 3, ignore_frac=0.1, device="cuda")
     mod = LinearCrossEntropyLoss(H, V, device="cuda", dtype=dtype, ignore_index=-1, init_method=lambda t: t.data.copy_(w))
     mod.monitoring = True
-    want = mod(x.clone().requires_grad_(), y).detach()
-    want_max = mod.latest_metrics["logit_max"]
-    torch.cuda.synchronize()
-    torch.cuda.reset_peak_memory_stats()
-    before = torch.cuda.memory_allocated()
-    if mode == "detached":
-        mod.weight.requires_grad_(False)
-        loss = mod(x, y)
-    else:
-        with torch.no_grad() if mode == "no_grad" else torch.inference_mode():
+    if dtype == torch.bfloat16:  # (fp32 activations have no such route)
+        prob = _lib.make_problem(N, H, V, H, V, H, V, dtype, dtype, dtype, dtype, -1, 1.0, 0.0, mod.N_chunk_size, True, 0,
+                                 _lib.PACK_AUTO, 0, _lib.W_HV, _lib.ROUTE_ONE_PASS)
+        assert _lib.forward_backward_plan(prob)[0] > 0
+    token = ops.one_pass.set("always")
+    try:
+        want = mod(x.clone().requires_grad_(), y).detach()
+        want_max = mod.latest_metrics["logit_max"]
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        if mode == "detached":
+            mod.weight.requires_grad_(False)
             loss = mod(x, y)
-    torch.cuda.synchronize()
+        else:
+            with torch.no_grad() if mode == "no_grad" else torch.inference_mode():
+                loss = mod(x, y)
+        torch.cuda.synchronize()
+    finally:
+        ops.one_pass.reset(token)
     assert not loss.requires_grad
-    # (fp32 takes one product of bf16 pairs at a time either way; bf16 sums of the loss may be cut at other places)
+    # (the same fp32 logits; sums over columns cut at other places)
     assert torch.allclose(loss, want, rtol=1e-6, atol=0)
     assert torch.allclose(mod.latest_metrics["logit_max"], want_max, rtol=1e-6, atol=0)
     if dtype == torch.bfloat16:
         assert torch.cuda.max_memory_allocated() - before < H * V * 2
 
 
-@pytest.mark.parametrize("transform", ["forward_ad", "vmap"])
-def test_loss_without_gradients_refuses_transforms(transform):
+@pytest.mark.parametrize("transform, error, message", [("forward_ad", NotImplementedError, "jvp"),
+                                                       ("vmap", RuntimeError, "setup_context staticmethod")])
+def test_loss_without_gradients_refuses_transforms(transform, error, message):
     """Also where no input needs a gradient: a tangent is not dropped and a batch dimension not misread, the call is refused as
     the autograd Function refuses it."""
     from linear_cross_entropy_loss_amd import linear_cross_entropy
 
     x, y, w = make_inputs(64, 64, 256, torch.bfloat16, 3, device="cuda")
-    with torch.no_grad(), pytest.raises(Exception):
+    with torch.no_grad(), pytest.raises(error, match=message):
         if transform == "vmap":
             torch.func.vmap(lambda xx: linear_cross_entropy(xx, y, w)[0])(x[None])
         else:
@@ -97,11 +106,15 @@ def test_packing_counts_and_order(N, ignored):
             x.grad = None
             xx = x.detach().requires_grad_()
             loss = linear_cross_entropy(xx, y, w, -1, 0.0, 1.0, 65536)[0]
-            got[mode] = (loss.detach(), torch.autograd.grad(loss, xx)[0])
+            lse = torch.ops.lce_amd.forward(x, y, w, -1, 0.0, 1.0, 65536, False, mode)[1]
+            got[mode] = (loss.detach(), torch.autograd.grad(loss, xx)[0], lse)
         finally:
             ops.pack_rows.reset(token)
             ops.one_pass.reset(route)
-    (la, da), (lb, db) = got[_lib.PACK_ALWAYS], got[_lib.PACK_NEVER]
+    (la, da, lse_a), (lb, db, lse_b) = got[_lib.PACK_ALWAYS], got[_lib.PACK_NEVER]
+    assert not lse_a[y == -1].any() and not lse_b[y == -1].any()
+    # (the same logits and the same slices of columns, in tiles at other places: the last bit of an exponential's argument)
+    assert torch.allclose(lse_a, lse_b, rtol=1e-6, atol=0)
     if ignored == 1.0:
         assert torch.isnan(la) and torch.isnan(lb) and not da.any() and not db.any()
         return

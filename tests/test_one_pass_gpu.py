@@ -456,3 +456,42 @@ def test_one_pass_is_deterministic_at_the_headline_shape(layout):
     for o in runs[1:]:
         for k in o:
             assert torch.equal(o[k], runs[0][k]), k
+
+
+# fp32 sums of dW over chunks in the caller's buffer: the last column piece of four whole or cut, the last rows, one tile and
+# more, both layouts of the weight; row strides that leave pieces past the last one
+@pytest.mark.parametrize("N,H,V,n_chunk,layout", [
+    (1500, 257, 2049, 1024, 0), (1500, 260, 2052, 1024, 0), (1500, 264, 2051, 1024, 1), (900, 264, 301, 900, 0),
+    (900, 264, 301, 900, 1), (700, 256, 2304, 600, 0), (700, 256, 2304, 600, 1),
+])
+def test_fp32_sums_of_dw_keep_to_their_columns(N, H, V, n_chunk, layout):
+    from linear_cross_entropy_loss_amd import _lib, ops
+    from oracle import lce_forward_backward_fp64
+
+    lib = _lib.load()
+    x, y, w = make_inputs(N, H, V, torch.bfloat16, 13, ignore_frac=0.1, w_dtype=torch.float32, device="cuda")
+    xr = ops._aligned_rows(x)
+    wr = ops._aligned_rows(w.t().contiguous() if layout else w)
+    rows, cols = wr.shape
+    lddw = -(-cols // 4) * 4 + 12
+    dw = torch.full((rows + 1, lddw), 3.0, device="cuda")
+    dx = torch.empty((N, -(-H // 8) * 8), dtype=torch.bfloat16, device="cuda")
+    prob = _lib.make_problem(N, H, V, xr.stride(0), wr.stride(0), dx.stride(0), lddw, torch.bfloat16, torch.float32,
+                             torch.bfloat16, torch.float32, -1, 1.0, 0.0, n_chunk, False, 0, _lib.PACK_AUTO, 0, layout,
+                             _lib.ROUTE_ONE_PASS)
+    chunks, _ = _lib.forward_backward_plan(prob)
+    assert chunks > 1  # (else there are no sums)
+    ws = torch.empty(_lib.forward_backward_workspace_bytes(prob), dtype=torch.uint8, device="cuda")
+    g = torch.ones(1, device="cuda")
+    lse, out5 = torch.empty(N, device="cuda"), torch.empty(5, device="cuda")
+    nv = torch.empty(1, dtype=torch.int64, device="cuda")
+    rc = lib.lce_forward_backward(ctypes.byref(prob), P(xr), P(wr), P(y), P(g), P(lse), P(out5), P(nv), P(dx), P(dw), P(ws),
+                                  ws.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, (rc, lib.lce_last_hip_error())
+    used = -(-cols // 4) * 4
+    assert (dw[:rows, used:] == 3.0).all() and (dw[rows:] == 3.0).all()
+    ref = lce_forward_backward_fp64(x, y, w.to(torch.bfloat16), -1, 0.0, 1.0, chunk=n_chunk)
+    got = dw[:rows, :cols].t() if layout else dw[:rows, :cols]
+    # (dz is rounded to bf16 twice before the contraction, 2^-8 of an entry at most each: some 2e-3 of the 2-norm)
+    emax, el2 = rel_errors(got, ref.dw)
+    assert emax < 2e-2 and el2 < 5e-3
