@@ -350,14 +350,14 @@ int lce_scale(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const 
  * *out (1 float, device) = the largest power of two that is not above the
  * number of labels in y[0 .. N) that are not ignore_index (1 if there is none):
  * the grad_out to give lce_forward_backward for fp16 gradients whose upstream
- * gradient arrives later.  1 <= N <= 2^30.
+ * gradient arrives later.  1 <= N <= 2^30.  From version 600 on.
  */
 int lce_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, void* stream);
 
 /*
  * dst[r][c] = src[r][c] for c < cols, 0 for cols <= c < dst_ld: a copy of a matrix whose rows do not start on 16-byte
  * boundaries that the other calls can read.  Row strides in elements; src at any element boundary, rows of dst on 16-byte
- * boundaries.
+ * boundaries.  From version 600 on.
  */
 int lce_pad_rows(const void* src, int dtype, int64_t rows, int64_t cols, int64_t ld, void* dst, int64_t dst_ld,
                  void* stream);

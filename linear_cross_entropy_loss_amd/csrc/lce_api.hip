@@ -779,7 +779,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
 
 extern "C" {
 
-int lce_version(void) { return 500; }  // 0.5.0: lce_problem.route, lce_forward_backward, lce_scale
+int lce_version(void) { return 600; }  // 0.6.0: lce_stand_in, lce_pad_rows
 
 const char* lce_strerror(int status) {
   switch (status) {
