@@ -79,6 +79,10 @@ struct PackPlan {
 bool splits(const lce_problem* p) { return p->x_dtype == LCE_F32; }
 
 // Whether the tokens with an ignored label are packed away before the tile kernels run (lce.h).
+// The line is where 5 % of ignored labels, a usual share, pay for the packing, the gathers and the scatter (how many there are is
+// not known on the host).  bf16, us with / without packing, N x H x V = 2^36 (N=4096, H=1024): none ignored 442 / 423, 5 % 437 / 424,
+// 10 % 416 / 424, 30 % 350 / 418; 2^37: 817 / 801, 805 / 801, 772 / 800, 640 / 792; 2^38: 1555 / 1539, 1532 / 1541, 1464 / 1537,
+// 1231 / 1531; loss alone at 2^38: 451 / 444, 447 / 442, 422 / 442, 339 / 440.
 bool packs_rows(const lce_problem* p) {
   if (p->pack_rows == LCE_PACK_ALWAYS) return true;
   if (p->pack_rows == LCE_PACK_NEVER) return false;
