@@ -413,7 +413,7 @@ LCE_DEV double wave_join(int q, double v) {
   return v;
 }
 
-// Row merge: one workgroup = 64 tokens (lanes) x kMergeGroups strided groups of slices (waves).  Bound by latency: a few
+// Row merge: one workgroup = 64 tokens (lanes) x 16 strided groups of slices (waves).  Bound by latency: a few
 // workgroups (64 for a chunk of 4096 rows), each a chain of batches of 8 loads in flight, so a token's slices go to 16 waves.
 // Against 4 waves, us a launch: 394 slices 9 / 13 (64 workgroups) and 6.7 / 10.4 (4), 512 slices 10 / 17 (64), 1002 slices
 // with monitoring 46 / 80 (128), 32 slices 5.0 / 4.0 (4), 8 slices 5.1 / 4.7 (256): what 16 cost at few slices is less than a
@@ -423,14 +423,44 @@ LCE_DEV double wave_join(int q, double v) {
 // kernel spilled 16 of them to memory.)
 //   The block sums are added up by a launch of its own (below).  Folded into the last workgroup to be done -- a fence, a count
 // in memory, a second fence -- they cost 4.5 us on 4 workgroups, 6.5 on 64 and 10 on 256, against 2.3 to 5 for the launch.
-constexpr int kMergeGroups = 16;
-__global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdArgs a) {
-  constexpr int G = kMergeGroups;
-  __shared__ float sh_m[G][kMergeRows], sh_s[G][kMergeRows], sh_lse[kMergeRows];
-  __shared__ float sh_pz[G][kMergeRows], sh_sq[G][kMergeRows], sh_mx[G][kMergeRows];
-  __shared__ double sh_q[kMergeRows][kSums + 2];  // (rows of 9: those of 8 lanes that write together are in different banks)
-  const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const int64_t tokl = (int64_t)blockIdx.x * kMergeRows + r;  // row inside the chunk of this launch
+//   FINAL: one workgroup has all the tokens there are and goes on to the final sums, with barriers alone in between: no second
+// launch for the smallest calls, which wait for the host (a launch is 3 of the 35 us of a loss alone).  Up to 64 tokens it has
+// their block (394 slices: 6.9 us against 6.4 + 2.3), up to 256 all four blocks of a tile, four waves each, which one compute
+// unit reads at the rate of several up to 128 slices: 32 slices 4.4 against 4.8 + 2.4, 64 4.8 / 4.5 + 2.2, 128 6.3 / 4.9 + 2.3,
+// but 256 9.8 / 5.4 + 2.2 and 394 13.2 / 6.8 + 3.7.
+constexpr int kMergeWaves = 16;
+constexpr int kOneTileBlocks = kTile / kMergeRows;
+
+// From the totals of the seven quantities in lanes 0 .. 6 of a wave to the five scalars and the count.
+LCE_DEV void store_results(const FwdArgs& a, double v) {
+  const double ce_sum = __shfl(v, 0), zr_sum = __shfl(v, 1), ent_sum = __shfl(v, 2), nrm_sum = __shfl(v, 3);
+  const double z_max = __shfl(v, kMaxAt), R = __shfl(v, 5);  // 0 valid labels -> 0/0 = NaN, as F.cross_entropy gives
+  // Labels outside [0, V) that are not ignore_index have no column to match; the reference lets
+  // them contribute lse alone, silently.  Here they turn the loss into NaN (F.cross_entropy
+  // raises a device-side assert for them) -- visible to the caller, no synchronisation needed.
+  const bool bad_labels = __shfl(v, 6) != 0.0;
+  if ((threadIdx.x & 63) == 0) {
+    const double ce = ce_sum / R, zr = zr_sum / R;
+    a.out5[0] = bad_labels ? __builtin_nanf("") : (float)(ce + (double)a.z_reg * zr);
+    a.out5[1] = (float)zr;
+    a.out5[2] = a.monitoring ? (float)z_max : 0.f;
+    a.out5[3] = a.monitoring ? (float)(ent_sum / R) : 0.f;
+    a.out5[4] = a.monitoring ? (float)(nrm_sum / (double)a.N) : 0.f;
+    a.n_valid[0] = (int64_t)R;
+  }
+}
+
+// BLOCKS: blocks of 64 tokens in a workgroup, kMergeWaves / BLOCKS waves for each.
+template <int BLOCKS, bool FINAL>
+__global__ __launch_bounds__(64 * kMergeWaves) void fwd_rows_kernel(const FwdArgs a) {
+  constexpr int G = kMergeWaves / BLOCKS;  // groups of slices
+  __shared__ float sh_m[kMergeWaves][kMergeRows], sh_s[kMergeWaves][kMergeRows], sh_lse[BLOCKS][kMergeRows];
+  __shared__ float sh_pz[kMergeWaves][kMergeRows], sh_sq[kMergeWaves][kMergeRows], sh_mx[kMergeWaves][kMergeRows];
+  __shared__ double sh_q[BLOCKS * kMergeRows][kSums + 2];  // (rows of 9: those of 8 lanes that write together are in different banks)
+  __shared__ double sh_fin[BLOCKS][8];
+  const int r = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int block = wave / G, g = wave % G, w0 = block * G;  // block of the workgroup, group of slices, the block's first wave
+  const int64_t tokl = ((int64_t)blockIdx.x * BLOCKS + block) * kMergeRows + r;  // row inside the chunk of this launch
   const int64_t tok = a.row0 + tokl;  // < Np; rows that do not exist only keep the block sums aligned
   const int64_t rows = a.n_rows ? packed_rows(a.n_rows, a.N) : a.N;
   const bool exists = tok < rows;
@@ -461,18 +491,18 @@ __global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdAr
     S = S * fast_exp2((M - Mn) * kLog2e) + sb * fast_exp2((mb - Mn) * kLog2e);
     M = Mn;
   }
-  sh_m[g][r] = M;
-  sh_s[g][r] = S;
+  sh_m[wave][r] = M;
+  sh_s[wave][r] = S;
   __syncthreads();
   if (g == 0) {
-    float Mt = sh_m[0][r], St = 0.f;
+    float Mt = sh_m[w0][r], St = 0.f;
 #pragma unroll 4
-    for (int i = 1; i < G; ++i) Mt = fmaxf(Mt, sh_m[i][r]);
+    for (int i = 1; i < G; ++i) Mt = fmaxf(Mt, sh_m[w0 + i][r]);
 #pragma unroll 4
     for (int i = 0; i < G; ++i)
-      if (sh_s[i][r] != 0.f) St += sh_s[i][r] * fast_exp2((sh_m[i][r] - Mt) * kLog2e);
+      if (sh_s[w0 + i][r] != 0.f) St += sh_s[w0 + i][r] * fast_exp2((sh_m[w0 + i][r] - Mt) * kLog2e);
     const float lse = Mt + fast_log(St);
-    sh_lse[r] = lse;
+    sh_lse[block][r] = lse;
     if (a.lse_rows != nullptr) a.lse_rows[tok] = lse;
     // lse[i] of a token with an ignored label is 0, whether its row was computed (all rows are when they are not
     // packed) or not: a caller sees one thing.  (sh_lse keeps the value: logit_entropy is taken over valid rows only,
@@ -481,7 +511,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdAr
   }
   if (a.monitoring) {
     __syncthreads();
-    const float lse = sh_lse[r];
+    const float lse = sh_lse[block][r];
     float pz = 0.f, sq = 0.f, mx = -INFINITY;
     for (int c0 = g; c0 < nslices; c0 += 8 * G) {
       float pl[8], pp[8], ps[8], pm[8];
@@ -502,53 +532,64 @@ __global__ __launch_bounds__(64 * kMergeGroups) void fwd_rows_kernel(const FwdAr
         mx = fmaxf(mx, pm[u]);
       }
     }
-    sh_pz[g][r] = pz;
-    sh_sq[g][r] = sq;
-    sh_mx[g][r] = mx;
+    sh_pz[wave][r] = pz;
+    sh_sq[wave][r] = sq;
+    sh_mx[wave][r] = mx;
     __syncthreads();
   }
   if (g == 0) {
     const bool valid = exists && a.y[tok] != a.ignore_index;
-    const double l = (double)sh_lse[r];
+    const double l = (double)sh_lse[block][r];
     double ent = 0.0, nrm = 0.0, mx = -INFINITY;
     if (a.monitoring && exists) {
       float pz = 0.f, sq = 0.f, m = -INFINITY;
 #pragma unroll 4
       for (int i = 0; i < G; ++i) {
-        pz += sh_pz[i][r];
-        sq += sh_sq[i][r];
-        m = fmaxf(m, sh_mx[i][r]);
+        pz += sh_pz[w0 + i][r];
+        sq += sh_sq[w0 + i][r];
+        m = fmaxf(m, sh_mx[w0 + i][r]);
       }
       mx = (double)m;
-      ent = valid ? (double)(sh_lse[r] - pz) : 0.0;
+      ent = valid ? (double)(sh_lse[block][r] - pz) : 0.0;
       nrm = (double)sqrtf(sq);
     }
+    double* mine = sh_q[block * kMergeRows + r];
     // tgt[tok] is written by the one tile that holds the target column; it is only read for a valid
     // label (for a valid label outside [0, V) nothing wrote it -- and the loss is NaN anyway)
-    sh_q[r][0] = valid ? l - (double)a.tgt[tok] : 0.0;
-    sh_q[r][1] = valid ? l * l : 0.0;
-    sh_q[r][2] = ent;
-    sh_q[r][3] = nrm;
-    sh_q[r][kMaxAt] = mx;
-    sh_q[r][5] = valid ? 1.0 : 0.0;
+    mine[0] = valid ? l - (double)a.tgt[tok] : 0.0;
+    mine[1] = valid ? l * l : 0.0;
+    mine[2] = ent;
+    mine[3] = nrm;
+    mine[kMaxAt] = mx;
+    mine[5] = valid ? 1.0 : 0.0;
     // a label that is neither ignore_index nor a column of W: poisons the loss (below)
-    sh_q[r][6] = (valid && (a.y[tok] < 0 || a.y[tok] >= a.V)) ? 1.0 : 0.0;
-    sh_q[r][kSums] = 0.0;
+    mine[6] = (valid && (a.y[tok] < 0 || a.y[tok] >= a.V)) ? 1.0 : 0.0;
+    mine[kSums] = 0.0;
     __threadfence_block();  // (written and read by this wave alone)
     __builtin_amdgcn_wave_barrier();
     const int q = r & 7;
     double v = no_sum(q);
 #pragma unroll
-    for (int i = 0; i < kMergeRows / 8; ++i) v = join_sums(q, v, sh_q[i * 8 + (r >> 3)][q]);
+    for (int i = 0; i < kMergeRows / 8; ++i) v = join_sums(q, v, sh_q[block * kMergeRows + i * 8 + (r >> 3)][q]);
     v = wave_join(q, v);
-    if (r < kSums) reinterpret_cast<double*>(a.blk)[(a.row0 / kMergeRows + (int64_t)blockIdx.x) * 8 + r] = v;
+    if (!FINAL) {
+      if (r < kSums) reinterpret_cast<double*>(a.blk)[(a.row0 / kMergeRows + (int64_t)blockIdx.x) * 8 + r] = v;
+    } else if (r < 8) {
+      sh_fin[block][r] = v;
+    }
+  }
+  if constexpr (FINAL) {  // the final sums, in the order of fwd_final_kernel
+    __syncthreads();
+    if (wave != 0) return;
+    const int q = r & 7, b = r >> 3;
+    store_results(a, wave_join(q, b < BLOCKS ? sh_fin[b][q] : no_sum(q)));
   }
 }
 
 // The block sums of all chunks into the five scalars, in a fixed order.  Bound by latency: one workgroup, a quantity to a lane
 // as above, eight workgroups' sums in one 512-byte load of a wave.
-__global__ __launch_bounds__(64 * kMergeGroups) void fwd_final_kernel(const FwdArgs a) {
-  constexpr int G = kMergeGroups;
+__global__ __launch_bounds__(64 * kMergeWaves) void fwd_final_kernel(const FwdArgs a) {
+  constexpr int G = kMergeWaves;
   const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
   const double* blk = reinterpret_cast<const double*>(a.blk);
   const int64_t nblk = a.Np / kMergeRows;
@@ -567,22 +608,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void fwd_final_kernel(const FwdA
 #pragma unroll
   for (int i = 0; i < G / 8; ++i) v = join_sums(q, v, sh_fin[i * 8 + (r >> 3)][q]);
   v = wave_join(q, v);
-  // lane 0 .. 6: the total of each quantity
-  const double ce_sum = __shfl(v, 0), zr_sum = __shfl(v, 1), ent_sum = __shfl(v, 2), nrm_sum = __shfl(v, 3);
-  const double z_max = __shfl(v, kMaxAt), R = __shfl(v, 5);  // 0 valid labels -> 0/0 = NaN, as F.cross_entropy gives
-  // Labels outside [0, V) that are not ignore_index have no column to match; the reference lets
-  // them contribute lse alone, silently.  Here they turn the loss into NaN (F.cross_entropy
-  // raises a device-side assert for them) -- visible to the caller, no synchronisation needed.
-  const bool bad_labels = __shfl(v, 6) != 0.0;
-  if (r == 0) {
-    const double ce = ce_sum / R, zr = zr_sum / R;
-    a.out5[0] = bad_labels ? __builtin_nanf("") : (float)(ce + (double)a.z_reg * zr);
-    a.out5[1] = (float)zr;
-    a.out5[2] = a.monitoring ? (float)z_max : 0.f;
-    a.out5[3] = a.monitoring ? (float)(ent_sum / R) : 0.f;
-    a.out5[4] = a.monitoring ? (float)(nrm_sum / (double)a.N) : 0.f;
-    a.n_valid[0] = (int64_t)R;
-  }
+  store_results(a, v);
 }
 
 template <class T, int TAIL, bool KMASK, bool WVH, bool MON>
@@ -624,14 +650,25 @@ hipError_t launch_fwd_tiles(const FwdArgs& a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
+// Blocks of the row merge that forms the final sums as well (see fwd_rows_kernel), or 0.
+static int final_merge_blocks(const FwdArgs& a) {
+  if (a.Np != kTile) return 0;
+  if (a.N <= kMergeRows && a.lse_rows == nullptr) return 1;  // (lse_rows is read for all rows of a tile)
+  return a.Vp / kChunkV <= 128 ? kOneTileBlocks : 0;
+}
+
 hipError_t launch_fwd_rows(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;
-  hipLaunchKernelGGL(fwd_rows_kernel, dim3((unsigned)((left < a.nc ? left : a.nc) / kMergeRows)), dim3(64 * kMergeGroups), 0, s, a);
+  const int whole = final_merge_blocks(a);
+  auto kern = whole == 0 ? fwd_rows_kernel<1, false> : whole == 1 ? fwd_rows_kernel<1, true> : fwd_rows_kernel<kOneTileBlocks, true>;
+  const int64_t grid = whole != 0 ? 1 : (left < a.nc ? left : a.nc) / kMergeRows;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kMergeWaves), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_fwd_final(const FwdArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(fwd_final_kernel, dim3(1), dim3(64 * kMergeGroups), 0, s, a);
+  if (final_merge_blocks(a) != 0) return hipSuccess;
+  hipLaunchKernelGGL(fwd_final_kernel, dim3(1), dim3(64 * kMergeWaves), 0, s, a);
   return hipGetLastError();
 }
 

@@ -198,7 +198,8 @@ __device__ __forceinline__ float final_factor_of(const BwdArgs& a) {
 }
 
 hipError_t launch_fwd_tiles(const FwdArgs& a, hipStream_t s);
-// Row merge of the current chunk (lse, per-block sums), and -- once, after the last chunk -- the final reduction.
+// Row merge of the current chunk (lse, per-block sums), and -- once, after the last chunk -- the final reduction (nothing to
+// do there where the row merge was one workgroup's).
 hipError_t launch_fwd_rows(const FwdArgs& a, hipStream_t s);
 hipError_t launch_fwd_final(const FwdArgs& a, hipStream_t s);
 hipError_t launch_bwd_dz(const BwdArgs& a, hipStream_t s);

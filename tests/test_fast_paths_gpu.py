@@ -175,8 +175,10 @@ def test_padded_copy_of_rows(dtype, rows, cols, offset, extra):
 
 
 # row merge and final sums: one token, a workgroup's 64 and their neighbours, more blocks than one trip of the final sums takes;
-# one slice of 128 columns, less and more than the 16 groups, and than the 128 slices of one trip
-@pytest.mark.parametrize("N,V", [(1, 1), (63, 129), (64, 2048), (65, 2049), (257, 16384), (300, 16385), (130, 40000), (9000, 1000), (70000, 300)])
+# one slice of 128 columns, less and more than the 16 groups, and than the 128 slices of one trip; the last token counts that one
+# workgroup merges by itself, the slices up to which it does, and the first beyond
+@pytest.mark.parametrize("N,V", [(1, 1), (63, 129), (64, 2048), (64, 40000), (65, 2049), (256, 16384), (256, 16385), (257, 16384),
+                                 (300, 16385), (130, 40000), (9000, 1000), (70000, 300)])
 @pytest.mark.parametrize("route", [False, "always"])
 def test_row_merge_and_final_sums(N, V, route):
     from linear_cross_entropy_loss_amd import linear_cross_entropy, ops
