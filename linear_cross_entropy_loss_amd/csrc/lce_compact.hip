@@ -111,7 +111,7 @@ __global__ __launch_bounds__(1024) void chunk_rows_kernel(const int64_t* n_rows,
 
 // All of it in one launch, for N <= 1024 * ITER: one workgroup of 16 waves, each on ITER * 64 consecutive tokens that it
 // holds in registers, counted and numbered by ballots.  Bound by latency, as the four kernels are that do it for any N (counts,
-// their scan, packing, the chunks' rows: one launch of about 5 us each, whatever N).
+// their scan, packing, the chunks' rows: 14 us of launches at N = 16384): 5 us up to N = 8192, 7.5 at 16384, 14.5 at 32768.
 template <int ITER>
 __global__ __launch_bounds__(1024) void compact_labels_kernel(const int64_t* y, int N, int64_t ignore_index, int64_t* n_rows,
                                                               int* perm, int64_t* yc, int64_t nc, int chunks,
