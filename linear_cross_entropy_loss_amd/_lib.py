@@ -156,11 +156,20 @@ def make_problem(N, H, V, ldx, ldw, lddx, lddw, x_dtype, w_dtype, dx_dtype, dw_d
 
 
 def workspace_bytes(prob: LceProblem) -> tuple[int, int]:
-    lib = load()
-    f, b = ctypes.c_size_t(0), ctypes.c_size_t(0)
-    raise_for_status(lib.lce_workspace_bytes(ctypes.byref(prob), ctypes.byref(f), ctypes.byref(b)),
-                     "lce_workspace_bytes")
-    return int(f.value), int(b.value)
+    return forward_workspace_bytes(prob), backward_workspace_bytes(prob)
+
+
+def forward_workspace_bytes(prob: LceProblem, what: str = "lce_workspace_bytes") -> int:
+    """Workspace of lce_forward alone: the backward is not planned for it.  `what` is named where the problem is refused."""
+    b = ctypes.c_size_t(0)
+    raise_for_status(load().lce_workspace_bytes(ctypes.byref(prob), ctypes.byref(b), None), what)
+    return b.value
+
+
+def backward_workspace_bytes(prob: LceProblem) -> int:
+    b = ctypes.c_size_t(0)
+    raise_for_status(load().lce_workspace_bytes(ctypes.byref(prob), None, ctypes.byref(b)), "lce_workspace_bytes")
+    return b.value
 
 
 def backward_plan(prob: LceProblem) -> tuple[int, int]:

@@ -21,6 +21,7 @@ logit tiles (``lce_backward``).  So does a second ``backward`` over the same gra
 """
 from __future__ import annotations
 
+import contextlib
 import contextvars
 import ctypes
 import math
@@ -72,8 +73,13 @@ def _route_mode() -> int:
     return 2 if v == "always" else (1 if v else 0)
 
 
+def _on_device(device):
+    """A context in which `device`, a tensor's, is the current one."""
+    return contextlib.nullcontext() if device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def _row_multiple(dtype):
@@ -131,9 +137,9 @@ def _aligned_rows(t, what=None):
     rows, cols = t.shape
     padded = torch.empty((rows, _padded_cols(cols, t.dtype)), dtype=t.dtype, device=t.device)
     if t.stride(1) == 1 and rows > 0 and cols > 0 and padded.is_cuda and t.data_ptr() % t.element_size() == 0:
-        with torch.cuda.device(t.device):
+        with _on_device(t.device):
             rc = _lib.load().lce_pad_rows(_ptr(t), _lib.dtype_code(t.dtype), rows, cols, t.stride(0), _ptr(padded),
-                                          padded.stride(0), ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream))
+                                          padded.stride(0), torch.cuda.current_stream(t.device).cuda_stream)
         _lib.raise_for_status(rc, "lce_pad_rows")
     else:  # (columns apart from each other)
         padded[:, :cols] = t
@@ -201,8 +207,7 @@ def _check_dtypes(x, At):
 
 
 def _problem_views(x_in, y, At):
-    """The (x, y, w) views the kernels read, w's layout, and the shapes (N, H, V)."""
-    _check_inputs(x_in, y, At)
+    """The (x, y, w) views the kernels read, w's layout, and the shapes (N, H, V).  (Of inputs that _check_inputs took.)"""
     _check_dtypes(x_in, At)
     x = _aligned_rows(x_in.reshape(-1, x_in.shape[-1]))
     y1 = y.reshape(-1).contiguous()
@@ -242,8 +247,8 @@ def _stand_in_gradient(x, y1, ignore_index):
     if x.dtype == torch.float16:
         pre = torch.empty(1, dtype=torch.float32, device=x.device)
         stream = torch.cuda.current_stream(x.device).cuda_stream
-        with torch.cuda.device(x.device):
-            rc = _lib.load().lce_stand_in(_ptr(y1), y1.numel(), int(ignore_index), _ptr(pre), ctypes.c_void_p(stream))
+        with _on_device(x.device):
+            rc = _lib.load().lce_stand_in(_ptr(y1), y1.numel(), int(ignore_index), _ptr(pre), stream)
         _lib.raise_for_status(rc, "lce_stand_in")
         return pre
     return torch.ones(1, dtype=torch.float32, device=x.device)
@@ -251,17 +256,18 @@ def _stand_in_gradient(x, y1, ignore_index):
 
 def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, need_dx,
                    need_dw, always=None):
-    """Runs lce_forward_backward when its one-pass route covers the problem.  Returns (done, views): `views` as of
-    _problem_views, for the other route to go on with; `done` None if the problem is not covered, else
-    (out5, lse, n_valid, x, y1, w, layout, dx, dw, pre): the gradients for an upstream gradient of `pre` (a device
-    scalar; None stands for 1).  `always`: take the route wherever it fits (default: what `one_pass` says)."""
+    """Runs lce_forward_backward when its one-pass route covers the problem.  Returns (done, given).  `done`: None if the problem
+    is not covered, else (out5, lse, n_valid, x, y1, w, layout, dx, dw, pre): the gradients for an upstream gradient of
+    `pre` (a device scalar; None stands for 1).  `given`, for the other route to go on with: the views as of
+    _problem_views and the checked problem (None if it was not made).  `always`: take the route wherever it fits (default: what `one_pass` says)."""
     if always is None:
         always = one_pass.get() == "always"
-    with torch.cuda.device(x_in.device):
+    _check_inputs(x_in, y, At)
+    with _on_device(x_in.device):
         views = _problem_views(x_in, y, At)
         x, y1, w, layout, N, H, V = views
         if x.dtype == torch.float32 or w.dtype not in (x.dtype, torch.float32):
-            return None, views
+            return None, (views, None)
         vh = layout == _lib.W_VH
         w_cols = H if vh else V
         prob = _lib.make_problem(
@@ -272,7 +278,7 @@ def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_c
         lib = _lib.load()
         _lib.raise_for_status(lib.lce_check_problem(ctypes.byref(prob)), "linear_cross_entropy")
         if _lib.forward_backward_plan(prob)[0] == 0:
-            return None, views
+            return None, (views, prob)
         dev = x.device
         dx, dw = _alloc_grads(x, w, layout, N, H, V, need_dx, need_dw)
         nbytes = _lib.forward_backward_workspace_bytes(prob)
@@ -283,10 +289,10 @@ def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_c
         pre = _stand_in_gradient(x, y1, ignore_index)  # (the upstream gradient is not known yet)
         stream = torch.cuda.current_stream(dev).cuda_stream
         rc = lib.lce_forward_backward(ctypes.byref(prob), _ptr(x), _ptr(w), _ptr(y1), _ptr(pre), _ptr(lse), _ptr(out5),
-                                      _ptr(n_valid), _ptr(dx), _ptr(dw), _ptr(ws), nbytes, ctypes.c_void_p(stream))
+                                      _ptr(n_valid), _ptr(dx), _ptr(dw), _ptr(ws), nbytes, stream)
         _lib.raise_for_status(rc, "lce_forward_backward")
         del ws
-    return (out5, lse, n_valid, x, y1, w, layout, dx, dw, (pre if x.dtype == torch.float16 else None)), views
+    return (out5, lse, n_valid, x, y1, w, layout, dx, dw, (pre if x.dtype == torch.float16 else None)), None
 
 
 def _scale_grad(t, grad_output):
@@ -294,29 +300,32 @@ def _scale_grad(t, grad_output):
     if t is None:
         return
     lib = _lib.load()
-    with torch.cuda.device(t.device):
+    with _on_device(t.device):
         g = grad_output.detach().to(device=t.device, dtype=torch.float32).reshape(1).contiguous()
         stream = torch.cuda.current_stream(t.device).cuda_stream
         rc = lib.lce_scale(_ptr(t), _lib.dtype_code(t.dtype), t.shape[0], t.shape[1], t.stride(0), _ptr(g),
-                           ctypes.c_void_p(stream))
+                           stream)
         _lib.raise_for_status(rc, "lce_scale")
 
 
-def _forward_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, views=None):
-    """Runs lce_forward.  Returns (out5, lse, n_valid), the (x, y, w) views the kernels read and w's layout.  `views`:
-    what _problem_views returned for these tensors, if the caller has them: a matrix that cannot be read in place is then
-    not copied again (N=1999, H=500, V=10007 in bf16: four launches, 20 us on the device and 45 us on the host)."""
-    _check_inputs(x_in, y, At)
-    with torch.cuda.device(x_in.device):
-        x, y1, w, layout, N, H, V = _problem_views(x_in, y, At) if views is None else views
-        lddw = (H if layout == _lib.W_VH else _padded_cols(V, w.dtype))  # (not used by the forward)
-        prob = _lib.make_problem(
-            N, H, V, x.stride(0), w.stride(0), _padded_cols(H, x.dtype), lddw, x.dtype, w.dtype, x.dtype, w.dtype,
-            ignore_index, logit_scale, z_regularization, N_chunk_size, monitoring, 0, pack, 0, layout,
-        )
+def _forward_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, given=None):
+    """Runs lce_forward.  Returns (out5, lse, n_valid), the (x, y, w) views the kernels read and w's layout.  `given`:
+    what _one_pass_impl returned for these arguments, if the caller has it: a matrix that cannot be read in place is then
+    not copied again (N=1999, H=500, V=10007 in bf16: four launches, 20 us on the device and 45 us on the host), nor the
+    problem made again."""
+    if given is None:
+        _check_inputs(x_in, y, At)
+    with _on_device(x_in.device):
+        views, prob = given if given is not None else (_problem_views(x_in, y, At), None)
+        x, y1, w, layout, N, H, V = views
         lib = _lib.load()
-        _lib.raise_for_status(lib.lce_check_problem(ctypes.byref(prob)), "linear_cross_entropy")
-        fwd_bytes, _ = _lib.workspace_bytes(prob)
+        if prob is None:
+            lddw = (H if layout == _lib.W_VH else _padded_cols(V, w.dtype))  # (not used by the forward)
+            prob = _lib.make_problem(
+                N, H, V, x.stride(0), w.stride(0), _padded_cols(H, x.dtype), lddw, x.dtype, w.dtype, x.dtype, w.dtype,
+                ignore_index, logit_scale, z_regularization, N_chunk_size, monitoring, 0, pack, 0, layout,
+            )
+        fwd_bytes = _lib.forward_workspace_bytes(prob, "linear_cross_entropy")  # (checks the problem)
         dev = x.device
         ws = torch.empty(fwd_bytes, dtype=torch.uint8, device=dev)
         lse = torch.empty(N, dtype=torch.float32, device=dev)
@@ -324,7 +333,7 @@ def _forward_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_ch
         n_valid = torch.empty(1, dtype=torch.int64, device=dev)
         stream = torch.cuda.current_stream(dev).cuda_stream
         rc = lib.lce_forward(ctypes.byref(prob), _ptr(x), _ptr(w), _ptr(y1), _ptr(lse), _ptr(out5),
-                             _ptr(n_valid), _ptr(ws), fwd_bytes, ctypes.c_void_p(stream))
+                             _ptr(n_valid), _ptr(ws), fwd_bytes, stream)
         _lib.raise_for_status(rc, "lce_forward")
         del ws
     return out5, lse, n_valid, x, y1, w, layout
@@ -338,7 +347,7 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
     vh = layout == _lib.W_VH
     V = w.shape[0] if vh else w.shape[1]
     w_cols = H if vh else V
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         dev = x.device
         dx = _empty_rows(N, H, x.dtype, dev) if need_dx else None
         dw = (_empty_rows(V, H, w.dtype, dev) if vh else _empty_rows(H, V, w.dtype, dev)) if need_dw else None
@@ -349,12 +358,12 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
                 ignore_index, logit_scale, z_regularization, N_chunk_size, False, 0, pack, 0, layout,
             )
             lib = _lib.load()
-            _, bwd_bytes = _lib.workspace_bytes(prob)
+            bwd_bytes = _lib.backward_workspace_bytes(prob)
             ws = torch.empty(bwd_bytes, dtype=torch.uint8, device=dev)
             g = grad_output.detach().to(device=dev, dtype=torch.float32).reshape(1).contiguous()
             stream = torch.cuda.current_stream(dev).cuda_stream
             rc = lib.lce_backward(ctypes.byref(prob), _ptr(x), _ptr(w), _ptr(y1), _ptr(lse), _ptr(n_valid),
-                                  _ptr(g), _ptr(dx), _ptr(dw), _ptr(ws), bwd_bytes, ctypes.c_void_p(stream))
+                                  _ptr(g), _ptr(dx), _ptr(dw), _ptr(ws), bwd_bytes, stream)
             _lib.raise_for_status(rc, "lce_backward")
             del ws
     if dx is not None and not dx.is_contiguous():
@@ -392,16 +401,16 @@ class LinearXentImplementation(torch.autograd.Function):
         x_in = _autocast_x(x_in, At)
         pack = _pack_mode()
         need_dx, need_dw = grad_mode and ctx.needs_input_grad[0], grad_mode and ctx.needs_input_grad[2]
-        done = views = None
+        done = given = None
         if (need_dx or need_dw) and one_pass.get():
-            done, views = _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring,
+            done, given = _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring,
                                          pack, need_dx, need_dw)
         if done is not None:
             out5, lse, n_valid, x, y1, w, layout, dx, dw, pre = done
             ctx.lce_grads = [dx, dw, pre]  # for the first backward; dropped there
         else:
             out5, lse, n_valid, x, y1, w, layout = _forward_impl(
-                x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, views)
+                x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, given)
             ctx.lce_grads = None
         ctx.save_for_backward(x, y1, w, lse, n_valid)
         ctx.lce_cfg = (ignore_index, z_regularization, logit_scale, N_chunk_size, pack, layout)
@@ -513,9 +522,7 @@ def _op_forward_grads(x: torch.Tensor, y: torch.Tensor, At: torch.Tensor, ignore
                       logit_scale: float, N_chunk_size: int, monitoring: bool, need_dx: bool, need_dw: bool,
                       pack_rows_mode: int = 0, always: bool = False
                       ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    _check_inputs(x, y, At)
-    _check_dtypes(x, At)
-    done, views = _one_pass_impl(x, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring,
+    done, given = _one_pass_impl(x, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring,
                                  pack_rows_mode, need_dx, need_dw, always)
     if done is not None:
         out5, lse, n_valid, x2, y1, _, layout, dx, dw, pre = done
@@ -524,7 +531,7 @@ def _op_forward_grads(x: torch.Tensor, y: torch.Tensor, At: torch.Tensor, ignore
             pre = torch.ones(1, dtype=torch.float32, device=x.device)
     else:  # (a problem the one-pass route does not cover: the two device calls, one after the other)
         out5, lse, n_valid, x2, y1, w, layout = _forward_impl(x, y, At, ignore_index, z_regularization, logit_scale,
-                                                              N_chunk_size, monitoring, pack_rows_mode, views)
+                                                              N_chunk_size, monitoring, pack_rows_mode, given)
         pre = _stand_in_gradient(x2, y1, ignore_index)
         dx, dw = _backward_impl(x2, y1, w, lse, n_valid, pre, ignore_index, z_regularization, logit_scale, N_chunk_size,
                                 need_dx, need_dw, pack_rows_mode, layout)
@@ -560,11 +567,11 @@ def _op_scale(t: torch.Tensor, factor: torch.Tensor) -> torch.Tensor:
     n = flat.numel()
     if n:
         lib = _lib.load()
-        with torch.cuda.device(t.device):
+        with _on_device(t.device):
             g = factor.detach().to(device=t.device, dtype=torch.float32).reshape(1).contiguous()
             stream = torch.cuda.current_stream(t.device).cuda_stream
             # (one row of n elements: any dense tensor, whatever its row length)
-            rc = lib.lce_scale(_ptr(flat), _lib.dtype_code(t.dtype), 1, n, n + (-n) % 8, _ptr(g), ctypes.c_void_p(stream))
+            rc = lib.lce_scale(_ptr(flat), _lib.dtype_code(t.dtype), 1, n, n + (-n) % 8, _ptr(g), stream)
             _lib.raise_for_status(rc, "lce_scale")
     return out
 

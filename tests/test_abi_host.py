@@ -645,3 +645,25 @@ def test_row_stride_of_own_matrices(dtype):
             assert row <= 2 * used and row % 128 == 0
         else:
             assert row % 128 == 0 or 2 * used < 128
+
+
+def test_device_is_switched_only_where_it_differs(monkeypatch):
+    from linear_cross_entropy_loss_amd import ops
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert isinstance(ops._on_device(torch.device("cuda", 0)), torch.cuda.device)
+    assert not isinstance(ops._on_device(torch.device("cuda", 1)), torch.cuda.device)
+
+
+def test_workspace_of_one_direction_is_that_of_both(lib):
+    """Each direction planned by itself: the same bytes, and the same problems refused."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    for kw in (dict(), dict(N=1), dict(N=70000, H=64, ldx=64, lddx=64, V=300, ldw=304, lddw=304), dict(monitoring=True),
+               dict(x_dtype=torch.float32, w_dtype=torch.float32, dx_dtype=torch.float32, dw_dtype=torch.float32)):
+        p = _prob(**kw)
+        f, b = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert lib.lce_workspace_bytes(ctypes.byref(p), ctypes.byref(f), ctypes.byref(b)) == 0
+        assert (_lib.forward_workspace_bytes(p), _lib.backward_workspace_bytes(p)) == (f.value, b.value)
+    with pytest.raises(ValueError, match="linear_cross_entropy: .*outside the range"):
+        _lib.forward_workspace_bytes(_prob(N=0), "linear_cross_entropy")
