@@ -256,10 +256,11 @@ def _stand_in_gradient(x, y1, ignore_index):
 
 def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, need_dx,
                    need_dw, always=None):
-    """Runs lce_forward_backward when its one-pass route covers the problem.  Returns (done, given).  `done`: None if the problem
-    is not covered, else (out5, lse, n_valid, x, y1, w, layout, dx, dw, pre): the gradients for an upstream gradient of
-    `pre` (a device scalar; None stands for 1).  `given`, for the other route to go on with: the views as of
-    _problem_views and the checked problem (None if it was not made).  `always`: take the route wherever it fits (default: what `one_pass` says)."""
+    """Runs lce_forward_backward when its one-pass route covers the problem.  Returns (done, given).  `done`: None if the
+    problem is not covered, else (out5, lse, n_valid, x, y1, w, layout, dx, dw, pre): the gradients for an upstream
+    gradient of `pre` (a device scalar; None stands for 1).  `given`, for the other route to go on with: the views as of
+    _problem_views and the checked problem (None if it was not made).  `always`: take the route wherever it fits (default:
+    what `one_pass` says)."""
     if always is None:
         always = one_pass.get() == "always"
     _check_inputs(x_in, y, At)
