@@ -345,8 +345,17 @@ struct FusedPlan {
   bool parts_on;
   bool dw_direct;  // fp32 dW: the chunks' terms are added in the caller's buffer, there is no plane
   bool lo8;        // the lower halves of a 16-bit dW's sums are cut to a byte (lce_bwd_dw.hip)
+  bool factors;    // the dx and dW kernels turn the staged e into dz (factors_in_gradients)
   double cost;     // modelled time of the plan (kernel_cost units)
 };
+
+// Whether the dx and dW kernels multiply the staged e by its factors themselves, on its way to LDS, or a pass over the stage
+// does it before them (lce_fuse.hip).  The pass costs 4 bytes of memory traffic per logit, whatever the hidden size; the
+// products cost vector work under the matrix work of both kernels, once for every tile of 256 hidden indices: 5 % of their
+// time at two of them, 13 % at eight.  bf16, ms a step, products / pass: N=8192, V=50304, H=768 2.03 / 2.17, 1024 2.48 /
+// 2.56, 1280 3.12 / 3.17, 1536 3.53 / 3.53, 2048 4.41 / 4.32; N=16384, V=131072 stored (V, H), H=768 9.46 / 10.13, 1024
+// 11.85 / 12.30, 1536 17.57 / 17.58; fp16, N=8192, V=50304, H=768 2.15 / 2.28, 1024 2.65 / 2.73, 1536 3.78 / 3.74.
+bool factors_in_gradients(const lce_problem* p) { return lce::padded_hidden(p->H) <= 1024; }
 
 bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, FusedPlan* f);
 
@@ -370,6 +379,8 @@ bool plan_fused(const lce_problem* p, bool want_dx, bool want_dw, FusedPlan* f) 
 bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, FusedPlan* f) {
   memset(f, 0, sizeof(*f));
   f->lo8 = lo8;
+  f->factors = factors_in_gradients(p);
+  const double mul = f->factors ? 1.06 : 1.0;
   const bool x16 = p->x_dtype == LCE_BF16 || p->x_dtype == LCE_F16;
   if (!x16 || (p->w_dtype != p->x_dtype && p->w_dtype != LCE_F32) || (p->route & ~LCE_ROUTE_EXACT_SUMS) == LCE_ROUTE_TWO_PASS) return false;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Vp = (size_t)lce::padded_vocab(p->V), Hp = (size_t)lce::padded_hidden(p->H);
@@ -444,8 +455,8 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
     const int64_t t_last = tiles - (chunks - 1) * t_even;
     auto chunk_cost = [&](double tt) -> double {
       return kernel_cost(tt * tv, (double)(lce::padded_k(p->H) / 64), 8.0, false) +
-             (want_dx ? kernel_cost(tt * th, (double)(Vp / 64), 5.0, true) : 0.0) +
-             (want_dw ? kernel_cost(tv * th, tt * 4.0, chunks > 1 ? (f->dw_direct ? 16.0 : lo8 ? 10.0 : 12.0) : 5.0, chunks == 1) : 0.0);
+             (want_dx ? kernel_cost(tt * th, mul * (double)(Vp / 64), 5.0, true) : 0.0) +
+             (want_dw ? kernel_cost(tv * th, mul * tt * 4.0, chunks > 1 ? (f->dw_direct ? 16.0 : lo8 ? 10.0 : 12.0) : 5.0, chunks == 1) : 0.0);
     };
     // (per chunk, besides the tile kernels: the row merge, the kernel that adds dx's K segments, launch gaps -- about 25 units)
     const double cost = (double)(chunks - 1) * chunk_cost((double)t_even) + chunk_cost((double)t_last) + 25.0 * (double)chunks;
@@ -464,7 +475,7 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
   // The two-pass route by the same model: the forward over all tokens, then the backward's plan.  It wins where the
   // scratch bound leaves only short chunks (every chunk adds a round trip of all the fp32 sums of dW).
   BwdPlan b;
-  const double scale_pass = (double)Np * (double)Vp * 4.0 / 8.0e6;
+  const double scale_pass = (double)Np * (double)Vp * (f->factors ? 16.0 / lce::kChunkV : 4.0) / 8.0e6;
   f->cost = best + scale_pass;
   if ((p->route & ~LCE_ROUTE_EXACT_SUMS) == LCE_ROUTE_AUTO && plan_bwd(p, &b) == LCE_OK) {
     const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false) + b.cost;
@@ -706,6 +717,9 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   b.nc = f.nc;
   b.dx_part = f.parts_on && dx ? (float*)(base + f.part) : nullptr;
   b.dw_part = f.parts_on && dw && f.chunks == 1 ? (float*)(base + f.part) : nullptr;
+  // the factors of the stage take the place of the partials once the rows' lse are known (lce_fuse.hip)
+  b.dx_f = f.factors ? b.part_lse : nullptr;
+  b.dw_f = f.factors ? b.part_max : nullptr;
   b.dw_plane = f.chunks > 1 && !f.dw_direct ? (void*)(base + f.plane) : nullptr;
   b.dw_plane_hi = f.chunks > 1 && !f.dw_direct && f.total != f.plane_hi ? (void*)(base + f.plane_hi) : nullptr;
 
@@ -754,7 +768,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
       if (e != hipSuccess) return hip_fail(e, "fwd_rows");
     }
     if ((dx || dw) && (ph & LCE_PHASE_BWD_DZ)) {
-      e = lce::launch_stage_scale(a, s);
+      e = f.factors ? lce::launch_stage_factors(a, s) : lce::launch_stage_scale(a, s);
       if (e != hipSuccess) return hip_fail(e, "stage_scale");
     }
     if (dx && (ph & LCE_PHASE_BWD_DX)) {

@@ -48,7 +48,8 @@ template <bool WVH> struct DwTileGeom {
 constexpr int kDwSliceBytes = kWaveTile * 128;
 static_assert(4 * kDwSliceBytes <= kMainloopLds - kStageBytes, "four wave slices must fit beside one stage");
 
-template <class T, bool F32OUT>
+// LATE: the accumulator is read as it is used, not ahead (the factors of the stage are held through the epilogue).
+template <class T, bool F32OUT, bool LATE>
 LCE_DEV void dw_store_rows_hv(const BwdArgs& a, f32x16_t (&acc)[kNB][kNB], int tp, int tq, char* scratch) {
   typedef typename elem_of<T>::type E;
   typedef typename std::conditional<F32OUT, float, E>::type O;
@@ -89,7 +90,12 @@ LCE_DEV void dw_store_rows_hv(const BwdArgs& a, f32x16_t (&acc)[kNB][kNB], int t
             // register quads gives each lane a whole run (16 bytes)
             float d[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) d[i] = blk[gq * 4 + i] * coef;
+            for (int i = 0; i < 8; ++i) {
+              float v;
+              if (LATE) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(blk[gq * 4 + i]));
+              else v = blk[gq * 4 + i];
+              d[i] = v * coef;
+            }
             const unsigned x0 = pack2<T>(d[0], d[1]), x1 = pack2<T>(d[2], d[3]);
             const unsigned y0 = pack2<T>(d[4], d[5]), y1 = pack2<T>(d[6], d[7]);
             const auto s0 = __builtin_amdgcn_permlane32_swap(x0, y0, false, false);
@@ -490,7 +496,9 @@ LCE_DEV DwPlan dw_plan(const BwdArgs& a, int64_t rows) {
 enum { kDwAll = 0, kDwStaged = 1, kDwTails = 2, kDwStaged32 = 3 };
 
 // ACC: what the plane of sums over chunks of token rows has to do with a tile (BwdArgs::dw_acc; whole tiles only).
-template <class T, bool WVH, int MODE, int ACC = 0> struct DwProblem {
+// SCALE: the stage holds e, which the factors of BwdArgs::dw_f turn into dz.
+template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
+  static constexpr bool kQScale = SCALE;
   static constexpr bool kSwapAB = !WVH;  // (H, V) output: dz, the Q operand, feeds the A side (v along registers)
   static constexpr bool kVarK = true;    // whole tiles and segment items have different K extents
   static constexpr bool kKMask = false;  // both operands have K as their slow index: nothing to mask
@@ -532,6 +540,17 @@ template <class T, bool WVH, int MODE, int ACC = 0> struct DwProblem {
     const int seg = (item - plan.full) % plan.nseg;
     return seg == plan.nseg - 1 ? plan.kt - seg * plan.kseg : plan.kseg;
   }
+  LCE_DEV const float* q_factors(int local) const {
+    if (local >= count) return a.dw_f;
+    int item, tp, tq, seg;
+    decode(local, item, tp, tq, seg);
+    return a.dw_f + (int64_t)tq * (kTile / kChunkV) * a.nc + (seg < 0 ? 0 : (int64_t)seg * plan.kseg * kBK);
+  }
+  LCE_DEV unsigned q_factor_offset() const {
+    const unsigned t = threadIdx.x;
+    return ((t >> 4) & 1) * (unsigned)(a.nc * 4) + (t >> 5) * 32;
+  }
+  LCE_DEV int64_t q_factor_step(int) const { return kBK; }
   LCE_DEV void origins(int local, const void*& p, const void*& q) const {
     int item, tp, tq, seg;
     decode(local, item, tp, tq, seg);
@@ -570,7 +589,7 @@ template <class T, bool WVH, int MODE, int ACC = 0> struct DwProblem {
       return;
     }
     if (MODE == kDwStaged || MODE == kDwStaged32) {
-      dw_store_rows_hv<T, MODE == kDwStaged32>(a, acc, tp, tq, scratch);
+      dw_store_rows_hv<T, MODE == kDwStaged32, SCALE>(a, acc, tp, tq, scratch);
     } else {
       float* part = seg >= 0 ? a.dw_part + (int64_t)(item - plan.full) * kTile * kTile : nullptr;
       dw_epilogue<T, WVH>(a, part, acc, tp, tq);
@@ -578,14 +597,15 @@ template <class T, bool WVH, int MODE, int ACC = 0> struct DwProblem {
   }
 };
 
-template <class T, bool WVH, int MODE, int ACC>
+template <class T, bool WVH, int MODE, int ACC, bool SCALE>
 __global__ __launch_bounds__(kThreads) void bwd_dw_persistent_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
-  DwProblem<T, WVH, MODE, ACC> prob(a);
+  typedef DwProblem<T, WVH, MODE, ACC, SCALE> Problem;
+  Problem prob(a);
   // (a chunk without a kept row adds nothing to the sums of the earlier chunks)
   if ((ACC == 2 || ACC == 4 || ACC == 7) && prob.rows == 0) return;
-  Pipe3<T, E, false, E, false, DwProblem<T, WVH, MODE, ACC>> pipe(prob);
+  Pipe3<T, E, false, E, false, Problem> pipe(prob);
   pipe.run(prob.ldx, a.vs / kBK, prob.plan.kt, lds, (int)blockIdx.x);
 }
 
@@ -623,13 +643,17 @@ __global__ __launch_bounds__(256) void dw_tail_kernel(const BwdArgs a) {
   }
 }
 
-template <class T, bool WVH, int MODE, int ACC = 0> hipError_t launch_tiles(const BwdArgs& a, hipStream_t s) {
-  auto kern = bwd_dw_persistent_kernel<T, WVH, MODE, ACC>;
+template <class T, bool WVH, int MODE, int ACC, bool SCALE> hipError_t launch_kernel(const BwdArgs& a, hipStream_t s) {
+  auto kern = bwd_dw_persistent_kernel<T, WVH, MODE, ACC, SCALE>;
   static LdsOptIn optin;
   hipError_t e = optin.ensure(reinterpret_cast<const void*>(kern), kMainloopLds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(a.dw_grid), dim3(kThreads), kMainloopLds, s, a);
   return hipGetLastError();
+}
+
+template <class T, bool WVH, int MODE, int ACC = 0> hipError_t launch_tiles(const BwdArgs& a, hipStream_t s) {
+  return a.dw_f != nullptr ? launch_kernel<T, WVH, MODE, ACC, true>(a, s) : launch_kernel<T, WVH, MODE, ACC, false>(a, s);
 }
 
 // Whole tiles that meet the plane of sums over chunks of token rows (nothing is split along K then).

@@ -155,8 +155,10 @@ enum { kDxFirst = 0, kDxMiddle = 1, kDxLast = 2, kDxOnly = 3, kDxTails = 4 };
 
 // WVH: the weight is stored (V, H) row-major: the P tile then has K = v as its slow index (read through the
 // LDS transpose path) and only dz, the K-contiguous operand, carries the K mask.
-template <class T, bool KMASK, bool WVH, int MODE> struct DxProblem {
+// SCALE: the stage holds e, which the factors of BwdArgs::dx_f turn into dz.
+template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem {
   static constexpr bool kKMask = KMASK;
+  static constexpr bool kQScale = SCALE;
   static constexpr bool kSwapAB = false;
   static constexpr bool kVarK = MODE == kDxTails;  // segment items have their own K extent
   static constexpr bool kQBlocked = true;          // dz is staged in blocks of 256 rows x 64 columns (BwdArgs::dz)
@@ -187,6 +189,15 @@ template <class T, bool KMASK, bool WVH, int MODE> struct DxProblem {
     tile_coords(tile, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
   }
   LCE_DEV int item_ktiles(int) const { return plan.kseg; }
+  // (a K tile is half a slice of 128 columns; work items start at even K tiles)
+  LCE_DEV const float* q_factors(int local) const {
+    if (local >= count) return a.dx_f;
+    int item, tp, tq, seg;
+    decode(local, item, tp, tq, seg);
+    return a.dx_f + k0_of(seg) / kChunkV * a.nc + (int64_t)tq * kTile;
+  }
+  LCE_DEV unsigned q_factor_offset() const { return (threadIdx.x >> 3) * 32; }
+  LCE_DEV int64_t q_factor_step(int k) const { return (k & 1) ? a.nc : 0; }
   LCE_DEV void prefetch(int) {}
   LCE_DEV int64_t k0_of(int seg) const { return seg < 0 ? 0 : (int64_t)seg * plan.kseg * kBK; }
   LCE_DEV void origins(int local, const void*& p, const void*& q) const {
@@ -223,12 +234,13 @@ template <class T, bool KMASK, bool WVH, int MODE> struct DxProblem {
   }
 };
 
-template <class T, bool KMASK, bool WVH, int MODE>
+template <class T, bool KMASK, bool WVH, int MODE, bool SCALE>
 __global__ __launch_bounds__(kThreads) void bwd_dx_persistent_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
-  DxProblem<T, KMASK, WVH, MODE> prob(a);
-  Pipe3<T, E, !WVH, E, true, DxProblem<T, KMASK, WVH, MODE>> pipe(prob);
+  typedef DxProblem<T, KMASK, WVH, MODE, SCALE> Problem;
+  Problem prob(a);
+  Pipe3<T, E, !WVH, E, true, Problem> pipe(prob);
   pipe.run(a.ldw, a.vs / kBK, MODE == kDxTails ? prob.plan.kseg : (int)(a.vs / kBK), lds, (int)blockIdx.x);
 }
 
@@ -278,8 +290,8 @@ __global__ __launch_bounds__(256) void dx_tail_kernel(const BwdArgs a) {
   }
 }
 
-template <class T, bool KMASK, bool WVH, int MODE> hipError_t launch_tiles(const BwdArgs& a, hipStream_t s) {
-  auto kern = bwd_dx_persistent_kernel<T, KMASK, WVH, MODE>;
+template <class T, bool KMASK, bool WVH, int MODE, bool SCALE = false> hipError_t launch_tiles(const BwdArgs& a, hipStream_t s) {
+  auto kern = bwd_dx_persistent_kernel<T, KMASK, WVH, MODE, SCALE>;
   static LdsOptIn optin;
   hipError_t e = optin.ensure(reinterpret_cast<const void*>(kern), kMainloopLds);
   if (e != hipSuccess) return e;
@@ -291,6 +303,12 @@ template <class T, bool KMASK, bool WVH> hipError_t launch_layout(const BwdArgs&
   // (a small problem whose tiles are all split along K has no whole tile to launch; known here when rows are not packed)
   const bool none_whole = tails && a.n_rows == nullptr &&
                           all_tiles_are_tails((a.Np / kTile) * (a.Hp / kTile), a.dx_grid, a.vs / kBK);
+  if (a.dx_f != nullptr) {
+    if (!a.first || !a.last) return hipErrorInvalidValue;
+    hipError_t e = none_whole ? hipSuccess : launch_tiles<T, KMASK, WVH, kDxOnly, true>(a, s);
+    if (e == hipSuccess && tails) e = launch_tiles<T, KMASK, WVH, kDxTails, true>(a, s);
+    return e;
+  }
   hipError_t e = none_whole ? hipSuccess
                : a.first ? (a.last ? launch_tiles<T, KMASK, WVH, kDxOnly>(a, s) : launch_tiles<T, KMASK, WVH, kDxFirst>(a, s))
                          : (a.last ? launch_tiles<T, KMASK, WVH, kDxLast>(a, s) : launch_tiles<T, KMASK, WVH, kDxMiddle>(a, s));

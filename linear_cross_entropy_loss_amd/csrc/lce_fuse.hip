@@ -10,8 +10,9 @@
 // in place, exact zeros for tokens with an ignored label and rows past the last one, and the target column
 // gets the rounding of the fp32 value 2^shift * (softmax * gain - 1), formed from the target logit the logit
 // kernel wrote, as in the kernel that recomputes the logits (lce_bwd_dz.hip).  The pass is bound by memory
-// traffic: 2 bytes read and 2 written per logit.
-#include "lce_gemm.h"
+// traffic: 2 bytes read and 2 written per logit.  For small hidden sizes, where that traffic is most of what the gradients
+// cost beyond their matrix work, it is not made: the dx and dW kernels form dz on the way to LDS (stage_factors_kernel).
+#include "lce_gemm3.h"
 #include "lce_internal.h"
 
 namespace lce {
@@ -19,10 +20,6 @@ namespace lce {
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
-
-template <class T> LCE_DEV float from_bits(unsigned short b);
-template <> LCE_DEV float from_bits<BF16>(unsigned short b) { return __builtin_bit_cast(float, (unsigned)b << 16); }
-template <> LCE_DEV float from_bits<F16>(unsigned short b) { return (float)__builtin_bit_cast(_Float16, b); }
 
 // One workgroup per block of the stage (256 token rows x 64 columns, 32 KiB, BwdArgs::dz): blockIdx.x = column
 // group, blockIdx.y = token tile.  Thread t first works out the factor of row t, then the block is
@@ -86,6 +83,83 @@ __global__ __launch_bounds__(256) void stage_scale_kernel(const BwdArgs a) {
   }
 }
 
+// The same without the pass over the stage: only the factors are worked out, and the dx and dW kernels multiply e by them on
+// its way to LDS (BwdArgs::dx_f, dw_f; the products and roundings are those of stage_scale_kernel).  The slice of 128 columns
+// that holds a token's target is rewritten here, with a factor of 1 from then on.  One workgroup per token tile and
+// kSlices slices; the two tables take the place of the partials (part_lse, part_max), which nothing reads any more.
+// Bound by launch and latency: 12 bytes per 128 logits and 512 per token.  (4096 tokens, us a launch against the pass over
+// the stage: V=32000 21 / 79, V=50257 22 / 129, V=65536 13 / 165; which problems take it: factors_in_gradients in lce_api.hip.)
+constexpr int kSlices = 8;
+template <class T>
+__global__ __launch_bounds__(256) void stage_factors_kernel(const BwdArgs a) {
+  __shared__ int sh_list[kTile];   // token rows whose target lies in one of this workgroup's slices
+  __shared__ float sh_f[kTile];
+  __shared__ unsigned short sh_tv[kTile];
+  __shared__ int sh_rel[kTile];    // target column, from the first of these slices on
+  __shared__ int sh_n;
+  typedef typename elem_of<T>::type E;
+  const int64_t rows = packed_rows(a.n_rows, a.N);
+  const int64_t t0 = (int64_t)blockIdx.y * kTile;
+  // (token tiles without a row were not written and are not read -- but for the first: dW's K extent is never empty, and zeros
+  // stand there in the place of e)
+  if (t0 >= rows && t0 > 0) return;
+  const int slices = (int)(a.vs / kChunkV), s0 = blockIdx.x * kSlices;
+  const int t = threadIdx.x;
+  const int64_t tok = t0 + t;
+  const bool exists = tok < rows;
+  const int64_t yy = exists ? a.y[tok] : a.ignore_index;
+  const bool valid = yy != a.ignore_index;
+  const float lse = valid ? a.lse[tok] : 0.f;
+  float gain = 1.f + 2.f * a.z_reg * lse;
+  if (a.dz_shift != 0) gain = fminf(fmaxf(gain, -63.f), 63.f);  // (as in lce_bwd_dz.hip)
+  if (t == 0) sh_n = 0;
+  float f[kSlices];
+#pragma unroll
+  for (int i = 0; i < kSlices; ++i) {
+    const float m = s0 + i < slices && valid ? a.part_max[(int64_t)(s0 + i) * a.nc + tok] : 0.f;
+    f[i] = valid ? __builtin_amdgcn_exp2f((m - lse) * kLog2e) * gain : 0.f;
+  }
+  __syncthreads();  // every partial has been read
+  const int64_t rel = valid ? yy - (int64_t)s0 * kChunkV : -1;
+  if (rel >= 0 && rel < kSlices * kChunkV && yy < a.vs) {
+    const float p = __builtin_amdgcn_exp2f(fmaf(a.tgt[tok] - lse, kLog2e, (float)a.dz_shift)) * gain;
+    const int at = atomicAdd(&sh_n, 1);
+    sh_list[at] = t;
+    sh_rel[at] = (int)rel;
+    sh_tv[at] = to_bits<T>(p - __builtin_bit_cast(float, (127 + a.dz_shift) << 23));
+#pragma unroll
+    for (int i = 0; i < kSlices; ++i)
+      if ((int)(rel / kChunkV) == i) {
+        sh_f[at] = f[i];
+        f[i] = 1.f;
+      }
+  }
+  // (the places of this tile's 256 tokens within a slice of either table)
+  const int64_t px = t0 + (t & 31) * 8 + (t >> 5), pw = t0 + (t & ~63) + (t & 7) * 8 + ((t & 63) >> 3);
+#pragma unroll
+  for (int i = 0; i < kSlices; ++i)
+    if (s0 + i < slices) {
+      const_cast<float*>(a.dx_f)[(int64_t)(s0 + i) * a.nc + px] = f[i];
+      const_cast<float*>(a.dw_f)[(int64_t)(s0 + i) * a.nc + pw] = f[i];
+    }
+  __syncthreads();
+  for (int e = t >> 4; e < sh_n; e += 16) {  // 16 threads rewrite the 128 columns of one token
+    const int r = sh_list[e], hit_col = sh_rel[e] & (kChunkV - 1), piece = t & 15;
+    const int s = s0 + (sh_rel[e] / kChunkV);
+    u32x4_t* at = reinterpret_cast<u32x4_t*>(reinterpret_cast<E*>(a.dz) + dz_block_offset(blockIdx.y, 2 * s + (piece >> 3), a.vs) +
+                                             r * 64 + (piece & 7) * 8);
+    const u32x4_t v = *at;
+    const int hit = hit_col - piece * 8;  // 0..7: the target is element `hit` of this piece
+    u32x4_t o = scaled_piece<T>(v, sh_f[e]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (hit == 2 * j) o[j] = (o[j] & 0xffff0000u) | sh_tv[e];
+      if (hit == 2 * j + 1) o[j] = (o[j] & 0x0000ffffu) | ((unsigned)sh_tv[e] << 16);
+    }
+    *at = o;
+  }
+}
+
 // t[r][c] *= g[0] for r < rows, c < cols (row stride ld, rows on 16-byte boundaries), the product formed in fp32;
 // nothing is read or written when g[0] is 1.  Pieces of 16 bytes, the last piece of a row element by element.
 // v * f rounded to fp32 before anything else happens to it (the compiler may otherwise fold the product into
@@ -143,6 +217,16 @@ hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(a.vs / 64), (unsigned)(a.Np / kTile));
   if (a.x_dtype == DT_BF16) hipLaunchKernelGGL(stage_scale_kernel<BF16>, grid, dim3(256), 0, s, a);
   else if (a.x_dtype == DT_F16) hipLaunchKernelGGL(stage_scale_kernel<F16>, grid, dim3(256), 0, s, a);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+hipError_t launch_stage_factors(const BwdArgs& a, hipStream_t s) {
+  if (a.split || a.v0 != 0 || a.part_max == nullptr || a.tgt == nullptr || a.lse == nullptr || a.dx_f == nullptr || a.dw_f == nullptr)
+    return hipErrorInvalidValue;
+  const dim3 grid((unsigned)((a.vs / kChunkV + kSlices - 1) / kSlices), (unsigned)(a.Np / kTile));
+  if (a.x_dtype == DT_BF16) hipLaunchKernelGGL(stage_factors_kernel<BF16>, grid, dim3(256), 0, s, a);
+  else if (a.x_dtype == DT_F16) hipLaunchKernelGGL(stage_factors_kernel<F16>, grid, dim3(256), 0, s, a);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

@@ -299,6 +299,7 @@ template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON> struct FwdProblem
   static constexpr bool kSwapAB = false;
   static constexpr bool kVarK = false;
   static constexpr bool kQBlocked = false;
+  static constexpr bool kQScale = false;
   static constexpr bool kColumnEpilogue = !VTAIL;
   const FwdArgs& a;
   int64_t rows, ldx;

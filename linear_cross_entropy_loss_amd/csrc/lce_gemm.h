@@ -69,6 +69,9 @@ template <class T> LCE_DEV unsigned short to_bits(float f) {
   typename elem_of<T>::type h = (typename elem_of<T>::type)f;
   return __builtin_bit_cast(unsigned short, h);
 }
+template <class T> LCE_DEV float from_bits(unsigned short b);
+template <> LCE_DEV float from_bits<BF16>(unsigned short b) { return __builtin_bit_cast(float, (unsigned)b << 16); }
+template <> LCE_DEV float from_bits<F16>(unsigned short b) { return (float)__builtin_bit_cast(_Float16, b); }
 // Two floats -> one dword of the 16-bit type (a single v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32).
 template <class T> LCE_DEV unsigned int pack2(float lo, float hi) {
   typedef float f32x2_t __attribute__((ext_vector_type(2)));

@@ -136,6 +136,15 @@ template <class T, class SrcT, bool KC, bool KMASK> struct Stager3 {
   }
 };
 
+// A 16-byte piece of a 16-bit operand times f: the products in fp32, rounded to nearest even.
+template <class T> LCE_DEV u32x4_t scaled_piece(u32x4_t v, float f) {
+  u32x4_t o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    o[j] = pack2<T>(from_bits<T>((unsigned short)(v[j] & 0xffffu)) * f, from_bits<T>((unsigned short)(v[j] >> 16)) * f);
+  return o;
+}
+
 // One past the last byte the loads of a row-major matrix may touch.  The range
 // check of a buffer load works on whole dwords, so for 16-bit elements the last
 // row is taken to end on a dword boundary: with an odd row length the element
@@ -159,6 +168,12 @@ template <class S> LCE_DEV const void* matrix_end(const void* base, int64_t rows
 //        of P block i and Q block j, with Q along its registers and P along its lanes)
 //   void prefetch(int tile)                       called three K tiles before the tile's epilogue: the place to issue loads
 //        of per-row data the epilogue starts with (kept in members), so that their latency is not exposed there
+//   static constexpr bool kQScale                 true if the (blocked) Q operand is multiplied on its way to LDS: by one fp32
+//        factor per row of the stage and slice of 128 columns, rounded once to the operand type.  The eight factors of a
+//        thread's chunks of a K tile lie next to each other; then
+//   const float* q_factors(int tile)              where the factors of the tile's first K tile start,
+//   unsigned q_factor_offset()                    this thread's byte offset from there,
+//   int64_t q_factor_step(int k)                  and what takes K tile k's start to that of K tile k + 1, in floats
 //   static constexpr bool kQBlocked               true if the Q operand is stored in blocks of 256 rows x 64 columns
 //        (Stager3::init_blocked); run() then takes the column groups per row of blocks in place of the Q row stride, and
 //   int  q_phase(int tile)                        (rows are the K index) says which of the four K tiles of a row of blocks
@@ -199,6 +214,13 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
   int q_phase;    // blocked Q operand with rows as its K index: K tile of the current row of blocks, 0..3
   int64_t q_jump; // and the bytes from the last K tile of a row of blocks to the first of the next
   static constexpr bool kQRowBlocks = Problem::kQBlocked && !Q_KC;
+  // Problem::kQScale: the factors of the K tile in the staging set and of the one after it ([LDS stage of the K tile]), and where
+  // those of the K tile being loaded are.
+  static constexpr bool kQScale = Problem::kQScale;
+  f32x4_t qfac[2][2];
+  const float* qfac_base;
+  unsigned qfac_off;
+  int qfac_k;
 
   static constexpr int kPReads = P_KC ? 4 : 8;  // LDS read instructions per k-step
   static constexpr int kQReads = Q_KC ? 4 : 8;
@@ -211,6 +233,11 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
   // barrier, the more time the first fragment reads of the next K tile have; with 16 of them
   // (both operands transposed) the barrier opens the step, otherwise one row precedes it.
   static constexpr int kPreRows = kReads > 12 ? 0 : 1;
+  // kQScale: vector ALU instructions behind each matrix instruction of the first three k-steps: a Q chunk takes about 20,
+  // three are stored in each of the first two k-steps.  (Factors loaded a K tile ahead, like the operands: loaded in the last
+  // k-step of the K tile before, they kept the kernel waiting for 35 % of its time.  Five instructions behind each but the
+  // first three: no difference.)
+  static constexpr int kScaleOps = 4;
 
   LCE_DEV Pipe3(Problem& p) : prob(p) {}
 
@@ -228,6 +255,10 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
       qs.end = qs.base;
     }
     k_rem = prob.k_valid(tile);
+    if constexpr (kQScale) {
+      qfac_base = prob.q_factors(tile);
+      qfac_k = 0;
+    }
     if constexpr (kQRowBlocks) q_phase = tile < prob.num_tiles() ? prob.q_phase(tile) : 0;
     ps.retarget(k_rem);
     qs.retarget(k_rem);
@@ -241,15 +272,50 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
       qs.base += qs.k_stride;
     }
     k_rem -= kBK;
+    if constexpr (kQScale) {
+      // (K tiles past the extent, which are zeros, keep the last factors: the table ends where the extent does)
+      qfac_base += k_rem > 0 ? prob.q_factor_step(qfac_k) : 0;
+      ++qfac_k;
+    }
     ps.retarget(k_rem);
     qs.retarget(k_rem);
   }
-  // chunks 0..7 of a staged K tile belong to P, 8..15 to Q
-  LCE_DEV void store_chunks(const PRegs& sp, const QRegs& sq, char* stage, int c0, int c1) {
+  // chunks 0..7 of a staged K tile belong to P, 8..15 to Q; with factors they alternate, so that the multiplications
+  // are spread over the k-steps
+  template <int STAGE> LCE_DEV void load_factors() {
+    if constexpr (kQScale) {
+      const __amdgpu_buffer_rsrc_t rsrc =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(qfac_base), 0, 0x7fffffff, 0x00020000);
+      qfac[STAGE][0] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)qfac_off, 0, 0));
+      qfac[STAGE][1] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)qfac_off, 16, 0));
+    }
+  }
+  template <int STAGE> LCE_DEV void store_chunks(const PRegs& sp, const QRegs& sq, char* stage, int c0, int c1) {
+    if constexpr (kQScale) {
+#pragma unroll
+      for (int c = c0; c < c1; ++c) {
+        if (c & 1) {
+          QRegs t;
+          t.v[c >> 1] = scaled_piece<T>(sq.v[c >> 1], qfac[STAGE][c >> 3][(c >> 1) & 3]);
+          qs.store(t, stage + kTileBytes, c >> 1, (c >> 1) + 1);
+        } else {
+          ps.store(sp, stage, c >> 1, (c >> 1) + 1);
+        }
+      }
+      return;
+    }
     if (c0 < 8) ps.store(sp, stage, c0, c1 < 8 ? c1 : 8);
     if (c1 > 8) qs.store(sq, stage + kTileBytes, c0 > 8 ? c0 - 8 : 0, c1 - 8);
   }
   LCE_DEV void load_chunks(PRegs& sp, QRegs& sq, int c0, int c1) {
+    if constexpr (kQScale) {
+#pragma unroll
+      for (int c = c0; c < c1; ++c) {
+        if (c & 1) qs.load(sq, c >> 1, (c >> 1) + 1);
+        else ps.load(sp, c >> 1, (c >> 1) + 1);
+      }
+      return;
+    }
     if (c0 < 8) ps.load(sp, c0, c1 < 8 ? c1 : 8);
     if (c1 > 8) qs.load(sq, c0 > 8 ? c0 - 8 : 0, c1 - 8);
   }
@@ -298,39 +364,44 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
 
     // k-step 0: MFMAs on buffer 0; fragment reads for step 1; LDS stores 0..5
     read_frags(1, cur, 1);
-    store_chunks(sp, sq, nxt, 0, 6);
+    store_chunks<STAGE ^ 1>(sp, sq, nxt, 0, 6);
     mfma_rows<FIRST>(acc, 0, 0, kNB);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       __builtin_amdgcn_sched_group_barrier(LCE_SG_MFMA, 1, 0);
       if (i < 4) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_RD, kReadsPerSlot, 0);
+      if (kQScale) __builtin_amdgcn_sched_group_barrier(LCE_SG_VALU, kScaleOps, 0);
       if (i >= 4 && (i & 1) == 0) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_WR, 1, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
 
     // k-step 1: MFMAs on buffer 1; reads for step 2; stores 6..11 (in slots the reads leave free); loads 0..5
     read_frags(0, cur, 2);
-    store_chunks(sp, sq, nxt, 6, 12);
+    store_chunks<STAGE ^ 1>(sp, sq, nxt, 6, 12);
+    load_factors<STAGE>();
     load_chunks(sp, sq, 0, 6);
     mfma_rows<false>(acc, 1, 0, kNB);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       __builtin_amdgcn_sched_group_barrier(LCE_SG_MFMA, 1, 0);
       if (i < 4) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_RD, kReadsPerSlot, 0);
+      if (kQScale) __builtin_amdgcn_sched_group_barrier(LCE_SG_VALU, kScaleOps, 0);
       if (i >= 5 && (i & 1) == 1) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_WR, 1, 0);
+      if (kQScale && (i == 1 || i == 3)) __builtin_amdgcn_sched_group_barrier(LCE_SG_VMEM_RD, 1, 0);  // the factors
       if (i >= 4 && (i & 1) == 0) __builtin_amdgcn_sched_group_barrier(LCE_SG_VMEM_RD, 1, 0);  // chunks 0..5: P
     }
     __builtin_amdgcn_sched_barrier(0);
 
     // k-step 2: MFMAs on buffer 0; reads for step 3; stores 12..15; loads 6..10
     read_frags(1, cur, 3);
-    store_chunks(sp, sq, nxt, 12, 16);
+    store_chunks<STAGE ^ 1>(sp, sq, nxt, 12, 16);
     load_chunks(sp, sq, 6, 11);
     mfma_rows<false>(acc, 0, 0, kNB);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       __builtin_amdgcn_sched_group_barrier(LCE_SG_MFMA, 1, 0);
       if (i < 4) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_RD, kReadsPerSlot, 0);
+      if (kQScale) __builtin_amdgcn_sched_group_barrier(LCE_SG_VALU, kScaleOps, 0);
       if (i >= 4 && i < 12 && (i & 1) == 0) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_WR, 1, 0);
       if (i >= 5 && i < 9 && (i & 1) == 1) __builtin_amdgcn_sched_group_barrier(LCE_SG_VMEM_RD, 1, 0);  // chunks 6, 7: P
       if (i >= 9 && i < 15 && (i & 1) == 1) __builtin_amdgcn_sched_group_barrier(LCE_SG_VMEM_RD, 1, 0);  // chunks 8..10: Q
@@ -400,7 +471,7 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
         const int slot = 4 * ks + i;
         acc[i][J] = Problem::kSwapAB ? mfma32<T>(qk[n & 1], pa[ks][i], acc[i][J])
                                      : mfma32<T>(pa[ks][i], qk[n & 1], acc[i][J]);
-        if (J == 0) store_chunks(sp, sq, lds, slot, slot + 1);
+        if (J == 0) store_chunks<0>(sp, sq, lds, slot, slot + 1);
         if (J == 1) load_chunks(sp, sq, slot, slot + 1);
         if constexpr (J > 0) prob.template epilogue_slot<J - 1>(tile, acc, slot, lds + kMainloopLds);
         __builtin_amdgcn_sched_barrier(0);
@@ -447,11 +518,14 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
 
     PRegs sp;
     QRegs sq;
+    if constexpr (kQScale) qfac_off = prob.q_factor_offset();
     stream_begin(first);
     load_chunks(sp, sq, 0, 16);
+    load_factors<0>();
     stream_advance();
-    store_chunks(sp, sq, lds, 0, 16);
+    store_chunks<0>(sp, sq, lds, 0, 16);
     load_chunks(sp, sq, 0, 16);
+    load_factors<1>();
     stream_advance();
     __syncthreads();
 

@@ -165,6 +165,11 @@ struct BwdArgs {
   float* part_sq;
   float* tgt;
   int64_t nc;
+  // Not null: the stage holds e, and the dx and dW kernels turn it into dz on its way to LDS, with one factor per token
+  // and slice of 128 columns, [Vp/128][nc]: dx_f has the 256 tokens of a tile in the order (token % 32) * 8 + token / 32,
+  // dw_f the 64 of a K tile in the order (token % 8) * 8 + token / 8, so that what one thread needs lies together.
+  const float* dx_f;
+  const float* dw_f;
   // rows of dx always go to the tokens perm[] names (the rows of a chunk can be all there and still not be the
   // tokens of the same numbers)
   int perm_always;
@@ -206,6 +211,9 @@ hipError_t launch_bwd_dz(const BwdArgs& a, hipStream_t s);
 // The logit kernel of lce_forward_backward and the pass that follows the row merge (see BwdArgs).
 hipError_t launch_fwd_stage(const BwdArgs& a, hipStream_t s);
 hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s);
+// The same with the factors only worked out (dx_f and dw_f of BwdArgs, in part_lse and part_max), and the slice of each
+// token's target column rewritten.
+hipError_t launch_stage_factors(const BwdArgs& a, hipStream_t s);
 // t[r][c] *= g[0] (device scalar), in fp32; nothing is touched when g[0] == 1.  Rows on 16-byte boundaries.
 hipError_t launch_scale_rows(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* g, int num_cus,
                              hipStream_t s);

@@ -122,6 +122,21 @@ CASES = [
     (8192, 1024, 32768, torch.bfloat16, 4096, 0.05, 0.0, 1.0, 0, 0, None, 1.0),     # mid size: 3 chunks
 ]
 
+# Up to four tiles of hidden indices the dx and dW kernels multiply the staged exponentials by their factors themselves, from
+# five on a pass over the stage does: both sides of that line, token tiles and slices of 128 columns that end anywhere, a
+# single row, chunks without a row, a gain that z_reg makes large.
+FACTOR_CASES = [
+    (1, 8, 520, torch.bfloat16, 4096, 0.0, 0.0, 1.0, 0, 0, None, 1.0),
+    (257, 1024, 1100, torch.bfloat16, 4096, 0.0, 0.0, 1.0, 0, 0, None, 1.0),
+    (257, 1025, 1100, torch.bfloat16, 4096, 0.0, 0.0, 1.0, 0, 0, None, 1.0),
+    (1700, 1024, 1281, torch.float16, 1024, 0.3, 1e-2, 2.0, 2, 0, None, 1.0),
+    (1700, 1032, 1281, torch.float16, 1024, 0.3, 1e-2, 2.0, 2, 1, None, 1.0),
+    (129, 64, 129, torch.bfloat16, 4096, 0.5, 0.1, 1.0, 2, 1, None, 1.0),
+    (5000, 256, 4000, torch.bfloat16, 1024, 0.9, 0.0, 1.0, 1, 0, None, 1.0),
+    (5000, 768, 2000, torch.bfloat16, 2048, 0.2, 0.0, 1.0, 1, 0, torch.float32, 1.0),
+    (640, 200, 40000, torch.float16, 4096, 0.0, 0.0, 1.0, 0, 0, None, 1.0),         # dx cut along K, the last segment masked
+]
+
 # fp32 master weight under 16-bit activations: N, H, V, dtype of x, n_chunk, ignored, z_reg, scale, pack, layout
 MASTER_CASES = [
     (4096, 512, 4096, torch.bfloat16, 2048, 0.1, 0.0, 1.0, 1, 0),
@@ -140,7 +155,7 @@ def test_one_pass_with_an_fp32_master_weight(N, H, V, dt, n_chunk, ign, z_reg, s
 
 
 @pytest.mark.pack_auto
-@pytest.mark.parametrize("N,H,V,dt,n_chunk,ign,z_reg,scale,pack,layout,dw_dt,grad_out", CASES)
+@pytest.mark.parametrize("N,H,V,dt,n_chunk,ign,z_reg,scale,pack,layout,dw_dt,grad_out", CASES + FACTOR_CASES)
 def test_one_pass_matches_two_pass_and_the_fp64_oracle(N, H, V, dt, n_chunk, ign, z_reg, scale, pack, layout, dw_dt, grad_out):
     inputs, a, b = _both_routes(N, H, V, dt, n_chunk, ign, z_reg, scale, pack, layout, dw_dt, grad_out)
     _check(inputs, a, b, z_reg, scale, grad_out, fp64=N * V <= 4096 * 8192)
