@@ -69,10 +69,8 @@ int check(const lce_problem* p, bool backward) {
 
 // Buffers of the packing pre-pass (tokens with an ignored label dropped), relative to `base`.
 struct PackPlan {
-  size_t cnt, n_rows, perm, yc, xc, xk, end;
-  int64_t ldxc;  // row stride of the packed copy of x, elements: rows of whole 16-byte pieces
-  int64_t ldxk;  // fp32 activations, backward: row stride of the copy stacked along the tokens (lce_compact.hip)
-  size_t xes;    // element size of the packed copy: that of x, or 2 for fp32 activations (stored as bf16 pairs)
+  size_t cnt, n_rows, perm, yc, xc, end;
+  int64_t ldxc;  // row stride of the packed copy of x, elements: rows of whole 16-byte pieces (pairs: twice that, [hi | lo])
 };
 
 // fp32 activations (and with them an fp32 weight) are computed as bf16 pairs, hi + lo (lce_gemm.h).
@@ -89,20 +87,16 @@ bool packs_rows(const lce_problem* p) {
   return 8.0 * (double)p->N * (double)p->H * (double)p->V >= 2199023255552.0;  // 2^41
 }
 
-PackPlan plan_pack(const lce_problem* p, size_t base, bool backward) {
+PackPlan plan_pack(const lce_problem* p, size_t base) {
   PackPlan k;
   const size_t N = (size_t)p->N, es = 2;
-  k.xes = es;
-  k.ldxc = lce::pad_to(splits(p) ? 3 * p->H : p->H, (int64_t)(16 / es));
-  k.ldxk = lce::pad_to(p->H, (int64_t)(16 / es));
+  k.ldxc = lce::pad_to(p->H, (int64_t)(16 / es)) * (splits(p) ? 2 : 1);
   size_t o = base;
   k.cnt = o; o += align_up((size_t)lce::compact_segments(p->N) * 4);
   k.n_rows = o; o += 256;
   k.perm = o; o += align_up(N * 4);
   k.yc = o; o += align_up(N * 8);
   k.xc = o; o += align_up(N * (size_t)k.ldxc * es);
-  k.xk = o;
-  if (splits(p) && backward) o += align_up(3 * (size_t)lce::padded_tokens(p->N) * (size_t)k.ldxk * es);
   k.end = o;
   return k;
 }
@@ -127,8 +121,15 @@ int64_t fwd_chunk_rows(const lce_problem* p) {
   return nc < Np ? nc : Np;
 }
 
-// 16-bit type the kernels compute in: that of the activations (bf16 for fp32 activations).
-int compute_dtype(const lce_problem* p) { return p->x_dtype == LCE_F16 ? LCE_F16 : LCE_BF16; }
+// Type the kernels compute in: that of 16-bit activations, pairs for fp32 ones.
+int compute_dtype(const lce_problem* p) {
+  return splits(p) ? lce::DT_PAIR : p->x_dtype == LCE_F16 ? lce::DT_F16 : lce::DT_BF16;
+}
+// 16-bit numbers per element of an operand in that type, and matrix products per K tile.
+int64_t parts_of(const lce_problem* p) { return splits(p) ? 2 : 1; }
+int products(const lce_problem* p) { return lce::products_of(compute_dtype(p)); }
+// Bytes of a row of the logit contraction's operands (lce::live_bands).
+int64_t logit_k_bytes(const lce_problem* p) { return lce::padded_k(parts_of(p) * p->H) * 2; }
 
 FwdPlan plan_fwd(const lce_problem* p) {
   FwdPlan f;
@@ -148,18 +149,18 @@ FwdPlan plan_fwd(const lce_problem* p) {
   // memory by all eight XCDs; over a long launch they drift apart and stop sharing what they fetch.  Launches
   // of 32768 columns bring them back in step (measured at N = 16384, H = 8192, V = 131072: 24.6 ms against 27.3
   // in one launch; no difference at H = 2048, where x stays in the cache).
-  // (fp32 activations reach the tile kernels as bf16 pairs, three times as wide)
-  if ((size_t)f.nc * (size_t)(splits(p) ? 3 * p->H : p->H) * 2 > ((size_t)128 << 20) && f.vs > 32768) f.vs = 32768;
+  // (fp32 activations reach the tile kernels as bf16 pairs, twice as wide)
+  if ((size_t)f.nc * (size_t)(parts_of(p) * p->H) * 2 > ((size_t)128 << 20) && f.vs > 32768) f.vs = 32768;
   if (p->w_dtype == LCE_F32) {
     // slab copies of at most 256 MiB (at least one tile column)
-    const int64_t hw = splits(p) ? 3 * p->H : p->H;  // rows of the copy
+    const int64_t hw = parts_of(p) * p->H;  // rows of the copy
     int64_t cols = ((int64_t)256 << 20) / (hw * 2) / 256 * 256;
     if (cols < 256) cols = 256;
     if (cols < f.vs) f.vs = cols;
     o += align_up((size_t)hw * (size_t)f.vs * 2);
   }
   if ((!p->monitoring && packs_rows(p)) || p->x_dtype == LCE_F32) {
-    f.pack = plan_pack(p, o, false);
+    f.pack = plan_pack(p, o);
     o = f.pack.end;
   }
   f.total = o;
@@ -179,14 +180,16 @@ struct BwdPlan {
 };
 
 // Bytes of the split-K partial sums of dx for slabs of `vs` columns (0 when dx is not split).
-size_t dx_part_bytes(size_t Np, size_t Hp, int64_t vs, int64_t last_vs) {
-  const int64_t b0 = lce::dx_tail_blocks((int64_t)Np, (int64_t)Hp, vs), b1 = lce::dx_tail_blocks((int64_t)Np, (int64_t)Hp, last_vs);
+size_t dx_part_bytes(size_t Np, size_t Hp, int64_t vs, int64_t last_vs, int products) {
+  const int64_t b0 = lce::dx_tail_blocks((int64_t)Np, (int64_t)Hp, vs, products);
+  const int64_t b1 = lce::dx_tail_blocks((int64_t)Np, (int64_t)Hp, last_vs, products);
   return (size_t)(b0 > b1 ? b0 : b1) * 256 * 256 * 4;
 }
 
 // The same for dW.
-size_t dw_part_bytes(size_t Np, size_t Hp, int64_t vs, int64_t last_vs) {
-  const int64_t b0 = lce::dw_tail_blocks((int64_t)Np, (int64_t)Hp, vs), b1 = lce::dw_tail_blocks((int64_t)Np, (int64_t)Hp, last_vs);
+size_t dw_part_bytes(size_t Np, size_t Hp, int64_t vs, int64_t last_vs, int products) {
+  const int64_t b0 = lce::dw_tail_blocks((int64_t)Np, (int64_t)Hp, vs, products);
+  const int64_t b1 = lce::dw_tail_blocks((int64_t)Np, (int64_t)Hp, last_vs, products);
   return (size_t)(b0 > b1 ? b0 : b1) * 256 * 256 * 4;
 }
 
@@ -233,7 +236,7 @@ int plan_bwd(const lce_problem* p, BwdPlan* b) {
   const int64_t cols = Vp / 256;
   const bool split = splits(p);
   const size_t dxes = p->dx_dtype == LCE_F32 ? 4 : 2;
-  b->pack = plan_pack(p, 0, true);
+  b->pack = plan_pack(p, 0);
   b->lddxc = lce::pad_to(p->H, 8);
   b->lse_c = b->pack.end;
   b->dxc = b->lse_c + align_up((size_t)p->N * 4);
@@ -243,14 +246,14 @@ int plan_bwd(const lce_problem* p, BwdPlan* b) {
   // memory bandwidth; 5 when it is written once) and 5 (dW) units.  The model ranks the slab
   // widths measured at N = 16384, H = 2048, V = 32768 and 65536 (2 ... 18 slabs) in their measured order.
   // bands of W tiles that bwd_dz keeps in flight (tile_coords in lce_gemm.h), and the slab width that is a whole group of them
-  const int live = lce::live_bands(lce::padded_k(split ? 3 * p->H : p->H) * 2);
+  const int live = lce::live_bands(logit_k_bytes(p));
   const int64_t gran = live < 8 ? (int64_t)256 * 8 * live : 256;
   auto slab_cost = [&](int64_t w, bool parts, bool sums) -> double {
     const double tq = (double)(Np / 256), th = (double)(Hp / 256), tv = (double)(w / 256), k3 = split ? 3.0 : 1.0;
     // (bwd_dz runs about 4 % slower on a slab that is not whole groups of the bands it keeps in flight when K is long)
     const double dz_order = live < 8 && (w / 256) % (8 * live) != 0 ? 1.04 : 1.0;
     return dz_order * kernel_cost(tq * tv, k3 * (double)((p->H + 63) / 64), 6.0, false) +
-           k3 * kernel_cost(tq * th, (double)(w / 64), sums ? 21.0 : 5.0, parts) +
+           kernel_cost(tq * th, k3 * (double)(w / 64), sums ? 21.0 : 5.0, parts) +
            kernel_cost(tv * th, k3 * (double)(Np / 64), 5.0, parts);
   };
 
@@ -269,14 +272,13 @@ int plan_bwd(const lce_problem* p, BwdPlan* b) {
     int64_t vs = (cols + s - 1) / s * 256;
     if (whole_groups) vs = (vs + gran - 1) / gran * gran;  // the next width that is whole groups of bands
     const int64_t slabs = (Vp + vs - 1) / vs;
-    // (bf16 pairs: three blocks of dz, and dx is summed over three passes per slab, so it always needs the running sum)
-    const size_t dz = align_up(Np * (size_t)vs * 2 * (split ? 3 : 1));
-    const size_t acc = slabs > 1 || split ? align_up(Np * Hp * 4) : 0;
+    const size_t dz = align_up(Np * (size_t)vs * 2 * (size_t)parts_of(p));
+    const size_t acc = slabs > 1 ? align_up(Np * Hp * 4) : 0;
     const int64_t last_vs = Vp - (slabs - 1) * vs;  // padded width of the last slab
-    const size_t dxp = lean ? 0 : dx_part_bytes(Np, Hp, vs, last_vs);  // at most 64 MiB
-    const size_t dwp = lean ? 0 : dw_part_bytes(split ? 3 * Np : Np, Hp, vs, last_vs);
+    const size_t dxp = lean ? 0 : dx_part_bytes(Np, Hp, vs, last_vs, products(p));  // at most 64 MiB
+    const size_t dwp = lean ? 0 : dw_part_bytes(Np, Hp, vs, last_vs, products(p));
     const size_t part = dxp > dwp ? dxp : dwp;  // one buffer: the dx kernels are done with it before the dW kernels start
-    const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)vs * 2 * (split ? 3 : 1)) : 0;  // 16-bit copy of the slab of W
+    const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)vs * 2 * (size_t)parts_of(p)) : 0;  // copy of the slab of W
     // the widened bound is for the staging proper; the split-K partial sums (at most 64 MiB, shared by dx
     // and dW) and the packed rows come on top of it there
     // (reserve: what the caller holds besides the workspace between forward and backward -- lse and a few scalars)
@@ -393,7 +395,7 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
   // (a 16-bit dW summed over chunks keeps the upper halves of its sums in dW itself, addressed through 32-bit
   // offsets that span the 256 rows of a tile: lce_bwd_dw.hip)
   const bool halves_ok = (size_t)p->lddw * 2 * 256 < ((size_t)1 << 31);
-  f->k = plan_pack(p, 0, false);
+  f->k = plan_pack(p, 0);
   size_t o = f->k.xc;  // the labels are always counted; the packed copy of x is made chunk by chunk (below)
   f->chunk_rows = o; o += align_up(2048 * 8);
   f->lse_rows = o; o += align_up(Np * 4);
@@ -418,9 +420,9 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
     out->part_sq = t; if (p->monitoring) t += part;
     out->stage = t; t += align_up((size_t)nc * Vp * 2);
     // split-K partial sums of dx (and, with a single chunk, of dW): one buffer
-    size_t pb = want_dx ? dx_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp) : 0;
+    size_t pb = want_dx ? dx_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp, products(p)) : 0;
     if (chunks == 1 && want_dw) {
-      const size_t w = dw_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp);
+      const size_t w = dw_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp, products(p));
       if (w > pb) pb = w;
     }
     out->part = t; t += pb;
@@ -555,7 +557,7 @@ int forward_impl(const lce_problem* p, const void* x, const void* w, const int64
   a.blk = (float*)(base + f.blk);
   rc = current_num_cus(&a.num_cus, p->max_workgroups);
   if (rc != LCE_OK) return rc;
-  a.live = lce::live_bands(lce::padded_k(splits(p) ? 3 * p->H : p->H) * 2);
+  a.live = lce::live_bands(logit_k_bytes(p));
 
   const int ph = p->phases ? p->phases : ~0;
   hipError_t e;
@@ -578,16 +580,16 @@ int forward_impl(const lce_problem* p, const void* x, const void* w, const int64
         if (e != hipSuccess) return hip_fail(e, "compact_labels");
       }
       e = x32 ? lce::launch_gather_rows_split((const float*)x, p->ldx, p->H, a.perm, a.n_rows, p->N, base + k.xc,
-                                              k.ldxc, nullptr, 0, nullptr, nullptr, a.num_cus, s)
+                                              k.ldxc, nullptr, nullptr, a.num_cus, s)
               : lce::launch_gather_rows(x, p->ldx * 2, p->H * 2, a.perm, a.n_rows, p->N, base + k.xc, k.ldxc * 2, nullptr, nullptr,
                                         a.num_cus, s);
       if (e != hipSuccess) return hip_fail(e, "gather_rows");
     }
-    if (x32) {  // the tile kernels read the copy in bf16 pairs ([hi | hi | lo], K = 3 H), whether or not rows were dropped
+    if (x32) {  // the tile kernels read the copy in bf16 pairs, whether or not rows were dropped
       a.x = a.xc;
       a.ldx = a.ldxc;
-      a.x_dtype = lce::DT_BF16;
-      a.H = 3 * p->H;
+      a.x_dtype = lce::DT_PAIR;
+      a.x_lo = a.ldxc / 2;
     }
   }
   // The tokens go through in chunks of f.nc rows (one chunk at the benchmark shapes): tile kernels, then the row
@@ -606,7 +608,7 @@ int forward_impl(const lce_problem* p, const void* x, const void* w, const int64
           e = a.w_vh ? lce::launch_convert_w_rows((const float*)w, p->ldw, p->H, v0, t.vw, base + f.w16, ld16,
                                                   compute_dtype(p), s)
                      : lce::launch_convert_w_slab((const float*)w, p->ldw, p->H, v0, t.vw, base + f.w16, ld16,
-                                                  compute_dtype(p), splits(p), s);
+                                                  compute_dtype(p), s);
           if (e != hipSuccess) return hip_fail(e, "convert_w");
           t.w = base + f.w16; t.ldw = ld16; t.w_dtype = compute_dtype(p); t.wv0 = v0; t.Vw = t.vw;
         } else {
@@ -689,7 +691,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
     if (ph & LCE_PHASE_PACK) {
       e = p->w_layout == LCE_W_VH
               ? lce::launch_convert_w_rows((const float*)w, p->ldw, p->H, 0, p->V, base + f.w16, f.ld16, compute_dtype(p), s)
-              : lce::launch_convert_w_slab((const float*)w, p->ldw, p->H, 0, p->V, base + f.w16, f.ld16, compute_dtype(p), false, s);
+              : lce::launch_convert_w_slab((const float*)w, p->ldw, p->H, 0, p->V, base + f.w16, f.ld16, compute_dtype(p), s);
       if (e != hipSuccess) return hip_fail(e, "convert_w");
     }
   }
@@ -898,12 +900,12 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
   // |lse| < 992 never reaches at z_reg <= 1/32)
   a.dz_shift = p->x_dtype == LCE_F16 && p->z_reg <= 0.03125f ? 10 : 0;
   a.dz = base + b.dz;
-  a.dx_acc = b.slabs > 1 || splits(p) ? (float*)(base + b.dx_acc) : nullptr;
+  a.dx_acc = b.slabs > 1 ? (float*)(base + b.dx_acc) : nullptr;
   a.dx_part = b.parts_on ? (float*)(base + b.dx_part) : nullptr;
   a.dw_part = b.parts_on ? (float*)(base + b.dw_part) : nullptr;
   rc = current_num_cus(&a.num_cus, p->max_workgroups);
   if (rc != LCE_OK) return rc;
-  a.live = lce::live_bands(lce::padded_k(splits(p) ? 3 * p->H : p->H) * 2);
+  a.live = lce::live_bands(logit_k_bytes(p));
   const int ph = p->phases ? p->phases : ~0;
 
   // Tokens with an ignored label have dz == 0: the kernels run on the other rows only, packed to the front.
@@ -930,7 +932,7 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
     }
     float* lse_c = pack ? (float*)(base + b.lse_c) : nullptr;
     e = x32 ? lce::launch_gather_rows_split((const float*)x, p->ldx, p->H, perm, a.n_rows, p->N, base + k.xc, k.ldxc,
-                                            base + k.xk, k.ldxk, pack ? lse : nullptr, lse_c, a.num_cus, s)
+                                            pack ? lse : nullptr, lse_c, a.num_cus, s)
             : lce::launch_gather_rows(x, p->ldx * 2, p->H * 2, perm, a.n_rows, p->N, base + k.xc, k.ldxc * 2, lse, lse_c,
                                       a.num_cus, s);
     if (e != hipSuccess) return hip_fail(e, "gather_rows");
@@ -938,10 +940,10 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
   if (x32) {  // fp32 activations reach the tile kernels as copies in bf16 pairs, whether or not rows were dropped
     a.x = a.xc;
     a.ldx = a.ldxc;
-    a.x_dtype = lce::DT_BF16;
+    a.x_dtype = lce::DT_PAIR;
+    a.x_lo = a.ldxc / 2;
   }
-  const bool split = splits(p);
-  a.dz_rows = split ? 3 * a.Np : a.Np;  // rows of the dz stage (BwdArgs::dz)
+  a.dz_rows = a.Np;  // rows of the dz stage (BwdArgs::dz)
 
   for (int64_t i = 0; i < b.slabs; ++i) {
     a.v0 = i * b.vs;
@@ -956,7 +958,7 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
         e = a.w_vh ? lce::launch_convert_w_rows((const float*)w, p->ldw, p->H, a.v0, a.vw, base + b.w16, p->H,
                                                 compute_dtype(p), s)
                    : lce::launch_convert_w_slab((const float*)w, p->ldw, p->H, a.v0, a.vw, base + b.w16, a.vs,
-                                                compute_dtype(p), split, s);
+                                                compute_dtype(p), s);
         if (e != hipSuccess) return hip_fail(e, "convert_w");
       }
       a.w = base + b.w16; a.ldw = a.w_vh ? p->H : a.vs; a.w_dtype = compute_dtype(p); a.wv0 = a.v0; a.Vw = a.vw;
@@ -965,56 +967,16 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
     }
     a.first = i == 0;
     a.last = i == b.slabs - 1;
-    if (!split) {
-      if (ph & LCE_PHASE_BWD_DZ) {
-        e = lce::launch_bwd_dz(a, s);
-        if (e != hipSuccess) return hip_fail(e, "bwd_dz");
-      }
-      if (dx && (ph & LCE_PHASE_BWD_DX)) {
-        e = lce::launch_bwd_dx(a, s);
-        if (e != hipSuccess) return hip_fail(e, "bwd_dx");
-      }
-      if (dw && (ph & LCE_PHASE_BWD_DW)) {
-        e = lce::launch_bwd_dw(a, s);
-        if (e != hipSuccess) return hip_fail(e, "bwd_dw");
-      }
-      continue;
-    }
-    // fp32 tensors as bf16 pairs (lce_gemm.h): x = [hi | hi | lo] against W = [hi ; lo ; hi] along a K axis of
-    // 3 H for the logits; dz comes back as three parts [hi ; lo ; hi] of Np rows.
-    char* dz0 = (char*)a.dz;
-    const int64_t blk = a.Np * a.vs * 2;  // bytes from the first row of a part to that of the next
     if (ph & LCE_PHASE_BWD_DZ) {
-      lce::BwdArgs z = a;
-      z.H = 3 * p->H;
-      z.split = 1;
-      e = lce::launch_bwd_dz(z, s);
+      e = lce::launch_bwd_dz(a, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_dz");
     }
     if (dx && (ph & LCE_PHASE_BWD_DX)) {
-      // dx += dz_hi W_hi^T + dz_lo W_hi^T + dz_hi W_lo^T: three passes over the running fp32 sum
-      const char* w_hi = (const char*)a.w;
-      const char* w_lo = w_hi + p->H * a.ldw * 2;
-      for (int pass = 0; pass < 3; ++pass) {
-        lce::BwdArgs d = a;
-        d.dz = dz0 + (pass == 1 ? blk : 0);
-        d.w = pass == 2 ? w_lo : w_hi;
-        d.first = a.first && pass == 0;
-        d.last = a.last && pass == 2;
-        e = lce::launch_bwd_dx(d, s);
-        if (e != hipSuccess) return hip_fail(e, "bwd_dx");
-      }
+      e = lce::launch_bwd_dx(a, s);
+      if (e != hipSuccess) return hip_fail(e, "bwd_dx");
     }
     if (dw && (ph & LCE_PHASE_BWD_DW)) {
-      // dW = x_hi^T dz_hi + x_hi^T dz_lo + x_lo^T dz_hi: one contraction over 3 Np token rows, the copy of x
-      // stacked [hi ; hi ; lo] against the three blocks of dz (rows past the last kept token are zeros in both)
-      lce::BwdArgs g = a;
-      g.x = base + k.xk;
-      g.ldx = k.ldxk;
-      g.n_rows = nullptr;
-      g.N = 3 * a.Np;
-      g.Np = 3 * a.Np;
-      e = lce::launch_bwd_dw(g, s);
+      e = lce::launch_bwd_dw(a, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_dw");
     }
   }

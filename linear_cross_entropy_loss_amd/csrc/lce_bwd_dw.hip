@@ -460,7 +460,7 @@ LCE_DEV void dw_epilogue_f32_sum(const BwdArgs& a, f32x16_t (&acc)[kNB][kNB], in
 struct DwPlan {
   int tiles, full, tail_tiles, nseg, kseg, kt;
 };
-LCE_DEV DwPlan dw_plan(const BwdArgs& a, int64_t rows) {
+template <class T> LCE_DEV DwPlan dw_plan(const BwdArgs& a, int64_t rows) {
   DwPlan p;
   const int G = a.dw_grid;
   const int64_t kt2 = (rows + 2 * kBK - 1) / (2 * kBK) * 2;  // K tiles: an even number, at least four, covering the rows
@@ -470,7 +470,7 @@ LCE_DEV DwPlan dw_plan(const BwdArgs& a, int64_t rows) {
   const int r = p.tiles - p.full, cap = G < kTailBlocks ? G : kTailBlocks;
   int s = 1;
   if (r > 0 && a.dw_part != nullptr)  // (no blocks for partial sums: nothing is split)
-    while (r * s * 2 <= cap && p.kt / (s * 2) >= 16) s *= 2;
+    while (r * s * 2 <= cap && (is_pair<T>::value ? 3 : 1) * p.kt / (s * 2) >= 16) s *= 2;
   if (s == 1) {
     p.full = p.tiles;
     p.tail_tiles = 0;
@@ -499,6 +499,9 @@ enum { kDwAll = 0, kDwStaged = 1, kDwTails = 2, kDwStaged32 = 3 };
 // SCALE: the stage holds e, which the factors of BwdArgs::dw_f turn into dz.
 template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
   static constexpr bool kQScale = SCALE;
+  static constexpr bool kSplit = is_pair<T>::value;
+  LCE_DEV int64_t p_lo() const { return a.x_lo * 2; }
+  LCE_DEV int64_t q_lo() const { return kDzBlockElems * 2; }
   static constexpr bool kSwapAB = !WVH;  // (H, V) output: dz, the Q operand, feeds the A side (v along registers)
   static constexpr bool kVarK = true;    // whole tiles and segment items have different K extents
   static constexpr bool kKMask = false;  // both operands have K as their slow index: nothing to mask
@@ -516,7 +519,7 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
     const bool packed = rows != a.N;
     x = reinterpret_cast<const E*>(packed ? a.xc : a.x);
     ldx = packed ? a.ldxc : a.ldx;
-    plan = dw_plan(a, rows);
+    plan = dw_plan<T>(a, rows);
     const int tails = plan.tail_tiles * plan.nseg;
     first = MODE == kDwTails ? plan.full : 0;
     count = MODE == kDwAll ? plan.full + tails : (MODE == kDwTails ? tails : plan.full);
@@ -535,10 +538,10 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
     tile_coords(tile, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
   }
   LCE_DEV int item_ktiles(int local) const {
-    const int item = first + local;
-    if (item < plan.full) return plan.kt;
+    const int item = first + local, products = kSplit ? 3 : 1;
+    if (item < plan.full) return products * plan.kt;
     const int seg = (item - plan.full) % plan.nseg;
-    return seg == plan.nseg - 1 ? plan.kt - seg * plan.kseg : plan.kseg;
+    return products * (seg == plan.nseg - 1 ? plan.kt - seg * plan.kseg : plan.kseg);
   }
   LCE_DEV const float* q_factors(int local) const {
     if (local >= count) return a.dw_f;
@@ -556,7 +559,8 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
     decode(local, item, tp, tq, seg);
     const int64_t k0 = seg < 0 ? 0 : (int64_t)seg * plan.kseg * kBK;  // first token of the segment
     p = x + k0 * ldx + (int64_t)tp * kTile;
-    q = reinterpret_cast<const E*>(a.dz) + dz_block_offset(k0 / kTile, (int64_t)tq * (kTile / kBK), a.vs) + (k0 % kTile) * kBK;
+    q = reinterpret_cast<const E*>(a.dz) + (kSplit ? 2 : 1) * dz_block_offset(k0 / kTile, (int64_t)tq * (kTile / kBK), a.vs) +
+        (k0 % kTile) * kBK;
   }
   // (segments start at even numbers of K tiles: in the first or the third quarter of a row of blocks)
   LCE_DEV int q_phase(int local) const {
@@ -567,9 +571,10 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
   // x rows past the last one read as zeros.  dz is written for whole token tiles of 256 rows, and the K tiles of
   // the plan end with the pair of K tiles that holds the last row (dw_plan), so none of them reaches past
   // the rows that were written -- except when there is no row at all: then dz reads as zeros too.
-  LCE_DEV const void* p_end() const { return matrix_end<E>(x, rows, ldx, a.H); }
+  // (pairs: hidden indices past H of a hi part are read as lo parts; nothing is stored for them)
+  LCE_DEV const void* p_end() const { return matrix_end<E>(x, rows, ldx, kSplit ? a.x_lo + a.H : a.H); }
   LCE_DEV const void* q_end() const {
-    return reinterpret_cast<const E*>(a.dz) + (rows > 0 ? a.dz_rows * a.vs : 0);
+    return reinterpret_cast<const E*>(a.dz) + (rows > 0 ? (kSplit ? 2 : 1) * a.dz_rows * a.vs : 0);
   }
   LCE_DEV int k_valid(int) const { return (int)a.Np; }
   LCE_DEV void prefetch(int) {}
@@ -606,7 +611,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dw_persistent_kernel(const BwdAr
   // (a chunk without a kept row adds nothing to the sums of the earlier chunks)
   if ((ACC == 2 || ACC == 4 || ACC == 7) && prob.rows == 0) return;
   Pipe3<T, E, false, E, false, Problem> pipe(prob);
-  pipe.run(prob.ldx, a.vs / kBK, prob.plan.kt, lds, (int)blockIdx.x);
+  pipe.run(prob.ldx, a.vs / kBK, (is_pair<T>::value ? 3 : 1) * prob.plan.kt, lds, (int)blockIdx.x);
 }
 
 // Second step for the tail tiles: kTailParts workgroups share tail tile b (16 of its rows each) -- they sum
@@ -615,7 +620,7 @@ constexpr int kTailParts = 16;
 template <class T, bool WVH>
 __global__ __launch_bounds__(256) void dw_tail_kernel(const BwdArgs a) {
   typedef typename elem_of<T>::type E;
-  const DwPlan plan = dw_plan(a, packed_rows(a.n_rows, a.N));
+  const DwPlan plan = dw_plan<T>(a, packed_rows(a.n_rows, a.N));
   const int b = (int)blockIdx.x / kTailParts, piece = (int)blockIdx.x % kTailParts;
   if (b >= plan.tail_tiles) return;
   int tp, tq;
@@ -653,7 +658,10 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> hipError_t launch_ke
 }
 
 template <class T, bool WVH, int MODE, int ACC = 0> hipError_t launch_tiles(const BwdArgs& a, hipStream_t s) {
-  return a.dw_f != nullptr ? launch_kernel<T, WVH, MODE, ACC, true>(a, s) : launch_kernel<T, WVH, MODE, ACC, false>(a, s);
+  if constexpr (is_pair<T>::value)
+    return a.dw_f != nullptr ? hipErrorInvalidValue : launch_kernel<T, WVH, MODE, ACC, false>(a, s);
+  else
+    return a.dw_f != nullptr ? launch_kernel<T, WVH, MODE, ACC, true>(a, s) : launch_kernel<T, WVH, MODE, ACC, false>(a, s);
 }
 
 // Whole tiles that meet the plane of sums over chunks of token rows (nothing is split along K then).
@@ -679,11 +687,12 @@ template <class T, bool WVH> hipError_t launch_persistent(const BwdArgs& a, hipS
     const bool cut = a.Hp != a.H || a.v0 + a.vs != a.V;
     if (a.dw_plane == nullptr || a.dw_part != nullptr || a.dw_dtype == DT_F32 || (cut && a.dw_plane_hi == nullptr))
       return hipErrorInvalidValue;
-    return launch_plane<T, WVH, kDwAll>(a, s);
+    if constexpr (is_pair<T>::value) return hipErrorInvalidValue;
+    else return launch_plane<T, WVH, kDwAll>(a, s);
   }
   // a last round of tiles may be split along K (the tile count does not depend on the rows; whether its K
   // extent is long enough to split is decided on the device, and a launch without items returns at once)
-  const bool tails = a.dw_part != nullptr && dw_tail_blocks(a.Np, a.Hp, a.vs) != 0 &&
+  const bool tails = a.dw_part != nullptr && dw_tail_blocks(a.Np, a.Hp, a.vs, products_of(a.x_dtype)) != 0 &&
                      has_split_tail((a.vs / kTile) * (a.Hp / kTile), a.dw_grid);
   hipError_t e = hipSuccess;
   if constexpr (WVH) {
@@ -692,8 +701,10 @@ template <class T, bool WVH> hipError_t launch_persistent(const BwdArgs& a, hipS
     // (a small problem whose tiles are all split along K has no whole tile to launch; known here when rows are not packed)
     const int64_t kt2 = (a.N + 2 * kBK - 1) / (2 * kBK) * 2;
     const bool none_whole = tails && a.n_rows == nullptr &&
-                            all_tiles_are_tails((a.vs / kTile) * (a.Hp / kTile), a.dw_grid, kt2 < 4 ? 4 : kt2);
-    if (!none_whole)
+                            all_tiles_are_tails((a.vs / kTile) * (a.Hp / kTile), a.dw_grid, products_of(a.x_dtype) * (kt2 < 4 ? 4 : kt2));
+    if (none_whole) e = hipSuccess;
+    else if constexpr (is_pair<T>::value) e = launch_tiles<T, false, kDwStaged32>(a, s);
+    else
       e = a.dw_dtype == DT_F32 ? launch_tiles<T, false, kDwStaged32>(a, s) : launch_tiles<T, false, kDwStaged>(a, s);
     if (e == hipSuccess && tails) e = launch_tiles<T, false, kDwTails>(a, s);
   }
@@ -709,6 +720,7 @@ template <class T, bool WVH> hipError_t launch_persistent(const BwdArgs& a, hipS
 hipError_t launch_bwd_dw(const BwdArgs& a, hipStream_t s) {
   if (a.x_dtype == DT_BF16) return a.w_vh ? launch_persistent<BF16, true>(a, s) : launch_persistent<BF16, false>(a, s);
   if (a.x_dtype == DT_F16) return a.w_vh ? launch_persistent<F16, true>(a, s) : launch_persistent<F16, false>(a, s);
+  if (a.x_dtype == DT_PAIR && a.dw_dtype == DT_F32 && !a.w_vh) return launch_persistent<BF16P, false>(a, s);
   return hipErrorInvalidValue;
 }
 

@@ -126,7 +126,7 @@ LCE_DEV void dx_store_segment(float* part, f32x16_t (&acc)[kNB][kNB]) {
 struct DxPlan {
   int tiles, full, tail_tiles, nseg, kseg;  // items [0, full) are whole tiles, then tail_tiles * nseg segment items
 };
-LCE_DEV DxPlan dx_plan(const BwdArgs& a, int tiles) {
+template <class T> LCE_DEV DxPlan dx_plan(const BwdArgs& a, int tiles) {
   DxPlan p;
   const int G = a.dx_grid, kt = (int)(a.vs / kBK);
   p.tiles = tiles;
@@ -134,7 +134,7 @@ LCE_DEV DxPlan dx_plan(const BwdArgs& a, int tiles) {
   const int r = tiles - p.full, cap = G < kTailBlocks ? G : kTailBlocks;
   int s = 1;
   if (r > 0 && a.dx_part != nullptr)  // (no blocks for partial sums: nothing is split)
-    while (r * s * 2 <= cap && kt / (s * 2) >= 16) s *= 2;
+    while (r * s * 2 <= cap && (is_pair<T>::value ? 3 : 1) * kt / (s * 2) >= 16) s *= 2;
   if (s == 1) {
     p.full = tiles;
     p.tail_tiles = 0;
@@ -159,6 +159,9 @@ enum { kDxFirst = 0, kDxMiddle = 1, kDxLast = 2, kDxOnly = 3, kDxTails = 4 };
 template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem {
   static constexpr bool kKMask = KMASK;
   static constexpr bool kQScale = SCALE;
+  static constexpr bool kSplit = is_pair<T>::value;
+  LCE_DEV int64_t p_lo() const { return a.H * a.ldw * 2; }
+  LCE_DEV int64_t q_lo() const { return kDzBlockElems * 2; }
   static constexpr bool kSwapAB = false;
   static constexpr bool kVarK = MODE == kDxTails;  // segment items have their own K extent
   static constexpr bool kQBlocked = true;          // dz is staged in blocks of 256 rows x 64 columns (BwdArgs::dz)
@@ -171,7 +174,7 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
   int first, count;  // this launch's items of the plan: [first, first + count)
   LCE_DEV DxProblem(const BwdArgs& a_) : a(a_), rows(packed_rows(a_.n_rows, a_.N)), tiles_p((int)(a_.Hp / kTile)) {
     tiles_q = (int)((rows + kTile - 1) / kTile);
-    plan = dx_plan(a, tiles_p * tiles_q);
+    plan = dx_plan<T>(a, tiles_p * tiles_q);
     first = MODE == kDxTails ? plan.full : 0;
     count = MODE == kDxTails ? plan.tail_tiles * plan.nseg : plan.full;
   }
@@ -188,7 +191,7 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
     }
     tile_coords(tile, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
   }
-  LCE_DEV int item_ktiles(int) const { return plan.kseg; }
+  LCE_DEV int item_ktiles(int) const { return kSplit ? 3 * plan.kseg : plan.kseg; }
   // (a K tile is half a slice of 128 columns; work items start at even K tiles)
   LCE_DEV const float* q_factors(int local) const {
     if (local >= count) return a.dx_f;
@@ -206,15 +209,15 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
     const int64_t k0 = k0_of(seg);
     p = WVH ? reinterpret_cast<const E*>(a.w) + ((a.v0 - a.wv0) + k0) * a.ldw + (int64_t)tp * kTile
             : reinterpret_cast<const E*>(a.w) + (int64_t)tp * kTile * a.ldw + (a.v0 - a.wv0) + k0;
-    q = reinterpret_cast<const E*>(a.dz) + dz_block_offset(tq, k0 / kBK, a.vs);  // (k0 is a multiple of 64)
+    q = reinterpret_cast<const E*>(a.dz) + (kSplit ? 2 : 1) * dz_block_offset(tq, k0 / kBK, a.vs);  // (k0 is a multiple of 64)
   }
   LCE_DEV const void* p_end() const {
-    return WVH ? matrix_end<E>(a.w, a.Vw, a.ldw, a.H) : matrix_end<E>(a.w, a.H, a.ldw, a.Vw);
+    return WVH ? matrix_end<E>(a.w, a.Vw, a.ldw, a.H) : matrix_end<E>(a.w, kSplit ? 2 * a.H : a.H, a.ldw, a.Vw);
   }
   // (only whole token tiles that were written are read.  K tiles past the slab -- the last segment of a split tail
   // tile may have some -- lie in the next row of blocks, or past the stage: the K mask gives those threads an
   // out-of-range offset, the other operand's are zeros)
-  LCE_DEV const void* q_end() const { return reinterpret_cast<const E*>(a.dz) + a.dz_rows * a.vs; }
+  LCE_DEV const void* q_end() const { return reinterpret_cast<const E*>(a.dz) + (kSplit ? 2 : 1) * a.dz_rows * a.vs; }
   LCE_DEV int k_valid(int local) const {
     int item, tp, tq, seg;
     decode(local, item, tp, tq, seg);
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dx_persistent_kernel(const BwdAr
   typedef DxProblem<T, KMASK, WVH, MODE, SCALE> Problem;
   Problem prob(a);
   Pipe3<T, E, !WVH, E, true, Problem> pipe(prob);
-  pipe.run(a.ldw, a.vs / kBK, MODE == kDxTails ? prob.plan.kseg : (int)(a.vs / kBK), lds, (int)blockIdx.x);
+  pipe.run(a.ldw, a.vs / kBK, (is_pair<T>::value ? 3 : 1) * (MODE == kDxTails ? prob.plan.kseg : (int)(a.vs / kBK)), lds, (int)blockIdx.x);
 }
 
 // Second step for the tail tiles: kTailParts workgroups share tail tile b (16 rows each) -- they sum its
@@ -252,7 +255,7 @@ __global__ __launch_bounds__(256) void dx_tail_kernel(const BwdArgs a) {
   typedef typename elem_of<T>::type E;
   const int64_t rows = packed_rows(a.n_rows, a.N);
   const int tiles_p = (int)(a.Hp / kTile), tiles_q = (int)((rows + kTile - 1) / kTile);
-  const DxPlan plan = dx_plan(a, tiles_p * tiles_q);
+  const DxPlan plan = dx_plan<T>(a, tiles_p * tiles_q);
   const int b = (int)blockIdx.x / kTailParts, piece = (int)blockIdx.x % kTailParts;
   if (b >= plan.tail_tiles) return;
   int tp, tq;
@@ -302,12 +305,16 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE = false> hipError_
 template <class T, bool KMASK, bool WVH> hipError_t launch_layout(const BwdArgs& a, bool tails, hipStream_t s) {
   // (a small problem whose tiles are all split along K has no whole tile to launch; known here when rows are not packed)
   const bool none_whole = tails && a.n_rows == nullptr &&
-                          all_tiles_are_tails((a.Np / kTile) * (a.Hp / kTile), a.dx_grid, a.vs / kBK);
+                          all_tiles_are_tails((a.Np / kTile) * (a.Hp / kTile), a.dx_grid, products_of(a.x_dtype) * (a.vs / kBK));
   if (a.dx_f != nullptr) {
-    if (!a.first || !a.last) return hipErrorInvalidValue;
-    hipError_t e = none_whole ? hipSuccess : launch_tiles<T, KMASK, WVH, kDxOnly, true>(a, s);
-    if (e == hipSuccess && tails) e = launch_tiles<T, KMASK, WVH, kDxTails, true>(a, s);
-    return e;
+    if constexpr (is_pair<T>::value) {
+      return hipErrorInvalidValue;
+    } else {
+      if (!a.first || !a.last) return hipErrorInvalidValue;
+      hipError_t e = none_whole ? hipSuccess : launch_tiles<T, KMASK, WVH, kDxOnly, true>(a, s);
+      if (e == hipSuccess && tails) e = launch_tiles<T, KMASK, WVH, kDxTails, true>(a, s);
+      return e;
+    }
   }
   hipError_t e = none_whole ? hipSuccess
                : a.first ? (a.last ? launch_tiles<T, KMASK, WVH, kDxOnly>(a, s) : launch_tiles<T, KMASK, WVH, kDxFirst>(a, s))
@@ -319,11 +326,15 @@ template <class T, bool KMASK, bool WVH> hipError_t launch_layout(const BwdArgs&
 template <class T> hipError_t launch_persistent(const BwdArgs& a, hipStream_t s) {
   // A last round of tiles may be split along K.  Without packed rows the tile count is known here; with them
   // it is decided on the device, and a launch without items returns at once.
-  const bool tails = a.dx_part != nullptr && dx_tail_blocks(a.Np, a.Hp, a.vs) != 0 &&
+  const bool tails = a.dx_part != nullptr && dx_tail_blocks(a.Np, a.Hp, a.vs, products_of(a.x_dtype)) != 0 &&
                      (a.n_rows != nullptr || has_split_tail((a.Np / kTile) * (a.Hp / kTile), a.dx_grid));
   // the K mask is only needed when the K tiles of a work item can run past the columns that exist
-  const bool exact_k = a.vw == a.vs && dx_segments_exact(a.vs);
-  hipError_t e = a.w_vh ? (exact_k ? launch_layout<T, false, true>(a, tails, s) : launch_layout<T, true, true>(a, tails, s))
+  const bool exact_k = a.vw == a.vs && dx_segments_exact(a.vs, products_of(a.x_dtype));
+  hipError_t e;
+  if constexpr (is_pair<T>::value)
+    e = exact_k ? launch_layout<T, false, false>(a, tails, s) : launch_layout<T, true, false>(a, tails, s);
+  else
+    e = a.w_vh ? (exact_k ? launch_layout<T, false, true>(a, tails, s) : launch_layout<T, true, true>(a, tails, s))
                         : (exact_k ? launch_layout<T, false, false>(a, tails, s) : launch_layout<T, true, false>(a, tails, s));
   if (e != hipSuccess || !tails) return e;
   // at most dx_grid / 2 tail tiles can be split (two segments each)
@@ -338,6 +349,7 @@ hipError_t launch_bwd_dx(const BwdArgs& a, hipStream_t s) {
   // (an fp32 weight arrives here as a 16-bit slab copy; x_dtype is the compute type by now)
   if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16) return launch_persistent<BF16>(a, s);
   if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16) return launch_persistent<F16>(a, s);
+  if (a.x_dtype == DT_PAIR && a.w_dtype == DT_PAIR && !a.w_vh) return launch_persistent<BF16P>(a, s);
   return hipErrorInvalidValue;
 }
 

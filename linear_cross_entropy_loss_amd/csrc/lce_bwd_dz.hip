@@ -58,9 +58,9 @@ constexpr int kDzStoreAux = LCE_DZ_STORE_AUX;  // cache policy of the dz stores:
 // one run that V cuts through is handled element by element.  Columns outside
 // are written as exact zeros.
 //
-// SPLIT (fp32 tensors carried as bf16 pairs, lce_gemm.h): dz is staged as hi = bf16(dz) and lo = bf16(dz - hi)
-// in three parts of Np rows, [hi ; lo ; hi], each lane storing its 16-byte runs itself (this
-// path serves accuracy, not speed).
+// SPLIT (fp32 tensors carried as bf16 pairs, lce_gemm.h): dz is staged as hi = bf16(dz) and lo = bf16(dz - hi), the block
+// of the lo parts behind each block of hi parts; the pieces of hi parts leave first, then, through the same LDS area,
+// those of lo parts, which wait in registers.
 // `pf_y`, `pf_lse`: label and lse of this lane's four tokens (DzProblem::prefetch), ignore_index / 0 for rows that do not exist.
 //
 // FUSE (launch_fwd_stage: the logits are computed once, for the loss and for the gradients): the tile leaves
@@ -70,7 +70,7 @@ constexpr int kDzStoreAux = LCE_DZ_STORE_AUX;  // cache policy of the dz stores:
 // switch ZREG stands for the monitoring values instead (the slice's sum softmax * z and sum z^2, as lce_fwd.hip forms them).
 constexpr int kNoLabel = -0x7fffffff - 1;  // ignore_index, or no such row
 constexpr int kOffLabel = -1;              // a label that is no column of W (V <= 2^30): matches nothing
-template <class T, bool ZREG, bool VTAIL, bool SPLIT, bool FUSE>
+template <class T, bool ZREG, bool VTAIL, bool FUSE>
 LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const float (&pf_lse)[kNB],
                               f32x16_t (&acc)[kNB][kNB], int tp, int tq, char* pieces) {
   typedef typename elem_of<T>::type E;
@@ -88,18 +88,18 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
   const int cut_mine = cut - 4 * half;  // elements of this lane's quad of the cut run that exist (<= 0: none)
   // This wave's 128 columns are two column groups (accumulator blocks 0, 1 and 2, 3), neighbouring blocks of the
   // stage; `row` = this lane's token row of block qb = 0 in the first of them.
-  constexpr int64_t grp = kDzBlockElems;  // elements from a block of the stage to the next column group's
+  constexpr bool SPLIT = is_pair<T>::value;
+  constexpr int kParts = SPLIT ? 2 : 1;
+  constexpr int64_t grp = kParts * kDzBlockElems;  // elements from a block of the stage to the next column group's
   const int wpu = __builtin_amdgcn_readfirstlane(wp), wqu = __builtin_amdgcn_readfirstlane(wq);  // (uniform, for the scalar unit)
-  E* wave_base = reinterpret_cast<E*>(a.dz) + dz_block_offset(tq, tp * (kTile / kGroup) + wpu * (kWaveTile / kGroup), a.vs) +
+  E* wave_base = reinterpret_cast<E*>(a.dz) + kParts * dz_block_offset(tq, tp * (kTile / kGroup) + wpu * (kWaveTile / kGroup), a.vs) +
                  wqu * kWaveTile * kGroup;
   E* row = wave_base + (lane & 31) * kGroup;
   constexpr bool MON = FUSE && ZREG;
-  const int64_t blk = a.Np * a.vs;  // SPLIT: elements between the three parts of the stage
   // Stores go through a buffer descriptor over this wave's part of the stage (scalar base, one 32-bit offset per
   // lane, the block's offset as a scalar): no 64-bit vector address arithmetic.  All offsets stay below 2^31
-  // (one block for the second column group, plus two parts of a bf16-pair stage).
+  // (one block for the second column group, twice that for the pairs' two parts).
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(wave_base, 0, 0x7fffffff, 0x00020000);
-  const unsigned lane_off = (unsigned)((lane & 31) * (kGroup * 2) + half * 16);
   // staging: this lane's line of a piece when it writes (its token), and line / chunk when it reads back: 8 lines
   // per instruction, 8 lanes each; the upper 32 lanes take their four lines in the order 5, 4, 7, 6 so that lanes
   // l and l+32 always sit in lines of opposite parity (opposite bank halves)
@@ -129,6 +129,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
 #pragma unroll
   for (int qb = 0; qb < kNB; ++qb) {
     float m = -INFINITY, ssum = 0.f, mpz = 0.f, msq = 0.f;
+    u32x4_t lo_part[SPLIT ? 8 : 1];  // this lane's 16-byte runs of lo parts
     if constexpr (FUSE) {
       // the largest of this token's logits in the slice: this lane's 64, then the other half's
 #pragma unroll
@@ -148,7 +149,6 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
     }
 #pragma unroll
     for (int pb = 0; pb < kNB; ++pb) {
-      const unsigned blk_off = (unsigned)((pb >> 1) * grp * 2) + qb * (kBlk * kGroup * 2);  // bytes, uniform
 #pragma unroll
       for (int g = 0; g < 4; g += 2) {
         float d[8];
@@ -204,11 +204,8 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
           o[3] = s1[1];
           // streaming stores (aux 2 = nt): dz (1 GiB per slab) is read back from memory by the next kernels anyway,
           // and a normal store would evict the W / x tiles the following main loop is about to reuse from L2
-          if constexpr (SPLIT) {
-            const unsigned voff = lane_off + (pb & 1) * (kBlk * 2) + g * 16;
-            const unsigned soff = blk_off + (part == 1 ? (unsigned)(blk * 2) : 0u);
-            __builtin_amdgcn_raw_buffer_store_b128(o, rsrc, (int)voff, (int)soff, kDzStoreAux);
-            if (part == 0) __builtin_amdgcn_raw_buffer_store_b128(o, rsrc, (int)voff, (int)(soff + (unsigned)(blk * 4)), kDzStoreAux);
+          if (SPLIT && part == 1) {
+            lo_part[SPLIT ? pb * 2 + (g >> 1) : 0] = o;
           } else {
             const int chunk = (pb & 1) * 4 + g + half;  // 16-byte chunk of the token's line
             *reinterpret_cast<u32x4_t*>(mine + (pb >> 1) * kPieceBytes + wline * (kGroup * 2) + ((chunk ^ wsw) << 4)) = o;
@@ -216,7 +213,15 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
         }
       }
     }
-    if constexpr (!SPLIT) {
+#pragma unroll
+    for (int part = 0; part < kParts; ++part) {
+      if (SPLIT && part == 1) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int pb = u >> 1, chunk = (pb & 1) * 4 + 2 * (u & 1) + half;
+          *reinterpret_cast<u32x4_t*>(mine + (pb >> 1) * kPieceBytes + wline * (kGroup * 2) + ((chunk ^ wsw) << 4)) = lo_part[SPLIT ? u : 0];
+        }
+      }
       // read the two pieces back as 128-byte lines and send them out
 #pragma unroll
       for (int gi = 0; gi < 2; ++gi)
@@ -225,7 +230,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
           const int line = i * 8 + rline;
           const u32x4_t v = *reinterpret_cast<const u32x4_t*>(mine + gi * kPieceBytes + line * (kGroup * 2) +
                                                               ((rchunk ^ (line & 7) ^ ((line >> 3) & 1)) << 4));
-          const unsigned soff = (unsigned)(gi * grp * 2) + qb * (kBlk * kGroup * 2);
+          const unsigned soff = (unsigned)(gi * grp * 2 + part * kDzBlockElems * 2) + qb * (kBlk * kGroup * 2);
           __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, line * (kGroup * 2) + rchunk * 16, (int)soff, kDzStoreAux);
         }
     }
@@ -284,10 +289,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
       const float tv = p - __builtin_bit_cast(float, (127 + a.dz_shift) << 23);  // the one, times 2^dz_shift
       E* at = row + (yl >> 6) * grp + qb * (kBlk * kGroup) + (yl & (kGroup - 1));
       *reinterpret_cast<unsigned short*>(at) = to_bits<T>(tv);
-      if (SPLIT) {
-        *reinterpret_cast<unsigned short*>(at + 2 * blk) = to_bits<T>(tv);
-        *reinterpret_cast<unsigned short*>(at + blk) = to_bits<T>(bf16_lo(tv));
-      }
+      if (SPLIT) *reinterpret_cast<unsigned short*>(at + kDzBlockElems) = to_bits<T>(bf16_lo(tv));
     }
   }
 }
@@ -300,13 +302,16 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
 // of the vocabulary to the end of the padded slab -- or, with BwdArgs::vtail_all, every column (the VTAIL code
 // is right for full columns too, only slower).
 // WVH: the weight is stored (V, H) row-major, so that the P operand runs along K in memory like x does.
-template <class T, bool ZREG, bool VTAIL, bool KMASK, bool SPLIT, bool WVH, bool FUSE = false> struct DzProblem {
+template <class T, bool ZREG, bool VTAIL, bool KMASK, bool WVH, bool FUSE = false> struct DzProblem {
   typedef typename elem_of<T>::type E;
   static constexpr bool kKMask = KMASK;
   static constexpr bool kSwapAB = false;
   static constexpr bool kVarK = false;
   static constexpr bool kQBlocked = false;
   static constexpr bool kQScale = false;
+  static constexpr bool kSplit = is_pair<T>::value;
+  LCE_DEV int64_t p_lo() const { return a.H * a.ldw * 2; }
+  LCE_DEV int64_t q_lo() const { return a.x_lo * 2; }
   static constexpr bool kColumnEpilogue = false;
   const BwdArgs& a;
   int64_t rows, ldx;  // token rows: all of x, or the packed rows (see BwdArgs)
@@ -319,9 +324,7 @@ template <class T, bool ZREG, bool VTAIL, bool KMASK, bool SPLIT, bool WVH, bool
     const bool packed = rows != a.N;
     x = reinterpret_cast<const E*>(packed ? a.xc : a.x);
     ldx = packed ? a.ldxc : a.ldx;
-    // SPLIT: the dW contraction runs through all Np rows of each of the three blocks of the stage, so every
-    // token tile is written (rows past the last kept token as zeros), not only those that hold kept tokens
-    tiles_q = SPLIT ? (int)(a.Np / kTile) : (int)((rows + kTile - 1) / kTile);
+    tiles_q = (int)((rows + kTile - 1) / kTile);
   }
   LCE_DEV int num_tiles() const { return tiles_p * tiles_q; }
   LCE_DEV void coords(int tile, int& tp, int& tq) const {
@@ -336,9 +339,9 @@ template <class T, bool ZREG, bool VTAIL, bool KMASK, bool SPLIT, bool WVH, bool
     q = x + (int64_t)tq * kTile * ldx;
   }
   LCE_DEV const void* p_end() const {
-    return WVH ? matrix_end<E>(a.w, a.Vw, a.ldw, a.H) : matrix_end<E>(a.w, a.H, a.ldw, a.Vw);
+    return WVH ? matrix_end<E>(a.w, a.Vw, a.ldw, a.H) : matrix_end<E>(a.w, kSplit ? 2 * a.H : a.H, a.ldw, a.Vw);
   }
-  LCE_DEV const void* q_end() const { return matrix_end<E>(x, rows, ldx, a.H); }
+  LCE_DEV const void* q_end() const { return matrix_end<E>(x, rows, ldx, kSplit ? a.x_lo + a.H : a.H); }
   LCE_DEV int k_valid(int) const { return (int)a.H; }
   // The epilogue starts with the label and lse of each of this lane's four tokens: fetched while the last K tiles
   // of the tile are still being multiplied, instead of one exposed round trip to memory per tile.
@@ -360,36 +363,36 @@ template <class T, bool ZREG, bool VTAIL, bool KMASK, bool SPLIT, bool WVH, bool
   LCE_DEV void epilogue(int tile, f32x16_t (&acc)[kNB][kNB], char* scratch) const {
     int tp, tq;
     coords(tile, tp, tq);
-    dz_epilogue_impl<T, ZREG, VTAIL, SPLIT, FUSE>(a, pf_y, pf_lse, acc, tp, tq, scratch + kStageBytes);  // (behind the main loop's stages)
+    dz_epilogue_impl<T, ZREG, VTAIL, FUSE>(a, pf_y, pf_lse, acc, tp, tq, scratch + kStageBytes);  // (behind the main loop's stages)
   }
 };
 
 // TAIL: the tile columns that the launch covers, as in the forward (fwd_tiles_persistent_kernel).
-template <class T, bool ZREG, int TAIL, bool KMASK, bool SPLIT, bool WVH, bool FUSE>
+template <class T, bool ZREG, int TAIL, bool KMASK, bool WVH, bool FUSE>
 __global__ __launch_bounds__(kThreads) void bwd_dz_persistent_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
   int first = (int)blockIdx.x;
   if constexpr (TAIL != kTailOnly) {
-    typedef DzProblem<T, ZREG, false, KMASK, SPLIT, WVH, FUSE> Full;
+    typedef DzProblem<T, ZREG, false, KMASK, WVH, FUSE> Full;
     Full prob(a);
     Pipe3<T, E, WVH, E, true, Full> pipe(prob);
-    if (TAIL == kNoTail || first < prob.num_tiles()) pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+    if (TAIL == kNoTail || first < prob.num_tiles()) pipe.run(a.ldw, prob.ldx, logit_ktiles<T>(a.H), lds, first);
     if (TAIL == kWithTail) first = first_tail_tile(first, (int)gridDim.x, prob.num_tiles());
   }
   if constexpr (TAIL != kNoTail) {
-    typedef DzProblem<T, ZREG, true, true, SPLIT, WVH, FUSE> Tail;
+    typedef DzProblem<T, ZREG, true, true, WVH, FUSE> Tail;
     Tail prob(a);
     if (first >= prob.num_tiles()) return;
     __syncthreads();  // (every wave is done with the main loop's LDS stages)
     Pipe3<T, E, WVH, E, true, Tail> pipe(prob);
-    pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+    pipe.run(a.ldw, prob.ldx, logit_ktiles<T>(a.H), lds, first);
   }
 }
 
-template <class T, bool ZREG, int TAIL, bool KMASK, bool SPLIT, bool WVH, bool FUSE = false>
+template <class T, bool ZREG, int TAIL, bool KMASK, bool WVH, bool FUSE = false>
 hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
-  auto kern = bwd_dz_persistent_kernel<T, ZREG, TAIL, KMASK, SPLIT, WVH, FUSE>;
+  auto kern = bwd_dz_persistent_kernel<T, ZREG, TAIL, KMASK, WVH, FUSE>;
   static LdsOptIn optin;
   hipError_t e = optin.ensure(reinterpret_cast<const void*>(kern), kLdsBytes);
   if (e != hipSuccess) return e;
@@ -399,59 +402,58 @@ hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
 }
 
 // All tile columns of the slab in one launch.
-template <class T, bool ZREG, bool SPLIT, bool WVH, bool FUSE = false>
+template <class T, bool ZREG, bool WVH, bool FUSE = false>
 hipError_t launch_persistent_z(const BwdArgs& a, hipStream_t s) {
   const int64_t tq = a.Np / kTile, full = a.vw / kTile, tail = a.vs / kTile - full;
-  const bool exact_k = padded_k(a.H) == a.H;  // the K tiles cover H exactly: no K mask needed
-  if (full == 0) return launch_one<T, ZREG, kTailOnly, true, SPLIT, WVH, FUSE>(a, tail * tq, s);
+  const bool exact_k = (is_pair<T>::value ? padded_k_pair(a.H) : padded_k(a.H)) == a.H;  // the K tiles cover H exactly: no K mask needed
+  if (full == 0) return launch_one<T, ZREG, kTailOnly, true, WVH, FUSE>(a, tail * tq, s);
   if constexpr (FUSE && ZREG) {
     // (the monitoring sums on top of the K mask do not fit the registers in the kernel for full columns: a hidden
     // size that is not a multiple of 128 sends every column through the kernel for the last one, which has both)
     if (!exact_k) {
       BwdArgs all = a;
       all.vtail_all = 1;
-      return launch_one<T, ZREG, kTailOnly, true, SPLIT, WVH, FUSE>(all, (a.vs / kTile) * tq, s);
+      return launch_one<T, ZREG, kTailOnly, true, WVH, FUSE>(all, (a.vs / kTile) * tq, s);
     }
-    return tail > 0 ? launch_one<T, ZREG, kWithTail, false, SPLIT, WVH, FUSE>(a, (full + tail) * tq, s)
-                    : launch_one<T, ZREG, kNoTail, false, SPLIT, WVH, FUSE>(a, full * tq, s);
+    return tail > 0 ? launch_one<T, ZREG, kWithTail, false, WVH, FUSE>(a, (full + tail) * tq, s)
+                    : launch_one<T, ZREG, kNoTail, false, WVH, FUSE>(a, full * tq, s);
   } else {
     if (tail > 0)
-      return exact_k ? launch_one<T, ZREG, kWithTail, false, SPLIT, WVH, FUSE>(a, (full + tail) * tq, s)
-                     : launch_one<T, ZREG, kWithTail, true, SPLIT, WVH, FUSE>(a, (full + tail) * tq, s);
-    return exact_k ? launch_one<T, ZREG, kNoTail, false, SPLIT, WVH, FUSE>(a, full * tq, s)
-                   : launch_one<T, ZREG, kNoTail, true, SPLIT, WVH, FUSE>(a, full * tq, s);
+      return exact_k ? launch_one<T, ZREG, kWithTail, false, WVH, FUSE>(a, (full + tail) * tq, s)
+                     : launch_one<T, ZREG, kWithTail, true, WVH, FUSE>(a, (full + tail) * tq, s);
+    return exact_k ? launch_one<T, ZREG, kNoTail, false, WVH, FUSE>(a, full * tq, s)
+                   : launch_one<T, ZREG, kNoTail, true, WVH, FUSE>(a, full * tq, s);
   }
 }
 
-template <class T, bool SPLIT, bool WVH> hipError_t launch_persistent(const BwdArgs& a, hipStream_t s) {
-  return a.z_reg != 0.f ? launch_persistent_z<T, true, SPLIT, WVH>(a, s)
-                        : launch_persistent_z<T, false, SPLIT, WVH>(a, s);
+template <class T, bool WVH> hipError_t launch_persistent(const BwdArgs& a, hipStream_t s) {
+  return a.z_reg != 0.f ? launch_persistent_z<T, true, WVH>(a, s) : launch_persistent_z<T, false, WVH>(a, s);
 }
 
 }  // namespace
 
 hipError_t launch_bwd_dz(const BwdArgs& a, hipStream_t s) {
   if (a.w_vh) {  // (never with bf16 pairs)
-    if (a.split) return hipErrorInvalidValue;
-    if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16) return launch_persistent<BF16, false, true>(a, s);
-    if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16) return launch_persistent<F16, false, true>(a, s);
+    if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16) return launch_persistent<BF16, true>(a, s);
+    if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16) return launch_persistent<F16, true>(a, s);
     return hipErrorInvalidValue;
   }
   if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16)
-    return a.split ? launch_persistent<BF16, true, false>(a, s) : launch_persistent<BF16, false, false>(a, s);
-  if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16) return launch_persistent<F16, false, false>(a, s);
-  // (an fp32 weight arrives here as a 16-bit slab copy, fp32 activations as bf16 pairs with split set)
+    return launch_persistent<BF16, false>(a, s);
+  if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16) return launch_persistent<F16, false>(a, s);
+  // (an fp32 weight arrives here as a copy in the compute type, fp32 activations as bf16 pairs)
+  if (a.x_dtype == DT_PAIR && a.w_dtype == DT_PAIR) return launch_persistent<BF16P, false>(a, s);
   return hipErrorInvalidValue;
 }
 
 template <class T, bool WVH> hipError_t launch_stage(const BwdArgs& a, hipStream_t s) {
   // (the second template argument: the monitoring values, see dz_epilogue_impl)
-  return a.part_pz != nullptr ? launch_persistent_z<T, true, false, WVH, true>(a, s)
-                              : launch_persistent_z<T, false, false, WVH, true>(a, s);
+  return a.part_pz != nullptr ? launch_persistent_z<T, true, WVH, true>(a, s)
+                              : launch_persistent_z<T, false, WVH, true>(a, s);
 }
 
 hipError_t launch_fwd_stage(const BwdArgs& a, hipStream_t s) {
-  if (a.split || a.part_lse == nullptr || a.part_max == nullptr || a.tgt == nullptr) return hipErrorInvalidValue;
+  if (a.part_lse == nullptr || a.part_max == nullptr || a.tgt == nullptr) return hipErrorInvalidValue;
   if ((a.part_pz == nullptr) != (a.part_sq == nullptr)) return hipErrorInvalidValue;
   if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16) return a.w_vh ? launch_stage<BF16, true>(a, s) : launch_stage<BF16, false>(a, s);
   if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16) return a.w_vh ? launch_stage<F16, true>(a, s) : launch_stage<F16, false>(a, s);

@@ -176,49 +176,42 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const char* x, int64_t
   }
 }
 
-// fp32 activations reach the tile kernels as bf16 pairs, x = hi + lo (lce_gemm.h), in two copies that are made
-// even when no token is dropped (`perm` / `n_rows` may be null: all rows, in their order):
-//   xc  [rows][3 H]       row j = [hi | hi | lo] of x[perm[j]]: the K axis of the logit contraction, three
-//                         times as long, against a weight copy laid out [hi ; lo ; hi]
-//   xk  [3][Np][H]        hi, hi, lo again, stacked along the TOKEN axis, which is the K axis of
-//                         dW = x^T dz (against dz staged as [hi ; lo ; hi]); rows from `rows` to Np of each
-//                         block are zeros, since K runs through them.  Null in the forward.
-// One workgroup per packed row (grid-stride); elements go out as single 16-bit stores, consecutive lanes to
-// consecutive addresses (H need not be a multiple of anything, so the three parts of a row of xc do not
-// start on 16-byte boundaries).
+// fp32 activations reach the tile kernels as bf16 pairs, x = hi + lo (lce_gemm.h), in a copy that is made even when no token is
+// dropped (`perm` / `n_rows` may be null: all rows, in their order): row j = [hi | lo] of x[perm[j]], each part `part` elements
+// long (a multiple of 8, zero-padded).  One workgroup per packed row (grid-stride), 8 elements to a thread: two 16-byte loads,
+// two 16-byte stores; the run that the end of a row cuts is read element by element.  Bound by memory traffic, 4 bytes read and
+// 4 written per element.
 __global__ __launch_bounds__(256) void gather_rows_split_kernel(const float* x, int64_t ldx, int64_t H, const int* perm,
-                                                                const int64_t* n_rows, int64_t N, int64_t Np,
-                                                                unsigned short* xc, int64_t ldxc, unsigned short* xk,
-                                                                int64_t ldxk, const float* lse, float* lse_c) {
+                                                                const int64_t* n_rows, int64_t N, unsigned short* xc,
+                                                                int64_t part, const float* lse, float* lse_c) {
   const int64_t rows = n_rows != nullptr ? packed_rows(n_rows, N) : N;
-  const int64_t jend = xk != nullptr ? Np : rows;
-  for (int64_t j = blockIdx.x; j < jend; j += gridDim.x) {
-    if (j >= rows) {  // K padding of the dW contraction
-      for (int64_t k = threadIdx.x; k < ldxk; k += 256)
-        xk[j * ldxk + k] = xk[(Np + j) * ldxk + k] = xk[(2 * Np + j) * ldxk + k] = 0;
-      continue;
-    }
+  for (int64_t j = blockIdx.x; j < rows; j += gridDim.x) {
     const int64_t src = perm != nullptr ? packed_token(perm, j, N) : j;
     if (lse != nullptr && threadIdx.x == 0) lse_c[j] = lse[src];
     const float* s = x + src * ldx;
-    unsigned short* c = xc + j * ldxc;
-    for (int64_t k = threadIdx.x; k < H; k += 256) {
-      const float v = s[k];
-      const unsigned short hi = to_bits<BF16>(v), lo = to_bits<BF16>(bf16_lo(v));
-      c[k] = hi;
-      c[H + k] = hi;
-      c[2 * H + k] = lo;
-      if (xk != nullptr) {
-        xk[j * ldxk + k] = hi;
-        xk[(Np + j) * ldxk + k] = hi;
-        xk[(2 * Np + j) * ldxk + k] = lo;
+    unsigned short* c = xc + j * 2 * part;
+    for (int64_t k = threadIdx.x * 8; k < part; k += 256 * 8) {
+      float v[8];
+      if (k + 8 <= H) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(s + k), b = *reinterpret_cast<const f32x4_t*>(s + k + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[i] = a[i];
+          v[4 + i] = b[i];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = k + i < H ? s[k + i] : 0.f;
       }
+      u32x4_t hi, lo;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        hi[i] = pack2<BF16>(v[2 * i], v[2 * i + 1]);
+        lo[i] = pack2<BF16>(bf16_lo(v[2 * i]), bf16_lo(v[2 * i + 1]));
+      }
+      *reinterpret_cast<u32x4_t*>(c + k) = hi;
+      *reinterpret_cast<u32x4_t*>(c + part + k) = lo;
     }
-    // stride padding is read by the tile kernels and must be finite
-    for (int64_t k = 3 * H + threadIdx.x; k < ldxc; k += 256) c[k] = 0;
-    if (xk != nullptr)
-      for (int64_t k = H + threadIdx.x; k < ldxk; k += 256)
-        xk[j * ldxk + k] = xk[(Np + j) * ldxk + k] = xk[(2 * Np + j) * ldxk + k] = 0;
   }
 }
 
@@ -332,12 +325,11 @@ hipError_t launch_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, fl
 }
 
 hipError_t launch_gather_rows_split(const float* x, int64_t ldx, int64_t H, const int* perm, const int64_t* n_rows,
-                                    int64_t N, void* xc, int64_t ldxc, void* xk, int64_t ldxk, const float* lse,
-                                    float* lse_c, int num_cus, hipStream_t s) {
-  const int64_t Np = padded_tokens(N);
-  hipLaunchKernelGGL(gather_rows_split_kernel, dim3(row_grid(Np, num_cus)), dim3(256), 0, s, x, ldx, H, perm, n_rows, N,
-                     Np, reinterpret_cast<unsigned short*>(xc), ldxc, reinterpret_cast<unsigned short*>(xk), ldxk, lse,
-                     lse_c);
+                                    int64_t N, void* xc, int64_t ldxc, const float* lse, float* lse_c, int num_cus,
+                                    hipStream_t s) {
+  if (ldxc % 16 != 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(gather_rows_split_kernel, dim3(row_grid(N, num_cus)), dim3(256), 0, s, x, ldx, H, perm, n_rows, N,
+                     reinterpret_cast<unsigned short*>(xc), ldxc / 2, lse, lse_c);
   return hipGetLastError();
 }
 

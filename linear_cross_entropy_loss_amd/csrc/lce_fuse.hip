@@ -213,7 +213,7 @@ hipError_t launch_scale_rows(void* t, int dtype, int64_t rows, int64_t cols, int
 }
 
 hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s) {
-  if (a.split || a.part_max == nullptr || a.tgt == nullptr || a.lse == nullptr) return hipErrorInvalidValue;
+  if (a.part_max == nullptr || a.tgt == nullptr || a.lse == nullptr) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(a.vs / 64), (unsigned)(a.Np / kTile));
   if (a.x_dtype == DT_BF16) hipLaunchKernelGGL(stage_scale_kernel<BF16>, grid, dim3(256), 0, s, a);
   else if (a.x_dtype == DT_F16) hipLaunchKernelGGL(stage_scale_kernel<F16>, grid, dim3(256), 0, s, a);
@@ -222,7 +222,7 @@ hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_stage_factors(const BwdArgs& a, hipStream_t s) {
-  if (a.split || a.v0 != 0 || a.part_max == nullptr || a.tgt == nullptr || a.lse == nullptr || a.dx_f == nullptr || a.dw_f == nullptr)
+  if (a.v0 != 0 || a.part_max == nullptr || a.tgt == nullptr || a.lse == nullptr || a.dx_f == nullptr || a.dw_f == nullptr)
     return hipErrorInvalidValue;
   const dim3 grid((unsigned)((a.vs / kChunkV + kSlices - 1) / kSlices), (unsigned)(a.Np / kTile));
   if (a.x_dtype == DT_BF16) hipLaunchKernelGGL(stage_factors_kernel<BF16>, grid, dim3(256), 0, s, a);

@@ -300,6 +300,9 @@ template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON> struct FwdProblem
   static constexpr bool kVarK = false;
   static constexpr bool kQBlocked = false;
   static constexpr bool kQScale = false;
+  static constexpr bool kSplit = is_pair<T>::value;
+  LCE_DEV int64_t p_lo() const { return a.H * a.ldw * 2; }
+  LCE_DEV int64_t q_lo() const { return a.x_lo * 2; }
   static constexpr bool kColumnEpilogue = !VTAIL;
   const FwdArgs& a;
   int64_t rows, ldx;
@@ -329,9 +332,9 @@ template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON> struct FwdProblem
     q = x + (a.row0 + (int64_t)tq * kTile) * ldx;
   }
   LCE_DEV const void* p_end() const {
-    return WVH ? matrix_end<E>(a.w, a.Vw, a.ldw, a.H) : matrix_end<E>(a.w, a.H, a.ldw, a.Vw);
+    return WVH ? matrix_end<E>(a.w, a.Vw, a.ldw, a.H) : matrix_end<E>(a.w, kSplit ? 2 * a.H : a.H, a.ldw, a.Vw);
   }
-  LCE_DEV const void* q_end() const { return matrix_end<E>(x, rows, ldx, a.H); }
+  LCE_DEV const void* q_end() const { return matrix_end<E>(x, rows, ldx, kSplit ? a.x_lo + a.H : a.H); }
   LCE_DEV int k_valid(int) const { return (int)a.H; }
   // Column epilogue: the labels of this lane's four tokens are fetched three K tiles ahead.
   int64_t pf_y[kNB];
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
     typedef FwdProblem<T, false, KMASK, WVH, MON> Full;
     Full prob(a);
     Pipe3<T, E, WVH, E, true, Full> pipe(prob);
-    if (TAIL == kNoTail || first < prob.num_tiles()) pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+    if (TAIL == kNoTail || first < prob.num_tiles()) pipe.run(a.ldw, prob.ldx, logit_ktiles<T>(a.H), lds, first);
     if (TAIL == kWithTail) first = first_tail_tile(first, (int)gridDim.x, prob.num_tiles());
   }
   if constexpr (TAIL != kNoTail) {
@@ -397,7 +400,7 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
     if (first >= prob.num_tiles()) return;
     __syncthreads();  // (every wave is done with the main loop's LDS stages)
     Pipe3<T, E, WVH, E, true, Tail> pipe(prob);
-    pipe.run(a.ldw, prob.ldx, (int)(padded_k(a.H) / kBK), lds, first);
+    pipe.run(a.ldw, prob.ldx, logit_ktiles<T>(a.H), lds, first);
   }
 }
 
@@ -627,7 +630,7 @@ hipError_t launch_one(const FwdArgs& a, int64_t tiles, hipStream_t s) {
 template <class T, bool WVH, bool MON> hipError_t launch_persistent(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;  // token tiles of this chunk at most
   const int64_t tq = (left < a.nc ? left : a.nc) / kTile, full = a.vw / kTile;
-  const bool exact_k = padded_k(a.H) == a.H;  // the K tiles cover H exactly: no K mask needed
+  const bool exact_k = (is_pair<T>::value ? padded_k_pair(a.H) : padded_k(a.H)) == a.H;  // the K tiles cover H exactly: no K mask needed
   const bool tail = a.vw % kTile != 0;        // a column that straddles V
   if (full == 0) return launch_one<T, kTailOnly, true, WVH, MON>(a, tq, s);
   if (tail)
@@ -647,7 +650,8 @@ hipError_t launch_fwd_tiles(const FwdArgs& a, hipStream_t s) {
     return a.w_vh ? launch_layout<BF16, true>(a, s) : launch_layout<BF16, false>(a, s);
   if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16)
     return a.w_vh ? launch_layout<F16, true>(a, s) : launch_layout<F16, false>(a, s);
-  // (an fp32 weight arrives here as a 16-bit slab copy, fp32 activations as the bf16 packed copy)
+  if (a.x_dtype == DT_PAIR && a.w_dtype == DT_PAIR && !a.w_vh) return launch_layout<BF16P, false>(a, s);
+  // (an fp32 weight arrives here as a copy in the compute type, fp32 activations as the packed copy in pairs)
   return hipErrorInvalidValue;
 }
 

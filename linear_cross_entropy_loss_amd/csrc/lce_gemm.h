@@ -49,16 +49,21 @@ constexpr int kMainloopLds = 2 * kStageBytes;      // double buffered: 128 KiB
 
 struct BF16 {};
 struct F16 {};
+struct BF16P {};  // fp32 values as bf16 pairs (below)
+template <class T> struct is_pair { static constexpr bool value = false; };
+template <> struct is_pair<BF16P> { static constexpr bool value = true; };
 
 template <class T> struct elem_of;
 template <> struct elem_of<BF16> { typedef __bf16 type; };
 template <> struct elem_of<F16> { typedef _Float16 type; };
+template <> struct elem_of<BF16P> { typedef __bf16 type; };
 
 template <class T> LCE_DEV f32x16_t mfma32(s16x8_t a, s16x8_t b, f32x16_t c);
 template <> LCE_DEV f32x16_t mfma32<BF16>(s16x8_t a, s16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
                                                  __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
+template <> LCE_DEV f32x16_t mfma32<BF16P>(s16x8_t a, s16x8_t b, f32x16_t c) { return mfma32<BF16>(a, b, c); }
 template <> LCE_DEV f32x16_t mfma32<F16>(s16x8_t a, s16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
                                                 __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
@@ -81,8 +86,8 @@ template <class T> LCE_DEV unsigned int pack2(float lo, float hi) {
 }
 // fp32 operands are carried as two bf16 numbers, v = hi + lo with hi = bf16(v) and lo = bf16(v - hi): 16
 // bits of mantissa instead of 8.  A product a*b is then taken as a_hi*b_hi + a_hi*b_lo + a_lo*b_hi (the
-// a_lo*b_lo term is of relative order 2^-18 and dropped), which the kernels get by running along a K axis
-// that is three times as long, over copies of the operands laid out as [hi | hi | lo] and [hi | lo | hi].
+// a_lo*b_lo term is of relative order 2^-18 and dropped), which the kernels get by going through every K tile
+// three times, over the parts of the operands that the term names (lce_gemm3.h, Problem::kSplit).
 LCE_DEV float bf16_hi(float v) {
   return __builtin_bit_cast(float, (unsigned)to_bits<BF16>(v) << 16);
 }

@@ -26,6 +26,7 @@
 #pragma once
 
 #include "lce_gemm.h"
+#include "lce_internal.h"
 
 namespace lce {
 
@@ -91,13 +92,14 @@ template <class T, class SrcT, bool KC, bool KMASK> struct Stager3 {
   // contiguous block of 128-byte rows, and the next K tile is the next block.  Otherwise (its rows are the K
   // index): the tile's 256 columns are four consecutive blocks, each thread stays in one; a K tile is 64 rows of
   // them, and after four K tiles the stream moves on to the next row of blocks (Pipe3::stream_advance).
-  LCE_DEV void init_blocked() {
+  // (`parts` = 2: every block is followed by the block of its lo part)
+  LCE_DEV void init_blocked(int parts) {
     init(kBK);
     if (KC) {
-      k_stride = kTile * (kBK * kEs);
+      k_stride = parts * kTile * (kBK * kEs);
     } else {
       const int t = threadIdx.x, c = t & 31, k = t >> 5;
-      voff = (unsigned)((c >> 3) * (kTile * kBK * kEs) + k * (kBK * kEs) + (c & 7) * 16);
+      voff = (unsigned)((c >> 3) * parts * (kTile * kBK * kEs) + k * (kBK * kEs) + (c & 7) * 16);
       voff_cur = voff;
       iter_stride = (unsigned)(8 * kBK * kEs);
       k_stride = (int64_t)kBK * kBK * kEs;
@@ -155,6 +157,11 @@ template <class S> LCE_DEV const void* matrix_end(const void* base, int64_t rows
   return reinterpret_cast<const S*>(base) + (rows - 1) * ld + c;
 }
 
+// K tiles of the logit contraction.
+template <class T> LCE_DEV int logit_ktiles(int64_t H) {
+  return (int)(is_pair<T>::value ? 3 * padded_k_pair(H) / kBK : padded_k(H) / kBK);
+}
+
 // What a kernel plugs into the persistent loop.
 //   int  num_tiles()                              output tiles in this launch
 //   void origins(int tile, const void*& p, const void*& q)
@@ -168,6 +175,13 @@ template <class S> LCE_DEV const void* matrix_end(const void* base, int64_t rows
 //        of P block i and Q block j, with Q along its registers and P along its lanes)
 //   void prefetch(int tile)                       called three K tiles before the tile's epilogue: the place to issue loads
 //        of per-row data the epilogue starts with (kept in members), so that their latency is not exposed there
+//   static constexpr bool kSplit                  true if both operands are bf16 pairs, stored as two parts each: a K tile is
+//        then multiplied three times in a row, as (P hi, Q hi), (P hi, Q lo), (P lo, Q hi), `ktiles` counts all three,
+//        and a blocked Q operand has the block of its lo part behind each block of its hi part
+//        (one contraction whose stream comes back to the same K tile, instead of copies of the operands with their hi parts
+//        twice and K three times as long, or three launches that add to a sum in memory: fp32 forward + backward, N=2048,
+//        H=2048, V=16384 2276 -> 1434 us, N=6784, H=333, V=93824 10.4 -> 6.1 ms; the parts a K tile needs again are in cache)
+//   int64_t p_lo(), q_lo()                        bytes from an operand's hi part to its lo part
 //   static constexpr bool kQScale                 true if the (blocked) Q operand is multiplied on its way to LDS: by one fp32
 //        factor per row of the stage and slice of 128 columns, rounded once to the operand type.  The eight factors of a
 //        thread's chunks of a K tile lie next to each other; then
@@ -216,6 +230,9 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
   static constexpr bool kQRowBlocks = Problem::kQBlocked && !Q_KC;
   // Problem::kQScale: the factors of the K tile in the staging set and of the one after it ([LDS stage of the K tile]), and where
   // those of the K tile being loaded are.
+  static constexpr bool kSplit = Problem::kSplit;
+  int split_s;         // kSplit: which of the K tile's three products the stream is at
+  int64_t p_lo, q_lo;  // and the bytes to the lo parts
   static constexpr bool kQScale = Problem::kQScale;
   f32x4_t qfac[2][2];
   const float* qfac_base;
@@ -255,6 +272,7 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
       qs.end = qs.base;
     }
     k_rem = prob.k_valid(tile);
+    if constexpr (kSplit) split_s = 0;
     if constexpr (kQScale) {
       qfac_base = prob.q_factors(tile);
       qfac_k = 0;
@@ -264,6 +282,18 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
     qs.retarget(k_rem);
   }
   LCE_DEV void stream_advance() {
+    if constexpr (kSplit) {
+      if (split_s != 2) {
+        ps.base += split_s == 0 ? 0 : p_lo;
+        qs.base += split_s == 0 ? q_lo : -q_lo;
+        ++split_s;
+        ps.retarget(k_rem);
+        qs.retarget(k_rem);
+        return;
+      }
+      ps.base -= p_lo;
+      split_s = 0;
+    }
     ps.base += ps.k_stride;
     if constexpr (kQRowBlocks) {
       qs.base += q_phase == 3 ? q_jump : qs.k_stride;
@@ -506,10 +536,10 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
     const int wave = threadIdx.x >> 6;
     ps.init(ldp);
     if constexpr (Problem::kQBlocked) {
-      qs.init_blocked();
+      qs.init_blocked(kSplit ? 2 : 1);
       // (ldq: column groups per row of blocks) what takes a stream whose K index is the rows from the last K tile of
       // a row of blocks to the first of the next
-      q_jump = ldq * (kTile * kBK * QStager::kEs) - 3 * qs.k_stride;
+      q_jump = ldq * ((kSplit ? 2 : 1) * kTile * kBK * QStager::kEs) - 3 * qs.k_stride;
     } else {
       qs.init(ldq);
     }
@@ -518,6 +548,10 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
 
     PRegs sp;
     QRegs sq;
+    if constexpr (kSplit) {
+      p_lo = prob.p_lo();
+      q_lo = prob.q_lo();
+    }
     if constexpr (kQScale) qfac_off = prob.q_factor_offset();
     stream_begin(first);
     load_chunks(sp, sq, 0, 16);

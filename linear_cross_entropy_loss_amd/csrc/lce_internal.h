@@ -10,6 +10,8 @@
 namespace lce {
 
 enum { DT_BF16 = 0, DT_F16 = 1, DT_F32 = 2 };
+// Compute type of fp32 tensors inside the library: bf16 pairs (lce_gemm.h).
+enum { DT_PAIR = 3 };
 
 // The tile kernels use more dynamic LDS than a kernel gets by default and have to opt in
 // (hipFuncAttributeMaxDynamicSharedMemorySize): once per kernel and device, not before every launch.  One object
@@ -43,6 +45,11 @@ constexpr int64_t padded_hidden(int64_t H) { return pad_to(H, 256); }   // hidde
 // K extent of the logit contraction: an even number of 64-wide K tiles, at least four
 constexpr int64_t padded_k(int64_t H) { return pad_to(H, 128) < 256 ? 256 : pad_to(H, 128); }
 
+// Pairs: three K tiles for each of these 64-wide ones, so two of them are enough
+constexpr int64_t padded_k_pair(int64_t H) { return pad_to(H, 128); }
+// Matrix products per K tile of the compute type.
+constexpr int products_of(int dtype) { return dtype == DT_PAIR ? 3 : 1; }
+
 // Which tile columns of the vocabulary a logit kernel covers: full ones, the one(s) from the column that straddles the end of
 // the vocabulary on, or both.
 enum { kNoTail = 0, kTailOnly = 1, kWithTail = 2 };
@@ -63,7 +70,9 @@ struct FwdArgs {
   // w_vh != 0: the weight is stored with the vocabulary as its row index, w[v * ldw + h] (the buffer `w` then
   // holds ROWS [wv0, wv0 + Vw)); otherwise w[h * ldw + v].
   int w_vh;
-  int x_dtype, w_dtype;  // compute type = x_dtype (bf16 / f16)
+  int x_dtype, w_dtype;  // compute type = x_dtype (bf16 / f16 / pairs)
+  // Pairs: x is rows of [hi | lo], the lo part x_lo elements behind the hi part, and w is H rows of hi, then H rows of lo.
+  int64_t x_lo;
   int64_t ignore_index;
   float scale, z_reg;
   int monitoring;
@@ -99,7 +108,8 @@ struct BwdArgs {
   const float* grad_out;
   int64_t N, H, V, ldx, ldw, lddx, lddw;
   int64_t Np, Hp;  // padded_tokens(N), padded_hidden(H)
-  int x_dtype, w_dtype, dx_dtype, dw_dtype;
+  int x_dtype, w_dtype, dx_dtype, dw_dtype;  // compute type = x_dtype, as in FwdArgs
+  int64_t x_lo;  // pairs, as in FwdArgs
   int64_t ignore_index;
   float scale, z_reg;
   void* dx;
@@ -114,8 +124,8 @@ struct BwdArgs {
   // Staged dz in the compute type (exact zeros outside N x vw), stored in blocks of 256 rows x 64 columns,
   // [rows / 256][vs / 64][256][64] (dz_block_offset below): the 64-deep K tiles of the dx contraction (K = v) are
   // consecutive 32 KiB blocks, the K tiles of the dW contraction (K = tokens) quarters of four neighbouring blocks,
-  // and a token's 64 columns of a group are one 128-byte line.  dz_rows = Np rows, or 3 Np when dz is carried as
-  // bf16 pairs (`split` below).
+  // and a token's 64 columns of a group are one 128-byte line.  dz_rows = Np rows.  Pairs: the block of the lo parts follows
+  // each block of hi parts.
   void* dz;
   int64_t dz_rows;
   float* dx_acc;    // [Np][Hp] fp32 running dx (null when there is a single slab)
@@ -138,10 +148,6 @@ struct BwdArgs {
   int first, last;  // slab position
   int num_cus;      // compute units of the device: grid size of the persistent kernels
   int live;         // bwd_dz: bands of W that the XCDs keep in flight together (lce_gemm.h, tile_coords)
-  // fp32 tensors carried as bf16 pairs (lce_gemm.h): the stage holds three parts of Np rows each, [hi ; lo ; hi];
-  // only bwd_dz looks at this flag (the dx and dW launches get plain 16-bit problems over these parts: dx with `dz`
-  // pointing at the first row of a part, dW with 3 Np token rows).
-  int split;
   // Packed rows (tokens with an ignored label dropped; n_rows == null: the call works on all rows).
   // *n_rows (device) rows are worked on.  When *n_rows != N they are the rows of xc (row stride ldxc) and
   // row j of dx belongs to token perm[j]: the dx kernels store it there themselves, or -- dxc != null, a dx
@@ -220,9 +226,9 @@ hipError_t launch_scale_rows(void* t, int dtype, int64_t rows, int64_t cols, int
 hipError_t launch_bwd_dx(const BwdArgs& a, hipStream_t s);
 hipError_t launch_bwd_dw(const BwdArgs& a, hipStream_t s);
 // dst[h][c] = 16-bit rounding of src[h * ld + v0 + c] for c < vw, 0 for vw <= c < dst_ld; h < H.
-// compute_dtype: DT_BF16 or DT_F16.  split: dst has 3 H rows, [bf16 hi ; bf16 lo ; bf16 hi] of the fp32 values.
+// compute_dtype: DT_BF16, DT_F16 or DT_PAIR: dst then has 2 H rows, [bf16 hi ; bf16 lo] of the fp32 values.
 hipError_t launch_convert_w_slab(const float* src, int64_t ld, int64_t H, int64_t v0, int64_t vw, void* dst,
-                                 int64_t dst_ld, int compute_dtype, bool split, hipStream_t s);
+                                 int64_t dst_ld, int compute_dtype, hipStream_t s);
 // The same for a weight stored (V, H) row-major (H a multiple of 8): rows [v0, v0 + vw) go to dst[vw][dst_ld].
 hipError_t launch_convert_w_rows(const float* src, int64_t ld, int64_t H, int64_t v0, int64_t vw, void* dst,
                                  int64_t dst_ld, int compute_dtype, hipStream_t s);
@@ -261,13 +267,12 @@ hipError_t launch_compact_labels(const int64_t* y, int64_t N, int64_t ignore_ind
 hipError_t launch_gather_rows(const void* x, int64_t ldx_bytes, int64_t row_bytes, const int* perm,
                               const int64_t* n_rows, int64_t N, void* xc, int64_t ldxc_bytes, const float* lse,
                               float* lse_c, int num_cus, hipStream_t s, bool always = false);
-// fp32 activations: xc[j] = [hi | hi | lo] of x[perm[j]] as bf16 (3 H elements per row, row stride ldxc), and
-// -- xk not null -- the same three parts stacked along the tokens, xk[b * Np + j] (row stride ldxk, rows from
-// *n_rows to Np of each block zeroed).  Always made, also when no token is dropped; perm / n_rows may be null
-// (all N rows in their order).  Strides in elements.
+// fp32 activations: xc[j] = [hi | lo] of x[perm[j]] as bf16 pairs, each part half of the row stride ldxc (a multiple of 16)
+// and zero-padded to it.  Always made, also when no token is dropped; perm / n_rows may be null (all N rows in their
+// order).  Strides in elements; rows of x on 16-byte boundaries.
 hipError_t launch_gather_rows_split(const float* x, int64_t ldx, int64_t H, const int* perm, const int64_t* n_rows,
-                                    int64_t N, void* xc, int64_t ldxc, void* xk, int64_t ldxk, const float* lse,
-                                    float* lse_c, int num_cus, hipStream_t s);
+                                    int64_t N, void* xc, int64_t ldxc, const float* lse, float* lse_c, int num_cus,
+                                    hipStream_t s);
 // dx[perm[j]] = dxc[j] for j < *n_rows (skipped when dxc is null) and dx[i] = 0 for every token i with
 // y[i] == ignore_index, in 8-byte pieces covering row_bytes; nothing when *n_rows == N.
 hipError_t launch_scatter_rows(const void* dxc, int64_t lddxc_bytes, const int* perm, const int64_t* n_rows,
@@ -293,8 +298,9 @@ inline int64_t max_k_segments(int64_t kt) {
   while (kt / (s * 2) >= 16 && s * 2 <= kTailBlocks) s *= 2;
   return s;
 }
-inline int64_t dx_tail_blocks(int64_t Np, int64_t Hp, int64_t vs) {
-  const int64_t s = max_k_segments(vs / 64);
+// (`products`: products_of the compute type)
+inline int64_t dx_tail_blocks(int64_t Np, int64_t Hp, int64_t vs, int products) {
+  const int64_t s = max_k_segments(products * vs / 64);
   if (s == 1) return 0;
   const int64_t most = (Np / 256) * (Hp / 256) * s;
   return most < kTailBlocks ? most : kTailBlocks;
@@ -310,11 +316,11 @@ inline bool all_tiles_are_tails(int64_t T, int64_t G, int64_t kt) {
   return T < G && has_split_tail(T, G) && kt / 2 >= 16;
 }
 // true if every split the dx kernel may choose cuts the K tiles of a slab into equal, even segments
-inline bool dx_segments_exact(int64_t vs) { return (vs / 64) % (2 * max_k_segments(vs / 64)) == 0; }
+inline bool dx_segments_exact(int64_t vs, int products) { return (vs / 64) % (2 * max_k_segments(products * vs / 64)) == 0; }
 // dW of one slab: (vs/256) x (Hp/256) tiles, K = at most Np tokens.  The same bound for the dW kernel, whose
 // segments need not divide the K tiles evenly.
-inline int64_t dw_tail_blocks(int64_t Np, int64_t Hp, int64_t vs) {
-  const int64_t s = max_k_segments(Np / 64);
+inline int64_t dw_tail_blocks(int64_t Np, int64_t Hp, int64_t vs, int products) {
+  const int64_t s = max_k_segments(products * Np / 64);
   if (s == 1) return 0;
   const int64_t most = (vs / 256) * (Hp / 256) * s;
   return most < kTailBlocks ? most : kTailBlocks;
