@@ -205,7 +205,7 @@ double kernel_cost(double T, double L, double e, bool parts) {
   double cost = full * (L + e) + 10.0;
   if (r > 0) {
     double seg = 1;
-    if (parts) while (r * seg * 2 <= kPlanCUs && L / (seg * 2) >= 16) seg *= 2;
+    if (parts) seg = lce::k_segments((int)r, (int)kPlanCUs, (int)L);
     const double f = r * seg / kPlanCUs;
     cost += (L / seg + e) / (1.0 + 0.9 * (1.0 - f)) + (seg > 1 ? 12.0 : 0.0);
   }
@@ -477,7 +477,8 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
   // The two-pass route by the same model: the forward over all tokens, then the backward's plan.  It wins where the
   // scratch bound leaves only short chunks (every chunk adds a round trip of all the fp32 sums of dW).
   BwdPlan b;
-  const double scale_pass = (double)Np * (double)Vp * (f->factors ? 16.0 / lce::kChunkV : 4.0) / 8.0e6;
+  // (the factors instead: hardly any traffic, but a launch of some 15 us per chunk that starts from cold)
+  const double scale_pass = f->factors ? 12.0 * (double)f->chunks : (double)Np * (double)Vp * 4.0 / 8.0e6;
   f->cost = best + scale_pass;
   if ((p->route & ~LCE_ROUTE_EXACT_SUMS) == LCE_ROUTE_AUTO && plan_bwd(p, &b) == LCE_OK) {
     const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false) + b.cost;

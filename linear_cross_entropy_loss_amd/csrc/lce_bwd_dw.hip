@@ -453,12 +453,12 @@ LCE_DEV void dw_epilogue_f32_sum(const BwdArgs& a, f32x16_t (&acc)[kNB][kNB], in
 
 // How one launch divides its work: as for dx (lce_bwd_dx.hip).  The T = (vs/256) x (Hp/256) output tiles
 // go to G persistent workgroups in rounds; a last round with r <= G/2 tiles is cut along K = tokens into
-// `nseg` segments of `kseg` K tiles (r * nseg <= G, at least 16 K tiles each), whose fp32 sums meet in
+// `nseg` segments (r * nseg <= G, at least 16 K tiles each), whose fp32 sums meet in
 // 256 x 256 blocks of dw_part and are added, in segment order, by dw_tail_kernel.  With few tiles in all
 // (a small vocabulary slab times a small hidden size) every tile is a tail tile.  The K extent comes from
 // the row count on the device, so the plan is made there; the segments cover the K tiles exactly.
 struct DwPlan {
-  int tiles, full, tail_tiles, nseg, kseg, kt;
+  int tiles, full, tail_tiles, nseg, kt;
 };
 template <class T> LCE_DEV DwPlan dw_plan(const BwdArgs& a, int64_t rows) {
   DwPlan p;
@@ -467,22 +467,11 @@ template <class T> LCE_DEV DwPlan dw_plan(const BwdArgs& a, int64_t rows) {
   p.kt = (int)(kt2 < 4 ? 4 : kt2);
   p.tiles = (int)(a.vs / kTile) * (int)(a.Hp / kTile);
   p.full = p.tiles / G * G;
-  const int r = p.tiles - p.full, cap = G < kTailBlocks ? G : kTailBlocks;
-  int s = 1;
-  if (r > 0 && a.dw_part != nullptr)  // (no blocks for partial sums: nothing is split)
-    while (r * s * 2 <= cap && (is_pair<T>::value ? 3 : 1) * p.kt / (s * 2) >= 16) s *= 2;
-  if (s == 1) {
-    p.full = p.tiles;
-    p.tail_tiles = 0;
-    p.nseg = 1;
-    p.kseg = p.kt;
-  } else {
-    // s segments that cover the K tiles exactly: an even number each, the last one takes what is left over
-    // (fewer than 2 s K tiles more than the others)
-    p.tail_tiles = r;
-    p.kseg = (p.kt / s) & ~1;
-    p.nseg = s;
-  }
+  const int r = p.tiles - p.full;
+  // (no blocks for partial sums: nothing is split)
+  p.nseg = a.dw_part != nullptr ? k_segments(r, G, (is_pair<T>::value ? 3 : 1) * p.kt) : 1;
+  p.tail_tiles = p.nseg > 1 ? r : 0;
+  if (p.nseg == 1) p.full = p.tiles;
   return p;
 }
 
@@ -541,13 +530,13 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
     const int item = first + local, products = kSplit ? 3 : 1;
     if (item < plan.full) return products * plan.kt;
     const int seg = (item - plan.full) % plan.nseg;
-    return products * (seg == plan.nseg - 1 ? plan.kt - seg * plan.kseg : plan.kseg);
+    return products * (segment_start(seg + 1, plan.nseg, plan.kt) - segment_start(seg, plan.nseg, plan.kt));
   }
   LCE_DEV const float* q_factors(int local) const {
     if (local >= count) return a.dw_f;
     int item, tp, tq, seg;
     decode(local, item, tp, tq, seg);
-    return a.dw_f + (int64_t)tq * (kTile / kChunkV) * a.nc + (seg < 0 ? 0 : (int64_t)seg * plan.kseg * kBK);
+    return a.dw_f + (int64_t)tq * (kTile / kChunkV) * a.nc + (seg < 0 ? 0 : (int64_t)segment_start(seg, plan.nseg, plan.kt) * kBK);
   }
   LCE_DEV unsigned q_factor_offset() const {
     const unsigned t = threadIdx.x;
@@ -557,7 +546,7 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
   LCE_DEV void origins(int local, const void*& p, const void*& q) const {
     int item, tp, tq, seg;
     decode(local, item, tp, tq, seg);
-    const int64_t k0 = seg < 0 ? 0 : (int64_t)seg * plan.kseg * kBK;  // first token of the segment
+    const int64_t k0 = seg < 0 ? 0 : (int64_t)segment_start(seg, plan.nseg, plan.kt) * kBK;  // first token of the segment
     p = x + k0 * ldx + (int64_t)tp * kTile;
     q = reinterpret_cast<const E*>(a.dz) + (kSplit ? 2 : 1) * dz_block_offset(k0 / kTile, (int64_t)tq * (kTile / kBK), a.vs) +
         (k0 % kTile) * kBK;
@@ -566,7 +555,7 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
   LCE_DEV int q_phase(int local) const {
     int item, tp, tq, seg;
     decode(local, item, tp, tq, seg);
-    return seg < 0 ? 0 : (seg * plan.kseg) & 3;
+    return seg < 0 ? 0 : segment_start(seg, plan.nseg, plan.kt) & 3;
   }
   // x rows past the last one read as zeros.  dz is written for whole token tiles of 256 rows, and the K tiles of
   // the plan end with the pair of K tiles that holds the last row (dw_plan), so none of them reaches past
@@ -709,8 +698,7 @@ template <class T, bool WVH> hipError_t launch_persistent(const BwdArgs& a, hipS
     if (e == hipSuccess && tails) e = launch_tiles<T, false, kDwTails>(a, s);
   }
   if (e != hipSuccess || !tails) return e;
-  // at most dw_grid / 2 tail tiles can be split (two segments each)
-  const unsigned tail_most = (unsigned)(a.dw_grid / 2 > 0 ? a.dw_grid / 2 : 1);
+  const unsigned tail_most = (unsigned)((a.vs / kTile) * (a.Hp / kTile) % a.dw_grid);
   hipLaunchKernelGGL((dw_tail_kernel<T, WVH>), dim3(tail_most * kTailParts), dim3(256), 0, s, a);
   return hipGetLastError();
 }

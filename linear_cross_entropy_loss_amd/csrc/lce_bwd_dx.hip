@@ -118,34 +118,26 @@ LCE_DEV void dx_store_segment(float* part, f32x16_t (&acc)[kNB][kNB]) {
 
 // How one launch divides its work.  The output tiles (T of them, from the row count on the device) go to G
 // persistent workgroups in rounds of G.  A last round that would keep only r < G workgroups busy is cut along K
-// instead: its r tiles are split into `nseg` segments of `kseg` K tiles each (a power of two, r * nseg <= G, at
-// least 16 K tiles per segment), one work item per (tile, segment), so that the round is 1/nseg as long and
-// nearly all workgroups take part.  The segments' fp32 partial sums go to dx_part, one 256 x 256 block per
+// instead: its r tiles are split into `nseg` segments each (r * nseg <= G, at least 16 K tiles per segment),
+// one work item per (tile, segment), so that the round is 1/nseg as long and nearly all workgroups take part.
+// (Any number of segments, not only powers of two: N=8192, H=768, V=50257, where a chunk's 48 tiles are cut in five on 240
+// of 256 compute units and not in four on 192: 320 -> 288 us a launch.)  The segments' fp32 partial sums go to dx_part, one 256 x 256 block per
 // item, and dx_tail_kernel adds them in segment order -- deterministic, no atomics.  With few tiles in total
 // (small token counts) every tile is such a tail tile.
 struct DxPlan {
-  int tiles, full, tail_tiles, nseg, kseg;  // items [0, full) are whole tiles, then tail_tiles * nseg segment items
+  int tiles, full, tail_tiles, nseg, kt;  // items [0, full) are whole tiles, then tail_tiles * nseg segment items
 };
 template <class T> LCE_DEV DxPlan dx_plan(const BwdArgs& a, int tiles) {
   DxPlan p;
-  const int G = a.dx_grid, kt = (int)(a.vs / kBK);
+  const int G = a.dx_grid;
+  p.kt = (int)(a.vs / kBK);
   p.tiles = tiles;
   p.full = tiles / G * G;
-  const int r = tiles - p.full, cap = G < kTailBlocks ? G : kTailBlocks;
-  int s = 1;
-  if (r > 0 && a.dx_part != nullptr)  // (no blocks for partial sums: nothing is split)
-    while (r * s * 2 <= cap && (is_pair<T>::value ? 3 : 1) * kt / (s * 2) >= 16) s *= 2;
-  if (s == 1) {
-    p.full = tiles;
-    p.tail_tiles = 0;
-    p.nseg = 1;
-    p.kseg = kt;
-  } else {
-    // an even number of K tiles per segment; a last segment that runs past the slab is masked (K mask)
-    p.tail_tiles = r;
-    p.kseg = ((kt + s - 1) / s + 1) & ~1;
-    p.nseg = (kt + p.kseg - 1) / p.kseg;
-  }
+  const int r = tiles - p.full;
+  // (no blocks for partial sums: nothing is split)
+  p.nseg = a.dx_part != nullptr ? k_segments(r, G, (is_pair<T>::value ? 3 : 1) * p.kt) : 1;
+  p.tail_tiles = p.nseg > 1 ? r : 0;
+  if (p.nseg == 1) p.full = tiles;
   return p;
 }
 
@@ -191,7 +183,10 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
     }
     tile_coords(tile, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
   }
-  LCE_DEV int item_ktiles(int) const { return kSplit ? 3 * plan.kseg : plan.kseg; }
+  LCE_DEV int item_ktiles(int local) const {
+    const int seg = local % plan.nseg;  // (segment items only)
+    return (kSplit ? 3 : 1) * (segment_start(seg + 1, plan.nseg, plan.kt) - segment_start(seg, plan.nseg, plan.kt));
+  }
   // (a K tile is half a slice of 128 columns; work items start at even K tiles)
   LCE_DEV const float* q_factors(int local) const {
     if (local >= count) return a.dx_f;
@@ -202,7 +197,7 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
   LCE_DEV unsigned q_factor_offset() const { return (threadIdx.x >> 3) * 32; }
   LCE_DEV int64_t q_factor_step(int k) const { return (k & 1) ? a.nc : 0; }
   LCE_DEV void prefetch(int) {}
-  LCE_DEV int64_t k0_of(int seg) const { return seg < 0 ? 0 : (int64_t)seg * plan.kseg * kBK; }
+  LCE_DEV int64_t k0_of(int seg) const { return seg < 0 ? 0 : (int64_t)segment_start(seg, plan.nseg, plan.kt) * kBK; }
   LCE_DEV void origins(int local, const void*& p, const void*& q) const {
     int item, tp, tq, seg;
     decode(local, item, tp, tq, seg);
@@ -214,9 +209,7 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
   LCE_DEV const void* p_end() const {
     return WVH ? matrix_end<E>(a.w, a.Vw, a.ldw, a.H) : matrix_end<E>(a.w, kSplit ? 2 * a.H : a.H, a.ldw, a.Vw);
   }
-  // (only whole token tiles that were written are read.  K tiles past the slab -- the last segment of a split tail
-  // tile may have some -- lie in the next row of blocks, or past the stage: the K mask gives those threads an
-  // out-of-range offset, the other operand's are zeros)
+  // (only whole token tiles that were written are read)
   LCE_DEV const void* q_end() const { return reinterpret_cast<const E*>(a.dz) + (kSplit ? 2 : 1) * a.dz_rows * a.vs; }
   LCE_DEV int k_valid(int local) const {
     int item, tp, tq, seg;
@@ -244,7 +237,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dx_persistent_kernel(const BwdAr
   typedef DxProblem<T, KMASK, WVH, MODE, SCALE> Problem;
   Problem prob(a);
   Pipe3<T, E, !WVH, E, true, Problem> pipe(prob);
-  pipe.run(a.ldw, a.vs / kBK, (is_pair<T>::value ? 3 : 1) * (MODE == kDxTails ? prob.plan.kseg : (int)(a.vs / kBK)), lds, (int)blockIdx.x);
+  pipe.run(a.ldw, a.vs / kBK, (is_pair<T>::value ? 3 : 1) * (int)(a.vs / kBK), lds, (int)blockIdx.x);
 }
 
 // Second step for the tail tiles: kTailParts workgroups share tail tile b (16 rows each) -- they sum its
@@ -328,8 +321,8 @@ template <class T> hipError_t launch_persistent(const BwdArgs& a, hipStream_t s)
   // it is decided on the device, and a launch without items returns at once.
   const bool tails = a.dx_part != nullptr && dx_tail_blocks(a.Np, a.Hp, a.vs, products_of(a.x_dtype)) != 0 &&
                      (a.n_rows != nullptr || has_split_tail((a.Np / kTile) * (a.Hp / kTile), a.dx_grid));
-  // the K mask is only needed when the K tiles of a work item can run past the columns that exist
-  const bool exact_k = a.vw == a.vs && dx_segments_exact(a.vs, products_of(a.x_dtype));
+  // the K mask is only needed when the K tiles run past the columns that exist
+  const bool exact_k = a.vw == a.vs;
   hipError_t e;
   if constexpr (is_pair<T>::value)
     e = exact_k ? launch_layout<T, false, false>(a, tails, s) : launch_layout<T, true, false>(a, tails, s);
@@ -337,8 +330,9 @@ template <class T> hipError_t launch_persistent(const BwdArgs& a, hipStream_t s)
     e = a.w_vh ? (exact_k ? launch_layout<T, false, true>(a, tails, s) : launch_layout<T, true, true>(a, tails, s))
                         : (exact_k ? launch_layout<T, false, false>(a, tails, s) : launch_layout<T, true, false>(a, tails, s));
   if (e != hipSuccess || !tails) return e;
-  // at most dx_grid / 2 tail tiles can be split (two segments each)
-  const unsigned tail_most = (unsigned)(a.dx_grid / 2 > 0 ? a.dx_grid / 2 : 1);
+  // at most dx_grid / 2 tail tiles can be split (two segments each); without packed rows their number is known here
+  const unsigned tail_most = a.n_rows == nullptr ? (unsigned)((a.Np / kTile) * (a.Hp / kTile) % a.dx_grid)
+                                                 : (unsigned)(a.dx_grid / 2 > 0 ? a.dx_grid / 2 : 1);
   hipLaunchKernelGGL(dx_tail_kernel<T>, dim3(tail_most * kTailParts), dim3(256), 0, s, a);
   return hipGetLastError();
 }

@@ -293,10 +293,23 @@ inline int live_bands(int64_t k_bytes) {
 // blocks of partial sums that the device-side plan of the dx kernel can ask for (0: it never splits).
 constexpr int kTailBlocks = 256;
 // most segments per tile: a power of two that leaves at least 16 K tiles per segment
-inline int64_t max_k_segments(int64_t kt) {
+__host__ __device__ inline int64_t max_k_segments(int64_t kt) {
   int64_t s = 1;
   while (kt / (s * 2) >= 16 && s * 2 <= kTailBlocks) s *= 2;
   return s;
+}
+// Segments that each of r tiles with kt K tiles is cut into on G workgroups: as many as keep every workgroup busy once.  (1: not
+// cut.)
+__host__ __device__ inline int k_segments(int r, int G, int kt) {
+  const int cap = G < kTailBlocks ? G : kTailBlocks;
+  if (r <= 0 || 2 * r > cap) return 1;
+  const int s = cap / r, most = (int)max_k_segments(kt);
+  return s < most ? s : most;
+}
+// A segment's K tiles, of kt (an even number) in s segments: even numbers of them, as equal as that goes.
+__host__ __device__ inline int segment_start(int seg, int s, int kt) {
+  const int base = kt / 2 / s, rest = kt / 2 - base * s;
+  return 2 * (seg * base + (seg < rest ? seg : rest));
 }
 // (`products`: products_of the compute type)
 inline int64_t dx_tail_blocks(int64_t Np, int64_t Hp, int64_t vs, int products) {
@@ -315,10 +328,7 @@ inline bool has_split_tail(int64_t T, int64_t G) {
 inline bool all_tiles_are_tails(int64_t T, int64_t G, int64_t kt) {
   return T < G && has_split_tail(T, G) && kt / 2 >= 16;
 }
-// true if every split the dx kernel may choose cuts the K tiles of a slab into equal, even segments
-inline bool dx_segments_exact(int64_t vs, int products) { return (vs / 64) % (2 * max_k_segments(products * vs / 64)) == 0; }
-// dW of one slab: (vs/256) x (Hp/256) tiles, K = at most Np tokens.  The same bound for the dW kernel, whose
-// segments need not divide the K tiles evenly.
+// dW of one slab: (vs/256) x (Hp/256) tiles, K = at most Np tokens.  The same bound for the dW kernel.
 inline int64_t dw_tail_blocks(int64_t Np, int64_t Hp, int64_t vs, int products) {
   const int64_t s = max_k_segments(products * Np / 64);
   if (s == 1) return 0;
