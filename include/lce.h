@@ -362,6 +362,14 @@ int lce_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, 
 int lce_pad_rows(const void* src, int dtype, int64_t rows, int64_t cols, int64_t ld, void* dst, int64_t dst_ld,
                  void* stream);
 
+/*
+ * dst[r][c] = src[c * ld + r] for r < rows, c < cols, 0 for cols <= c < dst_ld: a row-major copy of a matrix that lies
+ * transposed, column after column, such as the view (H, V) of a weight stored (V, H) that lce_problem.w_layout cannot name.
+ * src at any element boundary, ld >= rows; rows of dst on 16-byte boundaries.  From version 700 on.
+ */
+int lce_transpose_rows(const void* src, int dtype, int64_t rows, int64_t cols, int64_t ld, void* dst, int64_t dst_ld,
+                       void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -35,6 +35,7 @@ EXPORTS = (
     "lce_scale",
     "lce_stand_in",
     "lce_pad_rows",
+    "lce_transpose_rows",
 )
 
 _DTYPES = {torch.bfloat16: LCE_BF16, torch.float16: LCE_F16, torch.float32: LCE_F32}
@@ -115,6 +116,8 @@ def load():
     lib.lce_stand_in.argtypes = [vp, ctypes.c_int64, ctypes.c_int64, vp, vp]
     lib.lce_pad_rows.restype = ctypes.c_int
     lib.lce_pad_rows.argtypes = [vp, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, vp, ctypes.c_int64, vp]
+    lib.lce_transpose_rows.restype = ctypes.c_int
+    lib.lce_transpose_rows.argtypes = lib.lce_pad_rows.argtypes
     _lib = lib
     return lib
 

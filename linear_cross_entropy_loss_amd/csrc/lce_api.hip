@@ -800,7 +800,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
 
 extern "C" {
 
-int lce_version(void) { return 600; }  // 0.6.0: lce_stand_in, lce_pad_rows
+int lce_version(void) { return 700; }  // 0.7.0: lce_transpose_rows
 
 const char* lce_strerror(int status) {
   switch (status) {
@@ -1019,6 +1019,18 @@ int lce_pad_rows(const void* src, int dtype, int64_t rows, int64_t cols, int64_t
     return LCE_EINVAL_ARG;
   hipError_t e = lce::launch_pad_rows(src, ld * es, rows, cols * es, dst, dst_ld * es, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "pad_rows");
+  return LCE_OK;
+}
+
+int lce_transpose_rows(const void* src, int dtype, int64_t rows, int64_t cols, int64_t ld, void* dst, int64_t dst_ld,
+                       void* stream) {
+  if (dtype != LCE_BF16 && dtype != LCE_F16 && dtype != LCE_F32) return LCE_EINVAL_DTYPE;
+  const int64_t es = dtype == LCE_F32 ? 4 : 2, most = (int64_t)1 << 40;
+  if (!src || !dst || misaligned(dst) || (uintptr_t)src % (uintptr_t)es != 0 || rows < 1 || cols < 1 || ld < rows || ld > most ||
+      dst_ld < cols || dst_ld > most || dst_ld * es % 16 != 0)
+    return LCE_EINVAL_ARG;
+  hipError_t e = lce::launch_transpose_rows(src, ld, rows, cols, (int)es, dst, dst_ld, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "transpose_rows");
   return LCE_OK;
 }
 

@@ -104,7 +104,66 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const char* src, int64_t 
   }
 }
 
+// dst[r][c] = src[c][r] for c < cols, zeros from there to the end of dst's rows: a matrix that lies transposed, with rows that may
+// start anywhere.  Bound by memory traffic, read once and written once.  A workgroup turns 64 x 64 elements over in LDS: 16 bytes
+// of a row of src to a thread, 8 rows apart by lane groups of 64 elements (loads of the source's alignment; the run that the end
+// of a row cuts goes element by element), then 16 bytes of a row of dst.  Rows of the LDS tile are one 16-byte piece longer than
+// 64 elements, so that the threads that gather a column meet different banks.
+// (V=235136, H=481 in bf16: 128 us, 3.5 TB/s, against 1990 of an elementwise copy.)
+template <class E>
+__global__ __launch_bounds__(256) void transpose_rows_kernel(const E* src, int64_t src_ld, int64_t rows, int64_t cols, E* dst,
+                                                             int64_t dst_ld) {
+  constexpr int kPer = 16 / (int)sizeof(E), kPieces = 64 / kPer, kLine = 64 + kPer;
+  __shared__ __attribute__((aligned(16))) E tile[64 * kLine];
+  const int64_t tiles_c = (dst_ld + 63) / 64, tiles = (rows + 63) / 64 * tiles_c;
+  for (int64_t b = blockIdx.x; b < tiles; b += gridDim.x) {
+    const int64_t r0 = b / tiles_c * 64, c0 = b % tiles_c * 64;
+#pragma unroll
+    for (int i = 0; i < 64 * kPieces / 256; ++i) {
+      const int p = i * 256 + threadIdx.x, c = p / kPieces, r = p % kPieces * kPer;
+      E v[kPer] = {};
+      const E* from = src + (c0 + c) * src_ld + r0 + r;
+      if (c0 + c < cols) {
+        if (r0 + r + kPer <= rows) {
+          __builtin_memcpy(v, from, 16);
+        } else {
+#pragma unroll
+          for (int j = 0; j < kPer; ++j)
+            if (r0 + r + j < rows) v[j] = from[j];
+        }
+      }
+      __builtin_memcpy(__builtin_assume_aligned(&tile[c * kLine + r], 16), v, 16);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 64 * kPieces / 256; ++i) {
+      const int p = i * 256 + threadIdx.x, r = p / kPieces, c = p % kPieces * kPer;
+      E v[kPer];
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) v[j] = tile[(c + j) * kLine + r];
+      // (dst_ld is a multiple of kPer)
+      if (r0 + r < rows && c0 + c < dst_ld)
+        __builtin_memcpy(__builtin_assume_aligned(dst + (r0 + r) * dst_ld + c0 + c, 16), v, 16);
+    }
+    __syncthreads();
+  }
+}
+
 }  // namespace
+
+hipError_t launch_transpose_rows(const void* src, int64_t src_ld, int64_t rows, int64_t cols, int es, void* dst, int64_t dst_ld,
+                                 hipStream_t s) {
+  if (rows < 1 || cols < 1 || (es != 2 && es != 4) || dst_ld < cols || dst_ld * es % 16 != 0) return hipErrorInvalidValue;
+  int64_t grid = (rows + 63) / 64 * ((dst_ld + 63) / 64);
+  if (grid > 65536) grid = 65536;
+  if (es == 2)
+    hipLaunchKernelGGL(transpose_rows_kernel<unsigned short>, dim3((unsigned)grid), dim3(256), 0, s,
+                       reinterpret_cast<const unsigned short*>(src), src_ld, rows, cols, reinterpret_cast<unsigned short*>(dst), dst_ld);
+  else
+    hipLaunchKernelGGL(transpose_rows_kernel<unsigned>, dim3((unsigned)grid), dim3(256), 0, s, reinterpret_cast<const unsigned*>(src),
+                       src_ld, rows, cols, reinterpret_cast<unsigned*>(dst), dst_ld);
+  return hipGetLastError();
+}
 
 hipError_t launch_convert_w_rows(const float* src, int64_t ld, int64_t H, int64_t v0, int64_t vw, void* dst,
                                  int64_t dst_ld, int compute_dtype, hipStream_t s) {

@@ -250,6 +250,10 @@ __device__ __forceinline__ int64_t packed_token(const int* perm, int64_t j, int6
 hipError_t launch_pad_rows(const void* src, int64_t src_ld, int64_t rows, int64_t row_bytes, void* dst, int64_t dst_ld,
                            hipStream_t s);
 
+// dst[r][c] = src[c * src_ld + r], c < cols, then zeros to dst_ld; es-byte elements, strides in elements (lce_convert.hip).
+hipError_t launch_transpose_rows(const void* src, int64_t src_ld, int64_t rows, int64_t cols, int es, void* dst, int64_t dst_ld,
+                                 hipStream_t s);
+
 // *out = the largest power of two not above the number of labels that are not ignore_index (lce_compact.hip).
 hipError_t launch_stand_in(const int64_t* y, int64_t N, int64_t ignore_index, float* out, hipStream_t s);
 

@@ -136,12 +136,14 @@ def _aligned_rows(t, what=None):
                                  f"multiples of {m} elements")
     rows, cols = t.shape
     padded = torch.empty((rows, _padded_cols(cols, t.dtype)), dtype=t.dtype, device=t.device)
-    if t.stride(1) == 1 and rows > 0 and cols > 0 and padded.is_cuda and t.data_ptr() % t.element_size() == 0:
+    by_rows, by_cols = t.stride(1) == 1, t.stride(0) == 1 and t.stride(1) >= rows
+    if (by_rows or by_cols) and rows > 0 and cols > 0 and padded.is_cuda and t.data_ptr() % t.element_size() == 0:
+        copy = _lib.load().lce_pad_rows if by_rows else _lib.load().lce_transpose_rows
         with _on_device(t.device):
-            rc = _lib.load().lce_pad_rows(_ptr(t), _lib.dtype_code(t.dtype), rows, cols, t.stride(0), _ptr(padded),
-                                          padded.stride(0), torch.cuda.current_stream(t.device).cuda_stream)
-        _lib.raise_for_status(rc, "lce_pad_rows")
-    else:  # (columns apart from each other)
+            rc = copy(_ptr(t), _lib.dtype_code(t.dtype), rows, cols, t.stride(0 if by_rows else 1), _ptr(padded), padded.stride(0),
+                      torch.cuda.current_stream(t.device).cuda_stream)
+        _lib.raise_for_status(rc, "lce_pad_rows" if by_rows else "lce_transpose_rows")
+    else:  # (elements apart in both directions)
         padded[:, :cols] = t
         padded[:, cols:] = 0  # (read, so it has to be finite)
     return padded[:, :cols]

@@ -174,6 +174,22 @@ def test_padded_copy_of_rows(dtype, rows, cols, offset, extra):
         assert not whole[:, cols:].any()
 
 
+# matrices that lie transposed: one element, edges of the 64 x 64 tiles and of 16-byte pieces, more tiles than workgroups; rows that
+# start anywhere, padded rows, and a stride between them that no kernel takes
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols,ld", [(1, 1, 1), (1, 65, 1), (63, 64, 63), (64, 63, 64), (65, 129, 65), (481, 1003, 481),
+                                          (100, 72, 104), (7, 33, 9), (3, 70000 * 64, 3), (200, 100, 199)])
+def test_copies_of_transposed_matrices(rows, cols, ld, dtype):
+    from linear_cross_entropy_loss_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    store = torch.randn(cols * ld + rows + 1, generator=g, device="cuda").to(dtype)
+    t = torch.as_strided(store, (rows, cols), (1, ld), 1)  # (ld < rows: rows that overlap, copied element by element)
+    out = ops._aligned_rows(t)
+    assert out.data_ptr() % 16 == 0 and out.stride(0) * out.element_size() % 16 == 0 and torch.equal(out, t)
+    assert not torch.as_strided(out, (rows, out.stride(0)), (out.stride(0), 1))[:, cols:].any()
+
+
 # row merge and final sums: one token, a workgroup's 64 and their neighbours, more blocks than one trip of the final sums takes;
 # one slice of 128 columns, less and more than the 16 groups, and than the 128 slices of one trip; the last token counts that one
 # workgroup merges by itself, the slices up to which it does, and the first beyond
