@@ -517,13 +517,15 @@ int static_scratch(void** out) {
   return LCE_OK;
 }
 
-// Compute units of the current device (grid size of the persistent kernels), capped by `cap` when that is positive.
-int current_num_cus(int* out, int cap) {
+// Compute units of the current device (grid size of the persistent kernels), capped by `cap` when that is positive; `small_wgs`:
+// lce::few_logit_tiles.
+int current_num_cus(int* out, int cap, int* small_wgs = nullptr) {
   int dev = 0, n = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
   if (e != hipSuccess) return hip_fail(e, "device query");
   *out = n > 0 ? n : 1;
+  if (small_wgs) *small_wgs = cap > 0 && cap < *out ? 0 : 2 * *out;
   if (cap > 0 && cap < *out) *out = cap;
   return LCE_OK;
 }
@@ -556,7 +558,7 @@ int forward_impl(const lce_problem* p, const void* x, const void* w, const int64
   a.part_sq = (float*)(base + f.part_sq);
   a.tgt = (float*)(base + f.tgt);
   a.blk = (float*)(base + f.blk);
-  rc = current_num_cus(&a.num_cus, p->max_workgroups);
+  rc = current_num_cus(&a.num_cus, p->max_workgroups, &a.small_wgs);
   if (rc != LCE_OK) return rc;
   a.live = lce::live_bands(logit_k_bytes(p));
 
@@ -640,8 +642,8 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   const PackPlan& k = f.k;
   const int64_t Np = lce::padded_tokens(p->N), Vp = lce::padded_vocab(p->V);
   const int64_t dxes = p->dx_dtype == LCE_F32 ? 4 : 2;
-  int num_cus = 0;
-  int rc = current_num_cus(&num_cus, p->max_workgroups);
+  int num_cus = 0, small_wgs = 0;
+  int rc = current_num_cus(&num_cus, p->max_workgroups, &small_wgs);
   if (rc != LCE_OK) return rc;
   int64_t* n_rows = (int64_t*)(base + k.n_rows);
   int* perm = (int*)(base + k.perm);
@@ -711,7 +713,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   b.dz = base + f.stage;
   b.v0 = 0; b.vw = p->V; b.vs = Vp; b.wv0 = 0; b.Vw = p->V;
   b.first = 1; b.last = 1;
-  b.num_cus = num_cus; b.dx_grid = num_cus; b.dw_grid = num_cus;
+  b.num_cus = num_cus; b.small_wgs = small_wgs; b.dx_grid = num_cus; b.dw_grid = num_cus;
   b.live = lce::live_bands(lce::padded_k(p->H) * 2);
   b.part_lse = (float*)(base + f.part_lse);
   b.part_max = (float*)(base + f.part_max);
@@ -904,7 +906,7 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
   a.dx_acc = b.slabs > 1 ? (float*)(base + b.dx_acc) : nullptr;
   a.dx_part = b.parts_on ? (float*)(base + b.dx_part) : nullptr;
   a.dw_part = b.parts_on ? (float*)(base + b.dw_part) : nullptr;
-  rc = current_num_cus(&a.num_cus, p->max_workgroups);
+  rc = current_num_cus(&a.num_cus, p->max_workgroups, &a.small_wgs);
   if (rc != LCE_OK) return rc;
   a.live = lce::live_bands(logit_k_bytes(p));
   const int ph = p->phases ? p->phases : ~0;

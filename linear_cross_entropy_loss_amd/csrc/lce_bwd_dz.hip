@@ -10,7 +10,7 @@
 // group are one 128-byte line, and dz leaves the compute unit as whole lines,
 // transposed through a small LDS area that the main loop does not use.
 // The kernel is persistent (one workgroup per CU, operand stream pipelined across tiles).
-#include "lce_gemm3.h"
+#include "lce_gemm_small.h"
 #include "lce_internal.h"
 
 namespace lce {
@@ -28,9 +28,10 @@ static_assert(kLdsBytes <= 160 * 1024, "a compute unit has 160 KiB of LDS");
 #endif
 constexpr int kDzStoreAux = LCE_DZ_STORE_AUX;  // cache policy of the dz stores: 2 = nt (streaming)
 
-// Turns the finished logit tile (tp, tq) into dz and writes it out.
+// Turns a wave's finished 128(v) x 32 NQ(token) logits -- the slice that starts at column slice_v0, the tokens from row tw of
+// the stage on (both uniform over the wave) -- into dz and writes it out.  `mine`: the wave's LDS area.
 //
-// Each lane owns 4 tokens (columns of the accumulator) x 64 vocabulary entries
+// Each lane owns NQ tokens (columns of the accumulator) x 64 vocabulary entries
 // per token, four consecutive entries per register quad; lanes l and l+32 hold
 // the two halves of every run of 8 entries.  One v_permlane32_swap per pair of
 // register quads hands each lane a full run of 8 (16 bytes in the 16-bit
@@ -70,16 +71,12 @@ constexpr int kDzStoreAux = LCE_DZ_STORE_AUX;  // cache policy of the dz stores:
 // switch ZREG stands for the monitoring values instead (the slice's sum softmax * z and sum z^2, as lce_fwd.hip forms them).
 constexpr int kNoLabel = -0x7fffffff - 1;  // ignore_index, or no such row
 constexpr int kOffLabel = -1;              // a label that is no column of W (V <= 2^30): matches nothing
-template <class T, bool ZREG, bool VTAIL, bool FUSE>
-LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const float (&pf_lse)[kNB],
-                              f32x16_t (&acc)[kNB][kNB], int tp, int tq, char* pieces) {
+template <class T, bool ZREG, bool VTAIL, bool FUSE, int NQ>
+LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[NQ], const float (&pf_lse)[NQ], f32x16_t (&acc)[kNB][NQ],
+                              int64_t slice_v0, int64_t tw, char* mine) {
   typedef typename elem_of<T>::type E;
-  const int64_t v0 = a.v0 + (int64_t)tp * kTile, t0 = (int64_t)tq * kTile;
-  const int tid = opaque_tid();
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wp = wave & 1, wq = wave >> 1;
+  const int lane = opaque_tid() & 63;
   const int half = lane >> 5;
-  const int64_t slice_v0 = v0 + wp * kWaveTile;
   const float c1 = a.scale * kLog2e;
   // columns of this wave's slice that exist: nq whole runs of 8, then `cut` more columns
   const int64_t left = a.v0 + a.vw - slice_v0;
@@ -91,9 +88,8 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
   constexpr bool SPLIT = is_pair<T>::value;
   constexpr int kParts = SPLIT ? 2 : 1;
   constexpr int64_t grp = kParts * kDzBlockElems;  // elements from a block of the stage to the next column group's
-  const int wpu = __builtin_amdgcn_readfirstlane(wp), wqu = __builtin_amdgcn_readfirstlane(wq);  // (uniform, for the scalar unit)
-  E* wave_base = reinterpret_cast<E*>(a.dz) + kParts * dz_block_offset(tq, tp * (kTile / kGroup) + wpu * (kWaveTile / kGroup), a.vs) +
-                 wqu * kWaveTile * kGroup;
+  E* wave_base = reinterpret_cast<E*>(a.dz) + kParts * dz_block_offset(tw / kTile, (slice_v0 - a.v0) / kGroup, a.vs) +
+                 (tw % kTile) * kGroup;
   E* row = wave_base + (lane & 31) * kGroup;
   constexpr bool MON = FUSE && ZREG;
   // Stores go through a buffer descriptor over this wave's part of the stage (scalar base, one 32-bit offset per
@@ -103,15 +99,14 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
   // staging: this lane's line of a piece when it writes (its token), and line / chunk when it reads back: 8 lines
   // per instruction, 8 lanes each; the upper 32 lanes take their four lines in the order 5, 4, 7, 6 so that lanes
   // l and l+32 always sit in lines of opposite parity (opposite bank halves)
-  char* mine = pieces + wave * kWaveLds;
   const int wline = lane & 31, wsw = (wline & 7) ^ ((wline >> 3) & 1);
   const int rline = (lane >> 3) + ((lane >> 5) ? 1 - 2 * ((lane >> 3) & 1) : 0), rchunk = lane & 7;
 
   // per-token scalars of this lane's four tokens
-  float nlse[kNB], gain[kNB];
-  int ykey[kNB];
+  float nlse[NQ], gain[NQ];
+  int ykey[NQ];
 #pragma unroll
-  for (int qb = 0; qb < kNB; ++qb) {
+  for (int qb = 0; qb < NQ; ++qb) {
     // (rows past the last one are staged as zeros, like ignored tokens)
     const int yy = pf_y[qb];  // the label as DzProblem::prefetch keeps it: kNoLabel, or the column (kOffLabel: none of W's)
     const int64_t rel = (int64_t)yy - slice_v0;
@@ -127,7 +122,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
   }
 
 #pragma unroll
-  for (int qb = 0; qb < kNB; ++qb) {
+  for (int qb = 0; qb < NQ; ++qb) {
     float m = -INFINITY, ssum = 0.f, mpz = 0.f, msq = 0.f;
     u32x4_t lo_part[SPLIT ? 8 : 1];  // this lane's 16-byte runs of lo parts
     if constexpr (FUSE) {
@@ -242,7 +237,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
     if constexpr (FUSE) {
       // the forward's partials of this slice for the token, and its target logit if it lies here
       ssum += __shfl_xor(ssum, 32);
-      const int64_t tokl = t0 + wq * kWaveTile + qb * kBlk + (lane & 31);
+      const int64_t tokl = tw + qb * kBlk + (lane & 31);
       const int64_t o = (slice_v0 / kChunkV) * a.nc + tokl;
       if (lane < 32) {
         // (no column of the slice inside the vocabulary: m = -inf, ssum = 0 -> -inf, nothing to add to the lse)
@@ -292,6 +287,14 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[kNB], const fl
       if (SPLIT) *reinterpret_cast<unsigned short*>(at + kDzBlockElems) = to_bits<T>(bf16_lo(tv));
     }
   }
+}
+
+// What the epilogue wants to know of a token: its label as one number, and its lse.
+template <bool FUSE> LCE_DEV void dz_row_scalars(const BwdArgs& a, int64_t rows, int64_t tok, int& y, float& lse) {
+  const bool exists = tok < rows;
+  const int64_t yy = exists ? a.y[tok] : a.ignore_index;
+  y = yy == a.ignore_index ? kNoLabel : (yy >= 0 && yy < a.V ? (int)yy : kOffLabel);
+  lse = exists && !FUSE ? a.lse[tok] : 0.f;
 }
 
 // ZREG (z_regularization != 0) is a compile-time switch of the kernels rather than a
@@ -352,18 +355,16 @@ template <class T, bool ZREG, bool VTAIL, bool KMASK, bool WVH, bool FUSE = fals
     coords(tile, tp, tq);
     const int lane = threadIdx.x & 63, wq = threadIdx.x >> 7;
 #pragma unroll
-    for (int qb = 0; qb < kNB; ++qb) {
-      const int64_t tok = (int64_t)tq * kTile + wq * kWaveTile + qb * kBlk + (lane & 31);
-      const bool exists = tok < rows;
-      const int64_t yy = exists ? a.y[tok] : a.ignore_index;
-      pf_y[qb] = yy == a.ignore_index ? kNoLabel : (yy >= 0 && yy < a.V ? (int)yy : kOffLabel);
-      pf_lse[qb] = exists && !FUSE ? a.lse[tok] : 0.f;
-    }
+    for (int qb = 0; qb < kNB; ++qb)
+      dz_row_scalars<FUSE>(a, rows, (int64_t)tq * kTile + wq * kWaveTile + qb * kBlk + (lane & 31), pf_y[qb], pf_lse[qb]);
   }
   LCE_DEV void epilogue(int tile, f32x16_t (&acc)[kNB][kNB], char* scratch) const {
     int tp, tq;
     coords(tile, tp, tq);
-    dz_epilogue_impl<T, ZREG, VTAIL, FUSE>(a, pf_y, pf_lse, acc, tp, tq, scratch + kStageBytes);  // (behind the main loop's stages)
+    const int wave = __builtin_amdgcn_readfirstlane(opaque_tid() >> 6);  // (uniform, for the scalar unit)
+    dz_epilogue_impl<T, ZREG, VTAIL, FUSE, kNB>(a, pf_y, pf_lse, acc, a.v0 + (int64_t)tp * kTile + (wave & 1) * kWaveTile,
+                                                (int64_t)tq * kTile + (wave >> 1) * kWaveTile,
+                                                scratch + kStageBytes + wave * kWaveLds);  // (behind the main loop's stages)
   }
 };
 
@@ -390,6 +391,40 @@ __global__ __launch_bounds__(kThreads) void bwd_dz_persistent_kernel(const BwdAr
   }
 }
 
+// The same on 128 x 128 tiles (lce_gemm_small.h): workgroup = one slice of 128 columns, 128 tokens; whole tiles of 256 tokens
+// are written, as the gradient kernels read them.  The pieces of the epilogue take the place of the K loop's stages.
+static_assert(4 * kWaveLds <= kSmallLds, "the pieces fit where the stages were");
+template <class T, bool ZREG, bool WVH, bool FUSE>
+__global__ __launch_bounds__(kThreads, 2) void dz_small_kernel(const BwdArgs a, int tiles_p, int tiles_q) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  typedef typename elem_of<T>::type E;
+  const int64_t rows = packed_rows(a.n_rows, a.N);
+  const bool packed = rows != a.N;
+  const E* x = reinterpret_cast<const E*>(packed ? a.xc : a.x);
+  const int64_t ldx = packed ? a.ldxc : a.ldx;
+  int tp, tq;
+  tile_coords((int)blockIdx.x, (int)gridDim.x, tiles_p, tiles_q, 8, 8, tp, tq);
+  const int64_t t0 = (int64_t)tq * kSmallTile;
+  if (t0 / kTile * kTile >= rows) return;
+  constexpr int kParts = is_pair<T>::value ? 2 : 1;
+  const int64_t v = (a.v0 - a.wv0) + (int64_t)tp * kSmallTile;
+  const E* w = reinterpret_cast<const E*>(a.w);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t slice_v0 = a.v0 + (int64_t)tp * kSmallTile, tw = t0 + wave * kBlk;
+  int pf_y[1];
+  float pf_lse[1];
+  dz_row_scalars<FUSE>(a, rows, tw + (threadIdx.x & 31), pf_y[0], pf_lse[0]);
+  SmallPipe<T, WVH> pipe;
+  f32x16_t acc[kNB][1];
+  // (the second half of a tile of 256 tokens may have none: logits of rows that do not exist are zeros)
+  pipe.run(w + (WVH ? v * a.ldw : v), WVH ? matrix_end<E>(w, a.Vw, a.ldw, a.H) : matrix_end<E>(w, kParts * a.H, a.ldw, a.Vw), a.ldw,
+           x + t0 * ldx, matrix_end<E>(x, rows, ldx, kParts == 2 ? a.x_lo + a.H : a.H), ldx, a.H,
+           t0 < rows ? logit_ktiles<T>(a.H) : 0, a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
+  char* mine = lds + wave * kWaveLds;
+  if (slice_v0 + kSmallTile <= a.v0 + a.vw) dz_epilogue_impl<T, ZREG, false, FUSE, 1>(a, pf_y, pf_lse, acc, slice_v0, tw, mine);
+  else dz_epilogue_impl<T, ZREG, true, FUSE, 1>(a, pf_y, pf_lse, acc, slice_v0, tw, mine);
+}
+
 template <class T, bool ZREG, int TAIL, bool KMASK, bool WVH, bool FUSE = false>
 hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
   auto kern = bwd_dz_persistent_kernel<T, ZREG, TAIL, KMASK, WVH, FUSE>;
@@ -404,6 +439,12 @@ hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
 // All tile columns of the slab in one launch.
 template <class T, bool ZREG, bool WVH, bool FUSE = false>
 hipError_t launch_persistent_z(const BwdArgs& a, hipStream_t s) {
+  if (few_logit_tiles(a.N <= kSmallTile ? a.N : a.Np, a.vw, logit_ktiles<T>(a.H), a.small_wgs)) {
+    const int tiles_p = (int)(a.vs / kSmallTile), tiles_q = (int)(a.Np / kSmallTile);
+    hipLaunchKernelGGL((dz_small_kernel<T, ZREG, WVH, FUSE>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a,
+                       tiles_p, tiles_q);
+    return hipGetLastError();
+  }
   const int64_t tq = a.Np / kTile, full = a.vw / kTile, tail = a.vs / kTile - full;
   const bool exact_k = (is_pair<T>::value ? padded_k_pair(a.H) : padded_k(a.H)) == a.H;  // the K tiles cover H exactly: no K mask needed
   if (full == 0) return launch_one<T, ZREG, kTailOnly, true, WVH, FUSE>(a, tail * tq, s);

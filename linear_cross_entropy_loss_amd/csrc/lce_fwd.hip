@@ -12,7 +12,7 @@
 // forms the per-token loss terms (ops.py:753-761); fwd_final_kernel sums them
 // in a fixed order into the five scalars of ops.py:802 and the valid-label
 // count of ops.py:705.  All reductions are order-deterministic.
-#include "lce_gemm3.h"
+#include "lce_gemm_small.h"
 #include "lce_internal.h"
 
 namespace lce {
@@ -25,8 +25,8 @@ constexpr float kLn2 = 0.6931471805599453f;
 LCE_DEV float fast_exp2(float v) { return __builtin_amdgcn_exp2f(v); }
 LCE_DEV float fast_log(float v) { return __builtin_amdgcn_logf(v) * kLn2; }
 
-// Reduces the finished 256(v) x 256(token) accumulator of tile (tp, tq) to the
-// per-slice partials.  Accumulator rows (v) lie along registers and columns
+// Reduces a wave's finished 128(v) x 32 NQ(token) accumulator -- the slice that starts at column slice_v0, the tokens from
+// row tw of this launch's chunk on -- to the per-slice partials.  Accumulator rows (v) lie along registers and columns
 // (tokens) along lanes, so each lane reduces its own tokens in registers and
 // meets the other half of the vocabulary slice in lane ^ 32.
 //
@@ -36,13 +36,9 @@ LCE_DEV float fast_log(float v) { return __builtin_amdgcn_logf(v) * kLn2; }
 // whole, uniformly over the wave, and is taken or skipped with a scalar branch;
 // the one run that V cuts through is handled element by element.
 // MON: the monitoring partials (slice max, sum softmax*z, sum z^2) are formed as well.
-template <class T, bool VTAIL, bool MON>
-LCE_DEV void fwd_epilogue(const FwdArgs& a, int64_t rows, f32x16_t (&acc)[kNB][kNB], int tp, int tq) {
-  const int64_t v0 = (int64_t)tp * kTile, t0 = (int64_t)tq * kTile;  // t0: inside the chunk of rows of this launch
-  const int tid = opaque_tid();
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wp = wave & 1, wq = wave >> 1;
-  const int64_t slice_v0 = v0 + wp * kWaveTile;
+template <class T, bool VTAIL, bool MON, int NQ>
+LCE_DEV void fwd_epilogue(const FwdArgs& a, int64_t rows, f32x16_t (&acc)[kNB][NQ], int64_t slice_v0, int64_t tw) {
+  const int lane = opaque_tid() & 63;
   // columns of this wave's slice inside the vocabulary: nq whole runs of 8, then `cut` more columns
   const int64_t left = a.V - slice_v0;
   const int vrem = VTAIL ? (int)(left < 0 ? 0 : (left > kWaveTile ? kWaveTile : left)) : kWaveTile;
@@ -52,8 +48,8 @@ LCE_DEV void fwd_epilogue(const FwdArgs& a, int64_t rows, f32x16_t (&acc)[kNB][k
   const float c1 = a.scale * kLog2e;
   const int64_t slice = slice_v0 / kChunkV;
 #pragma unroll
-  for (int qb = 0; qb < kNB; ++qb) {
-    const int64_t tokl = t0 + wq * kWaveTile + qb * kBlk + (lane & 31);  // row inside the chunk
+  for (int qb = 0; qb < NQ; ++qb) {
+    const int64_t tokl = tw + qb * kBlk + (lane & 31);  // row inside the chunk
     const int64_t tok = a.row0 + tokl;
     const int64_t o = slice * a.nc + tokl;
     if (VTAIL && vrem == 0) {  // nothing of this slice exists
@@ -156,7 +152,8 @@ LCE_DEV void fwd_epilogue(const FwdArgs& a, int64_t rows, f32x16_t (&acc)[kNB][k
 // The logit of the target column, written by the one lane that holds it (rare: a wave holds the target of
 // one token in a thousand at a vocabulary of 131072).  `yl`: the column inside this wave's 128-wide slice if
 // this lane's half holds it, else -1.
-LCE_DEV void fwd_store_target(const FwdArgs& a, f32x16_t (&acc)[kNB][kNB], int64_t tok, int qb, int yl) {
+template <int NQ>
+LCE_DEV void fwd_store_target(const FwdArgs& a, f32x16_t (&acc)[kNB][NQ], int64_t tok, int qb, int yl) {
   if (yl >= 0) {
     const int want = (yl >> 5) * 16 + ((yl >> 3) & 3) * 4 + (yl & 3);  // (block, register) index
     float zt = 0.f;
@@ -189,8 +186,8 @@ struct FwdColumnState {
 // Slot 0..15 of block column QB: the running (max, sum) of this lane's 64 values -- and, MON, the two monitoring
 // sums, which leave the arithmetic on (max, sum) as it is, so that the loss does not depend on the monitoring flag
 // bit for bit.  The exponentials of a slot are added up in the next one, when they are there.
-template <int QB, bool MON>
-LCE_DEV void fwd_slot_sum(const FwdArgs& a, FwdColumnState& st, f32x16_t (&acc)[kNB][kNB], int slot) {
+template <int QB, bool MON, int NQ>
+LCE_DEV void fwd_slot_sum(const FwdArgs& a, FwdColumnState& st, f32x16_t (&acc)[kNB][NQ], int slot) {
   const float c1 = a.scale * kLog2e;
   const int c = slot >> 3, sub = slot & 7;  // chunk c: accumulator blocks 2c, 2c + 1, slots 8c .. 8c + 7
   if (slot > 0) {
@@ -263,16 +260,15 @@ LCE_DEV void fwd_merge_halves(const FwdArgs& a, FwdColumnState& st) {
     st.sq = __builtin_bit_cast(float, q0u) + __builtin_bit_cast(float, q1u);
   }
 }
-template <class T, int QB, bool MON>
-LCE_DEV void fwd_epilogue_slot(const FwdArgs& a, FwdColumnState& st, f32x16_t (&acc)[kNB][kNB], int tp, int tq, int slot) {
-  fwd_slot_sum<QB, MON>(a, st, acc, slot);
+// tw: first token row of the wave inside this launch's chunk (like slice_v0 uniform over the wave).
+template <class T, int QB, bool MON, int NQ>
+LCE_DEV void fwd_epilogue_slot(const FwdArgs& a, FwdColumnState& st, f32x16_t (&acc)[kNB][NQ], int64_t slice_v0, int64_t tw, int slot) {
+  fwd_slot_sum<QB, MON, NQ>(a, st, acc, slot);
   if (slot == 15) {
     fwd_merge_halves<MON>(a, st);
     // one store per token and partial: the upper lanes get an offset that the range check of the buffer store drops
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t slice = ((int64_t)tp * kTile + (wave & 1) * kWaveTile) / kChunkV;
-    const int64_t o = slice * a.nc + (int64_t)tq * kTile + (wave >> 1) * kWaveTile + QB * kBlk;
+    const int lane = threadIdx.x & 63;
+    const int64_t o = slice_v0 / kChunkV * a.nc + tw + QB * kBlk;
     const int voff = lane < 32 ? lane * 4 : (int)0x80000000;
     auto store = [&](float* base, float v) {
       const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(base + o, 0, kBlk * 4, 0x00020000);
@@ -357,7 +353,9 @@ template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON> struct FwdProblem
   }
   FwdColumnState est;
   template <int J> LCE_DEV void epilogue_slot(int, f32x16_t (&acc)[kNB][kNB], int slot, char*) {
-    fwd_epilogue_slot<T, J, MON>(a, est, acc, etp, etq, slot);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    fwd_epilogue_slot<T, J, MON, kNB>(a, est, acc, (int64_t)etp * kTile + (wave & 1) * kWaveTile,
+                                      (int64_t)etq * kTile + (wave >> 1) * kWaveTile, slot);
   }
   LCE_DEV void epilogue_end(int, f32x16_t (&acc)[kNB][kNB], char*) const {
     const int tid = opaque_tid();
@@ -374,7 +372,9 @@ template <class T, bool VTAIL, bool KMASK, bool WVH, bool MON> struct FwdProblem
   LCE_DEV void epilogue(int tile, f32x16_t (&acc)[kNB][kNB], char*) const {
     int tp, tq;
     coords(tile, tp, tq);
-    fwd_epilogue<T, VTAIL, MON>(a, rows, acc, (int)(a.v0 / kTile) + tp, tq);
+    const int wave = opaque_tid() >> 6;
+    fwd_epilogue<T, VTAIL, MON, kNB>(a, rows, acc, a.v0 + (int64_t)tp * kTile + (wave & 1) * kWaveTile,
+                                     (int64_t)tq * kTile + (wave >> 1) * kWaveTile);
   }
 };
 
@@ -401,6 +401,44 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
     __syncthreads();  // (every wave is done with the main loop's LDS stages)
     Pipe3<T, E, WVH, E, true, Tail> pipe(prob);
     pipe.run(a.ldw, prob.ldx, logit_ktiles<T>(a.H), lds, first);
+  }
+}
+
+// The same on 128 x 128 tiles (lce_gemm_small.h): workgroup = one slice of 128 columns, 128 tokens.  tiles_p slices; those past
+// the vocabulary's end get partials as well, which the row merge reads.
+template <class T, bool WVH, bool MON>
+__global__ __launch_bounds__(kThreads, 2) void fwd_small_kernel(const FwdArgs a, int tiles_p, int tiles_q) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  typedef typename elem_of<T>::type E;
+  const int64_t rows = a.n_rows ? packed_rows(a.n_rows, a.N) : a.N;
+  const bool packed = rows != a.N;
+  const E* x = reinterpret_cast<const E*>(packed ? a.xc : a.x);
+  const int64_t ldx = packed ? a.ldxc : a.ldx;
+  int tp, tq;
+  tile_coords((int)blockIdx.x, (int)gridDim.x, tiles_p, tiles_q, 8, 8, tp, tq);
+  const int64_t t0 = (int64_t)tq * kSmallTile;
+  if (a.row0 + t0 >= rows) return;
+  constexpr int kParts = is_pair<T>::value ? 2 : 1;
+  const int64_t v = (a.v0 - a.wv0) + (int64_t)tp * kSmallTile;
+  const E* w = reinterpret_cast<const E*>(a.w);
+  SmallPipe<T, WVH> pipe;
+  f32x16_t acc[kNB][1];
+  pipe.run(w + (WVH ? v * a.ldw : v), WVH ? matrix_end<E>(w, a.Vw, a.ldw, a.H) : matrix_end<E>(w, kParts * a.H, a.ldw, a.Vw), a.ldw,
+           x + (a.row0 + t0) * ldx, matrix_end<E>(x, rows, ldx, kParts == 2 ? a.x_lo + a.H : a.H), ldx, a.H, logit_ktiles<T>(a.H),
+           a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
+  // (with the sums of the persistent kernel, bit for bit: by columns but in the tile of 256 columns that straddles the end)
+  const int64_t slice_v0 = a.v0 + (int64_t)tp * kSmallTile;
+  const int64_t tw = t0 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kBlk;
+  if (slice_v0 / kTile * kTile + kTile <= a.V) {
+    FwdColumnState st;
+#pragma unroll
+    for (int slot = 0; slot < 16; ++slot) fwd_epilogue_slot<T, 0, MON, 1>(a, st, acc, slice_v0, tw, slot);
+    const int lane = threadIdx.x & 63;
+    const int64_t tok = a.row0 + tw + (lane & 31), yy = tok < rows ? a.y[tok] : a.ignore_index, rel = yy - slice_v0;
+    const bool here = yy != a.ignore_index && rel >= 0 && rel < kWaveTile && ((rel >> 2) & 1) == (lane >> 5);
+    fwd_store_target<1>(a, acc, tok, 0, here ? (int)rel : -1);
+  } else {
+    fwd_epilogue<T, true, MON, 1>(a, rows, acc, slice_v0, tw);
   }
 }
 
@@ -629,6 +667,13 @@ hipError_t launch_one(const FwdArgs& a, int64_t tiles, hipStream_t s) {
 // All tile columns of the vocabulary in one launch.
 template <class T, bool WVH, bool MON> hipError_t launch_persistent(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;  // token tiles of this chunk at most
+  const int64_t here = left < a.nc ? left : a.nc, there = a.N - a.row0, rows = here < there ? here : there;
+  if (few_logit_tiles(rows, a.vw, logit_ktiles<T>(a.H), a.small_wgs)) {
+    const int tiles_p = (int)(pad_to(a.vw, kTile) / kSmallTile), tiles_q = (int)((rows + kSmallTile - 1) / kSmallTile);
+    hipLaunchKernelGGL((fwd_small_kernel<T, WVH, MON>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a, tiles_p,
+                       tiles_q);
+    return hipGetLastError();
+  }
   const int64_t tq = (left < a.nc ? left : a.nc) / kTile, full = a.vw / kTile;
   const bool exact_k = (is_pair<T>::value ? padded_k_pair(a.H) : padded_k(a.H)) == a.H;  // the K tiles cover H exactly: no K mask needed
   const bool tail = a.vw % kTile != 0;        // a column that straddles V

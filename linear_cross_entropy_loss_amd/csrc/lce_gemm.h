@@ -152,9 +152,10 @@ LCE_DEV int first_tail_tile(int wg, int grid, int full) {
 // Fragment readers: per-lane LDS offsets for the four 32-wide blocks of this
 // wave's 128-wide slice of an operand tile.
 // ---------------------------------------------------------------------------
-template <bool KC> struct FragReader;
+// COLS: columns of the operand tile (its P / Q extent).
+template <bool KC, int COLS = kTile> struct FragReader;
 
-template <> struct FragReader<true> {
+template <int COLS> struct FragReader<true, COLS> {
   int off[4];  // byte offset per k-step (block 0); blocks add 32 rows = 4096 bytes
   LCE_DEV void init(int wave_off /* first row of the wave's slice */) {
     const int l = threadIdx.x & 63;
@@ -169,7 +170,7 @@ template <> struct FragReader<true> {
   }
 };
 
-template <> struct FragReader<false> {
+template <int COLS> struct FragReader<false, COLS> {
   int off[4];  // byte offset per block at k-step 0, first half
   LCE_DEV void init(int wave_off /* first column of the wave's slice */) {
     const int l = threadIdx.x & 63;
@@ -179,13 +180,13 @@ template <> struct FragReader<false> {
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       const int colbyte = (wave_off + b * 32 + 16 * (g & 1) + 4 * c) * 2;
-      off[b] = krow * 512 + (colbyte ^ mask);
+      off[b] = krow * (COLS * 2) + (colbyte ^ mask);
     }
   }
   LCE_DEV s16x8_t read(const char* tile, int blk, int ks) const {
-    const char* p = tile + off[blk] + ks * (16 * 512);
+    const char* p = tile + off[blk] + ks * (16 * COLS * 2);
     const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LCE_LDS(s16x4_t)*)(p));
-    const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LCE_LDS(s16x4_t)*)(p + 4 * 512));
+    const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LCE_LDS(s16x4_t)*)(p + 4 * COLS * 2));
     s16x8_t v;
     v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
     v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];

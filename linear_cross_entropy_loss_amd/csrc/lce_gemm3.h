@@ -30,11 +30,12 @@
 
 namespace lce {
 
-// Register staging of one operand tile: 8 chunks of 8 elements (one 16-byte register quad) per thread.
+// Register staging of one operand tile of CHUNKS * 32 rows or columns: CHUNKS chunks of 8 elements (one 16-byte register quad)
+// per thread.
 // Operands are always 16-bit in memory: fp32 activations and weights are rounded to the compute type by
 // copy kernels before the tile kernels run.
-struct StageRegs {
-  u32x4_t v[8];
+template <int CHUNKS> struct StageRegs {
+  u32x4_t v[CHUNKS];
 };
 
 #define LCE_SG_VALU 0x002
@@ -49,10 +50,12 @@ struct StageRegs {
 // offset, and the stride between a thread's 8 chunks is a scalar offset, so a
 // load costs one instruction and no vector address arithmetic.
 // KMASK = false compiles the K mask out, for launches whose K tiles cover the K extent exactly.
-template <class T, class SrcT, bool KC, bool KMASK> struct Stager3 {
+template <class T, class SrcT, bool KC, bool KMASK, int CHUNKS = 8> struct Stager3 {
   static_assert(sizeof(SrcT) == 2, "operands are staged as 16-bit data");
   static constexpr int kEs = (int)sizeof(SrcT);
-  typedef StageRegs Regs;
+  typedef StageRegs<CHUNKS> Regs;
+  // a tile whose columns are its P / Q extent: pieces of 16 bytes in a row of it, rows that the workgroup stages at a time
+  static constexpr int kRowPieces = CHUNKS * 4, kRowsAtOnce = kThreads / kRowPieces;
   const char* base;      // uniform: first byte of the K tile being loaded
   const char* end;       // uniform: one past the last valid byte of the operand (loads beyond return 0)
   unsigned range;        // uniform: bytes from `base` to `end`, clamped to [0, 2^31)
@@ -74,13 +77,13 @@ template <class T, class SrcT, bool KC, bool KMASK> struct Stager3 {
       lds_off = r * 128 + ((c ^ sw) << 4);
       kpos = c * 8;
     } else {
-      const int c = t & 31, k = t >> 5;
+      const int c = t % kRowPieces, k = t / kRowPieces;
       voff = (unsigned)(((int64_t)k * ld + c * 8) * kEs);
-      iter_stride = (unsigned)(8 * ld * kEs);
+      iter_stride = (unsigned)(kRowsAtOnce * ld * kEs);
       k_stride = (int64_t)kBK * ld * kEs;
       const int j = k & 3;
       const int mask = ((j & 1) << 7) | ((j >> 1) << 6) | ((j & 1) << 5);
-      lds_off = k * 512 + ((c << 4) ^ mask);
+      lds_off = k * (kRowPieces * 16) + ((c << 4) ^ mask);
       kpos = 0;
     }
     voff_cur = voff;
@@ -132,7 +135,7 @@ template <class T, class SrcT, bool KC, bool KMASK> struct Stager3 {
       r.v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff_cur, (int)(i * iter_stride), 0);
   }
   LCE_DEV void store(const Regs& r, char* tile, int i0, int i1) const {
-    constexpr int step = KC ? 32 * 128 : 8 * 512;
+    constexpr int step = KC ? 32 * 128 : kRowsAtOnce * kRowPieces * 16;
 #pragma unroll
     for (int i = i0; i < i1; ++i) *reinterpret_cast<u32x4_t*>(tile + lds_off + i * step) = r.v[i];
   }
@@ -158,7 +161,7 @@ template <class S> LCE_DEV const void* matrix_end(const void* base, int64_t rows
 }
 
 // K tiles of the logit contraction.
-template <class T> LCE_DEV int logit_ktiles(int64_t H) {
+template <class T> __host__ LCE_DEV int logit_ktiles(int64_t H) {
   return (int)(is_pair<T>::value ? 3 * padded_k_pair(H) / kBK : padded_k(H) / kBK);
 }
 

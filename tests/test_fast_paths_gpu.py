@@ -271,3 +271,58 @@ def test_dense_fp32_gradients(N, H, V, n_chunk, x_dtype, route):
     # (fp32: products of bf16 pairs, 2^-16 relative to each operand, so some 2^-15 of the 2-norm; bf16: as above)
     for got, want in ((gx, ref.dx), (gw, ref.dw)):
         assert rel_errors(got, want)[1] < (3e-5 if x_dtype == torch.float32 else 5e-3)
+
+
+# Logit kernels on 128 x 128 tiles against the persistent ones, which a limit on the workgroups of a launch asks for: halves and
+# quarters of a tile that do not exist, vocabularies that end in any slice, hidden sizes that end in any K tile, one workgroup and
+# as many as the rule allows, both layouts, monitoring, pairs.
+SMALL_TILE_CASES = [
+    # N, H, V, dtype, monitoring, (V, H), ignored
+    (1, 8, 1, torch.bfloat16, False, 0, 0.0), (127, 72, 127, torch.float16, True, 0, 0.1), (128, 64, 128, torch.bfloat16, False, 1, 0.0),
+    (129, 200, 129, torch.bfloat16, True, 1, 0.2), (255, 130, 257, torch.float32, True, 0, 0.1), (257, 128, 255, torch.float16, False, 0, 0.0),
+    (300, 1000, 1001, torch.bfloat16, False, 0, 0.3), (300, 104, 4000, torch.float32, False, 0, 0.0), (1, 4, 300, torch.float32, False, 0, 0.0),
+    (2048, 256, 4096, torch.bfloat16, False, 0, 0.1), (4096, 2048, 2048, torch.float16, False, 1, 0.0), (100, 320, 70000, torch.bfloat16, True, 0, 0.1),
+]
+
+
+@pytest.mark.parametrize("route", ["two_pass", "one_pass"])
+@pytest.mark.parametrize("N,H,V,dtype,mon,layout,ignored", SMALL_TILE_CASES)
+def test_small_logit_tiles_match_the_persistent_kernels(N, H, V, dtype, mon, layout, ignored, route):
+    import ctypes
+
+    from linear_cross_entropy_loss_amd import _lib, ops
+
+    lib = _lib.load()
+    x, y, w = make_inputs(N, H, V, dtype, 17, ignore_frac=ignored, device="cuda")
+    y[0] = V - 1
+    x, w = ops._aligned_rows(x), ops._aligned_rows(w.t().contiguous() if layout else w)
+    outs = []
+    for limit in (0, torch.cuda.get_device_properties(0).multi_processor_count - 1):
+        dx, dw = ops._empty_rows(N, H, dtype, "cuda"), ops._empty_rows(*w.shape, dtype, "cuda")
+        prob = _lib.make_problem(N, H, V, x.stride(0), w.stride(0), dx.stride(0), dw.stride(0), dtype, dtype, dtype, dtype, -1, 1.5, 1e-3,
+                                 65536, mon, 0, _lib.PACK_NEVER, limit, layout,
+                                 _lib.ROUTE_ONE_PASS if route == "one_pass" else _lib.ROUTE_TWO_PASS)
+        if route == "one_pass" and _lib.forward_backward_plan(prob)[0] == 0:
+            pytest.skip("no such route for this problem")
+        nbytes = _lib.forward_backward_workspace_bytes(prob)
+        ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device="cuda")  # (NaN wherever it is read unwritten)
+        lse, out5 = torch.full((N,), 7.0, device="cuda"), torch.zeros(5, device="cuda")
+        nv, g = torch.zeros(1, dtype=torch.int64, device="cuda"), torch.ones(1, device="cuda")
+        rc = lib.lce_forward_backward(ctypes.byref(prob), x.data_ptr(), w.data_ptr(), y.data_ptr(), g.data_ptr(), lse.data_ptr(),
+                                      out5.data_ptr(), nv.data_ptr(), dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), nbytes,
+                                      torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        outs.append((lse, out5, nv, dx, dw))
+    (lse, out5, nv, dx, dw), (lse_p, out5_p, nv_p, dx_p, dw_p) = outs
+    # each logit is one accumulator's sum in the order of K, and a slice's sums are formed alike: the same bit for bit.  (dx and dW
+    # have the workgroups that the limit leaves, and cut along K accordingly: fp32 sums of terms of one rounding, in another order,
+    # and an fp32 sum next to the boundary of a 16-bit rounding may fall to either side, 2^-8 of it in bf16.)
+    assert nv.item() == nv_p.item() == int((y != -1).sum())
+    assert torch.equal(lse, lse_p) and torch.equal(out5, out5_p)
+    for got, want in ((dx, dx_p), (dw, dw_p)):
+        assert not torch.isnan(got).any()
+        if want.double().norm() > 0:
+            assert rel_errors(got, want)[1] <= (1e-6 if dtype == torch.float32 else 1e-3)
+        else:
+            assert not got.any()
