@@ -347,6 +347,19 @@ int lce_forward_backward(const lce_problem* p, const void* x, const void* w, con
 int lce_scale(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* factor, void* stream);
 
 /*
+ * *out = the address, on the current device, of a float that holds 1 for as long as the process lives: the grad_out of a caller
+ * that learns the upstream gradient later, without a buffer and a launch to fill it.  From version 800 on.
+ */
+int lce_unit_gradient(const float** out);
+
+/*
+ * lce_scale for both gradients of a call in one launch, by *factor / *divisor (divisor NULL: by *factor); either gradient may
+ * be NULL.  From version 800 on.
+ */
+int lce_scale_gradients(void* dx, int dx_dtype, int64_t dx_rows, int64_t dx_cols, int64_t lddx, void* dw, int dw_dtype,
+                        int64_t dw_rows, int64_t dw_cols, int64_t lddw, const float* factor, const float* divisor, void* stream);
+
+/*
  * *out (1 float, device) = the largest power of two that is not above the
  * number of labels in y[0 .. N) that are not ignore_index (1 if there is none):
  * the grad_out to give lce_forward_backward for fp16 gradients whose upstream

@@ -33,6 +33,8 @@ EXPORTS = (
     "lce_forward_backward_plan",
     "lce_forward_backward",
     "lce_scale",
+    "lce_scale_gradients",
+    "lce_unit_gradient",
     "lce_stand_in",
     "lce_pad_rows",
     "lce_transpose_rows",
@@ -112,6 +114,10 @@ def load():
     lib.lce_forward_backward.argtypes = [P, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
     lib.lce_scale.restype = ctypes.c_int
     lib.lce_scale.argtypes = [vp, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, vp, vp]
+    lib.lce_scale_gradients.restype = ctypes.c_int
+    lib.lce_scale_gradients.argtypes = [vp, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64] * 2 + [vp, vp, vp]
+    lib.lce_unit_gradient.restype = ctypes.c_int
+    lib.lce_unit_gradient.argtypes = [ctypes.POINTER(vp)]
     lib.lce_stand_in.restype = ctypes.c_int
     lib.lce_stand_in.argtypes = [vp, ctypes.c_int64, ctypes.c_int64, vp, vp]
     lib.lce_pad_rows.restype = ctypes.c_int
@@ -120,6 +126,13 @@ def load():
     lib.lce_transpose_rows.argtypes = lib.lce_pad_rows.argtypes
     _lib = lib
     return lib
+
+
+def unit_gradient() -> int:
+    """Address of a float on the current device that holds 1."""
+    p = ctypes.c_void_p(0)
+    raise_for_status(load().lce_unit_gradient(ctypes.byref(p)), "lce_unit_gradient")
+    return p.value
 
 
 def dtype_code(dt: torch.dtype) -> int:

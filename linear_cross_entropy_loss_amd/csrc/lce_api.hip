@@ -24,6 +24,28 @@ size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 bool is16(int d) { return d == LCE_BF16 || d == LCE_F16; }
 
+int route_of(const lce_problem* p) { return p->route & ~LCE_ROUTE_EXACT_SUMS; }
+
+// The last plan of a kind that this thread made.  A call asks for its plan up to three times (whether the route covers the
+// problem, the workspace, the launches), and a training step for the same one as the step before; a plan follows from the
+// problem's numbers alone, all of which are compared, and takes 1 to 4 us of the 30 to 60 that a call costs the host.
+template <class Plan> struct LastPlan {
+  lce_problem of;
+  bool made = false;
+  int result;
+  Plan plan;
+  template <class Make> int get(const lce_problem* p, Plan* out, Make make) {
+    if (!made || memcmp(&of, p, sizeof(of)) != 0) {
+      made = false;
+      result = make(p, &plan);
+      of = *p;
+      made = true;
+    }
+    *out = plan;
+    return result;
+  }
+};
+
 int check(const lce_problem* p, bool backward) {
   if (!p) return LCE_EINVAL_ARG;
   if (p->N <= 0 || p->H <= 0 || p->V <= 0 || p->n_chunk <= 0) return LCE_EINVAL_SHAPE;
@@ -39,9 +61,7 @@ int check(const lce_problem* p, bool backward) {
   if (p->pack_rows != LCE_PACK_AUTO && p->pack_rows != LCE_PACK_ALWAYS && p->pack_rows != LCE_PACK_NEVER) return LCE_EINVAL_ARG;
   if (p->max_workgroups < 0) return LCE_EINVAL_ARG;
   if (p->w_layout != LCE_W_HV && p->w_layout != LCE_W_VH) return LCE_EINVAL_ARG;
-  if ((p->route & ~LCE_ROUTE_EXACT_SUMS) != LCE_ROUTE_AUTO && (p->route & ~LCE_ROUTE_EXACT_SUMS) != LCE_ROUTE_ONE_PASS &&
-      (p->route & ~LCE_ROUTE_EXACT_SUMS) != LCE_ROUTE_TWO_PASS)
-    return LCE_EINVAL_ARG;
+  if (route_of(p) != LCE_ROUTE_AUTO && route_of(p) != LCE_ROUTE_ONE_PASS && route_of(p) != LCE_ROUTE_TWO_PASS) return LCE_EINVAL_ARG;
   const bool vh = p->w_layout == LCE_W_VH;
   // (V, H) weight: both operands of the logit contraction run along H in memory, so no 16-byte piece may
   // straddle the end of a row (H a multiple of 8), and there is no bf16-pair form of it
@@ -228,7 +248,7 @@ double kernel_cost(double T, double L, double e, bool parts) {
 // N * H * 4 bytes, the fp32 x_grad buffer the reference allocates next to its logits chunk (ops.py:693) and
 // this library does not -- and by the split-K partial sums.  If even that fails, the narrowest split is used:
 // the bound is a target, the operator never refuses a shape.
-int plan_bwd(const lce_problem* p, BwdPlan* b) {
+int make_plan_bwd(const lce_problem* p, BwdPlan* b) {
   const size_t strict = (size_t)p->n_chunk * (size_t)p->V * 4;
   const size_t dz_cap = (size_t)1 << 30;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Hp = (size_t)lce::padded_hidden(p->H);
@@ -328,6 +348,11 @@ int plan_bwd(const lce_problem* p, BwdPlan* b) {
   return LCE_EWORKSPACE;
 }
 
+int plan_bwd(const lce_problem* p, BwdPlan* b) {
+  static thread_local LastPlan<BwdPlan> last;
+  return last.get(p, b, make_plan_bwd);
+}
+
 // lce_forward_backward: the logits are computed once.  The tokens go through in chunks of `nc` rows against the
 // whole vocabulary: logit kernel (partials of the loss, and e = exp(z - slice max) into the stage), row merge
 // (lse), the pass that turns e into dz, then dx of the chunk (complete: K = the vocabulary) and the chunk's
@@ -367,15 +392,20 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
 // on one box: 5.9 % at config 3, 7-10 % at the output layers of Llama-3-8B / Llama-2-7B, 11-20 % at config 4's
 // N_chunk_size = 2048 points, 0.7 % at the headline shape (which keeps the halves).  Never with LCE_ROUTE_EXACT_SUMS.
 constexpr double kBytesMargin = 0.97;
-bool plan_fused(const lce_problem* p, bool want_dx, bool want_dw, FusedPlan* f) {
-  const bool halves = plan_fused_with(p, want_dx, want_dw, false, f);
-  if ((p->route & LCE_ROUTE_EXACT_SUMS) || !want_dw || p->dw_dtype == LCE_F32) return halves;
+int make_plan_fused(const lce_problem* p, FusedPlan* f) {
+  const bool halves = plan_fused_with(p, true, true, false, f);
+  if ((p->route & LCE_ROUTE_EXACT_SUMS) || p->dw_dtype == LCE_F32) return halves;
   FusedPlan b;
-  if (plan_fused_with(p, want_dx, want_dw, true, &b) && (!halves || b.cost < kBytesMargin * f->cost)) {
+  if (plan_fused_with(p, true, true, true, &b) && (!halves || b.cost < kBytesMargin * f->cost)) {
     *f = b;
     return true;
   }
   return halves;
+}
+// (for both gradients, whichever the caller wants: the workspace does not depend on that)
+bool plan_fused(const lce_problem* p, FusedPlan* f) {
+  static thread_local LastPlan<FusedPlan> last;
+  return last.get(p, f, make_plan_fused) != 0;
 }
 
 bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, FusedPlan* f) {
@@ -384,7 +414,7 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
   f->factors = factors_in_gradients(p);
   const double mul = f->factors ? 1.06 : 1.0;
   const bool x16 = p->x_dtype == LCE_BF16 || p->x_dtype == LCE_F16;
-  if (!x16 || (p->w_dtype != p->x_dtype && p->w_dtype != LCE_F32) || (p->route & ~LCE_ROUTE_EXACT_SUMS) == LCE_ROUTE_TWO_PASS) return false;
+  if (!x16 || (p->w_dtype != p->x_dtype && p->w_dtype != LCE_F32) || route_of(p) == LCE_ROUTE_TWO_PASS) return false;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Vp = (size_t)lce::padded_vocab(p->V), Hp = (size_t)lce::padded_hidden(p->H);
   const size_t dxes = p->dx_dtype == LCE_F32 ? 4 : 2;
   // (packed rows of dx go to their tokens through 32-bit offsets into dx)
@@ -480,7 +510,7 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
   // (the factors instead: hardly any traffic, but a launch of some 15 us per chunk that starts from cold)
   const double scale_pass = f->factors ? 12.0 * (double)f->chunks : (double)Np * (double)Vp * 4.0 / 8.0e6;
   f->cost = best + scale_pass;
-  if ((p->route & ~LCE_ROUTE_EXACT_SUMS) == LCE_ROUTE_AUTO && plan_bwd(p, &b) == LCE_OK) {
+  if (route_of(p) == LCE_ROUTE_AUTO && plan_bwd(p, &b) == LCE_OK) {
     const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false) + b.cost;
     // (sums of 24 bits have to be ahead of two passes, which are exact, by the margin as well)
     if (best + scale_pass > two * (lo8 ? kBytesMargin : 1.0)) {
@@ -498,20 +528,22 @@ bool misaligned(const void* p) { return ((uintptr_t)p & 15) != 0; }
 // device address is looked up once per device and kept in g_scratch_ptr.
 constexpr size_t kStaticScratchBytes = LCE_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
+// An upstream gradient of 1 (lce_unit_gradient).
+static __device__ float unit_gradient = 1.f;
 constexpr int kMaxDevices = 64;
-std::atomic<void*> g_scratch_ptr[kMaxDevices];
+std::atomic<void*> g_scratch_ptr[kMaxDevices], g_unit_ptr[kMaxDevices];
 
-// Device address of `scratch` on the current device (looked up on the first call per device).
-int static_scratch(void** out) {
+// Device address of `scratch` or `unit_gradient` on the current device (looked up on the first call per device).
+template <class Symbol> int static_address(std::atomic<void*>* known, const Symbol& symbol, void** out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
   if (dev < 0 || dev >= kMaxDevices) return LCE_EINVAL_ARG;
-  void* ptr = g_scratch_ptr[dev].load(std::memory_order_acquire);
+  void* ptr = known[dev].load(std::memory_order_acquire);
   if (ptr == nullptr) {
-    e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || ptr == nullptr) return hip_fail(e, "hipGetSymbolAddress(scratch)");
-    g_scratch_ptr[dev].store(ptr, std::memory_order_release);  // every thread finds the same address
+    e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(symbol));
+    if (e != hipSuccess || ptr == nullptr) return hip_fail(e, "hipGetSymbolAddress");
+    known[dev].store(ptr, std::memory_order_release);  // every thread finds the same address
   }
   *out = ptr;
   return LCE_OK;
@@ -802,7 +834,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
 
 extern "C" {
 
-int lce_version(void) { return 700; }  // 0.7.0: lce_transpose_rows
+int lce_version(void) { return 800; }  // 0.8.0: lce_scale_gradients, lce_unit_gradient
 
 const char* lce_strerror(int status) {
   switch (status) {
@@ -865,7 +897,7 @@ int lce_forward_static(const lce_problem* p, const void* x, const void* w, const
   if (rc != LCE_OK) return rc;
   if (plan_fwd(p).total > kStaticScratchBytes) return LCE_ESTATIC;  // before any device call
   void* ptr = nullptr;
-  rc = static_scratch(&ptr);
+  rc = static_address(g_scratch_ptr, scratch, &ptr);
   if (rc != LCE_OK) return rc;
   // Nothing in the forward scratch has to start at zero: every cell a kernel reads was written by an
   // earlier kernel of the same call, so the contents the previous call left behind are never looked at.
@@ -992,6 +1024,31 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
   return LCE_OK;
 }
 
+int lce_unit_gradient(const float** out) {
+  if (!out) return LCE_EINVAL_ARG;
+  void* one = nullptr;
+  const int rc = static_address(g_unit_ptr, unit_gradient, &one);
+  if (rc == LCE_OK) *out = (const float*)one;
+  return rc;
+}
+
+int lce_scale_gradients(void* dx, int dx_dtype, int64_t dx_rows, int64_t dx_cols, int64_t lddx, void* dw, int dw_dtype,
+                        int64_t dw_rows, int64_t dw_cols, int64_t lddw, const float* factor, const float* divisor, void* stream) {
+  if (!factor) return LCE_EINVAL_ARG;
+  const lce::ScaleTask t[2] = {{dx, dx_dtype, dx_rows, dx_cols, lddx}, {dw, dw_dtype, dw_rows, dw_cols, lddw}};
+  for (const lce::ScaleTask& k : t) {
+    if (!k.t) continue;
+    if (k.dtype != LCE_BF16 && k.dtype != LCE_F16 && k.dtype != LCE_F32) return LCE_EINVAL_DTYPE;
+    if (k.rows < 0 || k.cols < 0 || k.ld < k.cols || k.ld % (k.dtype == LCE_F32 ? 4 : 8) || misaligned(k.t)) return LCE_EINVAL_ARG;
+  }
+  int num_cus = 0;
+  int rc = current_num_cus(&num_cus, 0);
+  if (rc != LCE_OK) return rc;
+  hipError_t e = lce::launch_scale_two(t[0], t[1], factor, divisor, num_cus, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "scale_two");
+  return LCE_OK;
+}
+
 int lce_scale(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* factor, void* stream) {
   if (dtype != LCE_BF16 && dtype != LCE_F16 && dtype != LCE_F32) return LCE_EINVAL_DTYPE;
   if (rows < 0 || cols < 0 || ld < cols || ld % (dtype == LCE_F32 ? 4 : 8) || !factor) return LCE_EINVAL_ARG;
@@ -1041,7 +1098,7 @@ int lce_forward_backward_workspace_bytes(const lce_problem* p, size_t* bytes) {
   if (rc != LCE_OK) return rc;
   if (!bytes) return LCE_EINVAL_ARG;
   FusedPlan f;
-  if (plan_fused(p, true, true, &f)) { *bytes = f.total; return LCE_OK; }
+  if (plan_fused(p, &f)) { *bytes = f.total; return LCE_OK; }
   size_t fw = 0, bw = 0;
   rc = lce_workspace_bytes(p, &fw, &bw);
   if (rc != LCE_OK) return rc;
@@ -1053,7 +1110,7 @@ int lce_forward_backward_plan(const lce_problem* p, int64_t* chunks, int64_t* ch
   int rc = check(p, true);
   if (rc != LCE_OK) return rc;
   FusedPlan f;
-  const bool ok = plan_fused(p, true, true, &f);
+  const bool ok = plan_fused(p, &f);
   if (chunks) *chunks = ok ? f.chunks : 0;
   if (chunk_rows) *chunk_rows = ok ? f.nc : 0;
   return LCE_OK;
@@ -1067,7 +1124,7 @@ int lce_forward_backward(const lce_problem* p, const void* x, const void* w, con
   if (!x || !w || !y || !grad_out || !lse || !out5 || !n_valid) return LCE_EINVAL_ARG;
   if (misaligned(x) || misaligned(w) || misaligned(dx) || misaligned(dw)) return LCE_EINVAL_ARG;
   FusedPlan f;
-  if ((dx || dw) && plan_fused(p, true, true, &f)) {
+  if ((dx || dw) && plan_fused(p, &f)) {
     if (!ws || ws_bytes < f.total || misaligned(ws)) return LCE_EWORKSPACE;
     return fused_impl(p, f, x, w, y, grad_out, lse, out5, n_valid, dx, dw, ws, stream);
   }

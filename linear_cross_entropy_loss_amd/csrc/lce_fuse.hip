@@ -170,12 +170,9 @@ LCE_DEV float scaled(float v, float f) {
   return p;
 }
 
-template <class E, int PER>
-__global__ __launch_bounds__(256) void scale_rows_kernel(E* t, int64_t rows, int64_t cols, int64_t ld, const float* g) {
-  const float f = g[0];
-  if (f == 1.f) return;
+template <class E, int PER> LCE_DEV void scale_rows(E* t, int64_t rows, int64_t cols, int64_t ld, float f, int64_t first, int64_t step) {
   const int64_t pieces = (cols + PER - 1) / PER;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < rows * pieces; i += (int64_t)gridDim.x * 256) {
+  for (int64_t i = first; i < rows * pieces; i += step) {
     const int64_t r = i / pieces, c0 = (i - r * pieces) * PER;
     E* at = t + r * ld + c0;
     if (c0 + PER <= cols) {
@@ -191,25 +188,42 @@ __global__ __launch_bounds__(256) void scale_rows_kernel(E* t, int64_t rows, int
     }
   }
 }
+LCE_DEV void scale_task(const ScaleTask& t, float f, int64_t first, int64_t step) {
+  if (t.t == nullptr) return;
+  if (t.dtype == DT_BF16) scale_rows<__bf16, 8>((__bf16*)t.t, t.rows, t.cols, t.ld, f, first, step);
+  else if (t.dtype == DT_F16) scale_rows<_Float16, 8>((_Float16*)t.t, t.rows, t.cols, t.ld, f, first, step);
+  else scale_rows<float, 4>((float*)t.t, t.rows, t.cols, t.ld, f, first, step);
+}
+// Both gradients of a call in one launch: where the factor is 1, which is the rule, the launch is all there is to it.
+__global__ __launch_bounds__(256) void scale_two_kernel(const ScaleTask t0, const ScaleTask t1, const float* g, const float* d) {
+  const float f = d != nullptr ? g[0] / d[0] : g[0];
+  if (f == 1.f) return;
+  const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+  scale_task(t0, f, first, step);
+  scale_task(t1, f, first, step);
+}
 
 }  // namespace
 
-hipError_t launch_scale_rows(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* g, int num_cus,
-                             hipStream_t s) {
-  if (rows <= 0 || cols <= 0) return hipSuccess;
-  const int per = dtype == DT_F32 ? 4 : 8;
-  const int64_t work = rows * ((cols + per - 1) / per);
+hipError_t launch_scale_two(const ScaleTask& t0, const ScaleTask& t1, const float* g, const float* d, int num_cus, hipStream_t s) {
+  int64_t work = 0;
+  for (const ScaleTask* t : {&t0, &t1})
+    if (t->t != nullptr) {
+      if (t->dtype != DT_BF16 && t->dtype != DT_F16 && t->dtype != DT_F32) return hipErrorInvalidValue;
+      const int per = t->dtype == DT_F32 ? 4 : 8;
+      const int64_t w = t->rows * ((t->cols + per - 1) / per);
+      work = w > work ? w : work;
+    }
+  if (work <= 0) return hipSuccess;
   int64_t grid = (work + 255) / 256;
   if (grid > (int64_t)num_cus * 16) grid = (int64_t)num_cus * 16;
-  if (dtype == DT_BF16)
-    hipLaunchKernelGGL((scale_rows_kernel<__bf16, 8>), dim3((unsigned)grid), dim3(256), 0, s, (__bf16*)t, rows, cols, ld, g);
-  else if (dtype == DT_F16)
-    hipLaunchKernelGGL((scale_rows_kernel<_Float16, 8>), dim3((unsigned)grid), dim3(256), 0, s, (_Float16*)t, rows, cols, ld, g);
-  else if (dtype == DT_F32)
-    hipLaunchKernelGGL((scale_rows_kernel<float, 4>), dim3((unsigned)grid), dim3(256), 0, s, (float*)t, rows, cols, ld, g);
-  else
-    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(scale_two_kernel, dim3((unsigned)grid), dim3(256), 0, s, t0, t1, g, d);
   return hipGetLastError();
+}
+
+hipError_t launch_scale_rows(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* g, int num_cus,
+                             hipStream_t s) {
+  return launch_scale_two(ScaleTask{t, dtype, rows, cols, ld}, ScaleTask{}, g, nullptr, num_cus, s);
 }
 
 hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s) {

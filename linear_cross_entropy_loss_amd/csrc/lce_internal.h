@@ -238,6 +238,13 @@ hipError_t launch_stage_factors(const BwdArgs& a, hipStream_t s);
 // t[r][c] *= g[0] (device scalar), in fp32; nothing is touched when g[0] == 1.  Rows on 16-byte boundaries.
 hipError_t launch_scale_rows(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* g, int num_cus,
                              hipStream_t s);
+// The same for two matrices (either may be absent: t null) in one launch, by the factor g[0] / d[0] (d null: g[0]).
+struct ScaleTask {
+  void* t;
+  int dtype;
+  int64_t rows, cols, ld;
+};
+hipError_t launch_scale_two(const ScaleTask& t0, const ScaleTask& t1, const float* g, const float* d, int num_cus, hipStream_t s);
 hipError_t launch_bwd_dx(const BwdArgs& a, hipStream_t s);
 hipError_t launch_bwd_dw(const BwdArgs& a, hipStream_t s);
 // dst[h][c] = 16-bit rounding of src[h * ld + v0 + c] for c < vw, 0 for vw <= c < dst_ld; h < H.

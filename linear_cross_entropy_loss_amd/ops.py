@@ -73,9 +73,18 @@ def _route_mode() -> int:
     return 2 if v == "always" else (1 if v else 0)
 
 
+_no_context = contextlib.nullcontext()
+
+
 def _on_device(device):
     """A context in which `device`, a tensor's, is the current one."""
-    return contextlib.nullcontext() if device.index == torch.cuda.current_device() else torch.cuda.device(device)
+    return _no_context if device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
+def _stream(device):
+    """The current stream of `device`, a tensor's, as the C interface takes it (the number that
+    ``torch.cuda.current_stream(device).cuda_stream`` gives, without the two objects around it)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t):
@@ -141,7 +150,7 @@ def _aligned_rows(t, what=None):
         copy = _lib.load().lce_pad_rows if by_rows else _lib.load().lce_transpose_rows
         with _on_device(t.device):
             rc = copy(_ptr(t), _lib.dtype_code(t.dtype), rows, cols, t.stride(0 if by_rows else 1), _ptr(padded), padded.stride(0),
-                      torch.cuda.current_stream(t.device).cuda_stream)
+                      _stream(t.device))
         _lib.raise_for_status(rc, "lce_pad_rows" if by_rows else "lce_transpose_rows")
     else:  # (elements apart in both directions)
         padded[:, :cols] = t
@@ -177,7 +186,9 @@ def _weight_rows(At, layout):
 
 def _empty_rows(rows, cols, dtype, device):
     """Uninitialised (rows, cols) matrix whose row stride satisfies the kernels' alignment rule."""
-    return torch.empty((rows, _padded_cols(cols, dtype)), dtype=dtype, device=device)[:, :cols]
+    padded = _padded_cols(cols, dtype)
+    t = torch.empty((rows, padded), dtype=dtype, device=device)
+    return t if padded == cols else t[:, :cols]
 
 
 def _autocast_x(x, At):
@@ -248,9 +259,8 @@ def _stand_in_gradient(x, y1, ignore_index):
     of the order of the per-token gradient -- and divided by it again when the real one is multiplied in."""
     if x.dtype == torch.float16:
         pre = torch.empty(1, dtype=torch.float32, device=x.device)
-        stream = torch.cuda.current_stream(x.device).cuda_stream
         with _on_device(x.device):
-            rc = _lib.load().lce_stand_in(_ptr(y1), y1.numel(), int(ignore_index), _ptr(pre), stream)
+            rc = _lib.load().lce_stand_in(_ptr(y1), y1.numel(), int(ignore_index), _ptr(pre), _stream(x.device))
         _lib.raise_for_status(rc, "lce_stand_in")
         return pre
     return torch.ones(1, dtype=torch.float32, device=x.device)
@@ -289,26 +299,34 @@ def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_c
         lse = torch.empty(N, dtype=torch.float32, device=dev)
         out5 = torch.empty(5, dtype=torch.float32, device=dev)
         n_valid = torch.empty(1, dtype=torch.int64, device=dev)
-        pre = _stand_in_gradient(x, y1, ignore_index)  # (the upstream gradient is not known yet)
-        stream = torch.cuda.current_stream(dev).cuda_stream
-        rc = lib.lce_forward_backward(ctypes.byref(prob), _ptr(x), _ptr(w), _ptr(y1), _ptr(pre), _ptr(lse), _ptr(out5),
-                                      _ptr(n_valid), _ptr(dx), _ptr(dw), _ptr(ws), nbytes, stream)
+        # (the upstream gradient is not known yet)
+        pre = _stand_in_gradient(x, y1, ignore_index) if x.dtype == torch.float16 else None
+        g = _lib.unit_gradient() if pre is None else _ptr(pre)
+        rc = lib.lce_forward_backward(ctypes.byref(prob), _ptr(x), _ptr(w), _ptr(y1), g, _ptr(lse), _ptr(out5), _ptr(n_valid),
+                                      _ptr(dx), _ptr(dw), _ptr(ws), nbytes, _stream(dev))
         _lib.raise_for_status(rc, "lce_forward_backward")
         del ws
-    return (out5, lse, n_valid, x, y1, w, layout, dx, dw, (pre if x.dtype == torch.float16 else None)), None
+    return (out5, lse, n_valid, x, y1, w, layout, dx, dw, pre), None
 
 
-def _scale_grad(t, grad_output):
-    """t *= grad_output in place, the product formed in fp32 (nothing is touched when grad_output is 1)."""
-    if t is None:
-        return
-    lib = _lib.load()
-    with _on_device(t.device):
-        g = grad_output.detach().to(device=t.device, dtype=torch.float32).reshape(1).contiguous()
-        stream = torch.cuda.current_stream(t.device).cuda_stream
-        rc = lib.lce_scale(_ptr(t), _lib.dtype_code(t.dtype), t.shape[0], t.shape[1], t.stride(0), _ptr(g),
-                           stream)
-        _lib.raise_for_status(rc, "lce_scale")
+def _device_scalar(g, device):
+    """The one number of `g` in fp32 on `device`: `g` itself where it is that."""
+    if g.dtype == torch.float32 and g.device == device and g.numel() == 1:
+        return g
+    return g.detach().to(device=device, dtype=torch.float32).reshape(1).contiguous()
+
+
+def _scale_grads(dx, dw, grad_output, pre):
+    """dx and dw (either may be None) times grad_output / pre (None: 1) in place, quotient and products formed in fp32; nothing is
+    touched when that is 1."""
+    device = (dx if dx is not None else dw).device
+    with _on_device(device):
+        g = _device_scalar(grad_output, device)
+        tasks = [a for t in (dx, dw)
+                 for a in ((None, 0, 0, 0, 0) if t is None
+                           else (t.data_ptr(), _lib.dtype_code(t.dtype), t.shape[0], t.shape[1], t.stride(0)))]
+        rc = _lib.load().lce_scale_gradients(*tasks, _ptr(g), _ptr(pre), _stream(device))
+        _lib.raise_for_status(rc, "lce_scale_gradients")
 
 
 def _forward_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, given=None):
@@ -334,9 +352,8 @@ def _forward_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_ch
         lse = torch.empty(N, dtype=torch.float32, device=dev)
         out5 = torch.empty(5, dtype=torch.float32, device=dev)
         n_valid = torch.empty(1, dtype=torch.int64, device=dev)
-        stream = torch.cuda.current_stream(dev).cuda_stream
         rc = lib.lce_forward(ctypes.byref(prob), _ptr(x), _ptr(w), _ptr(y1), _ptr(lse), _ptr(out5),
-                             _ptr(n_valid), _ptr(ws), fwd_bytes, stream)
+                             _ptr(n_valid), _ptr(ws), fwd_bytes, _stream(dev))
         _lib.raise_for_status(rc, "lce_forward")
         del ws
     return out5, lse, n_valid, x, y1, w, layout
@@ -363,10 +380,9 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
             lib = _lib.load()
             bwd_bytes = _lib.backward_workspace_bytes(prob)
             ws = torch.empty(bwd_bytes, dtype=torch.uint8, device=dev)
-            g = grad_output.detach().to(device=dev, dtype=torch.float32).reshape(1).contiguous()
-            stream = torch.cuda.current_stream(dev).cuda_stream
+            g = _device_scalar(grad_output, dev)
             rc = lib.lce_backward(ctypes.byref(prob), _ptr(x), _ptr(w), _ptr(y1), _ptr(lse), _ptr(n_valid),
-                                  _ptr(g), _ptr(dx), _ptr(dw), _ptr(ws), bwd_bytes, stream)
+                                  _ptr(g), _ptr(dx), _ptr(dw), _ptr(ws), bwd_bytes, _stream(dev))
             _lib.raise_for_status(rc, "lce_backward")
             del ws
     if dx is not None and not dx.is_contiguous():
@@ -381,8 +397,9 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
 class LinearXentImplementation(torch.autograd.Function):
     """The reference's autograd Function (``ops.py:661-810``): same arguments, same 5-tuple."""
 
+    # (Not wrapped in torch.amp.custom_fwd / custom_bwd: forward casts by _autocast_x, and backward makes device calls and casts
+    # to float32 only, which autocast leaves alone; the wrappers' contexts cost the host 12 us of a forward + backward.)
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
     def forward(
         ctx,
         x_in,
@@ -424,7 +441,6 @@ class LinearXentImplementation(torch.autograd.Function):
         return loss, z_reg, logit_max, logit_ent, logit_norm
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, grad_output, void0=None, void1=None, void2=None, void3=None):
         x, y1, w, lse, n_valid = ctx.saved_tensors
         ignore_index, z_regularization, logit_scale, N_chunk_size, pack, layout = ctx.lce_cfg
@@ -435,9 +451,7 @@ class LinearXentImplementation(torch.autograd.Function):
             # computed in the forward for an upstream gradient of 1 (ops.py:810 does the same multiplication); a
             # later backward over the same graph finds nothing here and recomputes
             dx, dw, pre = grads
-            factor = grad_output.detach().to(torch.float32) if pre is None else grad_output.detach().to(torch.float32) / pre
-            _scale_grad(dx, factor)
-            _scale_grad(dw, factor)
+            _scale_grads(dx, dw, grad_output, pre)
             dx, dw = _finish_grads(dx, dw, layout)
         else:
             dx, dw = _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regularization, logit_scale,
@@ -572,9 +586,8 @@ def _op_scale(t: torch.Tensor, factor: torch.Tensor) -> torch.Tensor:
         lib = _lib.load()
         with _on_device(t.device):
             g = factor.detach().to(device=t.device, dtype=torch.float32).reshape(1).contiguous()
-            stream = torch.cuda.current_stream(t.device).cuda_stream
             # (one row of n elements: any dense tensor, whatever its row length)
-            rc = lib.lce_scale(_ptr(flat), _lib.dtype_code(t.dtype), 1, n, n + (-n) % 8, _ptr(g), stream)
+            rc = lib.lce_scale(_ptr(flat), _lib.dtype_code(t.dtype), 1, n, n + (-n) % 8, _ptr(g), _stream(t.device))
             _lib.raise_for_status(rc, "lce_scale")
     return out
 

@@ -667,3 +667,19 @@ def test_workspace_of_one_direction_is_that_of_both(lib):
         assert (_lib.forward_workspace_bytes(p), _lib.backward_workspace_bytes(p)) == (f.value, b.value)
     with pytest.raises(ValueError, match="linear_cross_entropy: .*outside the range"):
         _lib.forward_workspace_bytes(_prob(N=0), "linear_cross_entropy")
+
+
+def test_a_plan_belongs_to_its_problem_alone():
+    """The library keeps the last plan that a thread made: problems taken in turn get the plans they get by themselves."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    def prob(N, n_chunk, route):
+        dt = torch.bfloat16
+        return _lib.make_problem(N, 512, 32000, 512, 32000, 512, 32000, dt, dt, dt, dt, -1, 1.0, 0.0, n_chunk, False, 0, 0, 0, 0, route)
+
+    problems = [prob(N, c, r) for N in (300, 8192) for c in (512, 4096) for r in (_lib.ROUTE_ONE_PASS, _lib.ROUTE_TWO_PASS)]
+    plans = lambda p: (_lib.forward_backward_plan(p), _lib.forward_backward_workspace_bytes(p), _lib.backward_plan(p),  # noqa: E731
+                       _lib.backward_workspace_bytes(p))
+    alone = [[plans(p) for _ in range(2)][1] for p in problems]
+    assert [plans(p) for p in problems] == alone and [plans(p) for p in reversed(problems)] == alone[::-1]
+    assert len(set(alone)) > 4

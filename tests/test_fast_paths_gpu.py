@@ -326,3 +326,32 @@ def test_small_logit_tiles_match_the_persistent_kernels(N, H, V, dtype, mon, lay
             assert rel_errors(got, want)[1] <= (1e-6 if dtype == torch.float32 else 1e-3)
         else:
             assert not got.any()
+
+
+# both gradients times one factor in one launch: either absent, types apart, rows that end inside a 16-byte piece, one element, a
+# factor and a quotient of 1 (nothing touched), fp32 products rounded once more to the type
+@pytest.mark.parametrize("shapes,dtypes", [(((1, 1), None), (torch.bfloat16, None)), (((37, 101), (5, 260)), (torch.bfloat16, torch.float32)),
+                                           ((None, (300, 7)), (None, torch.float16)), (((70, 1003), (1003, 70)), (torch.float16, torch.float16))])
+@pytest.mark.parametrize("factor,divisor", [(1.0, None), (0.37, None), (4096.0, 4096.0), (3.0, 7.0)])
+def test_both_gradients_scaled_in_one_launch(shapes, dtypes, factor, divisor):
+    from linear_cross_entropy_loss_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    ts = []
+    for shape, dtype in zip(shapes, dtypes):
+        if shape is None:
+            ts.append(None)
+            continue
+        t = ops._empty_rows(*shape, dtype, "cuda")
+        torch.as_strided(t, (shape[0], t.stride(0)), (t.stride(0), 1)).fill_(7.0)
+        t.copy_(torch.randn(shape, generator=gen, device="cuda"))
+        ts.append(t)
+    g = torch.full((), factor, device="cuda")
+    d = None if divisor is None else torch.full((1,), divisor, device="cuda")
+    f = g if d is None else g / d[0]
+    want = [None if t is None else (t.float() * f).to(t.dtype) for t in ts]
+    ops._scale_grads(*ts, g, d)
+    for t, w in zip(ts, want):
+        if t is not None:
+            assert torch.equal(t, w)
+            assert (torch.as_strided(t, (t.shape[0], t.stride(0)), (t.stride(0), 1))[:, t.shape[1]:] == 7.0).all()
