@@ -107,22 +107,22 @@ __global__ __launch_bounds__(256) void stage_factors_kernel(const BwdArgs a) {
   const int t = threadIdx.x;
   const int64_t tok = t0 + t;
   const bool exists = tok < rows;
+  // (everything is asked for at once: a launch is a few latencies long)
   const int64_t yy = exists ? a.y[tok] : a.ignore_index;
+  const float lse = exists ? a.lse[tok] : 0.f, zt = a.tgt[tok];  // (tgt: written where the label is a column of W)
+  float f[kSlices];
+#pragma unroll
+  for (int i = 0; i < kSlices; ++i) f[i] = s0 + i < slices ? a.part_max[(int64_t)(s0 + i) * a.nc + tok] : 0.f;
   const bool valid = yy != a.ignore_index;
-  const float lse = valid ? a.lse[tok] : 0.f;
   float gain = 1.f + 2.f * a.z_reg * lse;
   if (a.dz_shift != 0) gain = fminf(fmaxf(gain, -63.f), 63.f);  // (as in lce_bwd_dz.hip)
   if (t == 0) sh_n = 0;
-  float f[kSlices];
 #pragma unroll
-  for (int i = 0; i < kSlices; ++i) {
-    const float m = s0 + i < slices && valid ? a.part_max[(int64_t)(s0 + i) * a.nc + tok] : 0.f;
-    f[i] = valid ? __builtin_amdgcn_exp2f((m - lse) * kLog2e) * gain : 0.f;
-  }
+  for (int i = 0; i < kSlices; ++i) f[i] = valid ? __builtin_amdgcn_exp2f((f[i] - lse) * kLog2e) * gain : 0.f;
   __syncthreads();  // every partial has been read
   const int64_t rel = valid ? yy - (int64_t)s0 * kChunkV : -1;
   if (rel >= 0 && rel < kSlices * kChunkV && yy < a.vs) {
-    const float p = __builtin_amdgcn_exp2f(fmaf(a.tgt[tok] - lse, kLog2e, (float)a.dz_shift)) * gain;
+    const float p = __builtin_amdgcn_exp2f(fmaf(zt - lse, kLog2e, (float)a.dz_shift)) * gain;
     const int at = atomicAdd(&sh_n, 1);
     sh_list[at] = t;
     sh_rel[at] = (int)rel;
@@ -143,20 +143,32 @@ __global__ __launch_bounds__(256) void stage_factors_kernel(const BwdArgs a) {
       const_cast<float*>(a.dw_f)[(int64_t)(s0 + i) * a.nc + pw] = f[i];
     }
   __syncthreads();
-  for (int e = t >> 4; e < sh_n; e += 16) {  // 16 threads rewrite the 128 columns of one token
-    const int r = sh_list[e], hit_col = sh_rel[e] & (kChunkV - 1), piece = t & 15;
-    const int s = s0 + (sh_rel[e] / kChunkV);
-    u32x4_t* at = reinterpret_cast<u32x4_t*>(reinterpret_cast<E*>(a.dz) + dz_block_offset(blockIdx.y, 2 * s + (piece >> 3), a.vs) +
-                                             r * 64 + (piece & 7) * 8);
-    const u32x4_t v = *at;
-    const int hit = hit_col - piece * 8;  // 0..7: the target is element `hit` of this piece
-    u32x4_t o = scaled_piece<T>(v, sh_f[e]);
+  // 16 threads rewrite the 128 columns of one token, four tokens of theirs in flight (frequent labels: up to all 256 tokens)
+  const int n = sh_n, piece = t & 15;
+  for (int e0 = t >> 4; e0 < n; e0 += 64) {
+    u32x4_t* at[4];
+    u32x4_t v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (hit == 2 * j) o[j] = (o[j] & 0xffff0000u) | sh_tv[e];
-      if (hit == 2 * j + 1) o[j] = (o[j] & 0x0000ffffu) | ((unsigned)sh_tv[e] << 16);
+    for (int u = 0; u < 4; ++u) {
+      const int e = e0 + 16 * u < n ? e0 + 16 * u : e0;
+      at[u] = reinterpret_cast<u32x4_t*>(reinterpret_cast<E*>(a.dz) +
+                                         dz_block_offset(blockIdx.y, 2 * (s0 + sh_rel[e] / kChunkV) + (piece >> 3), a.vs) +
+                                         sh_list[e] * 64 + (piece & 7) * 8);
+      v[u] = *at[u];
     }
-    *at = o;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = e0 + 16 * u;
+      if (e >= n) break;
+      const int hit = (sh_rel[e] & (kChunkV - 1)) - piece * 8;  // 0..7: the target is element `hit` of this piece
+      u32x4_t o = scaled_piece<T>(v[u], sh_f[e]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (hit == 2 * j) o[j] = (o[j] & 0xffff0000u) | sh_tv[e];
+        if (hit == 2 * j + 1) o[j] = (o[j] & 0x0000ffffu) | ((unsigned)sh_tv[e] << 16);
+      }
+      *at[u] = o;
+    }
   }
 }
 
