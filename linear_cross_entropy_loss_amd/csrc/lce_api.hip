@@ -51,8 +51,7 @@ int check(const lce_problem* p, bool backward) {
   if (p->N <= 0 || p->H <= 0 || p->V <= 0 || p->n_chunk <= 0) return LCE_EINVAL_SHAPE;
   // Any N, H, V; only the row strides are constrained (below).
   if (p->N > (int64_t)1 << 30 || p->V > (int64_t)1 << 30 || p->H > (int64_t)1 << 20) return LCE_EINVAL_SHAPE;
-  // bf16 pairs: bwd_dz reaches the three parts of its stage through 32-bit byte offsets (two parts of at least
-  // Np * 256 * 2 bytes each)
+  // (fp32 activations: a limit that the layout of their stage does not need any more; calls beyond it stay refused)
   if (p->x_dtype == LCE_F32 && p->N > (int64_t)1 << 20) return LCE_EINVAL_SHAPE;
   const int xd = p->x_dtype, wd = p->w_dtype;
   const bool ok = (is16(xd) && (wd == xd || wd == LCE_F32)) || (xd == LCE_F32 && wd == LCE_F32);
@@ -355,7 +354,7 @@ int plan_bwd(const lce_problem* p, BwdPlan* b) {
 
 // lce_forward_backward: the logits are computed once.  The tokens go through in chunks of `nc` rows against the
 // whole vocabulary: logit kernel (partials of the loss, and e = exp(z - slice max) into the stage), row merge
-// (lse), the pass that turns e into dz, then dx of the chunk (complete: K = the vocabulary) and the chunk's
+// (lse), the pass that turns e into dz (or the factors by which the next two kernels do), then dx of the chunk (complete: K = the vocabulary) and the chunk's
 // term of dW, which is summed over the chunks in fp32 (the reference's fp32 At_grad, ops.py:692): in the caller's
 // buffer if dW is fp32, else as 16-bit halves -- the upper ones in the caller's dW, the lower ones in a plane here.
 // Everything counts towards the bound n_chunk * V * 4 (the reference's logits chunk, ops.py:700): the chunk is
@@ -806,7 +805,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
     }
     if ((dx || dw) && (ph & LCE_PHASE_BWD_DZ)) {
       e = f.factors ? lce::launch_stage_factors(a, s) : lce::launch_stage_scale(a, s);
-      if (e != hipSuccess) return hip_fail(e, "stage_scale");
+      if (e != hipSuccess) return hip_fail(e, f.factors ? "stage_factors" : "stage_scale");
     }
     if (dx && (ph & LCE_PHASE_BWD_DX)) {
       e = lce::launch_bwd_dx(a, s);

@@ -179,7 +179,8 @@ struct BwdArgs {
   //     e[token][v] = 2^dz_shift * exp(z[token][v] - m[token][v / 128])
   // in the stage, m = the largest logit of the token in that slice of 128 columns, together with the forward's
   // per-slice partials of the chunk: part_lse, part_max = m ([Vp/128][nc], as in FwdArgs) and the target logits
-  // tgt (first row of the chunk).  Once the rows' lse are known, launch_stage_scale turns e into dz in place.
+  // tgt (first row of the chunk).  Once the rows' lse are known, launch_stage_scale turns e into dz in
+  // place, or the dx and dW kernels do on the way to LDS (dx_f, dw_f below).
   float* part_lse;
   float* part_max;
   float* part_pz;  // both null, or the monitoring partials of FwdArgs as well
