@@ -439,7 +439,7 @@ hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
 // All tile columns of the slab in one launch.
 template <class T, bool ZREG, bool WVH, bool FUSE = false>
 hipError_t launch_persistent_z(const BwdArgs& a, hipStream_t s) {
-  if (few_logit_tiles(a.N <= kSmallTile ? a.N : a.Np, a.vw, logit_ktiles<T>(a.H), a.small_wgs)) {
+  if (few_logit_tiles(a.N <= kSmallTile ? a.N : a.Np, a.vw, a.small_wgs)) {
     const int tiles_p = (int)(a.vs / kSmallTile), tiles_q = (int)(a.Np / kSmallTile);
     hipLaunchKernelGGL((dz_small_kernel<T, ZREG, WVH, FUSE>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a,
                        tiles_p, tiles_q);

@@ -668,7 +668,7 @@ hipError_t launch_one(const FwdArgs& a, int64_t tiles, hipStream_t s) {
 template <class T, bool WVH, bool MON> hipError_t launch_persistent(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;  // token tiles of this chunk at most
   const int64_t here = left < a.nc ? left : a.nc, there = a.N - a.row0, rows = here < there ? here : there;
-  if (few_logit_tiles(rows, a.vw, logit_ktiles<T>(a.H), a.small_wgs)) {
+  if (few_logit_tiles(rows, a.vw, a.small_wgs)) {
     const int tiles_p = (int)(pad_to(a.vw, kTile) / kSmallTile), tiles_q = (int)((rows + kSmallTile - 1) / kSmallTile);
     hipLaunchKernelGGL((fwd_small_kernel<T, WVH, MON>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a, tiles_p,
                        tiles_q);

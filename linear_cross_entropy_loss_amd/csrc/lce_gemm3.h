@@ -161,7 +161,7 @@ template <class S> LCE_DEV const void* matrix_end(const void* base, int64_t rows
 }
 
 // K tiles of the logit contraction.
-template <class T> __host__ LCE_DEV int logit_ktiles(int64_t H) {
+template <class T> LCE_DEV int logit_ktiles(int64_t H) {
   return (int)(is_pair<T>::value ? 3 * padded_k_pair(H) / kBK : padded_k(H) / kBK);
 }
 

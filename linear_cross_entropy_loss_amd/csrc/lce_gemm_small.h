@@ -35,9 +35,9 @@ template <class T, bool P_KC> struct SmallPipe {
   int k_rem, split_s;
   int64_t p_lo, q_lo;
 
-  LCE_DEV void fetch(int set) {  // the K tile the stream is at, and on to the next
-    ps.load(sp[set], 0, 4);
-    qs.load(sq[set], 0, 4);
+  s16x8_t pf[2][kNB], qf[2];     // fragments of this k-step and the next
+
+  LCE_DEV void advance() {
     if constexpr (kSplit) {
       if (split_s != 2) {
         ps.base += split_s == 0 ? 0 : p_lo;
@@ -56,17 +56,70 @@ template <class T, bool P_KC> struct SmallPipe {
     ps.retarget(k_rem);
     qs.retarget(k_rem);
   }
-  LCE_DEV void stash(int set, char* stage) {
-    ps.store(sp[set], stage, 0, 4);
-    qs.store(sq[set], stage + kSmallOperandBytes, 0, 4);
-  }
-  LCE_DEV void multiply(const char* stage, f32x16_t (&acc)[kNB][1]) {
+  // Chunks 0 .. 7 of a staged K tile: those of P and of Q in turn.
+  template <int SET> LCE_DEV void load_chunks(int c0, int c1) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const s16x8_t q = qr.read(stage + kSmallOperandBytes, 0, ks);
-#pragma unroll
-      for (int i = 0; i < kNB; ++i) acc[i][0] = mfma32<T>(pr.read(stage, i, ks), q, acc[i][0]);
+    for (int c = c0; c < c1; ++c) {
+      if (c & 1) qs.load(sq[SET], c >> 1, (c >> 1) + 1);
+      else ps.load(sp[SET], c >> 1, (c >> 1) + 1);
     }
+  }
+  template <int SET> LCE_DEV void store_chunks(char* stage, int c0, int c1) {
+#pragma unroll
+    for (int c = c0; c < c1; ++c) {
+      if (c & 1) qs.store(sq[SET], stage + kSmallOperandBytes, c >> 1, (c >> 1) + 1);
+      else ps.store(sp[SET], stage, c >> 1, (c >> 1) + 1);
+    }
+  }
+  LCE_DEV void read_frags(const char* stage, int ks) {
+    qf[ks & 1] = qr.read(stage + kSmallOperandBytes, 0, ks);
+#pragma unroll
+    for (int i = 0; i < kNB; ++i) pf[ks & 1][i] = pr.read(stage, i, ks);
+  }
+  LCE_DEV void multiply(int ks, f32x16_t (&acc)[kNB][1]) {
+#pragma unroll
+    for (int i = 0; i < kNB; ++i) acc[i][0] = mfma32<T>(pf[ks & 1][i], qf[ks & 1], acc[i][0]);
+  }
+  static constexpr int kReads = 1 + (P_KC ? 4 : 8);  // LDS reads of a k-step's fragments
+  // What goes behind each of a k-step's four matrix instructions: a quarter of the next one's reads, stores and loads in turn.
+  template <int STORES, int LOADS> LCE_DEV void order() {
+    __builtin_amdgcn_sched_group_barrier(LCE_SG_MFMA, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_RD, kReads - 3 * (kReads / 4), 0);
+    if (STORES > 0) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_WR, 1, 0);
+#pragma unroll
+    for (int i = 1; i < kNB; ++i) {
+      __builtin_amdgcn_sched_group_barrier(LCE_SG_MFMA, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_RD, kReads / 4, 0);
+      if (i < STORES) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_WR, 1, 0);
+      if (i >= kNB - LOADS) __builtin_amdgcn_sched_group_barrier(LCE_SG_VMEM_RD, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // One K tile, t, held in `cur`, the fragments of its first k-step in registers: K tile t + 1 goes from set SET to `next`, which
+  // takes K tile t + 3 in its place, chunk by chunk; the barrier opens the last k-step, and the fragments of K tile t + 1's
+  // first k-step are read during it.  (Left to the compiler, which put all stores first and all loads last: N=1536, V=2560, H=2048
+  // 31 us, so 24; N=48, V=50304, H=2048 43, so 39, which is 5.3 TB/s of weight.)
+  template <int SET> LCE_DEV void step(const char* cur, char* next, f32x16_t (&acc)[kNB][1]) {
+    read_frags(cur, 1);
+    store_chunks<SET>(next, 0, 3);
+    load_chunks<SET>(0, 3);
+    multiply(0, acc);
+    order<3, 3>();
+    read_frags(cur, 2);
+    store_chunks<SET>(next, 3, 6);
+    load_chunks<SET>(3, 6);
+    multiply(1, acc);
+    order<3, 3>();
+    read_frags(cur, 3);
+    store_chunks<SET>(next, 6, 8);
+    load_chunks<SET>(6, 8);
+    multiply(2, acc);
+    order<2, 2>();
+    advance();
+    __syncthreads();
+    read_frags(next, 0);
+    multiply(3, acc);
+    order<0, 0>();
   }
   // p, q: first element of the tile's operands; *_end: one past the last valid byte; ktiles: even, as in Pipe3, or 0.
   LCE_DEV void run(const void* p, const void* p_end, int64_t ldp, const void* q, const void* q_end, int64_t ldq, int64_t k_valid,
@@ -89,22 +142,21 @@ template <class T, bool P_KC> struct SmallPipe {
     for (int i = 0; i < kNB; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][0][r] = 0.f;
-    fetch(0);
-    fetch(1);
-    stash(0, lds);
-    fetch(0);
+    load_chunks<0>(0, 8);
+    advance();
+    load_chunks<1>(0, 8);
+    advance();
+    store_chunks<0>(lds, 0, 8);
+    load_chunks<0>(0, 8);
+    advance();
     __syncthreads();
+    read_frags(lds, 0);
     // (K tiles past the last one are fetched as zeros: masked in the K-contiguous operand, out of range in the other)
     for (int t = 0; t < ktiles; t += 2) {
-      stash(1, lds + kSmallStageBytes);
-      fetch(1);
-      multiply(lds, acc);
-      __syncthreads();
-      stash(0, lds);
-      fetch(0);
-      multiply(lds + kSmallStageBytes, acc);
-      __syncthreads();
+      step<1>(lds, lds + kSmallStageBytes, acc);
+      step<0>(lds + kSmallStageBytes, lds, acc);
     }
+    __syncthreads();  // (the epilogue may use the stages)
   }
 };
 

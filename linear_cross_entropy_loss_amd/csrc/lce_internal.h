@@ -51,16 +51,16 @@ constexpr int64_t padded_k_pair(int64_t H) { return pad_to(H, 128); }
 constexpr int products_of(int dtype) { return dtype == DT_PAIR ? 3 : 1; }
 
 // Whether a logit kernel runs on 128 x 128 tiles, one workgroup each (lce_gemm_small.h), or on the 256 x 256 tiles of the
-// persistent kernels: by the number of workgroups for `rows` token rows and `cols` columns and by `ktiles` K tiles.  `most`:
-// two workgroups for each compute unit (FwdArgs::small_wgs; 0: never).  The persistent kernel starts with 14 us of fetching its
-// code, the other with 5; up to one workgroup to a compute unit its K tile is the shorter one, up to two the same time for
-// 32 K tiles or so, beyond that half as long again.  Loss alone, bf16, us, 128 x 128 / 256 x 256: N=256, V=4096, H=256
-// 8.7 / 18.4, H=4096 46 / 74; N=2048, V=2048, H=1024 18.6 / 31.9; N=4096, V=2048 (512 workgroups) H=256 11.6 / 18.7, H=1024
-// 26 / 32, H=2048 49 / 49; N=5120, V=2048 (640) 20 / 20, 35 / 33, 61 / 50.  Of up to 128 tokens the persistent kernel's tiles
-// are half empty: N=48, V=100000, H=256 20 / 33, H=2048 94 / 110.
-inline bool few_logit_tiles(int64_t rows, int64_t cols, int ktiles, int most) {
+// persistent kernels: by the number of workgroups for `rows` token rows and `cols` columns.  `most`: two workgroups for each
+// compute unit (FwdArgs::small_wgs; 0: never).  The persistent kernel starts with 14 us of fetching its code, the other with 5;
+// up to one workgroup to a compute unit its K tile takes half as long, up to two the same time, beyond that half as long again.
+// Loss alone, bf16, us, 128 x 128 / 256 x 256: N=256, V=4096, H=256 8.7 / 18.4, H=4096 46 / 74; N=1536, V=2560 (240 workgroups),
+// H=256 10.5 / 19.6, H=2048 24 / 46; N=4096, V=2048 (512), H=256 12.5 / 18.7, H=1024 25 / 32, H=2048 42 / 49; N=5120, V=2048 (640)
+// 20 / 20, 35 / 33, 61 / 50.  Of up to 128 tokens the persistent kernel's tiles are half empty: N=48, V=100000, H=256 19 / 33,
+// H=2048 94 to 102 / 110.
+inline bool few_logit_tiles(int64_t rows, int64_t cols, int most) {
   const int64_t n = (rows + 127) / 128 * (pad_to(cols, 256) / 128);
-  return n <= most / 2 || (n <= most && ktiles <= 32) || (rows <= 128 && most > 0);
+  return n <= most || (rows <= 128 && most > 0);
 }
 
 // Which tile columns of the vocabulary a logit kernel covers: full ones, the one(s) from the column that straddles the end of
