@@ -514,28 +514,31 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
     count = MODE == kDwAll ? plan.full + tails : (MODE == kDwTails ? tails : plan.full);
   }
   LCE_DEV int num_tiles() const { return count; }
-  // `local` counts this launch's items; seg < 0: a whole tile
-  LCE_DEV void decode(int local, int& item, int& tp, int& tq, int& seg) const {
-    item = first + local;
-    int tile = item;
+  // `local` counts this launch's items; seg < 0: a whole tile.  block: the segment's place among the partial sums
+  LCE_DEV void decode(int local, int& block, int& tp, int& tq, int& seg) const {
+    const int item = first + local;
+    block = 0;
     seg = -1;
     if (item >= plan.full) {
-      const int j = item - plan.full;
-      tile = plan.full + j / plan.nseg;
-      seg = j % plan.nseg;
+      int b;
+      segment_coords(item - plan.full, plan.tail_tiles, plan.nseg, b, seg);
+      block = b * plan.nseg + seg;
+      tail_tile_coords(b, plan.full, plan.tiles, tiles_p, tiles_q, tp, tq);
+    } else {
+      tile_coords(item, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
     }
-    tile_coords(tile, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
   }
   LCE_DEV int item_ktiles(int local) const {
     const int item = first + local, products = kSplit ? 3 : 1;
     if (item < plan.full) return products * plan.kt;
-    const int seg = (item - plan.full) % plan.nseg;
+    int tile, seg;
+    segment_coords(item - plan.full, plan.tail_tiles, plan.nseg, tile, seg);
     return products * (segment_start(seg + 1, plan.nseg, plan.kt) - segment_start(seg, plan.nseg, plan.kt));
   }
   LCE_DEV const float* q_factors(int local) const {
     if (local >= count) return a.dw_f;
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     return a.dw_f + (int64_t)tq * (kTile / kChunkV) * a.nc + (seg < 0 ? 0 : (int64_t)segment_start(seg, plan.nseg, plan.kt) * kBK);
   }
   LCE_DEV unsigned q_factor_offset() const {
@@ -544,8 +547,8 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
   }
   LCE_DEV int64_t q_factor_step(int) const { return kBK; }
   LCE_DEV void origins(int local, const void*& p, const void*& q) const {
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     const int64_t k0 = seg < 0 ? 0 : (int64_t)segment_start(seg, plan.nseg, plan.kt) * kBK;  // first token of the segment
     p = x + k0 * ldx + (int64_t)tp * kTile;
     q = reinterpret_cast<const E*>(a.dz) + (kSplit ? 2 : 1) * dz_block_offset(k0 / kTile, (int64_t)tq * (kTile / kBK), a.vs) +
@@ -553,8 +556,8 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
   }
   // (segments start at even numbers of K tiles: in the first or the third quarter of a row of blocks)
   LCE_DEV int q_phase(int local) const {
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     return seg < 0 ? 0 : segment_start(seg, plan.nseg, plan.kt) & 3;
   }
   // x rows past the last one read as zeros.  dz is written for whole token tiles of 256 rows, and the K tiles of
@@ -568,8 +571,8 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
   LCE_DEV int k_valid(int) const { return (int)a.Np; }
   LCE_DEV void prefetch(int) {}
   LCE_DEV void epilogue(int local, f32x16_t (&acc)[kNB][kNB], char* scratch) const {
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     if constexpr (ACC == 3 || ACC == 4) {
       dw_epilogue_f32_sum<WVH, ACC == 4>(a, acc, tp, tq, scratch);
       return;
@@ -585,7 +588,7 @@ template <class T, bool WVH, int MODE, int ACC, bool SCALE> struct DwProblem {
     if (MODE == kDwStaged || MODE == kDwStaged32) {
       dw_store_rows_hv<T, MODE == kDwStaged32, SCALE>(a, acc, tp, tq, scratch);
     } else {
-      float* part = seg >= 0 ? a.dw_part + (int64_t)(item - plan.full) * kTile * kTile : nullptr;
+      float* part = seg >= 0 ? a.dw_part + (int64_t)block * kTile * kTile : nullptr;
       dw_epilogue<T, WVH>(a, part, acc, tp, tq);
     }
   }
@@ -613,7 +616,7 @@ __global__ __launch_bounds__(256) void dw_tail_kernel(const BwdArgs a) {
   const int b = (int)blockIdx.x / kTailParts, piece = (int)blockIdx.x % kTailParts;
   if (b >= plan.tail_tiles) return;
   int tp, tq;
-  tile_coords(plan.full + b, plan.tiles, (int)(a.Hp / kTile), (int)(a.vs / kTile), 8, 8, tp, tq);
+  tail_tile_coords(b, plan.full, plan.tiles, (int)(a.Hp / kTile), (int)(a.vs / kTile), tp, tq);
   const DwTileGeom<WVH> g(a, tp, tq);
   const float coef = final_factor_of(a);
   const float* part = a.dw_part + (int64_t)b * plan.nseg * kTile * kTile;

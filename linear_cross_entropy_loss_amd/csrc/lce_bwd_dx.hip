@@ -171,27 +171,30 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
     count = MODE == kDxTails ? plan.tail_tiles * plan.nseg : plan.full;
   }
   LCE_DEV int num_tiles() const { return count; }
-  // `local` counts this launch's items; seg < 0: a whole tile
-  LCE_DEV void decode(int local, int& item, int& tp, int& tq, int& seg) const {
-    item = first + local;
-    int tile = item;
+  // `local` counts this launch's items; seg < 0: a whole tile.  block: the segment's place among the partial sums
+  LCE_DEV void decode(int local, int& block, int& tp, int& tq, int& seg) const {
+    const int item = first + local;
+    block = 0;
     seg = -1;
     if (item >= plan.full) {
-      const int j = item - plan.full;
-      tile = plan.full + j / plan.nseg;
-      seg = j % plan.nseg;
+      int b;
+      segment_coords(item - plan.full, plan.tail_tiles, plan.nseg, b, seg);
+      block = b * plan.nseg + seg;
+      tail_tile_coords(b, plan.full, plan.tiles, tiles_p, tiles_q, tp, tq);
+    } else {
+      tile_coords(item, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
     }
-    tile_coords(tile, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
   }
   LCE_DEV int item_ktiles(int local) const {
-    const int seg = local % plan.nseg;  // (segment items only)
+    int tile, seg;
+    segment_coords(local, plan.tail_tiles, plan.nseg, tile, seg);  // (segment items only)
     return (kSplit ? 3 : 1) * (segment_start(seg + 1, plan.nseg, plan.kt) - segment_start(seg, plan.nseg, plan.kt));
   }
   // (a K tile is half a slice of 128 columns; work items start at even K tiles)
   LCE_DEV const float* q_factors(int local) const {
     if (local >= count) return a.dx_f;
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     return a.dx_f + k0_of(seg) / kChunkV * a.nc + (int64_t)tq * kTile;
   }
   LCE_DEV unsigned q_factor_offset() const { return (threadIdx.x >> 3) * 32; }
@@ -199,8 +202,8 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
   LCE_DEV void prefetch(int) {}
   LCE_DEV int64_t k0_of(int seg) const { return seg < 0 ? 0 : (int64_t)segment_start(seg, plan.nseg, plan.kt) * kBK; }
   LCE_DEV void origins(int local, const void*& p, const void*& q) const {
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     const int64_t k0 = k0_of(seg);
     p = WVH ? reinterpret_cast<const E*>(a.w) + ((a.v0 - a.wv0) + k0) * a.ldw + (int64_t)tp * kTile
             : reinterpret_cast<const E*>(a.w) + (int64_t)tp * kTile * a.ldw + (a.v0 - a.wv0) + k0;
@@ -212,16 +215,16 @@ template <class T, bool KMASK, bool WVH, int MODE, bool SCALE> struct DxProblem 
   // (only whole token tiles that were written are read)
   LCE_DEV const void* q_end() const { return reinterpret_cast<const E*>(a.dz) + (kSplit ? 2 : 1) * a.dz_rows * a.vs; }
   LCE_DEV int k_valid(int local) const {
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     const int64_t left = a.vw - k0_of(seg);
     return (int)(left < 0 ? 0 : left);
   }
   LCE_DEV void epilogue(int local, f32x16_t (&acc)[kNB][kNB], char*) const {
-    int item, tp, tq, seg;
-    decode(local, item, tp, tq, seg);
+    int block, tp, tq, seg;
+    decode(local, block, tp, tq, seg);
     if (MODE == kDxTails) {
-      dx_store_segment(a.dx_part + (int64_t)(item - plan.full) * kTile * kTile, acc);
+      dx_store_segment(a.dx_part + (int64_t)block * kTile * kTile, acc);
     } else {
       const bool packed = rows != a.N || a.perm_always != 0, copy = packed && a.dxc != nullptr;
       dx_epilogue<T, MODE == kDxMiddle || MODE == kDxLast, MODE == kDxLast || MODE == kDxOnly>(
@@ -252,7 +255,7 @@ __global__ __launch_bounds__(256) void dx_tail_kernel(const BwdArgs a) {
   const int b = (int)blockIdx.x / kTailParts, piece = (int)blockIdx.x % kTailParts;
   if (b >= plan.tail_tiles) return;
   int tp, tq;
-  tile_coords(plan.full + b, plan.tiles, tiles_p, tiles_q, 8, 8, tp, tq);
+  tail_tile_coords(b, plan.full, plan.tiles, tiles_p, tiles_q, tp, tq);
   const bool packed = rows != a.N || a.perm_always != 0, copy = packed && a.dxc != nullptr;
   void* out = copy ? a.dxc : a.dx;
   const int64_t ldo = copy ? a.lddxc : a.lddx;
