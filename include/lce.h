@@ -316,7 +316,9 @@ enum {
  * room for a chunk within the bound (a 16-bit dW with H near 4 * n_chunk or
  * above; lce_forward_backward_plan then reports 0 chunks).  `phases` selects kernels of either route; on the one-pass
  * route LCE_PHASE_FWD_TILES is the logit kernel and LCE_PHASE_BWD_DZ the pass
- * that turns e into dz (hidden sizes up to 1024: the kernel that works out the factors by which the dx and dW kernels do).
+ * that turns e into dz (hidden sizes up to 1024: the kernel that works out the factors by which the dx and dW kernels do).  A
+ * workspace holds one chunk's partials and stage at a time: the results of a restricted call are those of the full call only
+ * where the plan is one chunk (and the stage is rewritten as LCE_PHASE_BWD_DZ runs: FWD_TILES has to come before it again).
  *
  *   grad_out   device pointer to 1 float: upstream gradient of the loss
  *              (the reference multiplies it in afterwards, ops.py:810).  A

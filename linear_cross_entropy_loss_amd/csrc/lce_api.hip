@@ -366,7 +366,7 @@ struct FusedPlan {
   int64_t nc;
   int chunks;
   PackPlan k;
-  size_t chunk_rows, lse_rows, tgt, blk, w16, xc, part_lse, part_max, part_pz, part_sq, stage, plane, plane_hi, part, total;
+  size_t chunk_rows, lse_rows, tgt, blk, w16, xc, part_lse, part_max, part_pz, part_sq, dx_f, dw_f, stage, plane, plane_hi, part, total;
   int64_t ld16;    // row stride of the 16-bit copy of an fp32 weight
   bool parts_on;
   bool dw_direct;  // fp32 dW: the chunks' terms are added in the caller's buffer, there is no plane
@@ -410,8 +410,6 @@ bool plan_fused(const lce_problem* p, FusedPlan* f) {
 bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, FusedPlan* f) {
   memset(f, 0, sizeof(*f));
   f->lo8 = lo8;
-  f->factors = factors_in_gradients(p);
-  const double mul = f->factors ? 1.06 : 1.0;
   const bool x16 = p->x_dtype == LCE_BF16 || p->x_dtype == LCE_F16;
   if (!x16 || (p->w_dtype != p->x_dtype && p->w_dtype != LCE_F32) || route_of(p) == LCE_ROUTE_TWO_PASS) return false;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Vp = (size_t)lce::padded_vocab(p->V), Hp = (size_t)lce::padded_hidden(p->H);
@@ -447,6 +445,11 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
     out->part_max = t; t += part;
     out->part_pz = t; if (p->monitoring) t += part;
     out->part_sq = t; if (p->monitoring) t += part;
+    // The factors' tables: of a single chunk apart from the partials, which a later call restricted to the row merge reads again;
+    // of one chunk after another in the place of the partials, of which a workspace holds the last chunk's only.
+    const bool apart = chunks == 1 && out->factors;
+    out->dx_f = apart ? t : out->part_lse; if (apart) t += part;
+    out->dw_f = apart ? t : out->part_max; if (apart) t += part;
     out->stage = t; t += align_up((size_t)nc * Vp * 2);
     // split-K partial sums of dx (and, with a single chunk, of dW): one buffer
     size_t pb = want_dx ? dx_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp, products(p)) : 0;
@@ -481,8 +484,12 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
     if (t < tiles && (tiles + t) / (t + 1) == chunks) continue;  // a longer chunk gives the same number of chunks
     if (chunks > 1 && want_dw && !f->dw_direct && !halves_ok) continue;
     const int64_t t_even = (tiles + chunks - 1) / chunks;  // equal lengths
+    // (where the bound has no room for the tables of factors, the pass over the stage does the same)
     FusedPlan cand = *f;
+    cand.factors = factors_in_gradients(p);
+    if (cand.factors && total_for(t_even * 256, (int)chunks, &cand) + reserve > bound) cand.factors = false;
     if (total_for(t_even * 256, (int)chunks, &cand) + reserve > bound) continue;
+    const double mul = cand.factors ? 1.06 : 1.0;
     const int64_t t_last = tiles - (chunks - 1) * t_even;
     auto chunk_cost = [&](double tt) -> double {
       return kernel_cost(tt * tv, (double)(lce::padded_k(p->H) / 64), 8.0, false) +
@@ -753,9 +760,8 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   b.nc = f.nc;
   b.dx_part = f.parts_on && dx ? (float*)(base + f.part) : nullptr;
   b.dw_part = f.parts_on && dw && f.chunks == 1 ? (float*)(base + f.part) : nullptr;
-  // the factors of the stage take the place of the partials once the rows' lse are known (lce_fuse.hip)
-  b.dx_f = f.factors ? b.part_lse : nullptr;
-  b.dw_f = f.factors ? b.part_max : nullptr;
+  b.dx_f = f.factors ? (float*)(base + f.dx_f) : nullptr;
+  b.dw_f = f.factors ? (float*)(base + f.dw_f) : nullptr;
   b.dw_plane = f.chunks > 1 && !f.dw_direct ? (void*)(base + f.plane) : nullptr;
   b.dw_plane_hi = f.chunks > 1 && !f.dw_direct && f.total != f.plane_hi ? (void*)(base + f.plane_hi) : nullptr;
 

@@ -86,7 +86,8 @@ __global__ __launch_bounds__(256) void stage_scale_kernel(const BwdArgs a) {
 // The same without the pass over the stage: only the factors are worked out, and the dx and dW kernels multiply e by them on
 // its way to LDS (BwdArgs::dx_f, dw_f; the products and roundings are those of stage_scale_kernel).  The slice of 128 columns
 // that holds a token's target is rewritten here, with a factor of 1 from then on.  One workgroup per token tile and
-// kSlices slices; the two tables take the place of the partials (part_lse, part_max), which nothing reads any more.
+// kSlices slices.  (The two tables may be part_lse and part_max themselves: where there are several chunks, nothing reads
+// those any more.)
 // Bound by launch and latency: 12 bytes per 128 logits and 512 per token.  (4096 tokens, us a launch against the pass over
 // the stage: V=32000 21 / 79, V=50257 22 / 129, V=65536 13 / 165; which problems take it: factors_in_gradients in lce_api.hip.)
 constexpr int kSlices = 8;

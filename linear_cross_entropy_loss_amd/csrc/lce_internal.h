@@ -233,8 +233,8 @@ hipError_t launch_bwd_dz(const BwdArgs& a, hipStream_t s);
 // The logit kernel of lce_forward_backward and the pass that follows the row merge (see BwdArgs).
 hipError_t launch_fwd_stage(const BwdArgs& a, hipStream_t s);
 hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s);
-// The same with the factors only worked out (dx_f and dw_f of BwdArgs, in part_lse and part_max), and the slice of each
-// token's target column rewritten.
+// The same with the factors only worked out (dx_f and dw_f of BwdArgs), and the slice of each token's target column
+// rewritten.
 hipError_t launch_stage_factors(const BwdArgs& a, hipStream_t s);
 // t[r][c] *= g[0] (device scalar), in fp32; nothing is touched when g[0] == 1.  Rows on 16-byte boundaries.
 hipError_t launch_scale_rows(void* t, int dtype, int64_t rows, int64_t cols, int64_t ld, const float* g, int num_cus,

@@ -510,3 +510,33 @@ def test_fp32_sums_of_dw_keep_to_their_columns(N, H, V, n_chunk, layout):
     # (dz is rounded to bf16 twice before the contraction, 2^-8 of an entry at most each: some 2e-3 of the 2-norm)
     emax, el2 = rel_errors(got, ref.dw)
     assert emax < 2e-2 and el2 < 5e-3
+
+
+# one chunk, hidden sizes on either side of the line up to which the gradient kernels multiply by the factors: the partials that the
+# row merge reads are still there after a full call
+@pytest.mark.parametrize("mon", [False, True])
+@pytest.mark.parametrize("H", [256, 1024, 1280])
+def test_row_merge_alone_on_the_workspace_of_a_full_call(H, mon):
+    from linear_cross_entropy_loss_amd import _lib
+
+    lib = _lib.load()
+    N, V, dt = 700, 3000, torch.bfloat16
+    x, y, w = make_inputs(N, H, V, dt, 3, ignore_frac=0.1, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ws = g = dx = dw = None
+    results = []
+    for phases in (0, _lib.PHASE_FWD_REDUCE):
+        prob = _problem(N, H, V, x, w, dt, dt, 1e-3, 1.0, 4096, 0, 0, phases=phases, mon=mon)
+        if ws is None:
+            assert _lib.forward_backward_plan(prob)[0] == 1
+            ws = torch.empty(_lib.forward_backward_workspace_bytes(prob), dtype=torch.uint8, device="cuda")
+            g, dx, dw = torch.ones(1, device="cuda"), torch.empty_like(x), torch.empty_like(w)
+        lse, out5 = torch.full((N,), 7.0, device="cuda"), torch.full((5,), 7.0, device="cuda")
+        nv = torch.zeros(1, dtype=torch.int64, device="cuda")
+        rc = lib.lce_forward_backward(ctypes.byref(prob), P(x), P(w), P(y), P(g), P(lse), P(out5), P(nv), P(dx), P(dw), P(ws),
+                                      ws.numel(), st)
+        assert rc == 0
+        results.append((lse, out5, nv))
+    torch.cuda.synchronize()
+    for full, again in zip(*results):
+        assert torch.equal(full, again)
