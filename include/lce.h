@@ -307,7 +307,9 @@ enum {
  * lce_problem.route: LCE_ROUTE_AUTO takes this route when a model of the tile
  * kernels' rounds of workgroups says it is the faster one (short chunks are
  * not: every chunk costs a round trip of dW's fp32 sums, so small problems
- * and tight bounds take two passes); LCE_ROUTE_ONE_PASS takes it whenever it
+ * and tight bounds take two passes).  Which problems may be rounded as above
+ * does not follow the kernels' speed from one version to the next: the model
+ * has to say so with settled costs too.  LCE_ROUTE_ONE_PASS takes it whenever it
  * fits the bound; LCE_ROUTE_TWO_PASS never.
  *
  * Problems this route does not cover take the two calls above, one after the

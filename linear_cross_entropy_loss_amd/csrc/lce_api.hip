@@ -217,14 +217,16 @@ size_t dw_part_bytes(size_t Np, size_t Hp, int64_t vs, int64_t last_vs, int prod
 // fraction f of the compute units runs 1 + 0.9 (1 - f) times faster per compute unit (the part is limited by
 // power: measured 1.14 / 1.30 / 1.46 / 1.54 at f = 0.81 / 0.69 / 0.47 / 0.34), and is cut along K when the
 // partial-sum blocks exist (`parts`; a small kernel then adds the segments: 12 units).  `e`: the epilogue of a
-// tile; a launch costs about 10.
+// tile; a launch costs about 10.  `settled`: the costs by which make_plan_fused decides what may be rounded, with K segments in
+// powers of two.
 constexpr double kPlanCUs = 256.0;
-double kernel_cost(double T, double L, double e, bool parts) {
+double kernel_cost(double T, double L, double e, bool parts, bool settled) {
   const double full = (double)(int64_t)(T / kPlanCUs), r = T - full * kPlanCUs;
   double cost = full * (L + e) + 10.0;
   if (r > 0) {
     double seg = 1;
-    if (parts) seg = lce::k_segments((int)r, (int)kPlanCUs, (int)L);
+    if (parts && settled) while (r * seg * 2 <= kPlanCUs && L / (seg * 2) >= 16) seg *= 2;
+    else if (parts) seg = lce::k_segments((int)r, (int)kPlanCUs, (int)L);
     const double f = r * seg / kPlanCUs;
     cost += (L / seg + e) / (1.0 + 0.9 * (1.0 - f)) + (seg > 1 ? 12.0 : 0.0);
   }
@@ -247,7 +249,7 @@ double kernel_cost(double T, double L, double e, bool parts) {
 // N * H * 4 bytes, the fp32 x_grad buffer the reference allocates next to its logits chunk (ops.py:693) and
 // this library does not -- and by the split-K partial sums.  If even that fails, the narrowest split is used:
 // the bound is a target, the operator never refuses a shape.
-int make_plan_bwd(const lce_problem* p, BwdPlan* b) {
+int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
   const size_t strict = (size_t)p->n_chunk * (size_t)p->V * 4;
   const size_t dz_cap = (size_t)1 << 30;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Hp = (size_t)lce::padded_hidden(p->H);
@@ -271,9 +273,9 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b) {
     const double tq = (double)(Np / 256), th = (double)(Hp / 256), tv = (double)(w / 256), k3 = split ? 3.0 : 1.0;
     // (bwd_dz runs about 4 % slower on a slab that is not whole groups of the bands it keeps in flight when K is long)
     const double dz_order = live < 8 && (w / 256) % (8 * live) != 0 ? 1.04 : 1.0;
-    return dz_order * kernel_cost(tq * tv, k3 * (double)((p->H + 63) / 64), 6.0, false) +
-           kernel_cost(tq * th, k3 * (double)(w / 64), sums ? 21.0 : 5.0, parts) +
-           kernel_cost(tv * th, k3 * (double)(Np / 64), 5.0, parts);
+    return dz_order * kernel_cost(tq * tv, k3 * (double)((p->H + 63) / 64), 6.0, false, settled) +
+           kernel_cost(tq * th, k3 * (double)(w / 64), sums ? 21.0 : 5.0, parts, settled) +
+           kernel_cost(tv * th, k3 * (double)(Np / 64), 5.0, parts, settled);
   };
 
   // mode 0: everything; mode 1: lean (at the strict bound only); mode 2: everything, widened bound.
@@ -349,7 +351,7 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b) {
 
 int plan_bwd(const lce_problem* p, BwdPlan* b) {
   static thread_local LastPlan<BwdPlan> last;
-  return last.get(p, b, make_plan_bwd);
+  return last.get(p, b, [](const lce_problem* q, BwdPlan* out) { return make_plan_bwd(q, out, false); });
 }
 
 // lce_forward_backward: the logits are computed once.  The tokens go through in chunks of `nc` rows against the
@@ -383,23 +385,46 @@ struct FusedPlan {
 // 11.85 / 12.30, 1536 17.57 / 17.58; fp16, N=8192, V=50304, H=768 2.15 / 2.28, 1024 2.65 / 2.73, 1536 3.78 / 3.74.
 bool factors_in_gradients(const lce_problem* p) { return lce::padded_hidden(p->H) <= 1024; }
 
-bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, FusedPlan* f);
+bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, bool settled, int64_t most_chunks, FusedPlan* f);
+constexpr int64_t kMostChunks = 1024;  // (lce_compact.hip counts the rows of so many)
 
 // The lower halves of the fp32 sums of a 16-bit dW at 16 bits (the sums are then exact fp32) or at 8 (sums of 24
 // bits): the latter where the former does not fit the bound, or leaves so little of it to the chunks that the model
 // puts the plan with bytes at least 3 % ahead of the exact alternatives (the plan with halves, two passes) -- measured
 // on one box: 5.9 % at config 3, 7-10 % at the output layers of Llama-3-8B / Llama-2-7B, 11-20 % at config 4's
 // N_chunk_size = 2048 points, 0.7 % at the headline shape (which keeps the halves).  Never with LCE_ROUTE_EXACT_SUMS.
+// most_chunks: of the plan with bytes.
 constexpr double kBytesMargin = 0.97;
-int make_plan_fused(const lce_problem* p, FusedPlan* f) {
-  const bool halves = plan_fused_with(p, true, true, false, f);
+bool fastest_fused(const lce_problem* p, bool settled, int64_t most_chunks, FusedPlan* f) {
+  const bool halves = plan_fused_with(p, true, true, false, settled, kMostChunks, f);
   if ((p->route & LCE_ROUTE_EXACT_SUMS) || p->dw_dtype == LCE_F32) return halves;
   FusedPlan b;
-  if (plan_fused_with(p, true, true, true, &b) && (!halves || b.cost < kBytesMargin * f->cost)) {
+  if (plan_fused_with(p, true, true, true, settled, most_chunks, &b) && (!halves || b.cost < kBytesMargin * f->cost)) {
     *f = b;
     return true;
   }
   return halves;
+}
+
+// How far a plan rounds what two passes over the logits hold in fp32: not at all, the staged dz a second time, or the sums of dW
+// between chunks to 24 bits as well (each chunk after the first once more).
+enum { kAsTwoPasses = 0, kDzTwice = 1, kSums24 = 2 };
+int rounding_of(bool one_pass, const FusedPlan& f) { return !one_pass ? kAsTwoPasses : f.lo8 && f.chunks > 1 ? kSums24 : kDzTwice; }
+
+// A faster kernel on one route must not change how far a problem's gradients are rounded: what a plan may round is decided by
+// costs that stay as they are (`settled`: K segments in powers of two, dz formed by a pass over the stage at every hidden size),
+// and the fastest of what is allowed by the costs of the kernels as they are.  (By the latter alone 179 of 2255 problems drawn
+// over N = 128 ... 32768, H = 64 ... 8192, V = 256 ... 262144 are rounded further, nearly all of them with H <= 1024.  Error
+// against fp64 and time, one pass / two: bf16 under an fp32 weight, N=3285, H=320, V=40832 dW 5.20e-5 / 5.08e-5, dx 2.3540e-3 /
+// 2.3537e-3, 500 / 559 us; bf16, N=896, H=704, V=46592 dx 1.6475e-3 / 1.6474e-3, 291 / 327 us, N=3411, H=256, V=80256 779 / 735.)
+int make_plan_fused(const lce_problem* p, FusedPlan* f) {
+  bool ok = fastest_fused(p, false, kMostChunks, f);
+  if (!ok) return false;
+  FusedPlan settled;
+  const int allowed = rounding_of(fastest_fused(p, true, kMostChunks, &settled), settled);
+  if (allowed == kAsTwoPasses) return false;
+  if (allowed == kSums24 && rounding_of(ok, *f) == kSums24 && f->chunks > settled.chunks) ok = fastest_fused(p, false, settled.chunks, f);
+  return rounding_of(ok, *f) <= allowed ? ok : plan_fused_with(p, true, true, false, false, kMostChunks, f);
 }
 // (for both gradients, whichever the caller wants: the workspace does not depend on that)
 bool plan_fused(const lce_problem* p, FusedPlan* f) {
@@ -407,7 +432,7 @@ bool plan_fused(const lce_problem* p, FusedPlan* f) {
   return last.get(p, f, make_plan_fused) != 0;
 }
 
-bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, FusedPlan* f) {
+bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, bool settled, int64_t most_chunks, FusedPlan* f) {
   memset(f, 0, sizeof(*f));
   f->lo8 = lo8;
   const bool x16 = p->x_dtype == LCE_BF16 || p->x_dtype == LCE_F16;
@@ -480,21 +505,21 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
   int64_t first = 0;  // chunks of the longest chunk that fits
   for (int64_t t = tiles; t >= 1; --t) {
     const int64_t chunks = (tiles + t - 1) / t;
-    if (chunks > 1024 || (first != 0 && chunks > 4 * first + 8)) break;
+    if (chunks > most_chunks || (first != 0 && chunks > 4 * first + 8)) break;
     if (t < tiles && (tiles + t) / (t + 1) == chunks) continue;  // a longer chunk gives the same number of chunks
     if (chunks > 1 && want_dw && !f->dw_direct && !halves_ok) continue;
     const int64_t t_even = (tiles + chunks - 1) / chunks;  // equal lengths
     // (where the bound has no room for the tables of factors, the pass over the stage does the same)
     FusedPlan cand = *f;
-    cand.factors = factors_in_gradients(p);
+    cand.factors = !settled && factors_in_gradients(p);
     if (cand.factors && total_for(t_even * 256, (int)chunks, &cand) + reserve > bound) cand.factors = false;
     if (total_for(t_even * 256, (int)chunks, &cand) + reserve > bound) continue;
     const double mul = cand.factors ? 1.06 : 1.0;
     const int64_t t_last = tiles - (chunks - 1) * t_even;
     auto chunk_cost = [&](double tt) -> double {
-      return kernel_cost(tt * tv, (double)(lce::padded_k(p->H) / 64), 8.0, false) +
-             (want_dx ? kernel_cost(tt * th, mul * (double)(Vp / 64), 5.0, true) : 0.0) +
-             (want_dw ? kernel_cost(tv * th, mul * tt * 4.0, chunks > 1 ? (f->dw_direct ? 16.0 : lo8 ? 10.0 : 12.0) : 5.0, chunks == 1) : 0.0);
+      return kernel_cost(tt * tv, (double)(lce::padded_k(p->H) / 64), 8.0, false, settled) +
+             (want_dx ? kernel_cost(tt * th, mul * (double)(Vp / 64), 5.0, true, settled) : 0.0) +
+             (want_dw ? kernel_cost(tv * th, mul * tt * 4.0, chunks > 1 ? (f->dw_direct ? 16.0 : lo8 ? 10.0 : 12.0) : 5.0, chunks == 1, settled) : 0.0);
     };
     // (per chunk, besides the tile kernels: the row merge, the kernel that adds dx's K segments, launch gaps -- about 25 units)
     const double cost = (double)(chunks - 1) * chunk_cost((double)t_even) + chunk_cost((double)t_last) + 25.0 * (double)chunks;
@@ -516,8 +541,8 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
   // (the factors instead: hardly any traffic, but a launch of some 15 us per chunk that starts from cold)
   const double scale_pass = f->factors ? 12.0 * (double)f->chunks : (double)Np * (double)Vp * 4.0 / 8.0e6;
   f->cost = best + scale_pass;
-  if (route_of(p) == LCE_ROUTE_AUTO && plan_bwd(p, &b) == LCE_OK) {
-    const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false) + b.cost;
+  if (route_of(p) == LCE_ROUTE_AUTO && (settled ? make_plan_bwd(p, &b, true) : plan_bwd(p, &b)) == LCE_OK) {
+    const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false, settled) + b.cost;
     // (sums of 24 bits have to be ahead of two passes, which are exact, by the margin as well)
     if (best + scale_pass > two * (lo8 ? kBytesMargin : 1.0)) {
       f->ok = false;  // (f->chunks stays: a plan fitted)

@@ -683,3 +683,34 @@ def test_a_plan_belongs_to_its_problem_alone():
     alone = [[plans(p) for _ in range(2)][1] for p in problems]
     assert [plans(p) for p in problems] == alone and [plans(p) for p in reversed(problems)] == alone[::-1]
     assert len(set(alone)) > 4
+
+
+# N, H, V, dtype, n_chunk, stored (V, H), fp32 weight, monitoring, what is rounded (below): problems for which one pass, or sums of 24
+# bits, became the faster plan as the kernels for hidden sizes up to 1024 and the cuts along K did, on either side of them ones that
+# the benchmark and its sweeps run
+ROUNDINGS = [
+    (457, 384, 126208, torch.bfloat16, 8192, 1, 0, 0, 0), (896, 704, 46592, torch.bfloat16, 8192, 1, 0, 0, 0),
+    (2432, 384, 30195, torch.float16, 4096, 0, 0, 0, 0), (3285, 320, 40832, torch.bfloat16, 4096, 0, 1, 1, 0),
+    (5248, 563, 206720, torch.bfloat16, 2048, 0, 0, 0, 0), (26345, 4480, 204544, torch.bfloat16, 2048, 1, 0, 1, 0),
+    (11328, 640, 164352, torch.float16, 2048, 1, 0, 0, 1),
+    (1999, 500, 10007, torch.bfloat16, 4096, 0, 0, 0, 0), (4096, 1024, 32000, torch.bfloat16, 4096, 1, 0, 0, 1),
+    (8192, 768, 50257, torch.bfloat16, 4096, 0, 0, 0, 1), (16384, 2048, 131072, torch.bfloat16, 4096, 0, 0, 0, 1),
+    (16384, 4096, 131072, torch.float16, 4096, 0, 0, 1, 2), (32768, 4096, 262144, torch.float16, 8192, 0, 1, 0, 1),
+]
+
+
+@pytest.mark.parametrize("N,H,V,dt,n_chunk,vh,master,mon,rounded", ROUNDINGS)
+def test_speed_does_not_decide_how_far_gradients_are_rounded(N, H, V, dt, n_chunk, vh, master, mon, rounded):
+    """0: as two passes round; 1: the staged dz twice (one pass); 2: sums of dW at 24 bits between chunks as well."""
+    from linear_cross_entropy_loss_amd import _lib, ops
+
+    wt = torch.float32 if master else dt
+    cols = ops._padded_cols(H if vh else V, wt)
+
+    def plan(route):
+        p = _lib.make_problem(N, H, V, ops._padded_cols(H, dt), cols, ops._dx_cols(H, dt), cols, dt, wt, dt, wt, -1, 1.0, 0.0, n_chunk,
+                              mon, 0, 0, 0, vh, route)
+        return _lib.forward_backward_plan(p) + (_lib.forward_backward_workspace_bytes(p),)
+
+    auto, exact = plan(_lib.ROUTE_AUTO), plan(_lib.ROUTE_AUTO | _lib.ROUTE_EXACT_SUMS)
+    assert (0 if auto[0] == 0 else 2 if auto != exact and auto[0] > 1 else 1) == rounded
