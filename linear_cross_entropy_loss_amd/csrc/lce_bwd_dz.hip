@@ -378,7 +378,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dz_persistent_kernel(const BwdAr
     typedef DzProblem<T, ZREG, false, KMASK, WVH, FUSE> Full;
     Full prob(a);
     Pipe3<T, E, WVH, E, true, Full> pipe(prob);
-    if (TAIL == kNoTail || first < prob.num_tiles()) pipe.run(a.ldw, prob.ldx, logit_ktiles<T>(a.H), lds, first);
+    pipe.run(a.ldw, prob.ldx, logit_ktiles<T>(a.H), lds, first);
     if (TAIL == kWithTail) first = first_tail_tile(first, (int)gridDim.x, prob.num_tiles());
   }
   if constexpr (TAIL != kNoTail) {

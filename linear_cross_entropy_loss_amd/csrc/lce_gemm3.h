@@ -270,11 +270,12 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
       qs.base = reinterpret_cast<const char*>(q);
       ps.end = reinterpret_cast<const char*>(prob.p_end());
       qs.end = reinterpret_cast<const char*>(prob.q_end());
-    } else {
+      k_rem = prob.k_valid(tile);
+    } else {  // (the problem is not asked about tiles that it does not have: its plan may have none to divide by)
       ps.end = ps.base;  // nothing left to fetch: every load returns 0
       qs.end = qs.base;
+      k_rem = 0;
     }
-    k_rem = prob.k_valid(tile);
     if constexpr (kSplit) split_s = 0;
     if constexpr (kQScale) {
       qfac_base = prob.q_factors(tile);
@@ -534,6 +535,7 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
 
   // `first`: this workgroup's first output tile (the next ones follow at the distance of the grid).
   LCE_DEV void run(int64_t ldp, int64_t ldq, int ktiles_, char* lds_, int first) {
+    if (first >= prob.num_tiles()) return;  // (the whole workgroup: there is no address to start the fetch stream at)
     lds = lds_;
     ktiles = ktiles_;
     const int wave = threadIdx.x >> 6;

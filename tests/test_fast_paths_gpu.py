@@ -355,3 +355,34 @@ def test_both_gradients_scaled_in_one_launch(shapes, dtypes, factor, divisor):
         if t is not None:
             assert torch.equal(t, w)
             assert (torch.as_strided(t, (t.shape[0], t.stride(0)), (t.stride(0), 1))[:, t.shape[1]:] == 7.0).all()
+
+
+# dx and dW launches whose plan has nothing to cut along K (as many tiles as workgroups, K too short), more workgroups than items, and no
+# item at all (every label ignored): the fetch stream of every workgroup ends past the last item of its launch
+@pytest.mark.parametrize("route", ["always", False])
+@pytest.mark.parametrize("N,H,V,dtype,ignored", [
+    (4096, 4096, 2304, torch.bfloat16, 0.0), (300, 512, 1024, torch.bfloat16, 0.0), (300, 512, 1024, torch.float32, 0.0),
+    (2100, 300, 2100, torch.float16, 0.2), (600, 1100, 4096, torch.bfloat16, 1.0), (600, 72, 4096, torch.float32, 1.0),
+])
+def test_launches_without_work_cut_along_k(N, H, V, dtype, ignored, route):
+    from linear_cross_entropy_loss_amd import linear_cross_entropy, ops
+
+    x, y, w = make_inputs(N, H, V, dtype, 23, ignore_frac=ignored, device="cuda")
+    x, w = x.requires_grad_(), w.requires_grad_()
+    token = ops.one_pass.set(route)
+    try:
+        loss = linear_cross_entropy(x, y, w, -1)[0]
+        dx, dw = torch.autograd.grad(loss, (x, w))
+    finally:
+        ops.one_pass.reset(token)
+    keep = y != -1
+    if not keep.any():
+        assert torch.isnan(loss) and not dx.any() and not dw.any()
+        return
+    xd, wd = x.detach().double(), w.detach().double()
+    p = torch.softmax(xd @ wd, 1)
+    p[torch.arange(N, device="cuda"), y.clamp(min=0)] -= 1
+    p *= keep[:, None] / keep.sum()
+    # (the operator's tolerance of gradients in 16 bits; pairs: 2^-16 relative to each operand, some 2^-15 of the 2-norm)
+    for got, want in ((dx, p @ wd.t()), (dw, xd.t() @ p)):
+        assert rel_errors(got, want)[1] < (3e-5 if dtype == torch.float32 else 5e-3)
