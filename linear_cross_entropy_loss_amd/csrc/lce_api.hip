@@ -385,7 +385,7 @@ struct FusedPlan {
 // 11.85 / 12.30, 1536 17.57 / 17.58; fp16, N=8192, V=50304, H=768 2.15 / 2.28, 1024 2.65 / 2.73, 1536 3.78 / 3.74.
 bool factors_in_gradients(const lce_problem* p) { return lce::padded_hidden(p->H) <= 1024; }
 
-bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, bool settled, int64_t most_chunks, FusedPlan* f);
+bool plan_fused_with(const lce_problem* p, bool lo8, bool settled, int64_t most_chunks, FusedPlan* f);
 constexpr int64_t kMostChunks = 1024;  // (lce_compact.hip counts the rows of so many)
 
 // The lower halves of the fp32 sums of a 16-bit dW at 16 bits (the sums are then exact fp32) or at 8 (sums of 24
@@ -396,10 +396,10 @@ constexpr int64_t kMostChunks = 1024;  // (lce_compact.hip counts the rows of so
 // most_chunks: of the plan with bytes.
 constexpr double kBytesMargin = 0.97;
 bool fastest_fused(const lce_problem* p, bool settled, int64_t most_chunks, FusedPlan* f) {
-  const bool halves = plan_fused_with(p, true, true, false, settled, kMostChunks, f);
+  const bool halves = plan_fused_with(p, false, settled, kMostChunks, f);
   if ((p->route & LCE_ROUTE_EXACT_SUMS) || p->dw_dtype == LCE_F32) return halves;
   FusedPlan b;
-  if (plan_fused_with(p, true, true, true, settled, most_chunks, &b) && (!halves || b.cost < kBytesMargin * f->cost)) {
+  if (plan_fused_with(p, true, settled, most_chunks, &b) && (!halves || b.cost < kBytesMargin * f->cost)) {
     *f = b;
     return true;
   }
@@ -424,7 +424,7 @@ int make_plan_fused(const lce_problem* p, FusedPlan* f) {
   const int allowed = rounding_of(fastest_fused(p, true, kMostChunks, &settled), settled);
   if (allowed == kAsTwoPasses) return false;
   if (allowed == kSums24 && rounding_of(ok, *f) == kSums24 && f->chunks > settled.chunks) ok = fastest_fused(p, false, settled.chunks, f);
-  return rounding_of(ok, *f) <= allowed ? ok : plan_fused_with(p, true, true, false, false, kMostChunks, f);
+  return rounding_of(ok, *f) <= allowed ? ok : plan_fused_with(p, false, false, kMostChunks, f);
 }
 // (for both gradients, whichever the caller wants: the workspace does not depend on that)
 bool plan_fused(const lce_problem* p, FusedPlan* f) {
@@ -432,7 +432,7 @@ bool plan_fused(const lce_problem* p, FusedPlan* f) {
   return last.get(p, f, make_plan_fused) != 0;
 }
 
-bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8, bool settled, int64_t most_chunks, FusedPlan* f) {
+bool plan_fused_with(const lce_problem* p, bool lo8, bool settled, int64_t most_chunks, FusedPlan* f) {
   memset(f, 0, sizeof(*f));
   f->lo8 = lo8;
   const bool x16 = p->x_dtype == LCE_BF16 || p->x_dtype == LCE_F16;
@@ -477,18 +477,18 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
     out->dw_f = apart ? t : out->part_max; if (apart) t += part;
     out->stage = t; t += align_up((size_t)nc * Vp * 2);
     // split-K partial sums of dx (and, with a single chunk, of dW): one buffer
-    size_t pb = want_dx ? dx_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp, products(p)) : 0;
-    if (chunks == 1 && want_dw) {
+    size_t pb = dx_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp, products(p));
+    if (chunks == 1) {
       const size_t w = dw_part_bytes((size_t)nc, Hp, (int64_t)Vp, (int64_t)Vp, products(p));
       if (w > pb) pb = w;
     }
     out->part = t; t += pb;
     out->parts_on = pb != 0;
     out->plane = t;
-    if (chunks > 1 && want_dw && !f->dw_direct) t += align_up(Hp * Vp * (lo8 ? 1 : 2));
+    if (chunks > 1 && !f->dw_direct) t += align_up(Hp * Vp * (lo8 ? 1 : 2));
     // (upper halves of the tiles that the edge of dW cuts: the last tile row over h, the last over v)
     out->plane_hi = t;
-    if (chunks > 1 && want_dw && !f->dw_direct)
+    if (chunks > 1 && !f->dw_direct)
       t += align_up(((Hp != (size_t)p->H ? Vp / 256 : 0) + (Vp != (size_t)p->V ? Hp / 256 : 0)) * (size_t)(256 * 256 * 2));
     out->total = t;
     return t;
@@ -507,7 +507,7 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
     const int64_t chunks = (tiles + t - 1) / t;
     if (chunks > most_chunks || (first != 0 && chunks > 4 * first + 8)) break;
     if (t < tiles && (tiles + t) / (t + 1) == chunks) continue;  // a longer chunk gives the same number of chunks
-    if (chunks > 1 && want_dw && !f->dw_direct && !halves_ok) continue;
+    if (chunks > 1 && !f->dw_direct && !halves_ok) continue;
     const int64_t t_even = (tiles + chunks - 1) / chunks;  // equal lengths
     // (where the bound has no room for the tables of factors, the pass over the stage does the same)
     FusedPlan cand = *f;
@@ -518,8 +518,8 @@ bool plan_fused_with(const lce_problem* p, bool want_dx, bool want_dw, bool lo8,
     const int64_t t_last = tiles - (chunks - 1) * t_even;
     auto chunk_cost = [&](double tt) -> double {
       return kernel_cost(tt * tv, (double)(lce::padded_k(p->H) / 64), 8.0, false, settled) +
-             (want_dx ? kernel_cost(tt * th, mul * (double)(Vp / 64), 5.0, true, settled) : 0.0) +
-             (want_dw ? kernel_cost(tv * th, mul * tt * 4.0, chunks > 1 ? (f->dw_direct ? 16.0 : lo8 ? 10.0 : 12.0) : 5.0, chunks == 1, settled) : 0.0);
+             kernel_cost(tt * th, mul * (double)(Vp / 64), 5.0, true, settled) +
+             kernel_cost(tv * th, mul * tt * 4.0, chunks > 1 ? (f->dw_direct ? 16.0 : lo8 ? 10.0 : 12.0) : 5.0, chunks == 1, settled);
     };
     // (per chunk, besides the tile kernels: the row merge, the kernel that adds dx's K segments, launch gaps -- about 25 units)
     const double cost = (double)(chunks - 1) * chunk_cost((double)t_even) + chunk_cost((double)t_last) + 25.0 * (double)chunks;
