@@ -514,6 +514,7 @@ def test_fp32_sums_of_dw_keep_to_their_columns(N, H, V, n_chunk, layout):
 
 # one chunk, hidden sizes on either side of the line up to which the gradient kernels multiply by the factors: the partials that the
 # row merge reads are still there after a full call
+@pytest.mark.pack_auto
 @pytest.mark.parametrize("mon", [False, True])
 @pytest.mark.parametrize("H", [256, 1024, 1280])
 def test_row_merge_alone_on_the_workspace_of_a_full_call(H, mon):
@@ -540,3 +541,42 @@ def test_row_merge_alone_on_the_workspace_of_a_full_call(H, mon):
     torch.cuda.synchronize()
     for full, again in zip(*results):
         assert torch.equal(full, again)
+
+
+# The products and roundings of the two ways of forming dz are the same: hidden states and weight as they are (H up to 1024: dx and dW
+# multiply by the factors) and with rows of zeros added up to H = 1032 (a pass over the stage) give the same bits.  K too short to be
+# cut (less than 32 K tiles), so that the sums are formed in one order; 128 x 128 and 256 x 256 logit tiles (`limit`), one chunk and
+# several, a frequent label.
+@pytest.mark.pack_auto
+@pytest.mark.parametrize("N,H,V,dt,n_chunk,ign,z_reg,pack,layout,mon,limit", [
+    (1700, 1024, 1700, torch.bfloat16, 8192, 0.1, 0.0, 2, 0, False, 0), (1700, 1024, 1792, torch.float16, 8192, 0.0, 1e-2, 2, 1, False, 255),
+    (257, 200, 1001, torch.bfloat16, 4096, 0.3, 1e-3, 2, 0, True, 255), (700, 8, 300, torch.float16, 65536, 0.0, 0.0, 2, 1, False, 0),
+    (6000, 768, 1500, torch.bfloat16, 4096, 0.2, 0.0, 1, 0, False, 255), (6000, 520, 1790, torch.float16, 4096, 0.2, 1e-3, 1, 1, True, 255),
+])
+def test_factors_give_the_bits_of_the_pass_over_the_stage(N, H, V, dt, n_chunk, ign, z_reg, pack, layout, mon, limit):
+    from linear_cross_entropy_loss_amd import _lib, ops
+
+    lib = _lib.load()
+    x, y, w = make_inputs(N, H, V, dt, 29, ignore_frac=ign, device="cuda")
+    y[(y != -1) & (torch.arange(N, device="cuda") % 3 == 0)] = V - 1
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    plans, outs = [], []
+    for h in (H, 1032):
+        xh = torch.nn.functional.pad(x, (0, h - H))
+        wh = torch.nn.functional.pad(w, (0, 0, 0, h - H))
+        wh = ops._aligned_rows(wh.t().contiguous() if layout else wh)
+        dx, dw = torch.empty_like(xh), ops._empty_rows(*wh.shape, dt, "cuda")
+        prob = _lib.make_problem(N, h, V, xh.stride(0), wh.stride(0), h, dw.stride(0), dt, dt, dt, dt, -1, 1.5, z_reg, n_chunk, mon, 0,
+                                 pack, limit, layout, _lib.ROUTE_ONE_PASS | _lib.ROUTE_EXACT_SUMS)
+        plans.append(_lib.forward_backward_plan(prob))
+        ws = torch.full((_lib.forward_backward_workspace_bytes(prob),), 0xff, dtype=torch.uint8, device="cuda")
+        g, lse, out5 = torch.ones(1, device="cuda"), torch.empty(N, device="cuda"), torch.empty(5, device="cuda")
+        nv = torch.zeros(1, dtype=torch.int64, device="cuda")
+        rc = lib.lce_forward_backward(ctypes.byref(prob), P(xh), P(wh), P(y), P(g), P(lse), P(out5), P(nv), P(dx), P(dw), P(ws),
+                                      ws.numel(), st)
+        assert rc == 0
+        outs.append((lse, dx[:, :H], dw[:, :H] if layout else dw[:H]))
+    print(plans, flush=True)
+    assert plans[0] == plans[1] and plans[0][0] > 0
+    for few, many in zip(*outs):
+        assert torch.isfinite(few).all() and few.any() and torch.equal(few, many)
