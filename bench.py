@@ -97,8 +97,9 @@ def time_phases_one_pass(cfg, x, y, w, prob, chunks, torch, reps):
     out = {}
     for name, ph, flops, nbytes in (
         ("fwd_stage", _lib.PHASE_FWD_TILES, 2.0 * (N if cfg["monitoring"] else rows) * H * V / chunks, 0.0),
-        # 2 bytes read and 2 written per logit: bound by memory traffic, not by matrix instructions
-        ("stage_scale", _lib.PHASE_BWD_DZ, 0.0, 4.0 * rows * V / chunks),
+        # 2 bytes read and 2 written per logit: bound by memory traffic, not by matrix instructions (hidden sizes up to 1024: the
+        # factors are worked out alone, and the stage is not touched but for the slices of the target columns)
+        ("stage_scale", _lib.PHASE_BWD_DZ, 0.0, 4.0 * rows * V / chunks) if H > 1024 else ("stage_factors", _lib.PHASE_BWD_DZ, 0.0, 0.0),
         ("bwd_dx", _lib.PHASE_BWD_DX, 2.0 * rows * H * V / chunks, 0.0),
         # (with more than one chunk: the tile kernel adds into the fp32 sums of dW that are kept over the chunks; the last chunk's launch stores dW)
         ("bwd_dw", _lib.PHASE_BWD_DW, 2.0 * rows * H * V / chunks, 0.0),

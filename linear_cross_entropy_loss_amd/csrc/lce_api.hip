@@ -737,7 +737,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
     fa.n_rows = all_rows ? nullptr : n_rows; fa.perm = perm; fa.y0 = y; fa.y = yc;
   }
 
-  // (a call restricted to some kernels works on what a full call left in the workspace)
+  // (a call restricted to some kernels works on what a full call left in the workspace: of several chunks, the last one's)
   const int ph = p->phases ? p->phases : ~0;
   // the count of valid labels comes first (the gradients' factor needs it), with it the packing
   hipError_t e = hipSuccess;

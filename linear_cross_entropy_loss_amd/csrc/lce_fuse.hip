@@ -88,8 +88,10 @@ __global__ __launch_bounds__(256) void stage_scale_kernel(const BwdArgs a) {
 // that holds a token's target is rewritten here, with a factor of 1 from then on.  One workgroup per token tile and
 // kSlices slices.  (The two tables may be part_lse and part_max themselves: where there are several chunks, nothing reads
 // those any more.)
-// Bound by launch and latency: 12 bytes per 128 logits and 512 per token.  (4096 tokens, us a launch against the pass over
-// the stage: V=32000 21 / 79, V=50257 22 / 129, V=65536 13 / 165; which problems take it: factors_in_gradients in lce_api.hip.)
+// Bound by launch and latency: 12 bytes per 128 logits and 512 per token.  (4096 tokens, labels drawn uniformly, us a launch
+// against the pass over the stage: V=32000 10 / 79, V=50264 12 / 122, V=65536 12 / 168; labels of a Zipf distribution, whose
+// frequent ones give a workgroup many slices to rewrite: V=32000 17, V=50257 19.  Which problems take it: factors_in_gradients in
+// lce_api.hip.)
 constexpr int kSlices = 8;
 template <class T>
 __global__ __launch_bounds__(256) void stage_factors_kernel(const BwdArgs a) {

@@ -231,11 +231,11 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
   int q_phase;    // blocked Q operand with rows as its K index: K tile of the current row of blocks, 0..3
   int64_t q_jump; // and the bytes from the last K tile of a row of blocks to the first of the next
   static constexpr bool kQRowBlocks = Problem::kQBlocked && !Q_KC;
-  // Problem::kQScale: the factors of the K tile in the staging set and of the one after it ([LDS stage of the K tile]), and where
-  // those of the K tile being loaded are.
   static constexpr bool kSplit = Problem::kSplit;
   int split_s;         // kSplit: which of the K tile's three products the stream is at
   int64_t p_lo, q_lo;  // and the bytes to the lo parts
+  // Problem::kQScale: the factors of the K tile in the staging set and of the one after it ([LDS stage of the K tile]), and where
+  // those of the K tile being loaded are.
   static constexpr bool kQScale = Problem::kQScale;
   f32x4_t qfac[2][2];
   const float* qfac_base;
@@ -314,8 +314,6 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
     ps.retarget(k_rem);
     qs.retarget(k_rem);
   }
-  // chunks 0..7 of a staged K tile belong to P, 8..15 to Q; with factors they alternate, so that the multiplications
-  // are spread over the k-steps
   template <int STAGE> LCE_DEV void load_factors() {
     if constexpr (kQScale) {
       const __amdgpu_buffer_rsrc_t rsrc =
@@ -324,6 +322,8 @@ template <class T, class PSrc, bool P_KC, class QSrc, bool Q_KC, class Problem> 
       qfac[STAGE][1] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)qfac_off, 16, 0));
     }
   }
+  // chunks 0..7 of a staged K tile belong to P, 8..15 to Q; with factors they alternate, so that the multiplications
+  // are spread over the k-steps
   template <int STAGE> LCE_DEV void store_chunks(const PRegs& sp, const QRegs& sq, char* stage, int c0, int c1) {
     if constexpr (kQScale) {
 #pragma unroll
