@@ -194,6 +194,8 @@ struct BwdPlan {
   bool stage_dx;
   bool pack_on;   // tokens with an ignored label are packed away in this backward
   bool parts_on;  // tail tiles of dx / dW may be split along K (partial-sum blocks exist)
+  bool small;     // dx and dW run on 128 x 128 tiles (small_grads_pay)
+  int64_t small_blocks;  // room for their partial sums
   int64_t lddxc;
   size_t dz, dx_acc, dx_part, dw_part, w16, total;
 };
@@ -220,6 +222,10 @@ size_t dw_part_bytes(size_t Np, size_t Hp, int64_t vs, int64_t last_vs, int prod
 // tile; a launch costs about 10.  `settled`: the costs by which make_plan_fused decides what may be rounded, with K segments in
 // powers of two.
 constexpr double kPlanCUs = 256.0;
+// A unit in us, and how much faster the gradients on small tiles have to be by the model, which is off by up to 10 %.  Narrow
+// hidden sizes, for which a tight bound leaves slabs of the vocabulary, gain most: a step of bf16 N=16384, H=256, V=4096 586 -> 372 us,
+// N=8192, H=512, V=8192 583 -> 394, fp16 N=18432, H=128, V=9344 800 -> 540, fp32 N=4096, H=512, V=2048 940 -> 463.
+constexpr double kUnitUs = 1.4, kSmallMargin = 0.93;
 double kernel_cost(double T, double L, double e, bool parts, bool settled) {
   const double full = (double)(int64_t)(T / kPlanCUs), r = T - full * kPlanCUs;
   double cost = full * (L + e) + 10.0;
@@ -269,6 +275,11 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
   // bands of W tiles that bwd_dz keeps in flight (tile_coords in lce_gemm.h), and the slab width that is a whole group of them
   const int live = lce::live_bands(logit_k_bytes(p));
   const int64_t gran = live < 8 ? (int64_t)256 * 8 * live : 256;
+  auto logits_cost = [&](int64_t w) -> double {
+    const int64_t kt = lce::small_logit_ktiles(p->H, products(p));
+    const double a = lce::persistent_logits_us(p->N, w, kt), c = lce::small_logits_us(p->N, w, kt);
+    return (a < c ? a : c) / kUnitUs;
+  };
   auto slab_cost = [&](int64_t w, bool parts, bool sums) -> double {
     const double tq = (double)(Np / 256), th = (double)(Hp / 256), tv = (double)(w / 256), k3 = split ? 3.0 : 1.0;
     // (bwd_dz runs about 4 % slower on a slab that is not whole groups of the bands it keeps in flight when K is long)
@@ -278,6 +289,7 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
            kernel_cost(tv * th, k3 * (double)(Np / 64), 5.0, parts, settled);
   };
 
+  bool full_fits = false;
   // mode 0: everything; mode 1: lean (at the strict bound only); mode 2: everything, widened bound.
   // Tries a split into `s` slabs of equal width (the last one may be narrower); cost: its modelled time.
   auto fits = [&](int mode, int64_t s, bool whole_groups, BwdPlan* out, double* cost) -> bool {
@@ -318,8 +330,34 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
     out->w16 = fixed + dz + acc + part;
     out->total = fixed + dz + acc + part + w16;
     // (a lean plan computes the tokens with an ignored label too; how many there are is not known here)
-    *cost = ((double)(slabs - 1) * slab_cost(vs, !lean, acc != 0) + slab_cost(last_vs, !lean, acc != 0)) *
-            (lean && packs_rows(p) ? 1.02 : 1.0);
+    const double extra = lean && packs_rows(p) ? 1.02 : 1.0;
+    *cost = ((double)(slabs - 1) * slab_cost(vs, !lean, acc != 0) + slab_cost(last_vs, !lean, acc != 0)) * extra;
+    out->small = false;
+    if (settled || p->max_workgroups != 0 || pack || (lean && full_fits)) return true;
+    // The gradients on small tiles instead: their partial sums take the place of the others', or, in a lean plan that is one
+    // because no other fits, what room the bound has left.
+    const size_t room = !lean ? part : budget - counted;
+    out->small_blocks = (int64_t)(room / lce::kSmallBlockBytes);
+    auto small_cost = [&](int64_t w) -> double {
+      if (lce::pad_to(p->N, 128) / 128 * (lce::pad_to(p->H, 128) / 128) > 1 << 14 || w / 128 * (lce::pad_to(p->H, 128) / 128) > 1 << 14)
+        return 1e300;
+      const lce::SmallGrads g = lce::plan_small_grads(p->N, p->H, w, products(p), out->small_blocks);
+      return logits_cost(w) + (g.us + (acc != 0 ? (double)(Np * Hp) * 1.6e-6 : 0.0)) / kUnitUs;
+    };
+    const double small = ((double)(slabs - 1) * small_cost(vs) + small_cost(last_vs)) * extra;
+    if (small < kSmallMargin * *cost) {
+      *cost = small;
+      out->small = true;
+      if (lean) {
+        const lce::SmallGrads g0 = lce::plan_small_grads(p->N, p->H, vs, products(p), out->small_blocks);
+        const lce::SmallGrads g1 = lce::plan_small_grads(p->N, p->H, last_vs, products(p), out->small_blocks);
+        const int64_t b0 = g0.dx_blocks + g0.dw_blocks, b1 = g1.dx_blocks + g1.dw_blocks;
+        out->small_blocks = b0 > b1 ? b0 : b1;
+        const size_t more = (size_t)(out->small_blocks * lce::kSmallBlockBytes);
+        out->w16 += more;
+        out->total += more;
+      }
+    }
     return true;
   };
   // The fewest slabs that fit, or a few more of them when the model says that their tiles fill the rounds of
@@ -341,7 +379,8 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
   };
   BwdPlan full = *b, lean = *b;
   double cost_full = 0, cost_lean = 0;
-  const bool ok_full = choose(0, &full, &cost_full), ok_lean = choose(1, &lean, &cost_lean);
+  const bool ok_full = full_fits = choose(0, &full, &cost_full);
+  const bool ok_lean = choose(1, &lean, &cost_lean);
   if (ok_full && (!ok_lean || cost_full <= cost_lean)) { *b = full; b->cost = cost_full; return LCE_OK; }
   if (ok_lean) { *b = lean; b->cost = cost_lean; return LCE_OK; }
   double wide = 0;
@@ -542,7 +581,10 @@ bool plan_fused_with(const lce_problem* p, bool lo8, bool settled, int64_t most_
   const double scale_pass = f->factors ? 12.0 * (double)f->chunks : (double)Np * (double)Vp * 4.0 / 8.0e6;
   f->cost = best + scale_pass;
   if (route_of(p) == LCE_ROUTE_AUTO && (settled ? make_plan_bwd(p, &b, true) : plan_bwd(p, &b)) == LCE_OK) {
-    const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false, settled) + b.cost;
+    // (at these sizes the model is a quarter to a third above what the other kernels take: N=1024, H=2048, V=8192 156 us in one
+    // pass, 179 in two with the gradients on small tiles)
+    const double two_bwd = b.small ? 1.4 * b.cost : b.cost;
+    const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false, settled) + two_bwd;
     // (sums of 24 bits have to be ahead of two passes, which are exact, by the margin as well)
     if (best + scale_pass > two * (lo8 ? kBytesMargin : 1.0)) {
       f->ok = false;  // (f->chunks stays: a plan fitted)
@@ -1036,11 +1078,19 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
       e = lce::launch_bwd_dz(a, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_dz");
     }
-    if (dx && (ph & LCE_PHASE_BWD_DX)) {
+    const bool want_dx = dx && (ph & LCE_PHASE_BWD_DX), want_dw = dw && (ph & LCE_PHASE_BWD_DW);
+    if (b.small) {
+      lce::SmallGrads g = lce::plan_small_grads(p->N, p->H, a.vw, products(p), b.small_blocks);
+      g.part = (float*)(base + b.dx_part);
+      e = lce::launch_bwd_grads_small(a, g, want_dx, want_dw, s);
+      if (e != hipSuccess) return hip_fail(e, "bwd_grads_small");
+      continue;
+    }
+    if (want_dx) {
       e = lce::launch_bwd_dx(a, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_dx");
     }
-    if (dw && (ph & LCE_PHASE_BWD_DW)) {
+    if (want_dw) {
       e = lce::launch_bwd_dw(a, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_dw");
     }

@@ -419,7 +419,7 @@ __global__ __launch_bounds__(kThreads, 2) void dz_small_kernel(const BwdArgs a, 
   // (the second half of a tile of 256 tokens may have none: logits of rows that do not exist are zeros)
   pipe.run(w + (WVH ? v * a.ldw : v), WVH ? matrix_end<E>(w, a.Vw, a.ldw, a.H) : matrix_end<E>(w, kParts * a.H, a.ldw, a.Vw), a.ldw,
            x + t0 * ldx, matrix_end<E>(x, rows, ldx, kParts == 2 ? a.x_lo + a.H : a.H), ldx, a.H,
-           t0 < rows ? logit_ktiles<T>(a.H) : 0, a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
+           t0 < rows ? (int)small_logit_ktiles(a.H, kParts == 2 ? 3 : 1) : 0, a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
   char* mine = lds + wave * kWaveLds;
   if (slice_v0 + kSmallTile <= a.v0 + a.vw) dz_epilogue_impl<T, ZREG, false, FUSE, 1>(a, pf_y, pf_lse, acc, slice_v0, tw, mine);
   else dz_epilogue_impl<T, ZREG, true, FUSE, 1>(a, pf_y, pf_lse, acc, slice_v0, tw, mine);
@@ -439,7 +439,7 @@ hipError_t launch_one(const BwdArgs& a, int64_t tiles, hipStream_t s) {
 // All tile columns of the slab in one launch.
 template <class T, bool ZREG, bool WVH, bool FUSE = false>
 hipError_t launch_persistent_z(const BwdArgs& a, hipStream_t s) {
-  if (few_logit_tiles(a.N <= kSmallTile ? a.N : a.Np, a.vw, a.small_wgs)) {
+  if (few_logit_tiles(a.N <= kSmallTile ? a.N : a.Np, a.vw, small_logit_ktiles(a.H, products_of(a.x_dtype)), a.small_wgs)) {
     const int tiles_p = (int)(a.vs / kSmallTile), tiles_q = (int)(a.Np / kSmallTile);
     hipLaunchKernelGGL((dz_small_kernel<T, ZREG, WVH, FUSE>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a,
                        tiles_p, tiles_q);

@@ -424,8 +424,8 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_small_kernel(const FwdArgs a,
   SmallPipe<T, WVH> pipe;
   f32x16_t acc[kNB][1];
   pipe.run(w + (WVH ? v * a.ldw : v), WVH ? matrix_end<E>(w, a.Vw, a.ldw, a.H) : matrix_end<E>(w, kParts * a.H, a.ldw, a.Vw), a.ldw,
-           x + (a.row0 + t0) * ldx, matrix_end<E>(x, rows, ldx, kParts == 2 ? a.x_lo + a.H : a.H), ldx, a.H, logit_ktiles<T>(a.H),
-           a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
+           x + (a.row0 + t0) * ldx, matrix_end<E>(x, rows, ldx, kParts == 2 ? a.x_lo + a.H : a.H), ldx, a.H,
+           (int)small_logit_ktiles(a.H, kParts == 2 ? 3 : 1), a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
   // (with the sums of the persistent kernel, bit for bit: by columns but in the tile of 256 columns that straddles the end)
   const int64_t slice_v0 = a.v0 + (int64_t)tp * kSmallTile;
   const int64_t tw = t0 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kBlk;
@@ -668,7 +668,7 @@ hipError_t launch_one(const FwdArgs& a, int64_t tiles, hipStream_t s) {
 template <class T, bool WVH, bool MON> hipError_t launch_persistent(const FwdArgs& a, hipStream_t s) {
   const int64_t left = a.Np - a.row0;  // token tiles of this chunk at most
   const int64_t here = left < a.nc ? left : a.nc, there = a.N - a.row0, rows = here < there ? here : there;
-  if (few_logit_tiles(rows, a.vw, a.small_wgs)) {
+  if (few_logit_tiles(rows, a.vw, small_logit_ktiles(a.H, products_of(a.x_dtype)), a.small_wgs)) {
     const int tiles_p = (int)(pad_to(a.vw, kTile) / kSmallTile), tiles_q = (int)((rows + kSmallTile - 1) / kSmallTile);
     hipLaunchKernelGGL((fwd_small_kernel<T, WVH, MON>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a, tiles_p,
                        tiles_q);

@@ -93,7 +93,7 @@ template <class T, class SrcT, bool KC, bool KMASK, int CHUNKS = 8> struct Stage
   // The operand is stored in blocks of 256 rows x 64 columns, [rows / 256][cols / 64][256][64] (the staged dz, see
   // BwdArgs::dz), instead of row-major.  KC (its columns are the K index): the 256 rows x 64 k of a K tile are one
   // contiguous block of 128-byte rows, and the next K tile is the next block.  Otherwise (its rows are the K
-  // index): the tile's 256 columns are four consecutive blocks, each thread stays in one; a K tile is 64 rows of
+  // index): the tile's 256 columns are four consecutive blocks (128 columns: two), each thread stays in one; a K tile is 64 rows of
   // them, and after four K tiles the stream moves on to the next row of blocks (Pipe3::stream_advance).
   // (`parts` = 2: every block is followed by the block of its lo part)
   LCE_DEV void init_blocked(int parts) {
@@ -101,10 +101,10 @@ template <class T, class SrcT, bool KC, bool KMASK, int CHUNKS = 8> struct Stage
     if (KC) {
       k_stride = parts * kTile * (kBK * kEs);
     } else {
-      const int t = threadIdx.x, c = t & 31, k = t >> 5;
+      const int t = threadIdx.x, c = t % kRowPieces, k = t / kRowPieces;
       voff = (unsigned)((c >> 3) * parts * (kTile * kBK * kEs) + k * (kBK * kEs) + (c & 7) * 16);
       voff_cur = voff;
-      iter_stride = (unsigned)(8 * kBK * kEs);
+      iter_stride = (unsigned)(kRowsAtOnce * kBK * kEs);
       k_stride = (int64_t)kBK * kBK * kEs;
     }
   }

@@ -21,21 +21,29 @@ constexpr int kSmallOperandBytes = kSmallTile * kBK * 2;
 constexpr int kSmallStageBytes = 2 * kSmallOperandBytes;
 constexpr int kSmallLds = 2 * kSmallStageBytes;  // 64 KiB: two workgroups to a compute unit
 
-template <class T, bool P_KC> struct SmallPipe {
+// NP, NQ: blocks of 32 P / Q rows of a wave, four accumulator blocks together: 4, 1 for the logits; 2, 2 for the gradients, whose
+// epilogues do not need a slice of the vocabulary in one wave and whose fragment reads are then four for four products.
+// Q_BLOCKED, SWAP: Problem::kQBlocked and kSwapAB of Pipe3.
+template <class T, bool P_KC, bool Q_KC = true, bool Q_BLOCKED = false, int NP = 4, int NQ = 1, bool SWAP = false> struct SmallPipe {
+  static_assert(NP * NQ == kNB, "four accumulator blocks to a wave");
   typedef typename elem_of<T>::type E;
   static constexpr bool kSplit = is_pair<T>::value;
+  static constexpr bool kQRowBlocks = Q_BLOCKED && !Q_KC;
+  static constexpr int kWavesP = kNB / NP;
   typedef Stager3<T, E, P_KC, true, 4> PStager;
-  typedef Stager3<T, E, true, true, 4> QStager;
+  typedef Stager3<T, E, Q_KC, true, 4> QStager;
   PStager ps;
   QStager qs;
   FragReader<P_KC, kSmallTile> pr;
-  FragReader<true, kSmallTile> qr;
+  FragReader<Q_KC, kSmallTile> qr;
   typename PStager::Regs sp[2];  // K tiles t + 1 and t + 2 while t is multiplied; set t & 1
   typename QStager::Regs sq[2];
   int k_rem, split_s;
   int64_t p_lo, q_lo;
+  int q_phase;     // as in Pipe3
+  int64_t q_jump;
 
-  s16x8_t pf[2][kNB], qf[2];     // fragments of this k-step and the next
+  s16x8_t pf[2][NP], qf[2][NQ];  // fragments of this k-step and the next
 
   LCE_DEV void advance() {
     if constexpr (kSplit) {
@@ -51,7 +59,12 @@ template <class T, bool P_KC> struct SmallPipe {
       split_s = 0;
     }
     ps.base += ps.k_stride;
-    qs.base += qs.k_stride;
+    if constexpr (kQRowBlocks) {
+      qs.base += q_phase == 3 ? q_jump : qs.k_stride;
+      q_phase = (q_phase + 1) & 3;
+    } else {
+      qs.base += qs.k_stride;
+    }
     k_rem -= kBK;
     ps.retarget(k_rem);
     qs.retarget(k_rem);
@@ -72,15 +85,21 @@ template <class T, bool P_KC> struct SmallPipe {
     }
   }
   LCE_DEV void read_frags(const char* stage, int ks) {
-    qf[ks & 1] = qr.read(stage + kSmallOperandBytes, 0, ks);
 #pragma unroll
-    for (int i = 0; i < kNB; ++i) pf[ks & 1][i] = pr.read(stage, i, ks);
-  }
-  LCE_DEV void multiply(int ks, f32x16_t (&acc)[kNB][1]) {
+    for (int j = 0; j < NQ; ++j) qf[ks & 1][j] = qr.read(stage + kSmallOperandBytes, j, ks);
 #pragma unroll
-    for (int i = 0; i < kNB; ++i) acc[i][0] = mfma32<T>(pf[ks & 1][i], qf[ks & 1], acc[i][0]);
+    for (int i = 0; i < NP; ++i) pf[ks & 1][i] = pr.read(stage, i, ks);
   }
-  static constexpr int kReads = 1 + (P_KC ? 4 : 8);  // LDS reads of a k-step's fragments
+  LCE_DEV void multiply(int ks, f32x16_t (&acc)[NP][NQ]) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+#pragma unroll
+      for (int jj = 0; jj < NQ; ++jj) {
+        const int j = (i & 1) ? NQ - 1 - jj : jj;
+        acc[i][j] = SWAP ? mfma32<T>(qf[ks & 1][j], pf[ks & 1][i], acc[i][j]) : mfma32<T>(pf[ks & 1][i], qf[ks & 1][j], acc[i][j]);
+      }
+  }
+  static constexpr int kReads = NQ * (Q_KC ? 1 : 2) + NP * (P_KC ? 1 : 2);  // LDS reads of a k-step's fragments
   // What goes behind each of a k-step's four matrix instructions: a quarter of the next one's reads, stores and loads in turn.
   template <int STORES, int LOADS> LCE_DEV void order() {
     __builtin_amdgcn_sched_group_barrier(LCE_SG_MFMA, 1, 0);
@@ -99,7 +118,7 @@ template <class T, bool P_KC> struct SmallPipe {
   // takes K tile t + 3 in its place, chunk by chunk; the barrier opens the last k-step, and the fragments of K tile t + 1's
   // first k-step are read during it.  (Left to the compiler, which put all stores first and all loads last: N=1536, V=2560, H=2048
   // 31 us, so 24; N=48, V=50304, H=2048 43, so 39, which is 5.3 TB/s of weight.)
-  template <int SET> LCE_DEV void step(const char* cur, char* next, f32x16_t (&acc)[kNB][1]) {
+  template <int SET> LCE_DEV void step(const char* cur, char* next, f32x16_t (&acc)[NP][NQ]) {
     read_frags(cur, 1);
     store_chunks<SET>(next, 0, 3);
     load_chunks<SET>(0, 3);
@@ -121,13 +140,21 @@ template <class T, bool P_KC> struct SmallPipe {
     multiply(3, acc);
     order<0, 0>();
   }
-  // p, q: first element of the tile's operands; *_end: one past the last valid byte; ktiles: even, as in Pipe3, or 0.
+  // p, q: first element of the tile's operands; *_end: one past the last valid byte; ktiles: even, or 0.  Q_BLOCKED: ldq and q_phase_
+  // as in Pipe3.
   LCE_DEV void run(const void* p, const void* p_end, int64_t ldp, const void* q, const void* q_end, int64_t ldq, int64_t k_valid,
-                   int ktiles, int64_t p_lo_, int64_t q_lo_, char* lds, f32x16_t (&acc)[kNB][1]) {
+                   int ktiles, int64_t p_lo_, int64_t q_lo_, char* lds, f32x16_t (&acc)[NP][NQ], int q_phase_ = 0) {
+    const int wave = (int)(threadIdx.x >> 6);
     ps.init(ldp);
-    qs.init(ldq);
-    pr.init(0);
-    qr.init((int)(threadIdx.x >> 6) * kBlk);
+    if constexpr (Q_BLOCKED) {
+      qs.init_blocked(kSplit ? 2 : 1);
+      q_jump = ldq * ((kSplit ? 2 : 1) * kTile * kBK * QStager::kEs) - 3 * qs.k_stride;
+      q_phase = q_phase_;
+    } else {
+      qs.init(ldq);
+    }
+    pr.init(wave % kWavesP * (NP * kBlk));
+    qr.init(wave / kWavesP * (NQ * kBlk));
     ps.base = reinterpret_cast<const char*>(p);
     ps.end = reinterpret_cast<const char*>(p_end);
     qs.base = reinterpret_cast<const char*>(q);
@@ -139,9 +166,11 @@ template <class T, bool P_KC> struct SmallPipe {
     ps.retarget(k_rem);
     qs.retarget(k_rem);
 #pragma unroll
-    for (int i = 0; i < kNB; ++i)
+    for (int i = 0; i < NP; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][0][r] = 0.f;
+      for (int j = 0; j < NQ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     load_chunks<0>(0, 8);
     advance();
     load_chunks<1>(0, 8);

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <string.h>
 
 #include <atomic>
 
@@ -49,18 +50,33 @@ constexpr int64_t padded_k(int64_t H) { return pad_to(H, 128) < 256 ? 256 : pad_
 constexpr int64_t padded_k_pair(int64_t H) { return pad_to(H, 128); }
 // Matrix products per K tile of the compute type.
 constexpr int products_of(int dtype) { return dtype == DT_PAIR ? 3 : 1; }
+// K tiles of the logit contraction on 128 x 128 tiles, which need no four of them (N=8192, H=128, V=8192: 60 us with four, 47 with two).
+__host__ __device__ constexpr int64_t small_logit_ktiles(int64_t H, int products) { return products * (pad_to(H, 128) / 64); }
 
-// Whether a logit kernel runs on 128 x 128 tiles, one workgroup each (lce_gemm_small.h), or on the 256 x 256 tiles of the
-// persistent kernels: by the number of workgroups for `rows` token rows and `cols` columns.  `most`: two workgroups for each
-// compute unit (FwdArgs::small_wgs; 0: never).  The persistent kernel starts with 14 us of fetching its code, the other with 5;
-// up to one workgroup to a compute unit its K tile takes half as long, up to two the same time, beyond that half as long again.
-// Loss alone, bf16, us, 128 x 128 / 256 x 256: N=256, V=4096, H=256 8.7 / 18.4, H=4096 46 / 74; N=1536, V=2560 (240 workgroups),
-// H=256 10.5 / 19.6, H=2048 24 / 46; N=4096, V=2048 (512), H=256 12.5 / 18.7, H=1024 25 / 32, H=2048 42 / 49; N=5120, V=2048 (640)
-// 20 / 20, 35 / 33, 61 / 50.  Of up to 128 tokens the persistent kernel's tiles are half empty: N=48, V=100000, H=256 19 / 33,
-// H=2048 94 to 102 / 110.
-inline bool few_logit_tiles(int64_t rows, int64_t cols, int most) {
+// Modelled time of a logit kernel for `rows` token rows, `cols` columns and `kt` 64-deep K tiles (times the products of a pair), us:
+// on 128 x 128 tiles, one workgroup each (lce_gemm_small.h), or on the 256 x 256 tiles of the persistent kernels.  The latter start
+// with 14 us of fetching their code, the former with 5; a round of 512 workgroups, two to a compute unit, takes 0.9 us a K tile and
+// 3.4 for prologue and epilogue, one of up to 256 little more than half of that a K tile, a round of 256 x 256 tiles 1.2 and 5,
+// less where it leaves compute units, and with them power, to the others.  Loss alone, bf16, us measured, 128 x 128 / 256 x 256:
+// N=256, V=4096, H=256 8.7 / 18.4, H=4096 46 / 74; N=1536, V=2560, H=2048 24 / 46; N=4096, V=2048, H=256 12.5 / 18.7, H=2048
+// 42 / 49; N=5120, V=2048, H=256 20 / 20, H=1024 35 / 33, H=2048 61 / 50; N=1999, V=10007, H=500 32 / 45; N=16384, V=1000, H=1024
+// 45 / 42; N=2048, V=16384, H=768 64 / 53; N=4096, V=16384, H=256 60 / 52.
+inline double small_logits_us(int64_t rows, int64_t cols, int64_t kt) {
+  const int64_t n = (rows + 127) / 128 * (pad_to(cols, 256) / 128), full = n / 512, rest = n % 512;
+  return 5.0 + (double)full * (0.9 * (double)kt + 3.4) + (rest == 0 ? 0.0 : (rest > 256 ? 0.9 : 0.5) * (double)kt + 3.4);
+}
+inline double persistent_logits_us(int64_t rows, int64_t cols, int64_t kt) {
+  const int64_t n = (rows + 255) / 256 * (pad_to(cols, 256) / 256), full = n / 256, rest = n % 256;
+  const double round = 1.2 * (double)(kt < 4 ? 4 : kt) + 5.0;
+  return 14.0 + (double)full * round + (rest == 0 ? 0.0 : round / (1.0 + 0.9 * (1.0 - (double)rest / 256.0)));
+}
+// Whether a logit kernel runs on 128 x 128 tiles: up to two workgroups to a compute unit, for up to 128 tokens (of which the other
+// tiles are half empty: N=48, V=100000, H=256 19 / 33, H=2048 94 to 102 / 110), and where the model puts them 8 % ahead (what it is
+// off by).  `most`: two workgroups for each compute unit (FwdArgs::small_wgs; 0: never).
+inline bool few_logit_tiles(int64_t rows, int64_t cols, int64_t kt, int most) {
   const int64_t n = (rows + 127) / 128 * (pad_to(cols, 256) / 128);
-  return n <= most || (rows <= 128 && most > 0);
+  if (most <= 0) return false;
+  return n <= most || rows <= 128 || (n < (int64_t)1 << 28 && small_logits_us(rows, cols, kt) < 0.92 * persistent_logits_us(rows, cols, kt));
 }
 
 // Which tile columns of the vocabulary a logit kernel covers: full ones, the one(s) from the column that straddles the end of
@@ -362,5 +378,84 @@ inline int64_t dw_tail_blocks(int64_t Np, int64_t Hp, int64_t vs, int products) 
   const int64_t most = (vs / 256) * (Hp / 256) * s;
   return most < kTailBlocks ? most : kTailBlocks;
 }
+
+// dx and dW of a single slab on 128 x 128 tiles, in one launch (lce_bwd_small.hip): workgroups [0, first_span) are the tiles of
+// one gradient times its stretches of K, the rest those of the other.  part: one block of 128 x 128 floats for each stretch, those
+// of dx (where it has several) first.  The plan is one for both gradients, whichever the caller wants, and for rows that are not
+// packed: sums of the same tokens are then cut the same way in every call.
+struct SmallGrads {
+  int dw_first, first_span, dx_nseg, dx_blocks, dw_nseg, dw_blocks;
+  double us;  // modelled time
+  float* part;
+};
+constexpr int64_t kSmallBlockBytes = 128 * 128 * 4;
+constexpr int kSmallSlots = 512;  // workgroups that the chip holds at a time, two to a compute unit
+// When the last of na items of la K tiles and then nb of lb (<= la) ends on the slots, each going to the first free one.
+inline double small_span(int64_t na, double la, int64_t nb, double lb) {
+  const int64_t S = kSmallSlots;
+  if (na + nb <= S) return la;
+  int64_t busy = na % S;                       // slots with one item more than the others
+  double low = (double)(na / S) * la, high = busy > 0 ? low + la : low;
+  if (busy == 0) busy = S;
+  int64_t left = nb;
+  double end = high;
+  // (slots that are level with the busiest after k more items of the other kind)
+  while (left > 0) {
+    const int64_t free_slots = S - busy;
+    if (free_slots > 0 && low + lb <= high) {
+      const int64_t rounds = (int64_t)((high - low) / lb), can = rounds * free_slots;
+      if (left <= can) return end;
+      left -= can;
+      low += (double)rounds * lb;
+      continue;
+    }
+    if (free_slots > 0 && low < high) {
+      end = low + lb > end ? low + lb : end;
+      left -= free_slots;
+      if (left <= 0) return end;
+      low = high;  // (those run a little behind the others from here on)
+    }
+    const int64_t rounds = left / S, rest = left - rounds * S;
+    return high + (double)(rounds + (rest > 0 ? 1 : 0)) * lb;
+  }
+  return end;
+}
+// The stretches of K: as many of each gradient as give the shortest launch, with what their sums cost on top, and fit `most_blocks`.
+// kLeastStretch: K tiles of the shortest.
+constexpr int64_t kLeastStretch = 8;
+inline SmallGrads plan_small_grads(int64_t N, int64_t H, int64_t V, int products, int64_t most_blocks) {
+  const int64_t th = (H + 127) / 128, tx = th * ((N + 127) / 128), tw = th * ((V + 127) / 128);
+  const int64_t kx = pad_to(V, 128) / 64, kw = pad_to(N, 128) / 64;
+  auto most = [&](int64_t t, int64_t k) -> int64_t {
+    const int64_t by_length = k / kLeastStretch, by_slots = 4 * kSmallSlots / t;
+    const int64_t m = by_length < by_slots ? by_length : by_slots;
+    return m < 1 ? 1 : m;
+  };
+  SmallGrads g;
+  memset(&g, 0, sizeof(g));
+  g.us = -1;
+  const int64_t mx = most(tx, kx), mw = most(tw, kw);
+  auto next = [](int64_t n) { return n < 16 ? n + 1 : n + n / 8; };
+  for (int64_t nx = 1; nx <= mx; nx = next(nx))
+    for (int64_t nw = 1; nw <= mw; nw = next(nw)) {
+      const int64_t bx = nx > 1 ? tx * nx : 0, bw = nw > 1 ? tw * nw : 0;
+      if (bx + bw > most_blocks) continue;
+      const double lx = (double)((kx / 2 + nx - 1) / nx * 2 * products) + 4.0, lw = (double)((kw / 2 + nw - 1) / nw * 2 * products) + 4.0;
+      const bool wf = lw > lx;
+      double c = wf ? small_span(tw * nw, lw, tx * nx, lx) : small_span(tx * nx, lx, tw * nw, lw);
+      if (tx * nx + tw * nw <= kSmallSlots / 2) c *= 0.55;  // (one to a compute unit)
+      if (bx + bw > 0) c += 6.0 + (double)(bx + bw) * 0.03;
+      c = 5.0 + 0.9 * c;
+      if (g.us >= 0 && c >= g.us) continue;
+      g.us = c;
+      g.dw_first = wf;
+      g.dx_nseg = (int)nx;
+      g.dw_nseg = (int)nw;
+      g.dx_blocks = (int)bx;
+      g.dw_blocks = (int)bw;
+    }
+  return g;
+}
+hipError_t launch_bwd_grads_small(const BwdArgs& a, const SmallGrads& g, bool want_dx, bool want_dw, hipStream_t s);
 
 }  // namespace lce
