@@ -91,7 +91,7 @@ typedef struct lce_problem {
   int32_t pack_rows;    /* LCE_PACK_AUTO | LCE_PACK_ALWAYS | LCE_PACK_NEVER: see below        */
   int32_t max_workgroups; /* profiling aid: cap on the persistent workgroups of the tile kernels (0 = one per compute unit) */
   int32_t w_layout;     /* LCE_W_HV (0) | LCE_W_VH: how w and dw are stored, see below */
-  int32_t route;        /* lce_forward_backward only: LCE_ROUTE_AUTO (0) | LCE_ROUTE_ONE_PASS | LCE_ROUTE_TWO_PASS, [+ LCE_ROUTE_EXACT_SUMS], see there */
+  int32_t route;        /* lce_forward_backward only: LCE_ROUTE_AUTO (0) | LCE_ROUTE_ONE_PASS | LCE_ROUTE_TWO_PASS, [+ a flag], see there */
 } lce_problem;
 
 /*
@@ -268,7 +268,9 @@ enum {
   LCE_ROUTE_ONE_PASS = 1,
   LCE_ROUTE_TWO_PASS = 2,
   /* a flag, to be or-ed to one of the above: a 16-bit dW's sums over chunks are never kept at fewer than 32 bits */
-  LCE_ROUTE_EXACT_SUMS = 4
+  LCE_ROUTE_EXACT_SUMS = 4,
+  /* a flag for fp32 activations, which no other route of lce_forward_backward covers: see there.  From version 900 on. */
+  LCE_ROUTE_KEEP_LOGITS = 16
 };
 
 /*
@@ -311,6 +313,12 @@ enum {
  * does not follow the kernels' speed from one version to the next: the model
  * has to say so with settled costs too.  LCE_ROUTE_ONE_PASS takes it whenever it
  * fits the bound; LCE_ROUTE_TWO_PASS never.
+ *
+ * LCE_ROUTE_KEEP_LOGITS (fp32 activations): the logits are computed once as well, and rounded no further than by the
+ * two calls: the stage of a chunk holds them in fp32 (chunk_rows * V * 4 bytes, beside one copy of the weight as bf16
+ * pairs, H * V * 4), and dz as a pair takes their place.  dW is summed over the chunks in the caller's buffer.  Taken where
+ * that fits the bound and the model says it is faster; lce_forward_backward_plan reports the chunks, 0 of them without
+ * the flag.
  *
  * Problems this route does not cover take the two calls above, one after the
  * other on the same workspace, inside this entry point: fp32 activations, a

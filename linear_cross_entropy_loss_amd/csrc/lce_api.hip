@@ -24,7 +24,7 @@ size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 bool is16(int d) { return d == LCE_BF16 || d == LCE_F16; }
 
-int route_of(const lce_problem* p) { return p->route & ~LCE_ROUTE_EXACT_SUMS; }
+int route_of(const lce_problem* p) { return p->route & ~(LCE_ROUTE_EXACT_SUMS | LCE_ROUTE_KEEP_LOGITS); }
 
 // The last plan of a kind that this thread made.  A call asks for its plan up to three times (whether the route covers the
 // problem, the workspace, the launches), and a training step for the same one as the step before; a plan follows from the
@@ -61,6 +61,7 @@ int check(const lce_problem* p, bool backward) {
   if (p->max_workgroups < 0) return LCE_EINVAL_ARG;
   if (p->w_layout != LCE_W_HV && p->w_layout != LCE_W_VH) return LCE_EINVAL_ARG;
   if (route_of(p) != LCE_ROUTE_AUTO && route_of(p) != LCE_ROUTE_ONE_PASS && route_of(p) != LCE_ROUTE_TWO_PASS) return LCE_EINVAL_ARG;
+  if ((p->route & LCE_ROUTE_KEEP_LOGITS) && xd != LCE_F32) return LCE_EINVAL_ARG;
   const bool vh = p->w_layout == LCE_W_VH;
   // (V, H) weight: both operands of the logit contraction run along H in memory, so no 16-byte piece may
   // straddle the end of a row (H a multiple of 8), and there is no bf16-pair form of it
@@ -412,6 +413,10 @@ struct FusedPlan {
   bool parts_on;
   bool dw_direct;  // fp32 dW: the chunks' terms are added in the caller's buffer, there is no plane
   bool lo8;        // the lower halves of a 16-bit dW's sums are cut to a byte (lce_bwd_dw.hip)
+  bool kept;       // fp32: the stage holds the logits themselves (LCE_ROUTE_KEEP_LOGITS)
+  bool small;      // dx and dW run on 128 x 128 tiles
+  int dx_grid;     // workgroups of the dx kernel (0: one to a compute unit)
+  int64_t small_blocks;
   bool factors;    // the dx and dW kernels turn the staged e into dz (factors_in_gradients)
   double cost;     // modelled time of the plan (kernel_cost units)
 };
@@ -456,7 +461,9 @@ int rounding_of(bool one_pass, const FusedPlan& f) { return !one_pass ? kAsTwoPa
 // over N = 128 ... 32768, H = 64 ... 8192, V = 256 ... 262144 are rounded further, nearly all of them with H <= 1024.  Error
 // against fp64 and time, one pass / two: bf16 under an fp32 weight, N=3285, H=320, V=40832 dW 5.20e-5 / 5.08e-5, dx 2.3540e-3 /
 // 2.3537e-3, 500 / 559 us; bf16, N=896, H=704, V=46592 dx 1.6475e-3 / 1.6474e-3, 291 / 327 us, N=3411, H=256, V=80256 779 / 735.)
+bool plan_kept(const lce_problem* p, FusedPlan* f);
 int make_plan_fused(const lce_problem* p, FusedPlan* f) {
+  if (splits(p)) return plan_kept(p, f);
   bool ok = fastest_fused(p, false, kMostChunks, f);
   if (!ok) return false;
   FusedPlan settled;
@@ -465,6 +472,101 @@ int make_plan_fused(const lce_problem* p, FusedPlan* f) {
   if (allowed == kSums24 && rounding_of(ok, *f) == kSums24 && f->chunks > settled.chunks) ok = fastest_fused(p, false, settled.chunks, f);
   return rounding_of(ok, *f) <= allowed ? ok : plan_fused_with(p, false, false, kMostChunks, f);
 }
+// LCE_ROUTE_KEEP_LOGITS: chunks of token rows whose fp32 logits stay in the stage until their rows' lse are known.  Against two passes
+// a contraction (three products of bf16 pairs) is saved for 8 bytes of memory traffic per logit, and the weight is split into pairs
+// once and not twice; what it needs is room for all of that copy.
+bool plan_kept(const lce_problem* p, FusedPlan* f) {
+  memset(f, 0, sizeof(*f));
+  if (!(p->route & LCE_ROUTE_KEEP_LOGITS) || route_of(p) == LCE_ROUTE_TWO_PASS) return false;
+  const int64_t Np = lce::padded_tokens(p->N), Vp = lce::padded_vocab(p->V), Hp = lce::padded_hidden(p->H);
+  f->kept = f->dw_direct = true;
+  f->pack = packs_rows(p) && (size_t)p->N * (size_t)p->lddx * 4 < ((size_t)1 << 31);
+  f->k = plan_pack(p, 0);
+  size_t o = f->k.xc;
+  f->chunk_rows = o; o += align_up(2048 * 8);
+  f->lse_rows = o; o += align_up((size_t)Np * 4);
+  f->tgt = o; o += align_up((size_t)Np * 4);
+  f->blk = o; o += align_up((size_t)(Np / lce::kMergeRows) * 8 * sizeof(double));
+  f->ld16 = Vp;
+  f->w16 = o; o += align_up((size_t)(2 * p->H) * (size_t)Vp * 2);
+  const size_t fixed = o, bound = (size_t)p->n_chunk * (size_t)p->V * 4, reserve = align_up((size_t)p->N * 4) + 4096;
+  if (fixed + reserve > bound) return false;
+  const int64_t tiles = Np / 256, kt = lce::small_logit_ktiles(p->H, 3);
+  const double th = (double)(Hp / 256), tv = (double)(Vp / 256);
+  auto logits = [&](int64_t rows) -> double {
+    const double a = lce::persistent_logits_us(rows, p->V, kt), b = lce::small_logits_us(rows, p->V, kt);
+    return (a < b ? a : b) / kUnitUs;
+  };
+  int64_t first = 0;
+  for (int64_t t = tiles; t >= 1; --t) {
+    const int64_t chunks = (tiles + t - 1) / t;
+    if (chunks > kMostChunks || (first != 0 && chunks > 2 * first + 4)) break;
+    if (t < tiles && (tiles + t) / (t + 1) == chunks) continue;  // a longer chunk gives the same number of chunks
+    const int64_t even = (tiles + chunks - 1) / chunks, nc = even * 256, last = tiles - (chunks - 1) * even;
+    FusedPlan c = *f;
+    size_t m = fixed;
+    c.xc = m; m += align_up((size_t)nc * (size_t)f->k.ldxc * 2);
+    const size_t part = align_up((size_t)(Vp / lce::kChunkV) * (size_t)nc * 4);
+    c.part_lse = m; m += part;
+    c.part_max = m; m += part;
+    c.part_pz = m; if (p->monitoring) m += part;
+    c.part_sq = m; if (p->monitoring) m += part;
+    c.stage = m; m += align_up((size_t)nc * (size_t)Vp * 4);
+    if (m + reserve > bound) continue;
+    c.part = c.plane = c.plane_hi = m;
+    size_t parts = dx_part_bytes((size_t)nc, (size_t)Hp, Vp, Vp, 3);
+    if (chunks == 1) {
+      const size_t w = dw_part_bytes((size_t)nc, (size_t)Hp, Vp, Vp, 3);
+      if (w > parts) parts = w;
+    }
+    const size_t left = bound - reserve - m;
+    // (with less room than the partial sums ask for, a chunk's dx runs on as many workgroups as there are blocks)
+    const int64_t blocks = (int64_t)(left / (256 * 256 * 4));
+    const bool fewer = parts > left && chunks > 1 && blocks >= 128 && 2 * even * (Hp / 256) <= blocks;
+    c.dx_grid = fewer ? (int)blocks : 0;
+    if (fewer) parts = (size_t)blocks * 256 * 256 * 4;
+    c.parts_on = parts != 0 && parts <= left;
+    const double add = chunks > 1 ? 16.0 : 5.0;
+    auto large = [&](double tt) -> double {
+      return kernel_cost(tt * th, 3.0 * (double)(Vp / 64), 5.0, c.parts_on, false) * (fewer ? 256.0 / (double)blocks : 1.0) +
+             kernel_cost(tv * th, 12.0 * tt, add, c.parts_on && chunks == 1, false);
+    };
+    double cost = (double)(chunks - 1) * large((double)even) + large((double)last);
+    c.small_blocks = (int64_t)(left / lce::kSmallBlockBytes) < 1024 ? (int64_t)(left / lce::kSmallBlockBytes) : 1024;
+    if (!f->pack && p->max_workgroups == 0 && even * 2 * ((p->H + 127) / 128) <= 1 << 14 && Vp / 128 * ((p->H + 127) / 128) <= 1 << 14) {
+      const lce::SmallGrads g0 = lce::plan_small_grads(chunks > 1 ? nc : p->N, p->H, p->V, 3, c.small_blocks);
+      const lce::SmallGrads g1 = lce::plan_small_grads(p->N - (chunks - 1) * nc, p->H, p->V, 3, c.small_blocks);
+      const double sums = chunks > 1 ? (double)(p->H * p->V) * 8e-6 / 5.0 : 0.0;  // us to add to dW
+      const double small = ((double)(chunks - 1) * (g0.us + sums) + g1.us + sums) / kUnitUs;
+      if (small < kSmallMargin * cost) {
+        cost = small;
+        c.small = true;
+        const int64_t b0 = g0.dx_blocks + g0.dw_blocks, b1 = g1.dx_blocks + g1.dw_blocks;
+        c.small_blocks = b0 > b1 ? b0 : b1;
+        c.parts_on = false;
+        c.dx_grid = 0;
+      }
+    }
+    cost += (double)(chunks - 1) * logits(nc) + logits(p->N - (chunks - 1) * nc) + 12.0 * (double)chunks +
+            (double)Np * (double)Vp * 8.0 / 8.0e6 + (double)p->H * (double)Vp * 8.0 / 8.0e6;
+    if (first == 0) first = chunks;
+    if (f->ok && cost >= f->cost) continue;
+    c.total = m + (c.small ? (size_t)(c.small_blocks * lce::kSmallBlockBytes) : c.parts_on ? parts : 0);
+    c.nc = nc;
+    c.chunks = (int)chunks;
+    c.cost = cost;
+    c.ok = true;
+    *f = c;
+  }
+  if (!f->ok) return false;
+  BwdPlan b;
+  if (route_of(p) == LCE_ROUTE_AUTO && plan_bwd(p, &b) == LCE_OK) {
+    const double two = logits(p->N) + b.cost + 12.0 + (double)p->H * (double)Vp * 16.0 / 8.0e6;
+    if (f->cost > kBytesMargin * two) f->ok = false;
+  }
+  return f->ok;
+}
+
 // (for both gradients, whichever the caller wants: the workspace does not depend on that)
 bool plan_fused(const lce_problem* p, FusedPlan* f) {
   static thread_local LastPlan<FusedPlan> last;
@@ -809,7 +911,8 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   b.w = wk; b.n_valid = n_rows; b.grad_out = grad_out;
   b.H = p->H; b.V = p->V; b.Hp = lce::padded_hidden(p->H);
   b.ldw = ldwk; b.lddx = p->lddx; b.lddw = p->lddw;
-  b.x_dtype = p->x_dtype; b.w_dtype = wk_dtype; b.dx_dtype = p->dx_dtype; b.dw_dtype = p->dw_dtype;
+  b.x_dtype = f.kept ? (int)lce::DT_PAIR : p->x_dtype; b.w_dtype = wk_dtype; b.dx_dtype = p->dx_dtype; b.dw_dtype = p->dw_dtype;
+  b.x_lo = f.kept ? k.ldxc / 2 : 0;
   b.w_vh = p->w_layout == LCE_W_VH;
   b.ignore_index = p->ignore_index;
   b.scale = p->logit_scale; b.z_reg = p->z_reg;
@@ -818,8 +921,9 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
   b.dz = base + f.stage;
   b.v0 = 0; b.vw = p->V; b.vs = Vp; b.wv0 = 0; b.Vw = p->V;
   b.first = 1; b.last = 1;
-  b.num_cus = num_cus; b.small_wgs = small_wgs; b.dx_grid = num_cus; b.dw_grid = num_cus;
-  b.live = lce::live_bands(lce::padded_k(p->H) * 2);
+  b.num_cus = num_cus; b.small_wgs = small_wgs; b.dw_grid = num_cus;
+  b.dx_grid = f.dx_grid > 0 && f.dx_grid < num_cus ? f.dx_grid : num_cus;
+  b.live = lce::live_bands(logit_k_bytes(p));
   b.part_lse = (float*)(base + f.part_lse);
   b.part_max = (float*)(base + f.part_max);
   b.part_pz = p->monitoring ? (float*)(base + f.part_pz) : nullptr;
@@ -850,8 +954,8 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
       a.dx = dx;
     } else {
       a.N = p->N - row0 < f.nc ? p->N - row0 : f.nc;
-      a.x = a.xc = (const char*)x + (size_t)row0 * (size_t)p->ldx * 2;
-      a.ldx = a.ldxc = p->ldx;
+      a.x = a.xc = f.kept ? base + f.xc : (const char*)x + (size_t)row0 * (size_t)p->ldx * 2;
+      a.ldx = a.ldxc = f.kept ? k.ldxc : p->ldx;
       a.y = y + row0;
       a.dx = dx ? (char*)dx + (size_t)row0 * (size_t)p->lddx * dxes : nullptr;
     }
@@ -859,7 +963,14 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
     // -- fp32 dW -- in the caller's buffer itself (3: store, 4: add)
     const bool last = c == f.chunks - 1;
     a.dw_acc = f.chunks == 1 ? 0 : f.dw_direct ? (c == 0 ? 3 : 4) : f.lo8 ? (c == 0 ? 6 : last ? 8 : 7) : (c == 0 ? 1 : last ? 5 : 2);
-    if (f.pack && (ph & (LCE_PHASE_PACK | LCE_PHASE_FWD_TILES | LCE_PHASE_BWD_DW))) {
+    if (f.kept && (ph & (LCE_PHASE_PACK | LCE_PHASE_FWD_TILES | LCE_PHASE_BWD_DW))) {
+      // the chunk's rows as pairs
+      e = f.pack ? lce::launch_gather_rows_split((const float*)x, p->ldx, p->H, perm + row0, chunk_rows + (all_rows ? 1024 : 0) + c, p->N,
+                                                 base + f.xc, k.ldxc, nullptr, nullptr, num_cus, s)
+                 : lce::launch_gather_rows_split((const float*)x + row0 * p->ldx, p->ldx, p->H, nullptr, nullptr, a.N, base + f.xc, k.ldxc,
+                                                 nullptr, nullptr, num_cus, s);
+      if (e != hipSuccess) return hip_fail(e, "gather_rows_split");
+    } else if (f.pack && (ph & (LCE_PHASE_PACK | LCE_PHASE_FWD_TILES | LCE_PHASE_BWD_DW))) {
       e = lce::launch_gather_rows(x, p->ldx * 2, p->H * 2, perm + row0, chunk_rows + (all_rows ? 1024 : 0) + c, p->N,
                                   base + f.xc, k.ldxc * 2, nullptr, nullptr, num_cus, s, true);
       if (e != hipSuccess) return hip_fail(e, "gather_rows");
@@ -877,8 +988,15 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
       if (e != hipSuccess) return hip_fail(e, "fwd_rows");
     }
     if ((dx || dw) && (ph & LCE_PHASE_BWD_DZ)) {
-      e = f.factors ? lce::launch_stage_factors(a, s) : lce::launch_stage_scale(a, s);
-      if (e != hipSuccess) return hip_fail(e, f.factors ? "stage_factors" : "stage_scale");
+      e = f.kept ? lce::launch_stage_pairs(a, s) : f.factors ? lce::launch_stage_factors(a, s) : lce::launch_stage_scale(a, s);
+      if (e != hipSuccess) return hip_fail(e, f.kept ? "stage_pairs" : f.factors ? "stage_factors" : "stage_scale");
+    }
+    if (f.small) {
+      lce::SmallGrads g = lce::plan_small_grads(a.N, p->H, p->V, products(p), f.small_blocks);
+      g.part = (float*)(base + f.part);
+      e = lce::launch_bwd_grads_small(a, g, dx && (ph & LCE_PHASE_BWD_DX), dw && (ph & LCE_PHASE_BWD_DW), s);
+      if (e != hipSuccess) return hip_fail(e, "bwd_grads_small");
+      continue;
     }
     if (dx && (ph & LCE_PHASE_BWD_DX)) {
       e = lce::launch_bwd_dx(a, s);
@@ -906,7 +1024,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
 
 extern "C" {
 
-int lce_version(void) { return 800; }  // 0.8.0: lce_scale_gradients, lce_unit_gradient
+int lce_version(void) { return 900; }  // 0.9.0: LCE_ROUTE_KEEP_LOGITS
 
 const char* lce_strerror(int status) {
   switch (status) {

@@ -69,6 +69,9 @@ constexpr int kDzStoreAux = LCE_DZ_STORE_AUX;  // cache policy of the dz stores:
 // every row, whatever its label; the wave also writes the forward's partials of its slice (m and
 // m + log sum exp(z - m)) and the target logit.  `pf_lse` is not used, and there is no gain to apply: under FUSE the
 // switch ZREG stands for the monitoring values instead (the slice's sum softmax * z and sum z^2, as lce_fwd.hip forms them).
+//
+// FUSE and SPLIT: the unscaled fp32 logits themselves are staged, in the place of the pairs to be (launch_stage_pairs makes them in
+// place): their upper 16 bits where the hi part will be, the lower 16 where the lo part will be.
 constexpr int kNoLabel = -0x7fffffff - 1;  // ignore_index, or no such row
 constexpr int kOffLabel = -1;              // a label that is no column of W (V <= 2^30): matches nothing
 template <class T, bool ZREG, bool VTAIL, bool FUSE, int NQ>
@@ -91,7 +94,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[NQ], const flo
   E* wave_base = reinterpret_cast<E*>(a.dz) + kParts * dz_block_offset(tw / kTile, (slice_v0 - a.v0) / kGroup, a.vs) +
                  (tw % kTile) * kGroup;
   E* row = wave_base + (lane & 31) * kGroup;
-  constexpr bool MON = FUSE && ZREG;
+  constexpr bool MON = FUSE && ZREG, KEEP = FUSE && SPLIT;
   // Stores go through a buffer descriptor over this wave's part of the stage (scalar base, one 32-bit offset per
   // lane, the block's offset as a scalar): no 64-bit vector address arithmetic.  All offsets stay below 2^31
   // (one block for the second column group, twice that for the pairs' two parts).
@@ -124,7 +127,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[NQ], const flo
 #pragma unroll
   for (int qb = 0; qb < NQ; ++qb) {
     float m = -INFINITY, ssum = 0.f, mpz = 0.f, msq = 0.f;
-    u32x4_t lo_part[SPLIT ? 8 : 1];  // this lane's 16-byte runs of lo parts
+    u32x4_t lo_part[SPLIT && !KEEP ? 8 : 1];  // this lane's 16-byte runs of lo parts
     if constexpr (FUSE) {
       // the largest of this token's logits in the slice: this lane's 64, then the other half's
 #pragma unroll
@@ -181,7 +184,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[NQ], const flo
         }
         if constexpr (FUSE) ssum += ((d[0] + d[1]) + (d[2] + d[3])) + ((d[4] + d[5]) + (d[6] + d[7]));
 #pragma unroll
-        for (int part = 0; part < (SPLIT ? 2 : 1); ++part) {
+        for (int part = 0; part < (SPLIT && !KEEP ? 2 : KEEP ? 0 : 1); ++part) {
           if (part == 1) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) d[i] = bf16_lo(d[i]);
@@ -200,7 +203,7 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[NQ], const flo
           // streaming stores (aux 2 = nt): dz (1 GiB per slab) is read back from memory by the next kernels anyway,
           // and a normal store would evict the W / x tiles the following main loop is about to reuse from L2
           if (SPLIT && part == 1) {
-            lo_part[SPLIT ? pb * 2 + (g >> 1) : 0] = o;
+            lo_part[SPLIT && !KEEP ? pb * 2 + (g >> 1) : 0] = o;
           } else {
             const int chunk = (pb & 1) * 4 + g + half;  // 16-byte chunk of the token's line
             *reinterpret_cast<u32x4_t*>(mine + (pb >> 1) * kPieceBytes + wline * (kGroup * 2) + ((chunk ^ wsw) << 4)) = o;
@@ -210,11 +213,32 @@ LCE_DEV void dz_epilogue_impl(const BwdArgs& a, const int (&pf_y)[NQ], const flo
     }
 #pragma unroll
     for (int part = 0; part < kParts; ++part) {
-      if (SPLIT && part == 1) {
+      if constexpr (KEEP) {
+        // (straight from the accumulator, once for each half of the logits: no registers that wait)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int pb = u >> 1, g = 2 * (u & 1), chunk = (pb & 1) * 4 + g + half;
+          unsigned zb[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            // (a volatile read: the compiler would otherwise keep the values of the sums above)
+            asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(zb[i]) : "a"(acc[pb][qb][g * 4 + i]));
+          }
+          const unsigned sel = part == 0 ? 0x07060302u : 0x05040100u;  // v_perm selectors: the upper / lower halves of (S0, S1)
+          const auto s0 = __builtin_amdgcn_permlane32_swap(__builtin_amdgcn_perm(zb[1], zb[0], sel), __builtin_amdgcn_perm(zb[5], zb[4], sel), false, false);
+          const auto s1 = __builtin_amdgcn_permlane32_swap(__builtin_amdgcn_perm(zb[3], zb[2], sel), __builtin_amdgcn_perm(zb[7], zb[6], sel), false, false);
+          u32x4_t o;
+          o[0] = s0[0];
+          o[1] = s1[0];
+          o[2] = s0[1];
+          o[3] = s1[1];
+          *reinterpret_cast<u32x4_t*>(mine + (pb >> 1) * kPieceBytes + wline * (kGroup * 2) + ((chunk ^ wsw) << 4)) = o;
+        }
+      } else if (SPLIT && part == 1) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
           const int pb = u >> 1, chunk = (pb & 1) * 4 + 2 * (u & 1) + half;
-          *reinterpret_cast<u32x4_t*>(mine + (pb >> 1) * kPieceBytes + wline * (kGroup * 2) + ((chunk ^ wsw) << 4)) = lo_part[SPLIT ? u : 0];
+          *reinterpret_cast<u32x4_t*>(mine + (pb >> 1) * kPieceBytes + wline * (kGroup * 2) + ((chunk ^ wsw) << 4)) = lo_part[SPLIT && !KEEP ? u : 0];
         }
       }
       // read the two pieces back as 128-byte lines and send them out
@@ -498,6 +522,7 @@ hipError_t launch_fwd_stage(const BwdArgs& a, hipStream_t s) {
   if ((a.part_pz == nullptr) != (a.part_sq == nullptr)) return hipErrorInvalidValue;
   if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16) return a.w_vh ? launch_stage<BF16, true>(a, s) : launch_stage<BF16, false>(a, s);
   if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16) return a.w_vh ? launch_stage<F16, true>(a, s) : launch_stage<F16, false>(a, s);
+  if (a.x_dtype == DT_PAIR && a.w_dtype == DT_PAIR && !a.w_vh) return launch_stage<BF16P, false>(a, s);
   return hipErrorInvalidValue;
 }
 

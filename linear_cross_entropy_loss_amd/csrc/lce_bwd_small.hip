@@ -23,63 +23,34 @@ namespace {
 // K tiles of the two contractions (even numbers).
 LCE_DEV int small_kt(int64_t k) { return (int)((k + 2 * kBK - 1) / (2 * kBK) * 2); }
 
-// One of the two gradients as the stored matrix that it is: where a quad (four consecutive columns) of a row goes.
-struct SmallOut {
-  void* out;
-  int64_t ld, rows, cols;   // limits: nothing is stored past them (a quad that the last column cuts is written whole)
-  int f32;
-  float coef;
-  float* sum;               // fp32 running sum of dx over slabs [.][sum_ld], or null
-  int64_t sum_ld;
-  int first, last;
-  template <class T> LCE_DEV void put(int64_t r, int64_t c, f32x4_t v) const {
-    typedef typename elem_of<T>::type E;
-    if (r >= rows || c >= cols) return;
-    if (sum != nullptr) {
-      f32x4_t* at = reinterpret_cast<f32x4_t*>(sum + r * sum_ld + c);
-      if (!first) v += *at;
-      if (!last) {
-        *at = v;
-        return;
-      }
-    }
-    const int64_t o = r * ld + c;
-    if (f32) {
-      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + o) = v * coef;
-    } else {
-      u32x2_t b;
-      b[0] = pack2<T>(v[0] * coef, v[1] * coef);
-      b[1] = pack2<T>(v[2] * coef, v[3] * coef);
-      *reinterpret_cast<u32x2_t*>(reinterpret_cast<E*>(out) + o) = b;
+// Four consecutive columns of row r of either gradient, as stored; nothing goes past its limits (a quad that the last column cuts
+// is written whole).  `sum`: the fp32 running sum of dx over slabs, or null.
+template <class T, bool WVH>
+LCE_DEV void small_put(const BwdArgs& a, bool is_dx, float* sum, float coef, int64_t r, int64_t c, f32x4_t v) {
+  typedef typename elem_of<T>::type E;
+  const int64_t rows = is_dx ? a.N : WVH ? a.V : a.H, cols = is_dx || WVH ? a.H : a.V;
+  if (r >= rows || c >= cols) return;
+  if (sum != nullptr) {
+    f32x4_t* at = reinterpret_cast<f32x4_t*>(sum + r * a.Hp + c);
+    if (!a.first) v += *at;
+    if (!a.last) {
+      *at = v;
+      return;
     }
   }
-};
-LCE_DEV SmallOut dx_out(const BwdArgs& a) {
-  SmallOut o;
-  o.out = a.dx;
-  o.ld = a.lddx;
-  o.rows = a.N;
-  o.cols = a.H;
-  o.f32 = a.dx_dtype == DT_F32;
-  o.coef = final_factor_of(a);
-  o.sum = a.first && a.last ? nullptr : a.dx_acc;
-  o.sum_ld = a.Hp;
-  o.first = a.first;
-  o.last = a.last;
-  return o;
-}
-template <bool WVH> LCE_DEV SmallOut dw_out(const BwdArgs& a) {
-  SmallOut o;
-  o.out = a.dw;
-  o.ld = a.lddw;
-  o.rows = WVH ? a.V : a.H;
-  o.cols = WVH ? a.H : a.V;
-  o.f32 = a.dw_dtype == DT_F32;
-  o.coef = final_factor_of(a);
-  o.sum = nullptr;
-  o.sum_ld = 0;
-  o.first = o.last = 1;
-  return o;
+  v *= coef;
+  char* out = reinterpret_cast<char*>(is_dx ? a.dx : a.dw);
+  const int64_t o = r * (is_dx ? a.lddx : a.lddw) + c;
+  if ((is_dx ? a.dx_dtype : a.dw_dtype) == DT_F32) {
+    f32x4_t* at = reinterpret_cast<f32x4_t*>(out + o * 4);
+    if (!is_dx && a.dw_acc == 4) v += *at;  // (dW summed over chunks of token rows)
+    *at = v;
+  } else {
+    u32x2_t b;
+    b[0] = pack2<T>(v[0], v[1]);
+    b[1] = pack2<T>(v[2], v[3]);
+    *reinterpret_cast<u32x2_t*>(out + o * 2) = b;
+  }
 }
 
 // A wave's 64 x 64 quarter of a tile to LDS, as the rows of the stored matrix: 128 rows of 128 floats, the 16-byte pieces of row r
@@ -105,15 +76,6 @@ template <bool SWAP> LCE_DEV void small_to_lds(char* lds, const f32x16_t (&acc)[
       }
 }
 
-// Tile and stretch of workgroup j of `tiles * nseg`; false: there is none.
-LCE_DEV bool small_item(int j, int tiles_p, int tiles_q, int nseg, int& tile, int& tp, int& tq, int& seg) {
-  const int tiles = tiles_p * tiles_q;
-  if (j >= tiles * nseg) return false;
-  segment_coords(j, tiles, nseg, tile, seg);
-  tile_coords(tile, 1, tiles_p, tiles_q, 8, 8, tp, tq);
-  return true;
-}
-
 template <class T, bool WVH>
 __global__ __launch_bounds__(kThreads, 2) void grads_small_kernel(const BwdArgs a, const SmallGrads g) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -121,12 +83,15 @@ __global__ __launch_bounds__(kThreads, 2) void grads_small_kernel(const BwdArgs 
   constexpr int kParts = is_pair<T>::value ? 2 : 1, kProducts = is_pair<T>::value ? 3 : 1;
   const E* dz = reinterpret_cast<const E*>(a.dz);
   const void* dz_end = dz + kParts * a.dz_rows * a.vs;
-  int tile, tp, tq, seg;
   const bool in_first = (int)blockIdx.x < g.first_span, is_dx = in_first != (g.dw_first != 0);
   const int j = (int)blockIdx.x - (in_first ? 0 : g.first_span);
   const int tiles_p = (int)((a.H + kSmallTile - 1) / kSmallTile);
   const int nseg = is_dx ? g.dx_nseg : g.dw_nseg;
-  if (!small_item(j, tiles_p, (int)(((is_dx ? a.N : a.vw) + kSmallTile - 1) / kSmallTile), nseg, tile, tp, tq, seg)) return;
+  const int tiles_q = (int)(((is_dx ? a.N : a.vw) + kSmallTile - 1) / kSmallTile);
+  if (j >= tiles_p * tiles_q * nseg) return;  // (the first kind's share is a multiple of 8)
+  int tile, tp, tq, seg;
+  segment_coords(j, tiles_p * tiles_q, nseg, tile, seg);
+  tile_coords(tile, 1, tiles_p, tiles_q, 8, 8, tp, tq);
   const int kt = small_kt(is_dx ? a.vw : a.N), s0 = segment_start(seg, nseg, kt), n = segment_start(seg + 1, nseg, kt) - s0;
   const int64_t k0 = (int64_t)s0 * kBK, h0 = (int64_t)tp * kSmallTile, q0 = (int64_t)tq * kSmallTile;
   f32x16_t acc[2][2];
@@ -151,7 +116,8 @@ __global__ __launch_bounds__(kThreads, 2) void grads_small_kernel(const BwdArgs 
   }
   __syncthreads();
   float* part = nseg > 1 ? g.part + ((is_dx ? 0 : (int64_t)g.dx_blocks) + (int64_t)tile * nseg + seg) * (kSmallTile * kSmallTile) : nullptr;
-  const SmallOut o = is_dx ? dx_out(a) : dw_out<WVH>(a);
+  float* sum = !is_dx || (a.first && a.last) ? nullptr : a.dx_acc;
+  const float coef = final_factor_of(a);
   const bool h_rows = !is_dx && !WVH;
   const int64_t qv = q0 + (is_dx ? 0 : a.v0), row0 = h_rows ? h0 : qv, col0 = h_rows ? qv : h0;
 #pragma unroll 2
@@ -159,7 +125,7 @@ __global__ __launch_bounds__(kThreads, 2) void grads_small_kernel(const BwdArgs 
     const int r = i / (kSmallTile / 4), c = i % (kSmallTile / 4) * 4;
     const f32x4_t v = *reinterpret_cast<const f32x4_t*>(small_piece(lds, r, c));
     if (part != nullptr) *reinterpret_cast<f32x4_t*>(part + i * 4) = v;
-    else o.put<T>(row0 + r, col0 + c, v);
+    else small_put<T, WVH>(a, is_dx, sum, coef, row0 + r, col0 + c, v);
   }
 }
 
@@ -178,7 +144,8 @@ __global__ __launch_bounds__(256) void grads_tail_kernel(const BwdArgs a, const 
   nseg = is_dx ? g.dx_nseg : g.dw_nseg;
   const float* part = g.part + ((is_dx ? 0 : (int64_t)g.dx_blocks) + (int64_t)tile * nseg) * (kSmallTile * kSmallTile);
   const int64_t h0 = (int64_t)tp * kSmallTile, q0 = (int64_t)tq * kSmallTile + (is_dx ? 0 : a.v0);
-  const SmallOut o = is_dx ? dx_out(a) : dw_out<WVH>(a);
+  float* sum = !is_dx || (a.first && a.last) ? nullptr : a.dx_acc;
+  const float coef = final_factor_of(a);
   const bool h_rows = !is_dx && !WVH;
   const int64_t row0 = h_rows ? h0 : q0, col0 = h_rows ? q0 : h0;
   constexpr int kQuads = kSmallTile * kSmallTile / 4 / kTailParts;
@@ -186,10 +153,16 @@ __global__ __launch_bounds__(256) void grads_tail_kernel(const BwdArgs a, const 
   for (int u = 0; u < kQuads / 256; ++u) {
     const int i = piece * kQuads + u * 256 + (int)threadIdx.x, r = i / (kSmallTile / 4), c = i % (kSmallTile / 4) * 4;
     const float* at = part + r * kSmallTile + c;
-    f32x4_t v = *reinterpret_cast<const f32x4_t*>(at);
-#pragma unroll 8
-    for (int s = 1; s < nseg; ++s) v += *reinterpret_cast<const f32x4_t*>(at + (int64_t)s * (kSmallTile * kSmallTile));
-    o.put<T>(row0 + r, col0 + c, v);
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < nseg; s0 += 8) {  // (eight in flight; those that there are not are read again and dropped)
+      f32x4_t t[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) t[k] = *reinterpret_cast<const f32x4_t*>(at + (int64_t)(s0 + k < nseg ? s0 + k : s0) * (kSmallTile * kSmallTile));
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (s0 + k < nseg) v += t[k];
+    }
+    small_put<T, WVH>(a, is_dx, sum, coef, row0 + r, col0 + c, v);
   }
 }
 
@@ -212,7 +185,7 @@ template <class T, bool WVH> hipError_t launch_small(const BwdArgs& a, SmallGrad
 }  // namespace
 
 hipError_t launch_bwd_grads_small(const BwdArgs& a, const SmallGrads& g, bool want_dx, bool want_dw, hipStream_t s) {
-  if (a.n_rows != nullptr || a.dx_f != nullptr || a.dw_f != nullptr || a.dw_acc != 0 || ((g.dx_nseg > 1 || g.dw_nseg > 1) && g.part == nullptr))
+  if (a.n_rows != nullptr || a.dx_f != nullptr || a.dw_f != nullptr || (a.dw_acc != 0 && a.dw_acc != 3 && a.dw_acc != 4) || (a.dw_acc != 0 && a.dw_dtype != DT_F32) || ((g.dx_nseg > 1 || g.dw_nseg > 1) && g.part == nullptr))
     return hipErrorInvalidValue;
   if (a.w_vh) {
     if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16) return launch_small<BF16, true>(a, g, want_dx, want_dw, s);

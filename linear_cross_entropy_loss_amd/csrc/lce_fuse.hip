@@ -175,6 +175,63 @@ __global__ __launch_bounds__(256) void stage_factors_kernel(const BwdArgs a) {
   }
 }
 
+// fp32 tensors: the stage holds the unscaled fp32 logits, halves apart (lce_bwd_dz.hip, KEEP), and dz as a bf16 pair takes their
+// place, with the arithmetic of the kernel that recomputes the logits, so that dz has the same bits as there.  A workgroup per block,
+// a thread on eight columns at a time.  Bound by memory traffic: 4 bytes read and 4 written per logit (1024 tokens, V=16384: 24 us, 5.6 TB/s).
+__global__ __launch_bounds__(256) void stage_pairs_kernel(const BwdArgs a) {
+  __shared__ float sh_nlse[kTile], sh_gain[kTile];
+  __shared__ int sh_col[kTile];  // target column inside the block, -1 or, for a row without gradient, kNoRow
+  constexpr int kNoRow = -0x7fffffff;
+  const int64_t rows = packed_rows(a.n_rows, a.N);
+  const int64_t t0 = (int64_t)blockIdx.y * kTile;
+  if (t0 >= rows && t0 > 0) return;  // (token tiles without a row are not read, but for the first: dW's K extent is never empty)
+  const int64_t v0 = (int64_t)blockIdx.x * 64;
+  {
+    const int64_t tok = t0 + threadIdx.x;
+    const bool exists = tok < rows;
+    const int64_t yy = exists ? a.y[tok] : a.ignore_index, rel = yy - v0;
+    const float lse = exists ? a.lse[tok] : 0.f;
+    sh_nlse[threadIdx.x] = fmaf(-lse, kLog2e, 0.f);
+    sh_gain[threadIdx.x] = 1.f + 2.f * a.z_reg * lse;
+    sh_col[threadIdx.x] = yy == a.ignore_index ? kNoRow : rel >= 0 && rel < 64 ? (int)rel : -1;
+  }
+  __syncthreads();
+  const float c1 = a.scale * kLog2e;
+  const int cols = a.vw - v0 < 64 ? (int)(a.vw - v0) : 64;  // (may be <= 0)
+  u32x4_t* blk = reinterpret_cast<u32x4_t*>(reinterpret_cast<unsigned short*>(a.dz) + 2 * dz_block_offset(blockIdx.y, blockIdx.x, a.vs));
+  constexpr int kLo = kDzBlockElems * 2 / 16;  // pieces to the block of the lo parts
+  u32x4_t zh[8], zl[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    zh[i] = blk[i * 256 + threadIdx.x];
+    zl[i] = blk[i * 256 + threadIdx.x + kLo];
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int piece = i * 256 + threadIdx.x, r = piece >> 3, c0 = (piece & 7) * 8;
+    const float nlse = sh_nlse[r], gain = sh_gain[r];
+    const int col = sh_col[r];
+    u32x4_t oh, ol;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float d[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const unsigned bits = __builtin_amdgcn_perm(zh[i][j], zl[i][j], e == 0 ? 0x05040100u : 0x07060302u);
+        const float z = __builtin_bit_cast(float, bits);
+        const int c = c0 + 2 * j + e;
+        float p = __builtin_amdgcn_exp2f(fmaf(z, c1, nlse)) * gain;
+        p = c == col ? p - 1.f : p;
+        d[e] = c < cols && col != kNoRow ? p : 0.f;
+      }
+      oh[j] = pack2<BF16>(d[0], d[1]);
+      ol[j] = pack2<BF16>(bf16_lo(d[0]), bf16_lo(d[1]));
+    }
+    blk[piece] = oh;
+    blk[piece + kLo] = ol;
+  }
+}
+
 // t[r][c] *= g[0] for r < rows, c < cols (row stride ld, rows on 16-byte boundaries), the product formed in fp32;
 // nothing is read or written when g[0] is 1.  Pieces of 16 bytes, the last piece of a row element by element.
 // v * f rounded to fp32 before anything else happens to it (the compiler may otherwise fold the product into
@@ -247,6 +304,12 @@ hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s) {
   if (a.x_dtype == DT_BF16) hipLaunchKernelGGL(stage_scale_kernel<BF16>, grid, dim3(256), 0, s, a);
   else if (a.x_dtype == DT_F16) hipLaunchKernelGGL(stage_scale_kernel<F16>, grid, dim3(256), 0, s, a);
   else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+hipError_t launch_stage_pairs(const BwdArgs& a, hipStream_t s) {
+  if (a.x_dtype != DT_PAIR || a.v0 != 0 || a.dz_shift != 0 || a.lse == nullptr) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(stage_pairs_kernel, dim3((unsigned)(a.vs / 64), (unsigned)(a.Np / kTile)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

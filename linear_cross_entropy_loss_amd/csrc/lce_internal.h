@@ -249,6 +249,8 @@ hipError_t launch_bwd_dz(const BwdArgs& a, hipStream_t s);
 // The logit kernel of lce_forward_backward and the pass that follows the row merge (see BwdArgs).
 hipError_t launch_fwd_stage(const BwdArgs& a, hipStream_t s);
 hipError_t launch_stage_scale(const BwdArgs& a, hipStream_t s);
+// The same for pairs, of which the stage holds the logits themselves.
+hipError_t launch_stage_pairs(const BwdArgs& a, hipStream_t s);
 // The same with the factors only worked out (dx_f and dw_f of BwdArgs), and the slice of each token's target column
 // rewritten.
 hipError_t launch_stage_factors(const BwdArgs& a, hipStream_t s);
@@ -445,7 +447,8 @@ inline SmallGrads plan_small_grads(int64_t N, int64_t H, int64_t V, int products
       double c = wf ? small_span(tw * nw, lw, tx * nx, lx) : small_span(tx * nx, lx, tw * nw, lw);
       if (tx * nx + tw * nw <= kSmallSlots / 2) c *= 0.55;  // (one to a compute unit)
       if (bx + bw > 0) c += 6.0 + (double)(bx + bw) * 0.03;
-      c = 5.0 + 0.9 * c;
+      // (a long launch runs into the power limit: the K tile's time goes from 0.9 us to 1.2)
+      c = 5.0 + 0.9 * c * (1.0 + 0.35 * (c < 40.0 ? 0.0 : c > 200.0 ? 1.0 : (c - 40.0) / 160.0));
       if (g.us >= 0 && c >= g.us) continue;
       g.us = c;
       g.dw_first = wf;

@@ -285,14 +285,15 @@ def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_c
     with _on_device(x_in.device):
         views = _problem_views(x_in, y, At)
         x, y1, w, layout, N, H, V = views
-        if x.dtype == torch.float32 or w.dtype not in (x.dtype, torch.float32):
+        if w.dtype not in (x.dtype, torch.float32):
             return None, (views, None)
         vh = layout == _lib.W_VH
         w_cols = H if vh else V
         prob = _lib.make_problem(
             N, H, V, x.stride(0), w.stride(0), _dx_cols(H, x.dtype), _padded_cols(w_cols, w.dtype), x.dtype, w.dtype,
             x.dtype, w.dtype, ignore_index, logit_scale, z_regularization, N_chunk_size, monitoring, 0, pack, 0, layout,
-            (_lib.ROUTE_ONE_PASS if always else _lib.ROUTE_AUTO) | (_lib.ROUTE_EXACT_SUMS if exact_dw_sums.get() else 0),
+            (_lib.ROUTE_ONE_PASS if always else _lib.ROUTE_AUTO) | (_lib.ROUTE_EXACT_SUMS if exact_dw_sums.get() else 0)
+            | (_lib.ROUTE_KEEP_LOGITS if x.dtype == torch.float32 else 0),
         )
         lib = _lib.load()
         _lib.raise_for_status(lib.lce_check_problem(ctypes.byref(prob)), "linear_cross_entropy")
