@@ -8,6 +8,7 @@ import torch
 
 _PKG_DIR = Path(__file__).resolve().parent
 LIB_PATH = _PKG_DIR / "liblce_gfx950.so"
+HOST_LIB_PATH = _PKG_DIR / "_lce_host.so"
 
 LCE_BF16, LCE_F16, LCE_F32 = 0, 1, 2
 LCE_OK = 0
@@ -127,6 +128,27 @@ def load():
     lib.lce_transpose_rows.argtypes = lib.lce_pad_rows.argtypes
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The extension that takes plain calls from tensors to the C ABI (csrc/lce_host.cpp); raises if it has not been built."""
+    global _host
+    if _host is None:
+        lib = load()
+        if not HOST_LIB_PATH.exists():
+            raise RuntimeError(
+                f"{HOST_LIB_PATH} is missing: the host extension has not been built. "
+                "Run `python -m linear_cross_entropy_loss_amd.build`. There is no fallback path.")
+        import torch  # noqa: F401  (the extension links against its libraries)
+
+        from linear_cross_entropy_loss_amd import _lce_host
+
+        _lce_host.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in EXPORTS})
+        _host = _lce_host
+    return _host
 
 
 def unit_gradient() -> int:

@@ -17,6 +17,10 @@ LIB_NAME = "liblce_gfx950.so"
 LIB_PATH = PKG_DIR / LIB_NAME
 
 SOURCES = ["lce_api.hip", "lce_fwd.hip", "lce_bwd_dz.hip", "lce_bwd_dx.hip", "lce_bwd_dw.hip", "lce_bwd_small.hip", "lce_convert.hip", "lce_compact.hip", "lce_fuse.hip"]
+# Host path of the Python operator: a CPython extension on torch's C++ interface, without device code.
+HOST_SOURCE = "lce_host.cpp"
+HOST_LIB_NAME = "_lce_host.so"
+HOST_LIB_PATH = PKG_DIR / HOST_LIB_NAME
 # Measurement probes (`bench.py --probe`): sources and library of their own, built on demand only.
 PROBE_DIR = PKG_DIR / "probes"
 PROBE_LIB_NAME = "liblce_probe_gfx950.so"
@@ -60,15 +64,35 @@ def _link(path: Path, objs) -> None:
     os.replace(tmp, path)
 
 
+def _build_host() -> None:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    libdir = Path(torch.__file__).resolve().parent / "lib"
+    tmp = HOST_LIB_PATH.with_suffix(".so.tmp")
+    includes = [f"-I{p}" for p in cpp_extension.include_paths()] + [f"-I{sysconfig.get_paths()['include']}"]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DTORCH_EXTENSION_NAME=_lce_host",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, str(CSRC / HOST_SOURCE), "-o", str(tmp),
+           f"-L{libdir}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SOURCE}:\n{r.stderr}")
+    os.replace(tmp, HOST_LIB_PATH)
+
+
 def build(force: bool = True, verbose: bool = False) -> Path:
     """Compile every kernel translation unit of the operator for gfx950 and link the library."""
-    if LIB_PATH.exists() and not force:
+    if LIB_PATH.exists() and HOST_LIB_PATH.exists() and not force:
         return LIB_PATH
     objdir = PKG_DIR / "build"
     objdir.mkdir(exist_ok=True)
     jobs = min(len(SOURCES), int(os.environ.get("MAX_JOBS", "8")))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(lambda s: _compile(CSRC, s, objdir), SOURCES))
+        host.result()
     _link(LIB_PATH, objs)
     if verbose:
         print(f"built {LIB_PATH}")

@@ -316,6 +316,19 @@ def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_c
     return (out5, lse, n_valid, x, y1, w, layout, dx, dw, pre), None
 
 
+def _native_forward(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, need_dx, need_dw):
+    """What _one_pass_impl and, where that route does not cover the problem, _forward_impl return, and whether it was the former,
+    by the host extension: one call for both, of the calls whose matrices are read in place.  None: any other call, for those."""
+    device = x_in.device
+    if device.type != "cuda" or device.index != torch._C._cuda_getDevice():
+        return None
+    done = _lib.host().forward(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, _route_mode(),
+                               exact_dw_sums.get(), need_dx, need_dw, _stream(device))
+    if done is not None and len(done) == 2:
+        _lib.raise_for_status(*done)
+    return done
+
+
 def _device_scalar(g, device):
     """The one number of `g` in fp32 on `device`: `g` itself where it is that."""
     if g.dtype == torch.float32 and g.device == device and g.numel() == 1:
@@ -376,8 +389,17 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
                    N_chunk_size, need_dx, need_dw, pack, layout=0):
     """Runs lce_backward on what _forward_impl returned.  dx is (N, H); dw is (H, V) -- for a weight stored
     (V, H) (layout W_VH) the transposed view of a gradient stored the same way; None when not needed."""
-    N, H = x.shape
     vh = layout == _lib.W_VH
+    if x.device.index == torch._C._cuda_getDevice():
+        g = _device_scalar(grad_output, x.device)
+        done = _lib.host().backward(x, y1, w, lse, n_valid, g, ignore_index, z_regularization, logit_scale, N_chunk_size, need_dx,
+                                    need_dw, pack, layout, _stream(x.device))
+        if done is not None:
+            if len(done) == 3:
+                _lib.raise_for_status(*done[:2])
+            dx, dw = done
+            return dx, dw.t() if vh and dw is not None else dw
+    N, H = x.shape
     V = w.shape[0] if vh else w.shape[1]
     w_cols = H if vh else V
     with _on_device(x.device):
@@ -435,14 +457,20 @@ class LinearXentImplementation(torch.autograd.Function):
         pack = _pack_mode()
         need_dx, need_dw = grad_mode and ctx.needs_input_grad[0], grad_mode and ctx.needs_input_grad[2]
         done = given = None
-        if (need_dx or need_dw) and one_pass.get():
+        native = _native_forward(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, need_dx,
+                                 need_dw)
+        if native is not None:
+            *done, one = native
+            if not one:
+                given, done = done[:7], None
+        elif (need_dx or need_dw) and one_pass.get():
             done, given = _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring,
                                          pack, need_dx, need_dw)
         if done is not None:
             out5, lse, n_valid, x, y1, w, layout, dx, dw, pre = done
             ctx.lce_grads = [dx, dw, pre]  # for the first backward; dropped there
         else:
-            out5, lse, n_valid, x, y1, w, layout = _forward_impl(
+            out5, lse, n_valid, x, y1, w, layout = given if native is not None else _forward_impl(
                 x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, given)
             ctx.lce_grads = None
         ctx.save_for_backward(x, y1, w, lse, n_valid)
