@@ -318,12 +318,12 @@ def _one_pass_impl(x_in, y, At, ignore_index, z_regularization, logit_scale, N_c
 
 def _native_forward(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, need_dx, need_dw):
     """What _one_pass_impl and, where that route does not cover the problem, _forward_impl return, and whether it was the former,
-    by the host extension: one call for both, of the calls whose matrices are read in place.  None: any other call, for those."""
+    by the host extension: one call for both.  None: no ordinary call (csrc/lce_host.cpp), or one that has a warning to give."""
     device = x_in.device
     if device.type != "cuda" or device.index != torch._C._cuda_getDevice():
         return None
     done = _lib.host().forward(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, _route_mode(),
-                               exact_dw_sums.get(), need_dx, need_dw, _stream(device))
+                               exact_dw_sums.get(), need_dx, need_dw, "weight" in _copy_warned, _stream(device))
     if done is not None and len(done) == 2:
         _lib.raise_for_status(*done)
     return done
