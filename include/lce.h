@@ -194,6 +194,8 @@ int lce_workspace_bytes(const lce_problem* p, size_t* fwd_bytes, size_t* bwd_byt
  * vocabulary slab at a time (`slab_width` columns, a multiple of 256; `slabs`
  * passes, the last one over whatever columns remain).  The counterpart of the reference's loop over N_chunk_size-row
  * groups (ops.py:721), which exists for the same purpose: bounding scratch.
+ * 16-bit activations with a hidden size of up to 128, rows not packed on demand: nothing is staged; one slab, wider than
+ * the vocabulary.
  */
 int lce_backward_plan(const lce_problem* p, int64_t* slabs, int64_t* slab_width);
 

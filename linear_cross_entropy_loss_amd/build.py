@@ -16,7 +16,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_NAME = "liblce_gfx950.so"
 LIB_PATH = PKG_DIR / LIB_NAME
 
-SOURCES = ["lce_api.hip", "lce_fwd.hip", "lce_bwd_dz.hip", "lce_bwd_dx.hip", "lce_bwd_dw.hip", "lce_bwd_small.hip", "lce_convert.hip", "lce_compact.hip", "lce_fuse.hip"]
+SOURCES = ["lce_api.hip", "lce_fwd.hip", "lce_bwd_dz.hip", "lce_bwd_dx.hip", "lce_bwd_dw.hip", "lce_bwd_small.hip", "lce_narrow.hip", "lce_convert.hip", "lce_compact.hip", "lce_fuse.hip"]
 # Host path of the Python operator: a CPython extension on torch's C++ interface, without device code.
 HOST_SOURCE = "lce_host.cpp"
 HOST_LIB_NAME = "_lce_host.so"

@@ -196,7 +196,8 @@ struct BwdPlan {
   bool pack_on;   // tokens with an ignored label are packed away in this backward
   bool parts_on;  // tail tiles of dx / dW may be split along K (partial-sum blocks exist)
   bool small;     // dx and dW run on 128 x 128 tiles (small_grads_pay)
-  int64_t small_blocks;  // room for their partial sums
+  bool narrow;    // no stage at all (lce_narrow.hip)
+  int64_t small_blocks;  // room for the partial sums of either
   int64_t lddxc;
   size_t dz, dx_acc, dx_part, dw_part, w16, total;
 };
@@ -256,7 +257,10 @@ double kernel_cost(double T, double L, double e, bool parts, bool settled) {
 // N * H * 4 bytes, the fp32 x_grad buffer the reference allocates next to its logits chunk (ops.py:693) and
 // this library does not -- and by the split-K partial sums.  If even that fails, the narrowest split is used:
 // the bound is a target, the operator never refuses a shape.
+bool plan_narrow(const lce_problem* p, BwdPlan* b);
 int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
+  memset(b, 0, sizeof(*b));
+  if (!settled && plan_narrow(p, b)) return LCE_OK;
   const size_t strict = (size_t)p->n_chunk * (size_t)p->V * 4;
   const size_t dz_cap = (size_t)1 << 30;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Hp = (size_t)lce::padded_hidden(p->H);
@@ -387,6 +391,28 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
   double wide = 0;
   if (choose(2, b, &wide)) { b->cost = wide; return LCE_OK; }
   return LCE_EWORKSPACE;
+}
+
+// Hidden sizes up to lce::kNarrowHidden: the gradients without a stage, one slab, nothing packed away.  Not where the caller asks for
+// packing, as the sums over the tokens are cut by their number in memory.
+bool plan_narrow(const lce_problem* p, BwdPlan* b) {
+  const int64_t tok = lce::pad_to(p->N, 128) / 128, voc = lce::pad_to(p->V, 128) / 128;
+  if (p->H > lce::kNarrowHidden || splits(p) || p->pack_rows == LCE_PACK_ALWAYS || p->max_workgroups != 0 || tok > 1 << 20 || voc > 1 << 20)
+    return false;
+  const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)lce::padded_vocab(p->V) * 2) : 0;
+  const size_t strict = (size_t)p->n_chunk * (size_t)p->V * 4, reserve = align_up((size_t)p->N * 4) + 4096;
+  const size_t block = (size_t)lce::narrow_block_bytes(p->H), room = strict > w16 + reserve ? strict - w16 - reserve : 0;
+  const int64_t most = (int64_t)(room / block) < 1024 ? (int64_t)(room / block) : 1024;
+  const lce::SmallGrads g = lce::plan_narrow_grads(p->N, p->H, p->V, most);
+  b->narrow = true;
+  b->slabs = 1;
+  b->vs = lce::padded_vocab(p->V) + 256;  // (one slab that ends past the vocabulary: nothing is staged, lce.h)
+  b->small_blocks = g.dx_blocks + g.dw_blocks;
+  b->w16 = align_up((size_t)b->small_blocks * block);
+  b->total = b->w16 + w16;
+  if (b->total == 0) b->total = 256;
+  b->cost = g.us / kUnitUs;
+  return true;
 }
 
 int plan_bwd(const lce_problem* p, BwdPlan* b) {
@@ -685,6 +711,10 @@ bool plan_fused_with(const lce_problem* p, bool lo8, bool settled, int64_t most_
   if (route_of(p) == LCE_ROUTE_AUTO && (settled ? make_plan_bwd(p, &b, true) : plan_bwd(p, &b)) == LCE_OK) {
     // (at these sizes the model is a quarter to a third above what the other kernels take: N=1024, H=2048, V=8192 156 us in one
     // pass, 179 in two with the gradients on small tiles)
+    if (b.narrow) {
+      f->ok = false;
+      return false;
+    }
     const double two_bwd = b.small ? 1.4 * b.cost : b.cost;
     const double two = kernel_cost((double)tiles * tv, (double)(lce::padded_k(p->H) / 64), 4.0, false, settled) + two_bwd;
     // (sums of 24 bits have to be ahead of two passes, which are exact, by the margin as well)
@@ -1192,11 +1222,18 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
     }
     a.first = i == 0;
     a.last = i == b.slabs - 1;
+    const bool want_dx = dx && (ph & LCE_PHASE_BWD_DX), want_dw = dw && (ph & LCE_PHASE_BWD_DW);
+    if (b.narrow) {
+      lce::SmallGrads g = lce::plan_narrow_grads(p->N, p->H, p->V, b.small_blocks);
+      g.part = (float*)base;
+      e = lce::launch_bwd_narrow(a, g, want_dx, want_dw, s);
+      if (e != hipSuccess) return hip_fail(e, "bwd_narrow");
+      continue;
+    }
     if (ph & LCE_PHASE_BWD_DZ) {
       e = lce::launch_bwd_dz(a, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_dz");
     }
-    const bool want_dx = dx && (ph & LCE_PHASE_BWD_DX), want_dw = dw && (ph & LCE_PHASE_BWD_DW);
     if (b.small) {
       lce::SmallGrads g = lce::plan_small_grads(p->N, p->H, a.vw, products(p), b.small_blocks);
       g.part = (float*)(base + b.dx_part);

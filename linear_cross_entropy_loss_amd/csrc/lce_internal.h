@@ -423,42 +423,66 @@ inline double small_span(int64_t na, double la, int64_t nb, double lb) {
   return end;
 }
 // The stretches of K: as many of each gradient as give the shortest launch, with what their sums cost on top, and fit `most_blocks`.
-// kLeastStretch: K tiles of the shortest.
-constexpr int64_t kLeastStretch = 8;
-inline SmallGrads plan_small_grads(int64_t N, int64_t H, int64_t V, int products, int64_t most_blocks) {
-  const int64_t th = (H + 127) / 128, tx = th * ((N + 127) / 128), tw = th * ((V + 127) / 128);
-  const int64_t kx = pad_to(V, 128) / 64, kw = pad_to(N, 128) / 64;
+// tx tiles of dx with kx units of K each, tw of dW with kw; stretches of whole pairs of `pair` units, `least` at the shortest; `item`:
+// what prologue and epilogue of a workgroup take, in units; block: what a stretch's sums cost.
+struct CutRule {
+  int64_t tx, kx, tw, kw, pair, least;
+  double products, item, block;
+};
+inline double plan_cuts(const CutRule& c, int64_t most_blocks, SmallGrads* g) {
   auto most = [&](int64_t t, int64_t k) -> int64_t {
-    const int64_t by_length = k / kLeastStretch, by_slots = 4 * kSmallSlots / t;
+    const int64_t by_length = k / c.least, by_slots = 4 * kSmallSlots / t;
     const int64_t m = by_length < by_slots ? by_length : by_slots;
     return m < 1 ? 1 : m;
   };
-  SmallGrads g;
-  memset(&g, 0, sizeof(g));
-  g.us = -1;
-  const int64_t mx = most(tx, kx), mw = most(tw, kw);
+  auto length = [&](int64_t k, int64_t n) { return (double)(((k + c.pair - 1) / c.pair + n - 1) / n * c.pair) * c.products + c.item; };
   auto next = [](int64_t n) { return n < 16 ? n + 1 : n + n / 8; };
+  memset(g, 0, sizeof(*g));
+  double best = -1;
+  const int64_t mx = most(c.tx, c.kx), mw = most(c.tw, c.kw);
   for (int64_t nx = 1; nx <= mx; nx = next(nx))
     for (int64_t nw = 1; nw <= mw; nw = next(nw)) {
-      const int64_t bx = nx > 1 ? tx * nx : 0, bw = nw > 1 ? tw * nw : 0;
+      const int64_t bx = nx > 1 ? c.tx * nx : 0, bw = nw > 1 ? c.tw * nw : 0;
       if (bx + bw > most_blocks) continue;
-      const double lx = (double)((kx / 2 + nx - 1) / nx * 2 * products) + 4.0, lw = (double)((kw / 2 + nw - 1) / nw * 2 * products) + 4.0;
+      const double lx = length(c.kx, nx), lw = length(c.kw, nw);
       const bool wf = lw > lx;
-      double c = wf ? small_span(tw * nw, lw, tx * nx, lx) : small_span(tx * nx, lx, tw * nw, lw);
-      if (tx * nx + tw * nw <= kSmallSlots / 2) c *= 0.55;  // (one to a compute unit)
-      if (bx + bw > 0) c += 6.0 + (double)(bx + bw) * 0.03;
-      // (a long launch runs into the power limit: the K tile's time goes from 0.9 us to 1.2)
-      c = 5.0 + 0.9 * c * (1.0 + 0.35 * (c < 40.0 ? 0.0 : c > 200.0 ? 1.0 : (c - 40.0) / 160.0));
-      if (g.us >= 0 && c >= g.us) continue;
-      g.us = c;
-      g.dw_first = wf;
-      g.dx_nseg = (int)nx;
-      g.dw_nseg = (int)nw;
-      g.dx_blocks = (int)bx;
-      g.dw_blocks = (int)bw;
+      double t = wf ? small_span(c.tw * nw, lw, c.tx * nx, lx) : small_span(c.tx * nx, lx, c.tw * nw, lw);
+      if (c.tx * nx + c.tw * nw <= kSmallSlots / 2) t *= 0.55;  // (one to a compute unit)
+      if (bx + bw > 0) t += 200.0 * c.block + (double)(bx + bw) * c.block;
+      if (best >= 0 && t >= best) continue;
+      best = t;
+      g->dw_first = wf;
+      g->dx_nseg = (int)nx;
+      g->dw_nseg = (int)nw;
+      g->dx_blocks = (int)bx;
+      g->dw_blocks = (int)bw;
     }
+  return best;
+}
+// A unit is a K tile of 64.
+inline SmallGrads plan_small_grads(int64_t N, int64_t H, int64_t V, int products, int64_t most_blocks) {
+  const int64_t th = (H + 127) / 128;
+  const CutRule c = {th * ((N + 127) / 128), pad_to(V, 128) / 64, th * ((V + 127) / 128), pad_to(N, 128) / 64, 2, 8, (double)products, 4.0, 0.03};
+  SmallGrads g;
+  const double t = plan_cuts(c, most_blocks, &g);
+  // (a long launch runs into the power limit: the K tile's time goes from 0.9 us to 1.2)
+  g.us = 5.0 + 0.9 * t * (1.0 + 0.35 * (t < 40.0 ? 0.0 : t > 200.0 ? 1.0 : (t - 40.0) / 160.0));
   return g;
 }
+// Hidden sizes up to this: no stage (lce_narrow.hip).  A unit is a tile of 128 rows that streams past the 128 that stay; a block of
+// sums has 128 rows of whole K tiles.
+constexpr int64_t kNarrowHidden = 128;
+inline int64_t narrow_block_bytes(int64_t H) { return 128 * (H <= 64 ? 64 : 128) * 4; }
+inline SmallGrads plan_narrow_grads(int64_t N, int64_t H, int64_t V, int64_t most_blocks) {
+  const int64_t tok = (N + 127) / 128, voc = (V + 127) / 128;
+  const CutRule c = {tok, voc, voc, tok, 1, 1, 1.0, 1.5, 0.0075};
+  SmallGrads g;
+  const double t = plan_cuts(c, most_blocks, &g);
+  g.us = 5.0 + (H <= 64 ? 3.2 : 4.6) * t;
+  return g;
+}
+hipError_t launch_fwd_narrow(const FwdArgs& a, int64_t rows, hipStream_t s);
+hipError_t launch_bwd_narrow(const BwdArgs& a, const SmallGrads& g, bool want_dx, bool want_dw, hipStream_t s);
 hipError_t launch_bwd_grads_small(const BwdArgs& a, const SmallGrads& g, bool want_dx, bool want_dw, hipStream_t s);
 
 }  // namespace lce

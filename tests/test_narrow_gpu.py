@@ -1,0 +1,75 @@
+"""Hidden sizes up to lce_internal.h's kNarrowHidden: forward and gradients without a stage (lce_narrow.hip) against the staged
+kernels, which run where a call limits its workgroups.
+
+The logits have the same bits (the same products along the same K order), and with them lse and dz; dx and dW add the same products in
+another order: fp32 rounding, which moves a 16-bit result by at most one unit in the last place and only next to a boundary -- below a
+quarter of such a unit in the 2-norm --, an fp32 one by 6000^0.5 * 2^-24 * 2 at most."""
+import ctypes
+
+import pytest
+import torch
+
+from helpers import make_inputs, rel_errors
+
+pytestmark = pytest.mark.gpu
+
+BOUND = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12, torch.float32: 1e-5}
+
+
+def P(t):
+    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+
+
+def _rows(t, extra=0):
+    """Rows on 16-byte boundaries, with the largest finite numbers of the type behind them."""
+    m = 4 if t.dtype == torch.float32 else 8
+    pad = torch.full((t.shape[0], t.shape[1] + (-t.shape[1]) % m + extra), torch.finfo(t.dtype).max if extra else 0, dtype=t.dtype, device="cuda")
+    pad[:, :t.shape[1] + (-t.shape[1]) % m] = 0
+    pad[:, :t.shape[1]] = t.cuda()
+    return pad[:, :t.shape[1]]
+
+
+@pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.bfloat16, None, 1), (torch.float16, None, 0),
+                                                  (torch.float16, torch.float32, 1), (torch.bfloat16, torch.float32, 0)])
+@pytest.mark.parametrize("N,H,V,extra,mon,z_reg", [
+    (1, 8, 8, 0, False, 0.0), (127, 64, 129, 0, True, 1e-3), (128, 72, 128, 16, False, 1e-3), (129, 128, 1003, 0, True, 0.0),
+    (700, 40, 5001, 8, False, 0.0), (3000, 104, 300, 0, False, 1e-3), (260, 120, 777, 8, True, 1e-3), (515, 56, 2050, 0, False, 0.0)])
+def test_narrow_hidden_sizes(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout):
+    from linear_cross_entropy_loss_amd import _lib
+
+    print(f"narrow N={N} H={H} V={V} {dtype} {w_dtype} layout={layout}", flush=True)
+    lib = _lib.load()
+    x, y, w = make_inputs(N, H, V, dtype, seed=N + V, ignore_frac=0.2 if N > 1 else 0.0, w_dtype=w_dtype)
+    x, w, y = _rows(x, extra), _rows(w.t() if layout else w, extra), y.cuda()
+    g = torch.full((1,), 1024.0 if dtype == torch.float16 else 1.5, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def run(workgroups, want_dx=True, want_dw=True):
+        lddx, cols = H + (-H) % 8, H if layout else V
+        lddw = cols + (-cols) % 8
+        prob = _lib.make_problem(N, H, V, x.stride(0), w.stride(0), lddx, lddw, dtype, w.dtype, dtype, w.dtype, -1, 0.7, z_reg, 4096,
+                                 mon, 0, _lib.PACK_NEVER, workgroups, layout)
+        fb, bb = _lib.workspace_bytes(prob)
+        ws = torch.empty(max(fb, bb), dtype=torch.uint8, device="cuda")
+        lse, out5 = torch.empty(N, device="cuda"), torch.empty(5, device="cuda")
+        n = torch.empty(1, dtype=torch.int64, device="cuda")
+        dx = torch.full((N, lddx), float("nan"), dtype=dtype, device="cuda") if want_dx else None
+        dw = torch.full((V if layout else H, lddw), float("nan"), dtype=w.dtype, device="cuda") if want_dw else None
+        a = (ctypes.byref(prob), P(x), P(w), P(y), P(lse))
+        _lib.raise_for_status(lib.lce_forward(*a, P(out5), P(n), P(ws), fb, st), "lce_forward")
+        _lib.raise_for_status(lib.lce_backward(*a, P(n), P(g), P(dx), P(dw), P(ws), bb, st), "lce_backward")
+        torch.cuda.synchronize()
+        return out5, lse, dx[:, :H] if want_dx else None, dw[:, :cols] if want_dw else None
+
+    out, lse, dx, dw = run(0)
+    # (64 workgroups: the persistent kernels, forward and backward)
+    out_p, lse_p, dx_p, dw_p = run(64)
+    k = 5 if mon else 2
+    assert torch.equal(lse[y != -1], lse_p[y != -1]) and torch.equal(out[:k], out_p[:k])
+    for got, ref in ((dx, dx_p), (dw, dw_p)):
+        assert torch.isfinite(got).all()
+        if ref.double().norm() > 0:
+            assert rel_errors(got, ref)[1] <= BOUND[got.dtype]
+    assert (dx[y == -1] == 0).all()
+    # one gradient alone: the same bits
+    assert torch.equal(run(0, want_dw=False)[2], dx) and torch.equal(run(0, want_dx=False)[3], dw)
