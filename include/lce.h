@@ -178,7 +178,7 @@ int lce_check_problem(const lce_problem* p);
  * The forward works through the tokens in chunks of max(n_chunk, 16384) rows
  * (65536 under an fp32 weight): V/32 bytes of partial sums per token of one
  * chunk (four times that with monitoring), plus a 16-bit copy of at most
- * 256 MiB of an fp32 weight, plus 12 bytes per token, plus -- when tokens are
+ * 256 MiB of an fp32 weight (none for few tokens, which read it as it is), plus 12 bytes per token, plus -- when tokens are
  * packed or x is fp32 -- a packed copy of x.
  * The backward size stays within n_chunk * V * 4 bytes -- the memory bound the
  * reference documents for N_chunk_size (ops.py:677, 700, 860) -- whenever the

@@ -71,7 +71,8 @@ int check(const lce_problem* p, bool backward) {
   const int64_t xa = xd == LCE_F32 ? 4 : 8, wa = wd == LCE_F32 ? 4 : 8;  // 16-byte rows
   if (p->ldx < p->H || p->ldx % xa || p->ldw < w_cols || p->ldw % wa) return LCE_EINVAL_ARG;
   // The kernels address a 256-row tile of x, of a 16-bit W and of dx with 32-bit byte offsets: 256 rows must
-  // stay below 2 GiB.  (An fp32 W is only read by the slab conversion, which uses 64-bit addresses.)
+  // stay below 2 GiB.  (An fp32 W is read by the slab conversion, which uses 64-bit addresses, and within
+  // limits of its own: fwd_reads_f32.)
   const int64_t tile_limit = ((int64_t)1 << 31) / 256;
   if (p->ldx * (xd == LCE_F32 ? 4 : 2) > tile_limit) return LCE_EINVAL_ARG;
   if (is16(wd) && p->ldw * 2 > tile_limit) return LCE_EINVAL_ARG;
@@ -151,6 +152,21 @@ int products(const lce_problem* p) { return lce::products_of(compute_dtype(p)); 
 // Bytes of a row of the logit contraction's operands (lce::live_bands).
 int64_t logit_k_bytes(const lce_problem* p) { return lce::padded_k(parts_of(p) * p->H) * 2; }
 
+// Whether the forward's tile kernel reads an fp32 weight as it is (StagerF32) instead of 16-bit copies of slabs of it.  With few
+// tokens the loss is one pass over the weight, and making the copy (6 bytes an element through memory, 8 with pairs, and a launch)
+// costs more than the pass itself; with more, every 128 tokens take the fp32 rows through L2 and the registers again, where the
+// copy is half as wide.  us of device time, as it is / copied: bf16 or fp16 activations N=47, H=4544, V=28288 97 / 201; N=200,
+// H=2048, V=32000 65 / 116; N=256, H=4096, V=32000 151 / 233, stored (V, H) 140 / 241; N=256, H=768, V=8192 19 / 25; N=500, H=4096,
+// V=32000 279 / 248.  Pairs read a row three times, as hi, hi and lo, and with few columns (few workgroups, each a chain of
+// waits) that is what the launch takes: N=16, H=1024, V=8192 52 / 50, N=100, H=1024, V=16384 56 / 61, N=256, H=768, V=50304 125 / 131,
+// N=128, H=1024, V=50304 90 / 150, N=64, H=3741, V=40832 281 / 532.  (With monitoring, pairs run out of registers.)
+// (By the problem alone, as the workspace's size is.  A tile's 128 rows lie within the 2 GiB that an offset reaches.)
+constexpr int64_t kRowsF32 = 256, kPairColsF32 = 12288;
+bool fwd_reads_f32(const lce_problem* p) {
+  return p->w_dtype == LCE_F32 && p->N <= kRowsF32 && (!splits(p) || (p->V >= kPairColsF32 && !p->monitoring)) &&
+         p->ldw < ((int64_t)1 << 22) && p->max_workgroups <= 0;
+}
+
 FwdPlan plan_fwd(const lce_problem* p) {
   FwdPlan f;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Vp = (size_t)lce::padded_vocab(p->V);
@@ -171,7 +187,7 @@ FwdPlan plan_fwd(const lce_problem* p) {
   // in one launch; no difference at H = 2048, where x stays in the cache).
   // (fp32 activations reach the tile kernels as bf16 pairs, twice as wide)
   if ((size_t)f.nc * (size_t)(parts_of(p) * p->H) * 2 > ((size_t)128 << 20) && f.vs > 32768) f.vs = 32768;
-  if (p->w_dtype == LCE_F32) {
+  if (p->w_dtype == LCE_F32 && !fwd_reads_f32(p)) {
     // slab copies of at most 256 MiB (at least one tile column)
     const int64_t hw = parts_of(p) * p->H;  // rows of the copy
     int64_t cols = ((int64_t)256 << 20) / (hw * 2) / 256 * 256;
@@ -837,13 +853,13 @@ int forward_impl(const lce_problem* p, const void* x, const void* w, const int64
   a.nc = f.nc;
   for (a.row0 = 0; a.row0 < a.Np; a.row0 += f.nc) {
     if (ph & LCE_PHASE_FWD_TILES) {
-      // One launch over the whole vocabulary, or -- fp32 weight -- one per slab, each on a
+      // One launch over the whole vocabulary, or -- fp32 weight, more than a few tokens -- one per slab, each on a
       // 16-bit copy of its columns made just before it (same stream, one buffer).
       for (int64_t v0 = 0; v0 < p->V; v0 += f.vs) {
         lce::FwdArgs t = a;
         t.v0 = v0;
         t.vw = p->V - v0 < f.vs ? p->V - v0 : f.vs;
-        if (p->w_dtype == LCE_F32) {
+        if (p->w_dtype == LCE_F32 && !fwd_reads_f32(p)) {
           const int64_t ld16 = a.w_vh ? p->H : lce::pad_to(t.vw, 256);
           e = a.w_vh ? lce::launch_convert_w_rows((const float*)w, p->ldw, p->H, v0, t.vw, base + f.w16, ld16,
                                                   compute_dtype(p), s)

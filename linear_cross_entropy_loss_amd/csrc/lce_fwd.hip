@@ -12,6 +12,8 @@
 // forms the per-token loss terms (ops.py:753-761); fwd_final_kernel sums them
 // in a fixed order into the five scalars of ops.py:802 and the valid-label
 // count of ops.py:705.  All reductions are order-deterministic.
+#include <type_traits>
+
 #include "lce_gemm_small.h"
 #include "lce_fwd_epilogue.h"
 #include "lce_internal.h"
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void fwd_tiles_persistent_kernel(const Fw
 
 // The same on 128 x 128 tiles (lce_gemm_small.h): workgroup = one slice of 128 columns, 128 tokens.  tiles_p slices; those past
 // the vocabulary's end get partials as well, which the row merge reads.
-template <class T, bool WVH, bool MON>
+template <class T, bool WVH, bool MON, bool WF32>
 __global__ __launch_bounds__(kThreads, 2) void fwd_small_kernel(const FwdArgs a, int tiles_p, int tiles_q) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename elem_of<T>::type E;
@@ -157,12 +159,14 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_small_kernel(const FwdArgs a,
   if (a.row0 + t0 >= rows) return;
   constexpr int kParts = is_pair<T>::value ? 2 : 1;
   const int64_t v = (a.v0 - a.wv0) + (int64_t)tp * kSmallTile;
-  const E* w = reinterpret_cast<const E*>(a.w);
-  SmallPipe<T, WVH> pipe;
+  typedef typename std::conditional<WF32, float, E>::type W;
+  constexpr int kRowsOf = WF32 ? 1 : kParts;  // (fp32: one part, which is both)
+  const W* w = reinterpret_cast<const W*>(a.w);
+  SmallPipe<T, WVH, true, false, 4, 1, false, WF32> pipe;
   f32x16_t acc[kNB][1];
-  pipe.run(w + (WVH ? v * a.ldw : v), WVH ? matrix_end<E>(w, a.Vw, a.ldw, a.H) : matrix_end<E>(w, kParts * a.H, a.ldw, a.Vw), a.ldw,
+  pipe.run(w + (WVH ? v * a.ldw : v), WVH ? matrix_end<W>(w, a.Vw, a.ldw, a.H) : matrix_end<W>(w, kRowsOf * a.H, a.ldw, a.Vw), a.ldw,
            x + (a.row0 + t0) * ldx, matrix_end<E>(x, rows, ldx, kParts == 2 ? a.x_lo + a.H : a.H), ldx, a.H,
-           (int)small_logit_ktiles(a.H, kParts == 2 ? 3 : 1), a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
+           (int)small_logit_ktiles(a.H, kParts == 2 ? 3 : 1), WF32 ? 0 : a.H * a.ldw * 2, a.x_lo * 2, lds, acc);
   // (with the sums of the persistent kernel, bit for bit: by columns but in the tile of 256 columns that straddles the end)
   const int64_t slice_v0 = a.v0 + (int64_t)tp * kSmallTile;
   const int64_t tw = t0 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kBlk;
@@ -406,11 +410,21 @@ template <class T, bool WVH, bool MON> hipError_t launch_persistent(const FwdArg
   const int64_t left = a.Np - a.row0;  // token tiles of this chunk at most
   const int64_t here = left < a.nc ? left : a.nc, there = a.N - a.row0, rows = here < there ? here : there;
   if constexpr (!is_pair<T>::value) {
-    if (a.H <= kNarrowHidden && a.small_wgs > 0) return launch_fwd_narrow(a, rows, s);
+    if (a.H <= kNarrowHidden && a.small_wgs > 0 && a.w_dtype != DT_F32) return launch_fwd_narrow(a, rows, s);
+  }
+  if (a.w_dtype == DT_F32) {  // read as it is (fwd_reads_f32)
+    if constexpr (is_pair<T>::value && MON) {
+      return hipErrorInvalidValue;
+    } else {
+      const int tiles_p = (int)(pad_to(a.vw, kTile) / kSmallTile), tiles_q = (int)((rows + kSmallTile - 1) / kSmallTile);
+      hipLaunchKernelGGL((fwd_small_kernel<T, WVH, MON, true>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a, tiles_p,
+                         tiles_q);
+      return hipGetLastError();
+    }
   }
   if (few_logit_tiles(rows, a.vw, small_logit_ktiles(a.H, products_of(a.x_dtype)), a.small_wgs)) {
     const int tiles_p = (int)(pad_to(a.vw, kTile) / kSmallTile), tiles_q = (int)((rows + kSmallTile - 1) / kSmallTile);
-    hipLaunchKernelGGL((fwd_small_kernel<T, WVH, MON>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a, tiles_p,
+    hipLaunchKernelGGL((fwd_small_kernel<T, WVH, MON, false>), dim3((unsigned)(tiles_p * tiles_q)), dim3(kThreads), kSmallLds, s, a, tiles_p,
                        tiles_q);
     return hipGetLastError();
   }
@@ -431,12 +445,12 @@ template <class T, bool WVH> hipError_t launch_layout(const FwdArgs& a, hipStrea
 }  // namespace
 
 hipError_t launch_fwd_tiles(const FwdArgs& a, hipStream_t s) {
-  if (a.x_dtype == DT_BF16 && a.w_dtype == DT_BF16)
-    return a.w_vh ? launch_layout<BF16, true>(a, s) : launch_layout<BF16, false>(a, s);
-  if (a.x_dtype == DT_F16 && a.w_dtype == DT_F16)
-    return a.w_vh ? launch_layout<F16, true>(a, s) : launch_layout<F16, false>(a, s);
-  if (a.x_dtype == DT_PAIR && a.w_dtype == DT_PAIR && !a.w_vh) return launch_layout<BF16P, false>(a, s);
-  // (an fp32 weight arrives here as a copy in the compute type, fp32 activations as the packed copy in pairs)
+  // (An fp32 weight arrives here as a copy in the compute type or, for few tokens, as it is; fp32 activations as the packed copy in
+  // pairs.)
+  const bool as_x = a.w_dtype == a.x_dtype || a.w_dtype == DT_F32;
+  if (a.x_dtype == DT_BF16 && as_x) return a.w_vh ? launch_layout<BF16, true>(a, s) : launch_layout<BF16, false>(a, s);
+  if (a.x_dtype == DT_F16 && as_x) return a.w_vh ? launch_layout<F16, true>(a, s) : launch_layout<F16, false>(a, s);
+  if (a.x_dtype == DT_PAIR && as_x && !a.w_vh) return launch_layout<BF16P, false>(a, s);
   return hipErrorInvalidValue;
 }
 

@@ -12,6 +12,8 @@
 // workgroups the loop is bound by the latency of memory, not by the matrix cores.
 #pragma once
 
+#include <type_traits>
+
 #include "lce_gemm3.h"
 
 namespace lce {
@@ -21,16 +23,86 @@ constexpr int kSmallOperandBytes = kSmallTile * kBK * 2;
 constexpr int kSmallStageBytes = 2 * kSmallOperandBytes;
 constexpr int kSmallLds = 2 * kSmallStageBytes;  // 64 KiB: two workgroups to a compute unit
 
+// The P operand from fp32 rows, rounded to the compute type (pairs: to the hi or the lo part that the step multiplies) on its way to
+// LDS, with the rounding of convert_w_slab_kernel.  As Stager3 otherwise: a thread moves eight numbers at a time, two loads and
+// one store, into the same LDS layouts.
+template <class T, bool KC, int CHUNKS> struct StagerF32 {
+  struct Regs {
+    u32x4_t v[CHUNKS][2];
+  };
+  static constexpr int kRowPieces = CHUNKS * 4, kRowsAtOnce = kThreads / kRowPieces;
+  const char* base;
+  const char* end;
+  unsigned range, voff, voff_cur, iter_stride;
+  int kpos, lds_off;
+  int64_t k_stride;
+  bool lo;  // pairs: which part of the numbers is stored
+
+  LCE_DEV void init(int64_t ld) {
+    const int t = threadIdx.x;
+    if (KC) {
+      const int c = t & 7, r = t >> 3;
+      voff = (unsigned)((r * ld + c * 8) * 4);
+      iter_stride = (unsigned)(32 * ld * 4);
+      k_stride = kBK * 4;
+      lds_off = r * 128 + ((c ^ (r & 7) ^ ((r >> 3) & 1)) << 4);
+      kpos = c * 8;
+    } else {
+      const int c = t % kRowPieces, k = t / kRowPieces, j = k & 3;
+      voff = (unsigned)((k * ld + c * 8) * 4);
+      iter_stride = (unsigned)(kRowsAtOnce * ld * 4);
+      k_stride = (int64_t)kBK * ld * 4;
+      lds_off = k * (kRowPieces * 16) + ((c << 4) ^ (((j & 1) << 7) | ((j >> 1) << 6) | ((j & 1) << 5)));
+      kpos = 0;
+    }
+    voff_cur = voff;
+    base = end = nullptr;
+    range = 0;
+    lo = false;
+  }
+  LCE_DEV void retarget(int k_rem) {
+    const int64_t left = end - base;
+    range = left <= 0 ? 0u : left > 0x7fffffff ? 0x7fffffffu : (unsigned)left;
+    if (KC) voff_cur = kpos < k_rem ? voff : 0x80000000u;
+  }
+  LCE_DEV void load(Regs& r, int i0, int i1) const {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, (int)range, 0x00020000);
+#pragma unroll
+    for (int i = i0; i < i1; ++i) {
+      r.v[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff_cur, (int)(i * iter_stride), 0);
+      r.v[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff_cur + 16, (int)(i * iter_stride), 0);
+    }
+  }
+  LCE_DEV void store(const Regs& r, char* tile, int i0, int i1) const {
+    constexpr int step = KC ? 32 * 128 : kRowsAtOnce * kRowPieces * 16;
+#pragma unroll
+    for (int i = i0; i < i1; ++i) {
+      float f[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const unsigned u = r.v[i][k >> 2][k & 3];
+        f[k] = __builtin_bit_cast(float, u);
+        if (is_pair<T>::value && lo) f[k] = bf16_lo(f[k]);
+      }
+      u32x4_t o;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = pack2<T>(f[2 * k], f[2 * k + 1]);
+      *reinterpret_cast<u32x4_t*>(tile + lds_off + i * step) = o;
+    }
+  }
+};
+
 // NP, NQ: blocks of 32 P / Q rows of a wave, four accumulator blocks together: 4, 1 for the logits; 2, 2 for the gradients, whose
 // epilogues do not need a slice of the vocabulary in one wave and whose fragment reads are then four for four products.
 // Q_BLOCKED, SWAP: Problem::kQBlocked and kSwapAB of Pipe3.
-template <class T, bool P_KC, bool Q_KC = true, bool Q_BLOCKED = false, int NP = 4, int NQ = 1, bool SWAP = false> struct SmallPipe {
+template <class T, bool P_KC, bool Q_KC = true, bool Q_BLOCKED = false, int NP = 4, int NQ = 1, bool SWAP = false,
+          bool P_F32 = false> struct SmallPipe {
   static_assert(NP * NQ == kNB, "four accumulator blocks to a wave");
   typedef typename elem_of<T>::type E;
   static constexpr bool kSplit = is_pair<T>::value;
   static constexpr bool kQRowBlocks = Q_BLOCKED && !Q_KC;
   static constexpr int kWavesP = kNB / NP;
-  typedef Stager3<T, E, P_KC, true, 4> PStager;
+  typedef typename std::conditional<P_F32, StagerF32<T, P_KC, 4>, Stager3<T, E, P_KC, true, 4>>::type PStager;
   typedef Stager3<T, E, Q_KC, true, 4> QStager;
   PStager ps;
   QStager qs;
@@ -51,12 +123,14 @@ template <class T, bool P_KC, bool Q_KC = true, bool Q_BLOCKED = false, int NP =
         ps.base += split_s == 0 ? 0 : p_lo;
         qs.base += split_s == 0 ? q_lo : -q_lo;
         ++split_s;
+        if constexpr (P_F32) ps.lo = split_s == 1;  // (the K tile stored next is two before the one loaded next: one after it, modulo 3)
         ps.retarget(k_rem);
         qs.retarget(k_rem);
         return;
       }
       ps.base -= p_lo;
       split_s = 0;
+      if constexpr (P_F32) ps.lo = false;
     }
     ps.base += ps.k_stride;
     if constexpr (kQRowBlocks) {
@@ -102,6 +176,10 @@ template <class T, bool P_KC, bool Q_KC = true, bool Q_BLOCKED = false, int NP =
   static constexpr int kReads = NQ * (Q_KC ? 1 : 2) + NP * (P_KC ? 1 : 2);  // LDS reads of a k-step's fragments
   // What goes behind each of a k-step's four matrix instructions: a quarter of the next one's reads, stores and loads in turn.
   template <int STORES, int LOADS> LCE_DEV void order() {
+    if constexpr (P_F32) {  // (with the conversions in between, left to the compiler)
+      __builtin_amdgcn_sched_barrier(0);
+      return;
+    }
     __builtin_amdgcn_sched_group_barrier(LCE_SG_MFMA, 1, 0);
     __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_RD, kReads - 3 * (kReads / 4), 0);
     if (STORES > 0) __builtin_amdgcn_sched_group_barrier(LCE_SG_DS_WR, 1, 0);

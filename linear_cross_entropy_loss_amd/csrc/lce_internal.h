@@ -94,7 +94,8 @@ struct FwdArgs {
   int64_t row0, nc;
   // Vocabulary columns [v0, v0 + vw) covered by this launch (v0 a multiple of 256), and the
   // window of W that the buffer `w` holds: columns [wv0, wv0 + Vw) of the weight, row stride ldw.
-  // (`w` is the caller's matrix, wv0 = 0, Vw = V -- or a 16-bit copy of one slab of an fp32 weight.)
+  // (`w` is the caller's matrix, wv0 = 0, Vw = V -- or a 16-bit copy of one slab of an fp32 weight; an fp32 weight
+  // itself for few tokens, w_dtype DT_F32.)
   int64_t v0, vw, wv0, Vw;
   // w_vh != 0: the weight is stored with the vocabulary as its row index, w[v * ldw + h] (the buffer `w` then
   // holds ROWS [wv0, wv0 + Vw)); otherwise w[h * ldw + v].
