@@ -323,7 +323,7 @@ enum {
  * the flag.
  *
  * Problems this route does not cover take the two calls above, one after the
- * other on the same workspace, inside this entry point: fp32 activations, a
+ * other on the same workspace, inside this entry point: fp32 activations without the flag above, a
  * weight that is neither of x's dtype nor fp32, and shapes whose sums of dW leave no
  * room for a chunk within the bound (a 16-bit dW with H near 4 * n_chunk or
  * above; lce_forward_backward_plan then reports 0 chunks).  `phases` selects kernels of either route; on the one-pass

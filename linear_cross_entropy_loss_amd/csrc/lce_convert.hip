@@ -1,6 +1,6 @@
 // An fp32 (master) weight is rounded to the 16-bit compute type one vocabulary
 // slab at a time, into a workspace buffer that the tile kernels of that slab
-// then read like a 16-bit weight.  The reference converts the whole weight to
+// then read like a 16-bit weight (the loss of few tokens reads the fp32 weight itself).  The reference converts the whole weight to
 // fp16 on entry (custom_fwd(cast_inputs=torch.float16), linear_cross_entropy/ops.py:665-667);
 // here the copy is one slab wide, is made in the compute type that the
 // activations have, and costs one read of the slab.  The rounding (nearest

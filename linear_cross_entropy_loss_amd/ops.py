@@ -14,8 +14,8 @@ The device work is done by hand-written gfx950 kernels behind the C ABI of
 When a gradient is wanted, ``forward`` computes it along with the loss from one
 evaluation of the logits (``lce_forward_backward``), as the reference's forward
 does (``ops.py:721-791``), and ``backward`` multiplies the upstream gradient in
-(``ops.py:810``).  Problems that route does not cover (fp32 activations,
-shapes whose scratch bound leaves no room for it) and forward-only calls compute
+(``ops.py:810``).  Problems that route does not cover (shapes whose scratch
+bound leaves no room for it or makes it the slower one) and forward-only calls compute
 only the loss in ``forward`` and save ``lse``; their ``backward`` recomputes the
 logit tiles (``lce_backward``).  So does a second ``backward`` over the same graph.
 """
