@@ -415,6 +415,10 @@ bool plan_narrow(const lce_problem* p, BwdPlan* b) {
   const int64_t tok = lce::pad_to(p->N, 128) / 128, voc = lce::pad_to(p->V, 128) / 128;
   if (p->H > lce::kNarrowHidden || splits(p) || p->pack_rows == LCE_PACK_ALWAYS || p->max_workgroups != 0 || tok > 1 << 20 || voc > 1 << 20)
     return false;
+  // The kernel reaches the rows of whole K tiles of a weight stored (H, V) by 32-bit offsets.  The caller's rows are short enough
+  // (check); those of the copy of an fp32 weight, as wide as the vocabulary here, have to be: else slabs of it.
+  if (p->w_dtype == LCE_F32 && p->w_layout == LCE_W_HV && lce::pad_to(p->H, 64) * lce::padded_vocab(p->V) * 2 >= (int64_t)1 << 31)
+    return false;
   const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)lce::padded_vocab(p->V) * 2) : 0;
   const size_t strict = (size_t)p->n_chunk * (size_t)p->V * 4, reserve = align_up((size_t)p->N * 4) + 4096;
   const size_t block = (size_t)lce::narrow_block_bytes(p->H), room = strict > w16 + reserve ? strict - w16 - reserve : 0;

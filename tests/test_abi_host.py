@@ -420,6 +420,26 @@ def test_backward_plan_invariants_on_random_problems():
         assert fwd <= part + Np * 16 + N * (split * H + 8) * 2 + slab_copy + N * 16 + 8192, (it, fwd)
 
 
+@pytest.mark.parametrize("H,wide", [(128, 8388608), (72, 8388608), (64, 16777216), (8, 16777216)])
+def test_narrow_plan_keeps_the_copy_of_an_fp32_weight_within_32_bit_offsets(H, wide):
+    """Hidden sizes up to 128: the 16-bit copy of an fp32 weight stored (H, V) is as wide as the vocabulary, and the kernel reaches
+    64 or 128 of its rows by 32-bit offsets.  Rows that together reach 2 GiB take slabs, whose rows do not."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    def plan(V, w_dtype=torch.float32, layout=_lib.W_HV):
+        ld = H if layout == _lib.W_VH else V
+        p = _prob(N=256, H=H, V=V, ldx=H, ldw=ld, lddx=H, lddw=ld, n_chunk=4096, w_dtype=w_dtype, dw_dtype=w_dtype, w_layout=layout)
+        return _lib.backward_plan(p)
+
+    assert plan(wide - 256) == (1, wide)  # (without a stage: wider than the vocabulary)
+    for V in (wide - 248, wide, 20000000):
+        slabs, width = plan(V)
+        assert slabs > 1 and 256 * width * 2 <= 1 << 31, (V, slabs, width)
+    # stored (V, H): rows of H, whatever the vocabulary; a 16-bit weight is read in place
+    assert plan(20000000, layout=_lib.W_VH)[0] == 1
+    assert plan(4194304, torch.bfloat16) == (1, 4194304 + 256)
+
+
 def test_vocabulary_major_weight_layout_is_checked_and_detected():
     """lce_problem.w_layout = LCE_W_VH: row strides are checked against H, fp32 activations and hidden sizes
     that are not multiples of 8 are refused; the Python host picks the layout from the strides alone."""
