@@ -46,6 +46,9 @@ template <class Plan> struct LastPlan {
   }
 };
 
+// The kernels address a 256-row tile of x, of a 16-bit W and of dx with 32-bit byte offsets: 256 rows must stay below 2 GiB.
+constexpr int64_t kTileLimit = ((int64_t)1 << 31) / 256;  // bytes of a row
+
 int check(const lce_problem* p, bool backward) {
   if (!p) return LCE_EINVAL_ARG;
   if (p->N <= 0 || p->H <= 0 || p->V <= 0 || p->n_chunk <= 0) return LCE_EINVAL_SHAPE;
@@ -70,12 +73,9 @@ int check(const lce_problem* p, bool backward) {
   const int64_t w_cols = vh ? p->H : p->V;  // row length of w and dw as stored
   const int64_t xa = xd == LCE_F32 ? 4 : 8, wa = wd == LCE_F32 ? 4 : 8;  // 16-byte rows
   if (p->ldx < p->H || p->ldx % xa || p->ldw < w_cols || p->ldw % wa) return LCE_EINVAL_ARG;
-  // The kernels address a 256-row tile of x, of a 16-bit W and of dx with 32-bit byte offsets: 256 rows must
-  // stay below 2 GiB.  (An fp32 W is read by the slab conversion, which uses 64-bit addresses, and within
-  // limits of its own: fwd_reads_f32.)
-  const int64_t tile_limit = ((int64_t)1 << 31) / 256;
-  if (p->ldx * (xd == LCE_F32 ? 4 : 2) > tile_limit) return LCE_EINVAL_ARG;
-  if (is16(wd) && p->ldw * 2 > tile_limit) return LCE_EINVAL_ARG;
+  // (An fp32 W is read by the slab conversion, which uses 64-bit addresses, and within limits of its own: fwd_reads_f32.)
+  if (p->ldx * (xd == LCE_F32 ? 4 : 2) > kTileLimit) return LCE_EINVAL_ARG;
+  if (is16(wd) && p->ldw * 2 > kTileLimit) return LCE_EINVAL_ARG;
   // tile and work-item counts are 32-bit
   if (lce::padded_tokens(p->N) / 256 * (lce::padded_vocab(p->V) / 256) > (int64_t)1 << 28) return LCE_EINVAL_SHAPE;
   if (backward) {
@@ -83,7 +83,7 @@ int check(const lce_problem* p, bool backward) {
     if (p->dw_dtype != wd && p->dw_dtype != LCE_F32) return LCE_EINVAL_DTYPE;
     // dx is stored in 8-byte (16-bit types) or 16-byte pieces, dW in 16-byte pieces
     if (p->lddx < p->H || p->lddx % 4 || p->lddw < w_cols || p->lddw % (p->dw_dtype == LCE_F32 ? 4 : 8)) return LCE_EINVAL_ARG;
-    if (p->lddx * (p->dx_dtype == LCE_F32 ? 4 : 2) > tile_limit) return LCE_EINVAL_ARG;
+    if (p->lddx * (p->dx_dtype == LCE_F32 ? 4 : 2) > kTileLimit) return LCE_EINVAL_ARG;
   }
   return LCE_OK;
 }
@@ -534,6 +534,7 @@ bool plan_kept(const lce_problem* p, FusedPlan* f) {
   f->tgt = o; o += align_up((size_t)Np * 4);
   f->blk = o; o += align_up((size_t)(Np / lce::kMergeRows) * 8 * sizeof(double));
   f->ld16 = Vp;
+  if (f->ld16 * 2 > kTileLimit) return false;  // (the weight's pairs have rows as wide as the vocabulary)
   f->w16 = o; o += align_up((size_t)(2 * p->H) * (size_t)Vp * 2);
   const size_t fixed = o, bound = (size_t)p->n_chunk * (size_t)p->V * 4, reserve = align_up((size_t)p->N * 4) + 4096;
   if (fixed + reserve > bound) return false;

@@ -440,6 +440,25 @@ def test_narrow_plan_keeps_the_copy_of_an_fp32_weight_within_32_bit_offsets(H, w
     assert plan(4194304, torch.bfloat16) == (1, 4194304 + 256)
 
 
+def test_kept_logits_plan_keeps_the_pairs_of_the_weight_within_32_bit_offsets():
+    """fp32 tensors, logits kept: the weight's bf16 pairs have rows as wide as the vocabulary, of which the kernels reach 256 by
+    32-bit offsets.  Rows of more than 8 MiB take two passes, in slabs whose rows are shorter."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    f32 = torch.float32
+
+    def prob(V, route):
+        return _prob(N=256, H=256, V=V, ldx=256, ldw=V, lddx=256, lddw=V, n_chunk=4096, x_dtype=f32, w_dtype=f32, dx_dtype=f32,
+                     dw_dtype=f32, route=route | _lib.ROUTE_KEEP_LOGITS)
+
+    for route in (_lib.ROUTE_AUTO, _lib.ROUTE_ONE_PASS):
+        assert _lib.forward_backward_plan(prob(4194304, route)) == (1, 256)
+        for V in (4194304 + 4, 5000000, 6000000):
+            p = prob(V, route)
+            assert _lib.forward_backward_plan(p) == (0, 0)
+            assert 256 * _lib.backward_plan(p)[1] * 2 <= 1 << 31
+
+
 def test_vocabulary_major_weight_layout_is_checked_and_detected():
     """lce_problem.w_layout = LCE_W_VH: row strides are checked against H, fp32 activations and hidden sizes
     that are not multiples of 8 are refused; the Python host picks the layout from the strides alone."""
