@@ -644,6 +644,7 @@ bool plan_fused_with(const lce_problem* p, bool lo8, bool settled, int64_t most_
   // an fp32 master weight is rounded to the compute type once per call, all of it
   const bool vh = p->w_layout == LCE_W_VH;
   f->ld16 = vh ? p->H : (int64_t)Vp;
+  if (p->w_dtype == LCE_F32 && f->ld16 * 2 > kTileLimit) return false;
   f->w16 = o;
   if (p->w_dtype == LCE_F32) o += align_up((vh ? (size_t)p->V : (size_t)p->H) * (size_t)f->ld16 * 2);
   const size_t fixed = o;

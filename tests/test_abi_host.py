@@ -459,6 +459,21 @@ def test_kept_logits_plan_keeps_the_pairs_of_the_weight_within_32_bit_offsets():
             assert 256 * _lib.backward_plan(p)[1] * 2 <= 1 << 31
 
 
+def test_one_pass_plan_keeps_the_copy_of_an_fp32_weight_within_32_bit_offsets():
+    """16-bit activations under an fp32 weight stored (H, V): the one-pass route's copy of the weight has rows as wide as the
+    vocabulary; of more than 8 MiB they would lie outside the 2 GiB that an offset spans.  (Stored (V, H): rows of H.)"""
+    from linear_cross_entropy_loss_amd import _lib
+
+    def chunks(V, layout=_lib.W_HV, route=_lib.ROUTE_ONE_PASS):
+        ld = 256 if layout == _lib.W_VH else V
+        return _lib.forward_backward_plan(_prob(N=256, H=256, V=V, ldx=256, ldw=ld, lddx=256, lddw=ld, n_chunk=4096, w_layout=layout,
+                                                w_dtype=torch.float32, dw_dtype=torch.float32, route=route))[0]
+
+    assert chunks(4194304) == 1 and chunks(5000000, layout=_lib.W_VH) == 1
+    for V in (4194304 + 8, 5000000, 20000000):
+        assert chunks(V) == 0 and chunks(V, route=_lib.ROUTE_AUTO) == 0
+
+
 def test_vocabulary_major_weight_layout_is_checked_and_detected():
     """lce_problem.w_layout = LCE_W_VH: row strides are checked against H, fp32 activations and hidden sizes
     that are not multiples of 8 are refused; the Python host picks the layout from the strides alone."""

@@ -38,6 +38,7 @@ def _exact(x, y, w, dtype, step=1 << 18):
 @pytest.mark.parametrize("N,H,V,dtype,route", [
     (100, 128, 8388608 + 1000, torch.bfloat16, True),  # a hidden size of the kernels without a stage
     (60, 256, 4194304 + 1000, torch.float32, True),  # fp32 tensors, whose logits are kept below that
+    (60, 256, 4194304 + 1000, torch.bfloat16, "always"),  # an fp32 weight under 16-bit activations, one pass below that
 ])
 def test_gradients_at_vocabularies_beyond_32_bit_offsets(N, H, V, dtype, route):
     from linear_cross_entropy_loss_amd import linear_cross_entropy, ops
