@@ -184,8 +184,9 @@ int lce_check_problem(const lce_problem* p);
  * reference documents for N_chunk_size (ops.py:677, 700, 860) -- whenever the
  * narrowest split (256-column slabs plus an fp32 running dx) fits in it; for
  * the remaining shapes (a small vocabulary with many tokens) that narrowest
- * split is used and its size reported: the bound is a target, not a reason
- * to refuse a shape the reference runs.
+ * split is used -- or, for hidden sizes up to 128, the kernels that stage
+ * nothing, in at most twice its size -- and its size reported: the bound is a
+ * target, not a reason to refuse a shape the reference runs.
  */
 int lce_workspace_bytes(const lce_problem* p, size_t* fwd_bytes, size_t* bwd_bytes);
 
@@ -194,8 +195,9 @@ int lce_workspace_bytes(const lce_problem* p, size_t* fwd_bytes, size_t* bwd_byt
  * vocabulary slab at a time (`slab_width` columns, a multiple of 256; `slabs`
  * passes, the last one over whatever columns remain).  The counterpart of the reference's loop over N_chunk_size-row
  * groups (ops.py:721), which exists for the same purpose: bounding scratch.
- * 16-bit activations with a hidden size of up to 128, rows not packed on demand: nothing is staged; one slab, wider than
- * the vocabulary.
+ * 16-bit activations with a hidden size of up to 128, rows not packed on demand: nothing is staged, where the bound has room for
+ * the copy of an fp32 weight and the partial sums, or else the library's model puts that ahead all the same; one slab, wider
+ * than the vocabulary.
  */
 int lce_backward_plan(const lce_problem* p, int64_t* slabs, int64_t* slab_width);
 

@@ -243,7 +243,7 @@ constexpr double kPlanCUs = 256.0;
 // A unit in us, and how much faster the gradients on small tiles have to be by the model, which is off by up to 10 %.  Narrow
 // hidden sizes, for which a tight bound leaves slabs of the vocabulary, gain most: a step of bf16 N=16384, H=256, V=4096 586 -> 372 us,
 // N=8192, H=512, V=8192 583 -> 394, fp16 N=18432, H=128, V=9344 800 -> 540, fp32 N=4096, H=512, V=2048 940 -> 463.
-constexpr double kUnitUs = 1.4, kSmallMargin = 0.93;
+constexpr double kUnitUs = 1.4, kSmallMargin = 0.93, kStarvedMargin = 0.6;
 double kernel_cost(double T, double L, double e, bool parts, bool settled) {
   const double full = (double)(int64_t)(T / kPlanCUs), r = T - full * kPlanCUs;
   double cost = full * (L + e) + 10.0;
@@ -273,11 +273,19 @@ double kernel_cost(double T, double L, double e, bool parts, bool settled) {
 // N * H * 4 bytes, the fp32 x_grad buffer the reference allocates next to its logits chunk (ops.py:693) and
 // this library does not -- and by the split-K partial sums.  If even that fails, the narrowest split is used:
 // the bound is a target, the operator never refuses a shape.
-bool plan_narrow(const lce_problem* p, BwdPlan* b);
+bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved);
 int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
-  memset(b, 0, sizeof(*b));
-  if (!settled && plan_narrow(p, b)) return LCE_OK;
+  BwdPlan narrow;
+  bool starved = false;
   const size_t strict = (size_t)p->n_chunk * (size_t)p->V * 4;
+  // what the caller holds besides the workspace between forward and backward: lse and a few scalars
+  const size_t reserve = align_up((size_t)p->N * 4) + 4096;
+  const bool narrow_fits = !settled && strict > reserve && plan_narrow(p, strict - reserve, &narrow, &starved);
+  if (narrow_fits && !starved) {
+    *b = narrow;
+    return LCE_OK;
+  }
+  memset(b, 0, sizeof(*b));
   const size_t dz_cap = (size_t)1 << 30;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Hp = (size_t)lce::padded_hidden(p->H);
   const int64_t Vp = lce::padded_vocab(p->V);
@@ -335,8 +343,6 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
     const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)vs * 2 * (size_t)parts_of(p)) : 0;  // copy of the slab of W
     // the widened bound is for the staging proper; the split-K partial sums (at most 64 MiB, shared by dx
     // and dW) and the packed rows come on top of it there
-    // (reserve: what the caller holds besides the workspace between forward and backward -- lse and a few scalars)
-    const size_t reserve = align_up((size_t)p->N * 4) + 4096;
     const size_t counted = dz + acc + w16 + (mode != 2 ? fixed + part + reserve : 0);
     if (!((counted <= budget && (dz <= dz_cap || vs == 256)) || (mode == 2 && vs == 256))) return false;
     out->slabs = slabs;
@@ -402,16 +408,34 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
   double cost_full = 0, cost_lean = 0;
   const bool ok_full = full_fits = choose(0, &full, &cost_full);
   const bool ok_lean = choose(1, &lean, &cost_lean);
-  if (ok_full && (!ok_lean || cost_full <= cost_lean)) { *b = full; b->cost = cost_full; return LCE_OK; }
-  if (ok_lean) { *b = lean; b->cost = cost_lean; return LCE_OK; }
+  if (ok_full || ok_lean) {
+    const bool take_full = ok_full && (!ok_lean || cost_full <= cost_lean);
+    *b = take_full ? full : lean;
+    b->cost = take_full ? cost_full : cost_lean;
+    // (The model's few long items, which a starved launch ends on, have a compute unit each and run up to twice as fast as that: us
+    // of a backward, without a stage / staged, and what the model says: bf16 under an fp32 weight, N=1977, H=112, V=126246, n_chunk = 64
+    // 806 / 1039 (1534 / 1078), N=191, H=112, V=42438, 64 105 / 113 (176 / 113), N=186, H=120, V=11847, 64 243 / 120 (244 / 135).)
+    if (narrow_fits && kStarvedMargin * narrow.cost <= b->cost) *b = narrow;
+    return LCE_OK;
+  }
   double wide = 0;
-  if (choose(2, b, &wide)) { b->cost = wide; return LCE_OK; }
-  return LCE_EWORKSPACE;
+  if (!choose(2, b, &wide)) return LCE_EWORKSPACE;
+  b->cost = wide;
+  // No staged plan meets the bound: the kernels without a stage get up to twice what this one takes.  us of a backward, without a stage
+  // in what the bound leaves / in that / staged: bf16 N=262144, H=64, V=32, n_chunk = 4096 4836 / 97 / 131, N=65536, H=64, V=10
+  // 1203 / 69 / 54, N=2^20, H=64, V=256 19443 / 311 / 510, N=32768, H=128, V=256, 2048 72 / 92 / 38; under an fp32 weight N=4737, H=96,
+  // V=54762, 32 no room / 548 / 5144.
+  const size_t twice = 2 * b->total;
+  if (narrow_fits && narrow.cost <= b->cost) *b = narrow;
+  if (!settled && plan_narrow(p, twice, &narrow, &starved) && narrow.cost <= b->cost) *b = narrow;
+  return LCE_OK;
 }
 
 // Hidden sizes up to lce::kNarrowHidden: the gradients without a stage, one slab, nothing packed away.  Not where the caller asks for
-// packing, as the sums over the tokens are cut by their number in memory.
-bool plan_narrow(const lce_problem* p, BwdPlan* b) {
+// packing, as the sums over the tokens are cut by their number in memory.  `budget`: bytes for the 16-bit copy of an fp32 weight and
+// the partial sums.  *starved: that leaves the sums so little room that the model puts the kernels 10 % or more behind what they
+// would take with all they ask for.
+bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved) {
   const int64_t tok = lce::pad_to(p->N, 128) / 128, voc = lce::pad_to(p->V, 128) / 128;
   if (p->H > lce::kNarrowHidden || splits(p) || p->pack_rows == LCE_PACK_ALWAYS || p->max_workgroups != 0 || tok > 1 << 20 || voc > 1 << 20)
     return false;
@@ -420,10 +444,19 @@ bool plan_narrow(const lce_problem* p, BwdPlan* b) {
   if (p->w_dtype == LCE_F32 && p->w_layout == LCE_W_HV && lce::pad_to(p->H, 64) * lce::padded_vocab(p->V) * 2 >= (int64_t)1 << 31)
     return false;
   const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)lce::padded_vocab(p->V) * 2) : 0;
-  const size_t strict = (size_t)p->n_chunk * (size_t)p->V * 4, reserve = align_up((size_t)p->N * 4) + 4096;
-  const size_t block = (size_t)lce::narrow_block_bytes(p->H), room = strict > w16 + reserve ? strict - w16 - reserve : 0;
-  const int64_t most = (int64_t)(room / block) < 1024 ? (int64_t)(room / block) : 1024;
+  if (w16 > budget) return false;
+  const size_t block = (size_t)lce::narrow_block_bytes(p->H);
+  constexpr int64_t kWished = 1024;  // blocks: at most 64 MiB
+  const int64_t room = (int64_t)((budget - w16) / block), most = room < kWished ? room : kWished;
   const lce::SmallGrads g = lce::plan_narrow_grads(p->N, p->H, p->V, most);
+  // (the kernel that adds a tile's parts goes through them eight at a time, one such after another: 0.2 us a part, N=10303, H=40, V=24
+  // with 81 of them 33 us against 30 with nine)
+  auto us = [](const lce::SmallGrads& c) -> double {
+    const int parts = c.dx_nseg > c.dw_nseg ? c.dx_nseg : c.dw_nseg;
+    return c.us + (parts > 8 ? 0.2 * (double)(parts - 8) : 0.0);
+  };
+  *starved = most < kWished && us(g) > 1.1 * us(lce::plan_narrow_grads(p->N, p->H, p->V, kWished));
+  memset(b, 0, sizeof(*b));
   b->narrow = true;
   b->slabs = 1;
   b->vs = lce::padded_vocab(p->V) + 256;  // (one slab that ends past the vocabulary: nothing is staged, lce.h)
@@ -431,7 +464,7 @@ bool plan_narrow(const lce_problem* p, BwdPlan* b) {
   b->w16 = align_up((size_t)b->small_blocks * block);
   b->total = b->w16 + w16;
   if (b->total == 0) b->total = 256;
-  b->cost = g.us / kUnitUs;
+  b->cost = us(g) / kUnitUs;
   return true;
 }
 

@@ -440,6 +440,31 @@ def test_narrow_plan_keeps_the_copy_of_an_fp32_weight_within_32_bit_offsets(H, w
     assert plan(4194304, torch.bfloat16) == (1, 4194304 + 256)
 
 
+def test_narrow_plan_has_room_for_its_sums_or_is_not_taken():
+    """Hidden sizes up to 128, nothing staged: few classes and many tokens leave the bound no room to cut the sums over the tokens, and
+    one or two workgroups would walk them all.  The sums then get room on top, at most twice what a staged plan takes where that
+    cannot meet the bound either, or the staged plan is taken; where a plan within the bound exists, the bound holds."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    def plan(N, H, V, nc, w_dtype=torch.bfloat16, **kw):
+        p = _prob(N=N, H=H, V=V, ldx=H, ldw=V + (-V) % 8, lddx=H, lddw=V + (-V) % 8, n_chunk=nc, w_dtype=w_dtype, dw_dtype=w_dtype, **kw)
+        return _lib.backward_plan(p)[1] > -(-V // 256) * 256, _lib.backward_workspace_bytes(p)
+
+    block = 128 * 64 * 4
+    for N, H, V, nc in ((262144, 64, 32, 4096), (65536, 64, 10, 4096), (1 << 20, 64, 256, 4096), (32768, 128, 256, 2048),
+                        (100000, 8, 3, 512)):
+        narrow, size = plan(N, H, V, nc)
+        staged = plan(N, H, V, nc, max_workgroups=1 << 20)[1]  # (a call that limits its workgroups is staged)
+        assert size <= 2 * staged
+        assert not narrow or size >= 64 * block, (N, H, V, size)  # 64 stretches of the tokens at least
+    # the copy of an fp32 weight alone is more than the bound, slabs of it are not
+    for nc in (32, 64):
+        narrow, size = plan(4096, 128, 50000, nc, torch.float32)
+        assert not narrow and size + 4096 * 4 + 4096 <= nc * 50000 * 4
+    # with room for both, nothing is staged
+    assert plan(4096, 128, 50000, 128, torch.float32)[0] and plan(16384, 128, 1000, 4096)[0]
+
+
 def test_kept_logits_plan_keeps_the_pairs_of_the_weight_within_32_bit_offsets():
     """fp32 tensors, logits kept: the weight's bf16 pairs have rows as wide as the vocabulary, of which the kernels reach 256 by
     32-bit offsets.  Rows of more than 8 MiB take two passes, in slabs whose rows are shorter."""
