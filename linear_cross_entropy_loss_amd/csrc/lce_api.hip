@@ -431,9 +431,9 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
   return LCE_OK;
 }
 
-// Hidden sizes up to lce::kNarrowHidden: the gradients without a stage, one slab, nothing packed away.  Not where the caller asks for
-// packing, as the sums over the tokens are cut by their number in memory.  `budget`: bytes for the 16-bit copy of an fp32 weight and
-// the partial sums.  *starved: that leaves the sums so little room that the model puts the kernels 10 % or more behind what they
+// Hidden sizes up to lce::kNarrowHidden: the gradients without a stage, one slab.  (Not where the caller asks for packing whatever the
+// size: that is the staged kernels' as before.)  `budget`: bytes for the packed rows, the 16-bit copy of an fp32 weight and the
+// partial sums.  *starved: that leaves the sums so little room that the model puts the kernels 10 % or more behind what they
 // would take with all they ask for.
 bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved) {
   const int64_t tok = lce::pad_to(p->N, 128) / 128, voc = lce::pad_to(p->V, 128) / 128;
@@ -444,10 +444,13 @@ bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved)
   if (p->w_dtype == LCE_F32 && p->w_layout == LCE_W_HV && lce::pad_to(p->H, 64) * lce::padded_vocab(p->V) * 2 >= (int64_t)1 << 31)
     return false;
   const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)lce::padded_vocab(p->V) * 2) : 0;
-  if (w16 > budget) return false;
+  const bool pack = packs_rows(p);
+  const PackPlan k = plan_pack(p, 0);
+  const size_t fixed = pack ? k.end + align_up((size_t)p->N * 4) : 0;
+  if (fixed + w16 > budget) return false;
   const size_t block = (size_t)lce::narrow_block_bytes(p->H);
   constexpr int64_t kWished = 1024;  // blocks: at most 64 MiB
-  const int64_t room = (int64_t)((budget - w16) / block), most = room < kWished ? room : kWished;
+  const int64_t room = (int64_t)((budget - fixed - w16) / block), most = room < kWished ? room : kWished;
   const lce::SmallGrads g = lce::plan_narrow_grads(p->N, p->H, p->V, most);
   // (the kernel that adds a tile's parts goes through them eight at a time, one such after another: 0.2 us a part, N=10303, H=40, V=24
   // with 81 of them 33 us against 30 with nine)
@@ -460,8 +463,12 @@ bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved)
   b->narrow = true;
   b->slabs = 1;
   b->vs = lce::padded_vocab(p->V) + 256;  // (one slab that ends past the vocabulary: nothing is staged, lce.h)
+  b->pack = k;
+  b->pack_on = pack;
+  b->lse_c = k.end;
   b->small_blocks = g.dx_blocks + g.dw_blocks;
-  b->w16 = align_up((size_t)b->small_blocks * block);
+  b->dx_part = fixed;
+  b->w16 = fixed + align_up((size_t)b->small_blocks * block);
   b->total = b->w16 + w16;
   if (b->total == 0) b->total = 256;
   b->cost = us(g) / kUnitUs;
@@ -1280,7 +1287,7 @@ int lce_backward(const lce_problem* p, const void* x, const void* w, const int64
     const bool want_dx = dx && (ph & LCE_PHASE_BWD_DX), want_dw = dw && (ph & LCE_PHASE_BWD_DW);
     if (b.narrow) {
       lce::SmallGrads g = lce::plan_narrow_grads(p->N, p->H, p->V, b.small_blocks);
-      g.part = (float*)base;
+      g.part = (float*)(base + b.dx_part);
       e = lce::launch_bwd_narrow(a, g, want_dx, want_dw, s);
       if (e != hipSuccess) return hip_fail(e, "bwd_narrow");
       continue;

@@ -13,6 +13,9 @@
 // An accumulator block of S has the streaming index along its registers, in the order that the fragments of the second product
 // want along K once lanes l and l + 32 have exchanged quads: dz goes from one matrix instruction to the next without LDS.
 // dz is rounded once to the compute type, as in the staged kernels, and has their bits.
+// Large problems have their tokens with an ignored label packed away first, as with the staged kernels (packs_rows in lce_api.hip): the
+// number of rows is read from the device, and the cuts of dW follow it.  bf16 N=65536, H=128, V=32768, us of a backward, all rows / packed:
+// none ignored 2088 / 2117, 5 % 2089 / 2078, 85 % 1845 / 739; staged 4206, 4052, 1414.
 //
 // Bound by vector instructions, of which an exponential is four, with the matrix instructions only partly under them: 128 x 128
 // logits take two workgroups of a compute unit 3.3 us for the forward and 3.1 for a gradient at a hidden size of 64 (0.6 of 1.4
@@ -236,8 +239,8 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_narrow_kernel(const FwdArgs a
 // the streaming ones are columns from v0 on; dW: the other way round, the tokens' scalars in LDS.
 constexpr int kNoColumn = -0x7fffffff;
 // (label: kNoColumn where there is no column to look for)
-LCE_DEV void narrow_scalars(const BwdArgs& a, int64_t tok, float& nlse, float& gain, int& label) {
-  const int64_t yy = tok < a.N ? a.y[tok] : a.ignore_index;
+LCE_DEV void narrow_scalars(const BwdArgs& a, int64_t rows, int64_t tok, float& nlse, float& gain, int& label) {
+  const int64_t yy = tok < rows ? a.y[tok] : a.ignore_index;
   const bool valid = yy != a.ignore_index;
   const float l = valid ? a.lse[tok] : 0.f;
   nlse = valid ? fmaf(-l, kLog2e, (float)a.dz_shift) : -INFINITY;
@@ -247,14 +250,16 @@ LCE_DEV void narrow_scalars(const BwdArgs& a, int64_t tok, float& nlse, float& g
 }
 
 // The gradient of one 128-row tile of the stationary matrix over streaming tiles [first, last): acc[hb], rows h along registers,
-// stationary rows along lanes.
+// stationary rows along lanes.  rows: the tokens that are worked on, all of x's or the packed ones.
 template <class T, bool WVH, bool DW, bool ZREG, int KT>
-LCE_DEV void narrow_gradient(const BwdArgs& a, int wave, int tile, int first, int last, char* lds, f32x16_t (&acc)[2 * KT]) {
+LCE_DEV void narrow_gradient(const BwdArgs& a, int64_t rows, int wave, int tile, int first, int last, char* lds, f32x16_t (&acc)[2 * KT]) {
   typedef typename elem_of<T>::type E;
   constexpr bool TRANS = !DW && !WVH;  // the streaming matrix is W stored (H, V)
-  const E* x = reinterpret_cast<const E*>(a.x);
+  const bool packed = rows != a.N;
+  const E* x = reinterpret_cast<const E*>(packed ? a.xc : a.x);
+  const int64_t ldx = packed ? a.ldxc : a.ldx;
   const E* w = reinterpret_cast<const E*>(a.w);
-  const void* x_end = matrix_end<E>(x, a.N, a.ldx, a.H);
+  const void* x_end = matrix_end<E>(x, rows, ldx, a.H);
   const void* w_end = WVH ? matrix_end<E>(w, a.Vw, a.ldw, a.H) : matrix_end<E>(w, a.H, a.ldw, a.Vw);
   const int tid = narrow_tid(wave), lane = tid & 63, half = lane >> 5;
   const int64_t r0 = (int64_t)tile * kNarrowTile, rw = r0 + wave * kBlk;
@@ -268,8 +273,8 @@ LCE_DEV void narrow_gradient(const BwdArgs& a, int wave, int tile, int first, in
   auto fetch = [&](int tc) {
     const int64_t c = (int64_t)tc * kNarrowTile;
     if (DW) {
-      next.load(x + c * a.ldx, x_end, 0);
-      narrow_scalars(a, c + (tid & (kNarrowTile - 1)), nlse, gain, label);
+      next.load(x + c * ldx, x_end, 0);
+      narrow_scalars(a, rows, c + (tid & (kNarrowTile - 1)), nlse, gain, label);
     } else {
       next.load(w + (WVH ? c * a.ldw : c), w_end, a.Vw - c);
     }
@@ -288,7 +293,7 @@ LCE_DEV void narrow_gradient(const BwdArgs& a, int wave, int tile, int first, in
   s16x8_t q[4 * KT];
   NarrowReader<TRANS> rd;
   rd.init();
-  next.init(wave, DW ? a.ldx : a.ldw, a.H);
+  next.init(wave, DW ? ldx : a.ldw, a.H);
   if (DW && !WVH) {
     // (the columns of W that stay, through LDS)
     NarrowTile<T, true, KT> stay;
@@ -306,7 +311,7 @@ LCE_DEV void narrow_gradient(const BwdArgs& a, int wave, int tile, int first, in
   } else if (DW) {
     narrow_stay<KT>(q, w + rw * a.ldw, w_end, a.ldw, a.H);
   } else {
-    narrow_stay<KT>(q, x + rw * a.ldx, x_end, a.ldx, a.H);
+    narrow_stay<KT>(q, x + rw * ldx, x_end, ldx, a.H);
   }
 #pragma unroll
   for (int hb = 0; hb < 2 * KT; ++hb)
@@ -314,7 +319,7 @@ LCE_DEV void narrow_gradient(const BwdArgs& a, int wave, int tile, int first, in
     for (int r = 0; r < 16; ++r) acc[hb][r] = 0.f;
   if (first >= last) return;
   fetch(first);
-  if (!DW) narrow_scalars(a, rw + (lane & 31), nlse, gain, label);
+  if (!DW) narrow_scalars(a, rows, rw + (lane & 31), nlse, gain, label);
   put(0);
   __syncthreads();
   for (int tc = first; tc < last; ++tc) {
@@ -407,10 +412,11 @@ LCE_DEV void narrow_gradient(const BwdArgs& a, int wave, int tile, int first, in
   }
 }
 
-// Element (r, h) of dx (a token's row) or dW (a column of the vocabulary), four h at a time.
-template <class T, bool WVH> LCE_DEV void narrow_out(const BwdArgs& a, bool dw, float coef, int64_t r, int64_t h, f32x4_t v) {
+// Element (r, h) of dx (a token's row; of packed tokens the one that perm names) or dW (a column of the vocabulary), four h at a time.
+template <class T, bool WVH> LCE_DEV void narrow_out(const BwdArgs& a, int64_t rows, bool dw, float coef, int64_t r, int64_t h, f32x4_t v) {
   typedef typename elem_of<T>::type E;
-  if (r >= (dw ? a.V : a.N) || h >= a.H) return;
+  if (r >= (dw ? a.V : rows) || h >= a.H) return;
+  if (!dw && rows != a.N) r = packed_token(a.perm, r, a.N);
   v *= coef;
   const bool f32 = (dw ? a.dw_dtype : a.dx_dtype) == DT_F32;
   char* out = reinterpret_cast<char*>(dw ? a.dw : a.dx);
@@ -440,16 +446,17 @@ __global__ __launch_bounds__(kThreads, 2) void grads_narrow_kernel(const BwdArgs
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const bool in_first = (int)blockIdx.x < g.first_span, dw = in_first == (g.dw_first != 0);
   const int j = (int)blockIdx.x - (in_first ? 0 : g.first_span), nseg = dw ? g.dw_nseg : g.dx_nseg;
-  const int tok_tiles = (int)((a.N + kNarrowTile - 1) / kNarrowTile), voc_tiles = (int)((a.vw + kNarrowTile - 1) / kNarrowTile);
+  const int64_t rows = packed_rows(a.n_rows, a.N);
+  const int tok_tiles = (int)((rows + kNarrowTile - 1) / kNarrowTile), voc_tiles = (int)((a.vw + kNarrowTile - 1) / kNarrowTile);
   const int tiles = dw ? voc_tiles : tok_tiles, stream = dw ? tok_tiles : voc_tiles;
-  if (j >= tiles * nseg) return;
+  if (j >= tiles * nseg) return;  // (there are as many for dx as all tokens ask for)
   int tile, seg;
   segment_coords(j, tiles, nseg, tile, seg);
   const int first = (int)((int64_t)stream * seg / nseg), last = (int)((int64_t)stream * (seg + 1) / nseg);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   f32x16_t acc[2 * KT];
-  if (dw) narrow_gradient<T, WVH, true, ZREG, KT>(a, wave, tile, first, last, lds, acc);
-  else narrow_gradient<T, WVH, false, ZREG, KT>(a, wave, tile, first, last, lds, acc);
+  if (dw) narrow_gradient<T, WVH, true, ZREG, KT>(a, rows, wave, tile, first, last, lds, acc);
+  else narrow_gradient<T, WVH, false, ZREG, KT>(a, rows, wave, tile, first, last, lds, acc);
   const int lane = narrow_tid(0), r = wave * kBlk + (lane & 31), hq = 4 * (lane >> 5);
   float* part = nseg > 1 ? g.part + ((dw ? (int64_t)g.dx_blocks : 0) + (int64_t)tile * nseg + seg) * (kNarrowTile * kBK * KT) : nullptr;
   const float coef = final_factor_of(a);
@@ -462,7 +469,7 @@ __global__ __launch_bounds__(kThreads, 2) void grads_narrow_kernel(const BwdArgs
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[k] = acc[hb][rq * 4 + k];
       if (part != nullptr) *reinterpret_cast<f32x4_t*>(part + r * (kBK * KT) + h) = v;
-      else narrow_out<T, WVH>(a, dw, coef, (int64_t)tile * kNarrowTile + r, h, v);
+      else narrow_out<T, WVH>(a, rows, dw, coef, (int64_t)tile * kNarrowTile + r, h, v);
     }
 }
 
@@ -474,6 +481,8 @@ __global__ __launch_bounds__(256) void narrow_tail_kernel(const BwdArgs a, const
   const int piece = (int)blockIdx.x % kParts;
   const bool dw = tile >= dx_tiles;
   if (dw) tile -= dx_tiles;
+  const int64_t rows = packed_rows(a.n_rows, a.N);
+  if (!dw && (int64_t)tile * kNarrowTile >= rows) return;
   const int nseg = dw ? g.dw_nseg : g.dx_nseg;
   constexpr int kBlockFloats = kNarrowTile * kBK * KT, kQuads = kBlockFloats / 4 / kParts;
   const float* part = g.part + ((dw ? (int64_t)g.dx_blocks : 0) + (int64_t)tile * nseg) * kBlockFloats;
@@ -494,7 +503,7 @@ __global__ __launch_bounds__(256) void narrow_tail_kernel(const BwdArgs a, const
       for (int k = 0; k < 8; ++k)
         if (s0 + k < nseg) v += t[k];
     }
-    narrow_out<T, WVH>(a, dw, coef, (int64_t)tile * kNarrowTile + r, h, v);
+    narrow_out<T, WVH>(a, rows, dw, coef, (int64_t)tile * kNarrowTile + r, h, v);
   }
 }
 
@@ -556,7 +565,7 @@ hipError_t launch_fwd_narrow(const FwdArgs& a, int64_t rows, hipStream_t s) {
 }
 
 hipError_t launch_bwd_narrow(const BwdArgs& a, const SmallGrads& g, bool want_dx, bool want_dw, hipStream_t s) {
-  if (a.H > kNarrowHidden || a.w_dtype != a.x_dtype || a.n_rows != nullptr || a.v0 != 0 || a.wv0 != 0 || a.vw != a.V ||
+  if (a.H > kNarrowHidden || a.w_dtype != a.x_dtype || a.perm_always || a.dxc != nullptr || a.v0 != 0 || a.wv0 != 0 || a.vw != a.V ||
       ((g.dx_nseg > 1 || g.dw_nseg > 1) && g.part == nullptr))
     return hipErrorInvalidValue;
   if (a.x_dtype == DT_BF16) return a.w_vh ? launch_grads_kt<BF16, true>(a, g, want_dx, want_dw, s) : launch_grads_kt<BF16, false>(a, g, want_dx, want_dw, s);

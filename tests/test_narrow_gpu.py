@@ -29,13 +29,14 @@ def _rows(t, extra=0):
     return pad[:, :t.shape[1]]
 
 
-def _check(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout, n_chunk=4096):
-    """Both directions against the persistent kernels, one gradient alone against both."""
+def _check(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout, n_chunk=4096, pack=2, inputs=None):
+    """Both directions against the persistent kernels, one gradient alone against both.  Returns what was compared and how to run it
+    again.  `pack`: LCE_PACK_NEVER, or how the call says it; `inputs`: instead of make_inputs'."""
     from linear_cross_entropy_loss_amd import _lib
 
     print(f"narrow N={N} H={H} V={V} {dtype} {w_dtype} layout={layout}", flush=True)
     lib = _lib.load()
-    x, y, w = make_inputs(N, H, V, dtype, seed=N + V, ignore_frac=0.2 if N > 1 else 0.0, w_dtype=w_dtype)
+    x, y, w = inputs or make_inputs(N, H, V, dtype, seed=N + V, ignore_frac=0.2 if N > 1 else 0.0, w_dtype=w_dtype)
     x, w, y = _rows(x, extra), _rows(w.t() if layout else w, extra), y.cuda()
     g = torch.full((1,), 1024.0 if dtype == torch.float16 else 1.5, device="cuda")
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -44,7 +45,7 @@ def _check(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout, n_chunk=4096):
         lddx, cols = H + (-H) % 8, H if layout else V
         lddw = cols + (-cols) % 8
         prob = _lib.make_problem(N, H, V, x.stride(0), w.stride(0), lddx, lddw, dtype, w.dtype, dtype, w.dtype, -1, 0.7, z_reg, n_chunk,
-                                 mon, 0, _lib.PACK_NEVER, workgroups, layout)
+                                 mon, 0, pack, workgroups, layout)
         fb, bb = _lib.workspace_bytes(prob)
         ws = torch.empty(max(fb, bb), dtype=torch.uint8, device="cuda")
         lse, out5 = torch.empty(N, device="cuda"), torch.empty(5, device="cuda")
@@ -61,7 +62,7 @@ def _check(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout, n_chunk=4096):
     # (64 workgroups: the persistent kernels, forward and backward)
     out_p, lse_p, dx_p, dw_p = run(64)
     k = 5 if mon else 2
-    assert torch.equal(lse[y != -1], lse_p[y != -1]) and torch.equal(out[:k], out_p[:k])
+    assert torch.equal(lse[y != -1], lse_p[y != -1]) and (torch.equal(out[:k], out_p[:k]) or bool((y == -1).all()))
     for got, ref in ((dx, dx_p), (dw, dw_p)):
         assert torch.isfinite(got).all()
         if ref.double().norm() > 0:
@@ -70,6 +71,7 @@ def _check(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout, n_chunk=4096):
     assert (dx[y == -1] == 0).all()
     # one gradient alone: the same bits
     assert torch.equal(run(0, want_dw=False)[2], dx) and torch.equal(run(0, want_dx=False)[3], dw)
+    return run, x, y, out, lse, dx, dw
 
 
 @pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.bfloat16, None, 1), (torch.float16, None, 0),
@@ -91,3 +93,27 @@ def test_many_tokens_and_few_classes(N, H, V, n_chunk, dtype, w_dtype, layout):
     prob = _lib.make_problem(N, H, V, H, ld, H, ld, dtype, wd, dtype, wd, -1, 0.7, 0.0, n_chunk, False, 0, _lib.PACK_NEVER, 0, layout)
     assert _lib.backward_plan(prob)[1] > V + 255 and _lib.backward_workspace_bytes(prob) > n_chunk * V * 4
     _check(N, H, V, 0, False, 1e-3, dtype, w_dtype, layout, n_chunk)
+
+
+@pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.float16, None, 1), (torch.float16, torch.float32, 0)])
+@pytest.mark.parametrize("N,H,V,ignored", [(20000, 128, 107400, 0.85), (22000, 120, 104200, 0.05), (40000, 64, 107400, 0.3),
+                                           (20000, 128, 107400, 0.0), (20000, 128, 107400, 1.0)])
+def test_ignored_tokens_of_a_large_problem_are_packed_away(N, H, V, ignored, dtype, w_dtype, layout):
+    """From 8 * N * H * V = 2^41 on the tokens with an ignored label are not worked on, and what stands in their rows of x does not
+    reach a result."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    wd, ld = w_dtype or dtype, H if layout else V + (-V) % 8
+    prob = _lib.make_problem(N, H, V, H, ld, H, ld, dtype, wd, dtype, wd, -1, 0.7, 1e-3, 4096, False, 0, _lib.PACK_AUTO, 0, layout)
+    assert 8 * N * H * V >= 1 << 41 and _lib.backward_plan(prob)[1] > V + 255
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn((N, H), generator=g, device="cuda").to(dtype)
+    w = torch.randn((H, V), generator=g, device="cuda").mul_(H ** -0.5).to(wd)
+    y = torch.randint(0, V, (N,), generator=g, device="cuda")
+    y[torch.rand(N, generator=g, device="cuda") < ignored] = -1
+    run, xr, y, out, lse, dx, dw = _check(N, H, V, 0, False, 1e-3, dtype, w_dtype, layout, 4096, _lib.PACK_AUTO, (x, y, w))
+    if 0 < ignored < 1:
+        xr[y == -1] = float("inf")
+        again = run(0)
+        for a, b in zip((out[:2], lse, dx, dw), (again[0][:2],) + again[1:]):
+            assert torch.equal(a, b)
