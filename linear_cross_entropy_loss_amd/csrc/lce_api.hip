@@ -260,8 +260,8 @@ double kernel_cost(double T, double L, double e, bool parts, bool settled) {
 // Vocabulary slabs (of a width that is a multiple of 256 columns; the last one may be narrower) whose staging
 // fits the scratch bound: the fewest that fit, or somewhat more of them when a model of the three kernels'
 // rounds of workgroups says that those run faster (slab_cost below).  The dz stage itself is additionally
-// capped at 1 GiB: wider slabs are not faster, so a generous N_chunk_size does not translate into a larger
-// footprint.
+// capped at 1 GiB (kStageCap): wider slabs are not faster, so a generous N_chunk_size does not translate into a larger
+// footprint of this call.  (lce_forward_backward's chunks of token rows are as long as pays, see there.)
 //
 // The bound is n_chunk * V * 4 bytes, what the reference spends on its logits
 // chunk (ops.py:700).  Everything counts towards it: the dz stage, the fp32 running dx, the packed rows and
@@ -273,6 +273,7 @@ double kernel_cost(double T, double L, double e, bool parts, bool settled) {
 // N * H * 4 bytes, the fp32 x_grad buffer the reference allocates next to its logits chunk (ops.py:693) and
 // this library does not -- and by the split-K partial sums.  If even that fails, the narrowest split is used:
 // the bound is a target, the operator never refuses a shape.
+constexpr size_t kStageCap = (size_t)1 << 30;
 bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved);
 int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
   BwdPlan narrow;
@@ -286,7 +287,6 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
     return LCE_OK;
   }
   memset(b, 0, sizeof(*b));
-  const size_t dz_cap = (size_t)1 << 30;
   const size_t Np = (size_t)lce::padded_tokens(p->N), Hp = (size_t)lce::padded_hidden(p->H);
   const int64_t Vp = lce::padded_vocab(p->V);
   const int64_t cols = Vp / 256;
@@ -344,7 +344,7 @@ int make_plan_bwd(const lce_problem* p, BwdPlan* b, bool settled) {
     // the widened bound is for the staging proper; the split-K partial sums (at most 64 MiB, shared by dx
     // and dW) and the packed rows come on top of it there
     const size_t counted = dz + acc + w16 + (mode != 2 ? fixed + part + reserve : 0);
-    if (!((counted <= budget && (dz <= dz_cap || vs == 256)) || (mode == 2 && vs == 256))) return false;
+    if (!((counted <= budget && (dz <= kStageCap || vs == 256)) || (mode == 2 && vs == 256))) return false;
     out->slabs = slabs;
     out->vs = vs;
     out->pack_on = pack;
@@ -561,6 +561,14 @@ int make_plan_fused(const lce_problem* p, FusedPlan* f) {
 // LCE_ROUTE_KEEP_LOGITS: chunks of token rows whose fp32 logits stay in the stage until their rows' lse are known.  Against two passes
 // a contraction (three products of bf16 pairs) is saved for 8 bytes of memory traffic per logit, and the weight is split into pairs
 // once and not twice; what it needs is room for all of that copy.
+// Long chunks are not faster beyond some length, and a stage far outside the caches costs more than the model says.  ms, kept (rows
+// of a chunk) / two passes, and the ratio by the model: N=4096, H=256, V=2^20 28.0 (2048) / 25.0 (0.93); N=8192, H=256, V=262144
+// 12.8 (4096), 12.7 (2816), 13.0 (2048) / 12.4 (0.94); N=11488, H=208, V=57592 3.91 (5888) / 4.03 (0.92); N=4400, H=208, V=169328
+// 4.75 (2304) / 4.49 (0.97); N=8192, H=1024, V=262144 34.6 (4096), 35.1 (2816), 36.6 (1280) / 40.2 (0.81 to 0.86); N=32768, H=512,
+// V=65536 19.5 (16384), 19.4 (8192), 19.7 (4096) / 21.4 (0.86); N=19592, H=2432, V=95640 74.5 (5120), 73.4 (2816).  So above kStageCap,
+// the staged backward's limit, chunks have to be half a per cent faster by the model for every GiB of their stage, and 8 % ahead of
+// two passes, which need less.
+constexpr double kKeptMargin = 0.92;
 bool plan_kept(const lce_problem* p, FusedPlan* f) {
   memset(f, 0, sizeof(*f));
   if (!(p->route & LCE_ROUTE_KEEP_LOGITS) || route_of(p) == LCE_ROUTE_TWO_PASS) return false;
@@ -585,9 +593,11 @@ bool plan_kept(const lce_problem* p, FusedPlan* f) {
     return (a < b ? a : b) / kUnitUs;
   };
   int64_t first = 0;
+  size_t stage = 0;   // of the plan so far
+  double least = 0;   // cost of the fastest so far
   for (int64_t t = tiles; t >= 1; --t) {
     const int64_t chunks = (tiles + t - 1) / t;
-    if (chunks > kMostChunks || (first != 0 && chunks > 2 * first + 4)) break;
+    if (chunks > kMostChunks || (first != 0 && chunks > 2 * first + 4 && stage <= kStageCap)) break;
     if (t < tiles && (tiles + t) / (t + 1) == chunks) continue;  // a longer chunk gives the same number of chunks
     const int64_t even = (tiles + chunks - 1) / chunks, nc = even * 256, last = tiles - (chunks - 1) * even;
     FusedPlan c = *f;
@@ -637,7 +647,10 @@ bool plan_kept(const lce_problem* p, FusedPlan* f) {
     cost += (double)(chunks - 1) * logits(nc) + logits(p->N - (chunks - 1) * nc) + 12.0 * (double)chunks +
             (double)Np * (double)Vp * 8.0 / 8.0e6 + (double)p->H * (double)Vp * 8.0 / 8.0e6;
     if (first == 0) first = chunks;
-    if (f->ok && cost >= f->cost) continue;
+    const double worth = 1.0 + 0.005 * (double)stage / (double)kStageCap;
+    if (f->ok && cost >= f->cost && !(stage > kStageCap && cost <= (worth < 1.05 ? worth : 1.05) * least)) continue;
+    if (!f->ok || cost < least) least = cost;
+    stage = c.part - c.stage;
     c.total = m + (c.small ? (size_t)(c.small_blocks * lce::kSmallBlockBytes) : c.parts_on ? parts : 0);
     c.nc = nc;
     c.chunks = (int)chunks;
@@ -649,7 +662,7 @@ bool plan_kept(const lce_problem* p, FusedPlan* f) {
   BwdPlan b;
   if (route_of(p) == LCE_ROUTE_AUTO && plan_bwd(p, &b) == LCE_OK) {
     const double two = logits(p->N) + b.cost + 12.0 + (double)p->H * (double)Vp * 16.0 / 8.0e6;
-    if (f->cost > kBytesMargin * two) f->ok = false;
+    if (f->cost > (stage > kStageCap ? kKeptMargin : kBytesMargin) * two) f->ok = false;
   }
   return f->ok;
 }

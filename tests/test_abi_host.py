@@ -465,6 +465,28 @@ def test_narrow_plan_has_room_for_its_sums_or_is_not_taken():
     assert plan(4096, 128, 50000, 128, torch.float32)[0] and plan(16384, 128, 1000, 4096)[0]
 
 
+def test_kept_logits_do_not_take_all_the_bound_allows():
+    """fp32 tensors: chunks beyond a stage of 1 GiB are no longer than pays, whatever the bound allows, and where they do not pay the
+    logits are not kept."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    f32 = torch.float32
+
+    def plan(N, H, V, n_chunk, route=_lib.ROUTE_AUTO):
+        p = _prob(N=N, H=H, V=V, ldx=H, ldw=V, lddx=H, lddw=V, n_chunk=n_chunk, x_dtype=f32, w_dtype=f32, dx_dtype=f32, dw_dtype=f32,
+                  route=route | _lib.ROUTE_KEEP_LOGITS)
+        return _lib.forward_backward_plan(p), _lib.forward_backward_workspace_bytes(p)
+
+    for V in (262144, 1 << 20, 1 << 22):
+        (chunks, _), size = plan(8192, 256, V, 4096)
+        assert chunks == 0 and size <= 3 << 29, (V, chunks, size)
+    for N, H, V, most in ((19592, 2432, 95640, 3), (65536, 1024, 32768, 2), (65536, 512, 131072, 4)):  # (GiB of stage)
+        (chunks, rows), size = plan(N, H, V, 65536)
+        assert chunks > 1 and rows * V * 4 <= most << 30 and size <= rows * V * 4 + H * V * 4 + (1 << 30), (N, H, V, chunks, rows, size)
+    # where a chunk of all tokens stays below that, it is taken as before
+    assert plan(2048, 2048, 16384, 8192)[0] == (1, 2048)
+
+
 def test_kept_logits_plan_keeps_the_pairs_of_the_weight_within_32_bit_offsets():
     """fp32 tensors, logits kept: the weight's bf16 pairs have rows as wide as the vocabulary, of which the kernels reach 256 by
     32-bit offsets.  Rows of more than 8 MiB take two passes, in slabs whose rows are shorter."""
