@@ -322,8 +322,10 @@ def _native_forward(x_in, y, At, ignore_index, z_regularization, logit_scale, N_
     device = x_in.device
     if device.type != "cuda" or device.index != torch._C._cuda_getDevice():
         return None
-    done = _lib.host().forward(x_in, y, At, ignore_index, z_regularization, logit_scale, N_chunk_size, monitoring, pack, _route_mode(),
-                               exact_dw_sums.get(), need_dx, need_dw, "weight" in _copy_warned, _stream(device))
+    # (numbers as make_problem takes them: whoever applies the Function itself may pass 4096.0 for a size)
+    done = _lib.host().forward(x_in, y, At, int(ignore_index), float(z_regularization), float(logit_scale), int(N_chunk_size),
+                               bool(monitoring), pack, _route_mode(), bool(exact_dw_sums.get()), need_dx, need_dw,
+                               "weight" in _copy_warned, _stream(device))
     if done is not None and len(done) == 2:
         _lib.raise_for_status(*done)
     return done
@@ -392,8 +394,8 @@ def _backward_impl(x, y1, w, lse, n_valid, grad_output, ignore_index, z_regulari
     vh = layout == _lib.W_VH
     if x.device.index == torch._C._cuda_getDevice():
         g = _device_scalar(grad_output, x.device)
-        done = _lib.host().backward(x, y1, w, lse, n_valid, g, ignore_index, z_regularization, logit_scale, N_chunk_size, need_dx,
-                                    need_dw, pack, layout, _stream(x.device))
+        done = _lib.host().backward(x, y1, w, lse, n_valid, g, int(ignore_index), float(z_regularization), float(logit_scale),
+                                    int(N_chunk_size), need_dx, need_dw, pack, layout, _stream(x.device))
         if done is not None:
             if len(done) == 3:
                 _lib.raise_for_status(*done[:2])

@@ -111,3 +111,26 @@ def test_errors_are_those_of_the_operators_own_host_code(what, monkeypatch):
             linear_cross_entropy(x, y, w, -100, 0.0, -1.0 if what == "scale" else 1.0, 4096)
         said.append((type(e.value), str(e.value)))
     assert said[0] == said[1]
+
+
+@pytest.mark.parametrize("always", [False, True])
+def test_numbers_of_any_kind_for_the_function_itself(always):
+    """linear_cross_entropy converts its numbers; the autograd Function takes them as they come."""
+    import numpy as np
+
+    from linear_cross_entropy_loss_amd import ops
+
+    x = _mat(N, H, torch.bfloat16, 1).requires_grad_(True)
+    w = _mat(H, V, torch.bfloat16, 2).requires_grad_(True)
+    y = torch.randint(0, V, (N,), generator=torch.Generator().manual_seed(3)).cuda()
+    ops.one_pass.set("always" if always else False)
+
+    def run(*numbers):
+        out = ops.LinearXentImplementation.apply(x, y, w, *numbers)
+        return [o.detach() for o in out] + list(torch.autograd.grad(out[0], (x, w)))
+
+    plain = run(-100, 1e-4, 0.5, 4096, True)
+    for numbers in ((-100.0, np.float64(1e-4), np.float32(0.5), 4096.0, 1),
+                    (torch.tensor(-100), torch.tensor(1e-4), torch.tensor(0.5), np.int64(4096), np.bool_(True))):
+        for a, b in zip(plain, run(*numbers)):
+            assert torch.allclose(a, b, rtol=1e-6)
