@@ -408,7 +408,7 @@ def main():
         from pathlib import Path
 
         _lib.LIB_PATH = Path(args.library).resolve()
-    if not _lib.LIB_PATH.exists():  # normally built beforehand and shipped with the tree
+    if not _lib.is_built():  # normally built beforehand and shipped with the tree
         from linear_cross_entropy_loss_amd.build import build
 
         build(force=True)

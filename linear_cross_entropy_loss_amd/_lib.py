@@ -76,6 +76,11 @@ class LceProblem(ctypes.Structure):
 _lib = None
 
 
+def is_built() -> bool:
+    """Whether both libraries that a call needs are there: the kernels' and the host path's."""
+    return LIB_PATH.exists() and HOST_LIB_PATH.exists()
+
+
 def load():
     """Load the shared library; raises if it has not been built."""
     global _lib

@@ -15,10 +15,10 @@ def pytest_configure(config):
 
 
 def pytest_sessionstart(session):
-    """Load what is built; compile the library only when there is none (hipcc cross-compiles without a GPU)."""
+    """Load what is built; compile the libraries only when one is missing (hipcc cross-compiles without a GPU)."""
     from linear_cross_entropy_loss_amd import _lib
 
-    if not _lib.LIB_PATH.exists():
+    if not _lib.is_built():
         from linear_cross_entropy_loss_amd.build import build
 
         build(force=True)

@@ -720,6 +720,20 @@ def _kernel_notes(path, tmp_path):
     return found
 
 
+def test_a_tree_with_one_of_the_two_libraries_is_not_built(tmp_path, monkeypatch):
+    """Every eager call goes through both; what builds on demand (the tests, the benchmark) has to look for both."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    assert _lib.is_built()
+    for name in ("LIB_PATH", "HOST_LIB_PATH"):
+        with monkeypatch.context() as m:
+            m.setattr(_lib, name, tmp_path / "missing.so")
+            assert not _lib.is_built()
+    for path in ("tests/conftest.py", "__graft_entry__.py", "bench.py"):
+        with open(os.path.join(ROOT, path)) as f:
+            assert "_lib.is_built()" in f.read(), path
+
+
 def test_no_kernel_keeps_registers_in_memory(lib, tmp_path):
     """Every kernel's registers fit: none has private memory for spilled ones, which would put memory round trips into
     loops whose loads are counted."""
