@@ -202,6 +202,23 @@ int lce_workspace_bytes(const lce_problem* p, size_t* fwd_bytes, size_t* bwd_byt
 int lce_backward_plan(const lce_problem* p, int64_t* slabs, int64_t* slab_width);
 
 /*
+ * Testing and profiling aid: which kernels form the gradients of problem `p` -- in lce_backward, or (one_pass != 0) on the one-pass
+ * route of lce_forward_backward -- and how the first slab's (chunk's) sums along K are cut.  Host side only.  From version 901 on.
+ *   kernels     LCE_GRADS_LARGE (256 x 256 tiles, persistent), LCE_GRADS_SMALL (128 x 128 tiles, dx and dW in one launch),
+ *               LCE_GRADS_NARROW (nothing staged), LCE_GRADS_NONE: no such plan
+ *   dx_cuts, dw_cuts  stretches of K to a tile, 1 where it is not cut (LARGE: 0, which tiles are cut is decided on the device)
+ *   dx_workgroups     LARGE: workgroups of the dx kernel where the scratch allows fewer than one to a compute unit, else 0
+ */
+enum {
+  LCE_GRADS_NONE = -1,
+  LCE_GRADS_LARGE = 0,
+  LCE_GRADS_SMALL = 1,
+  LCE_GRADS_NARROW = 2
+};
+int lce_gradient_kernels(const lce_problem* p, int32_t one_pass, int32_t* kernels, int32_t* dx_cuts, int32_t* dw_cuts,
+                         int32_t* dx_workgroups);
+
+/*
  * Forward.  Replaces the launch of linear_xent_fwd_prep_bwd_kernel_matmul_t
  * (ops.py:722-752) and the torch reductions around it (ops.py:705, 753-761,
  * 793-794, 802), without ever writing logits to memory.

@@ -17,6 +17,7 @@ PACK_AUTO, PACK_ALWAYS, PACK_NEVER = 0, 1, 2
 ROUTE_AUTO, ROUTE_ONE_PASS, ROUTE_TWO_PASS = 0, 1, 2  # lce_problem.route (lce_forward_backward)
 ROUTE_EXACT_SUMS = 4  # a flag for the same field: dW's sums over chunks never at fewer than 32 bits
 ROUTE_KEEP_LOGITS = 16  # another, for fp32 activations: the logits computed once and kept in fp32
+GRADS_NONE, GRADS_LARGE, GRADS_SMALL, GRADS_NARROW = -1, 0, 1, 2  # gradient_kernels
 W_HV, W_VH = 0, 1  # lce_problem.w_layout: weight stored (H, V) / (V, H) row-major
 LCE_EINVAL_SHAPE, LCE_EINVAL_DTYPE, LCE_EINVAL_ARG, LCE_EWORKSPACE, LCE_EHIP, LCE_ESTATIC = -1, -2, -3, -4, -5, -6
 STATIC_SCRATCH_BYTES = 64 << 20
@@ -28,6 +29,7 @@ EXPORTS = (
     "lce_check_problem",
     "lce_workspace_bytes",
     "lce_backward_plan",
+    "lce_gradient_kernels",
     "lce_forward",
     "lce_forward_static",
     "lce_backward",
@@ -107,6 +109,8 @@ def load():
     lib.lce_workspace_bytes.argtypes = [P, ctypes.POINTER(sz), ctypes.POINTER(sz)]
     lib.lce_backward_plan.restype = ctypes.c_int
     lib.lce_backward_plan.argtypes = [P, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)]
+    lib.lce_gradient_kernels.restype = ctypes.c_int
+    lib.lce_gradient_kernels.argtypes = [P, ctypes.c_int32] + [ctypes.POINTER(ctypes.c_int32)] * 4
     lib.lce_forward.restype = ctypes.c_int
     lib.lce_forward.argtypes = [P, vp, vp, vp, vp, vp, vp, vp, sz, vp]
     lib.lce_forward_static.restype = ctypes.c_int
@@ -222,6 +226,13 @@ def backward_plan(prob: LceProblem) -> tuple[int, int]:
     n, w = ctypes.c_int64(0), ctypes.c_int64(0)
     raise_for_status(lib.lce_backward_plan(ctypes.byref(prob), ctypes.byref(n), ctypes.byref(w)), "lce_backward_plan")
     return int(n.value), int(w.value)
+
+
+def gradient_kernels(prob: LceProblem, one_pass: bool = False) -> tuple[int, int, int, int]:
+    """(GRADS_*, cuts of dx, cuts of dW, limit of dx's workgroups) of lce_backward or of the one-pass route (lce.h)."""
+    out = [ctypes.c_int32(0) for _ in range(4)]
+    raise_for_status(load().lce_gradient_kernels(ctypes.byref(prob), int(one_pass), *map(ctypes.byref, out)), "lce_gradient_kernels")
+    return tuple(v.value for v in out)
 
 
 def forward_backward_workspace_bytes(prob: LceProblem) -> int:

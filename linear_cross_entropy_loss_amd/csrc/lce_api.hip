@@ -1129,7 +1129,7 @@ int fused_impl(const lce_problem* p, const FusedPlan& f, const void* x, const vo
 
 extern "C" {
 
-int lce_version(void) { return 900; }  // 0.9.0: LCE_ROUTE_KEEP_LOGITS
+int lce_version(void) { return 901; }  // 0.9.1: lce_gradient_kernels
 
 const char* lce_strerror(int status) {
   switch (status) {
@@ -1178,6 +1178,35 @@ int lce_backward_plan(const lce_problem* p, int64_t* slabs, int64_t* slab_width)
   if (rc != LCE_OK) return rc;
   if (slabs) *slabs = b.slabs;
   if (slab_width) *slab_width = b.vs;
+  return LCE_OK;
+}
+
+int lce_gradient_kernels(const lce_problem* p, int32_t one_pass, int32_t* kernels, int32_t* dx_cuts, int32_t* dw_cuts,
+                         int32_t* dx_workgroups) {
+  int rc = check(p, true);
+  if (rc != LCE_OK) return rc;
+  int kind = LCE_GRADS_NONE, workgroups = 0;
+  lce::SmallGrads g;
+  memset(&g, 0, sizeof(g));
+  if (one_pass) {
+    FusedPlan f;
+    if (plan_fused(p, &f)) {
+      kind = f.small ? LCE_GRADS_SMALL : LCE_GRADS_LARGE;
+      workgroups = f.dx_grid;
+      if (f.small) g = lce::plan_small_grads(p->N < f.nc ? p->N : f.nc, p->H, p->V, products(p), f.small_blocks);
+    }
+  } else {
+    BwdPlan b;
+    rc = plan_bwd(p, &b);
+    if (rc != LCE_OK) return rc;
+    kind = b.narrow ? LCE_GRADS_NARROW : b.small ? LCE_GRADS_SMALL : LCE_GRADS_LARGE;
+    if (b.narrow) g = lce::plan_narrow_grads(p->N, p->H, p->V, b.small_blocks);
+    else if (b.small) g = lce::plan_small_grads(p->N, p->H, p->V < b.vs ? p->V : b.vs, products(p), b.small_blocks);
+  }
+  if (kernels) *kernels = kind;
+  if (dx_cuts) *dx_cuts = g.dx_nseg;
+  if (dw_cuts) *dw_cuts = g.dw_nseg;
+  if (dx_workgroups) *dx_workgroups = workgroups;
   return LCE_OK;
 }
 

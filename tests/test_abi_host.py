@@ -440,6 +440,29 @@ def test_narrow_plan_keeps_the_copy_of_an_fp32_weight_within_32_bit_offsets(H, w
     assert plan(4194304, torch.bfloat16) == (1, 4194304 + 256)
 
 
+def test_gradient_kernels_names_what_the_plans_choose(lib):
+    from linear_cross_entropy_loss_amd import _lib
+
+    f32 = torch.float32
+
+    def kernels(N, H, V, n_chunk=4096, one_pass=False, dt=torch.bfloat16, **kw):
+        return _lib.gradient_kernels(_prob(N=N, H=H, V=V, ldx=H, ldw=V, lddx=H, lddw=V, n_chunk=n_chunk, x_dtype=dt, w_dtype=dt,
+                                           dx_dtype=dt, dw_dtype=dt, **kw), one_pass)
+
+    assert kernels(16384, 2048, 131072)[0] == _lib.GRADS_LARGE
+    assert kernels(16384, 2048, 131072, one_pass=True) == (_lib.GRADS_LARGE, 0, 0, 0)
+    kind, dx, dw, _ = kernels(300, 520, 9000)
+    assert kind == _lib.GRADS_SMALL and dx > 1 and dw == 1
+    assert kernels(300, 520, 9000, max_workgroups=64)[0] == _lib.GRADS_LARGE
+    assert kernels(300, 128, 9000)[0] == _lib.GRADS_NARROW
+    assert kernels(300, 128, 9000, one_pass=True)[0] == _lib.GRADS_NONE
+    keep = dict(dt=f32, one_pass=True, route=_lib.ROUTE_KEEP_LOGITS)
+    assert kernels(2048, 2048, 16384, **keep)[0] == _lib.GRADS_LARGE and kernels(700, 300, 5000, **keep)[0] == _lib.GRADS_SMALL
+    bad = _prob(N=0)
+    assert lib.lce_gradient_kernels(ctypes.byref(bad), 0, None, None, None, None) == _lib.LCE_EINVAL_SHAPE
+    assert lib.lce_gradient_kernels(ctypes.byref(_prob()), 0, None, None, None, None) == _lib.LCE_OK
+
+
 def test_narrow_plan_has_room_for_its_sums_or_is_not_taken():
     """Hidden sizes up to 128, nothing staged: few classes and many tokens leave the bound no room to cut the sums over the tokens, and
     one or two workgroups would walk them all.  The sums then get room on top, at most twice what a staged plan takes where that

@@ -31,7 +31,8 @@ def _rows(t, extra=0):
 
 def _check(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout, n_chunk=4096, pack=2, inputs=None):
     """Both directions against the persistent kernels, one gradient alone against both.  Returns what was compared and how to run it
-    again.  `pack`: LCE_PACK_NEVER, or how the call says it; `inputs`: instead of make_inputs'."""
+    again.  `pack`: LCE_PACK_NEVER, or how the call says it (LCE_PACK_ALWAYS: the backward is staged); `inputs`: instead of
+    make_inputs'."""
     from linear_cross_entropy_loss_amd import _lib
 
     print(f"narrow N={N} H={H} V={V} {dtype} {w_dtype} layout={layout}", flush=True)
@@ -46,6 +47,8 @@ def _check(N, H, V, extra, mon, z_reg, dtype, w_dtype, layout, n_chunk=4096, pac
         lddw = cols + (-cols) % 8
         prob = _lib.make_problem(N, H, V, x.stride(0), w.stride(0), lddx, lddw, dtype, w.dtype, dtype, w.dtype, -1, 0.7, z_reg, n_chunk,
                                  mon, 0, pack, workgroups, layout)
+        if workgroups == 0 and pack != _lib.PACK_ALWAYS:
+            assert _lib.gradient_kernels(prob)[0] == _lib.GRADS_NARROW
         fb, bb = _lib.workspace_bytes(prob)
         ws = torch.empty(max(fb, bb), dtype=torch.uint8, device="cuda")
         lse, out5 = torch.empty(N, device="cuda"), torch.empty(5, device="cuda")
@@ -91,8 +94,17 @@ def test_many_tokens_and_few_classes(N, H, V, n_chunk, dtype, w_dtype, layout):
 
     wd, ld = w_dtype or dtype, H if layout else V + (-V) % 8
     prob = _lib.make_problem(N, H, V, H, ld, H, ld, dtype, wd, dtype, wd, -1, 0.7, 0.0, n_chunk, False, 0, _lib.PACK_NEVER, 0, layout)
-    assert _lib.backward_plan(prob)[1] > V + 255 and _lib.backward_workspace_bytes(prob) > n_chunk * V * 4
+    assert _lib.gradient_kernels(prob)[2] > 1 and _lib.backward_workspace_bytes(prob) > n_chunk * V * 4
     _check(N, H, V, 0, False, 1e-3, dtype, w_dtype, layout, n_chunk)
+
+
+def _on_device(N, H, V, dtype, w_dtype, ignored):
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn((N, H), generator=g, device="cuda").to(dtype)
+    w = torch.randn((H, V), generator=g, device="cuda").mul_(H ** -0.5).to(w_dtype or dtype)
+    y = torch.randint(0, V, (N,), generator=g, device="cuda")
+    y[torch.rand(N, generator=g, device="cuda") < ignored] = -1
+    return x, y, w
 
 
 @pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.float16, None, 1), (torch.float16, torch.float32, 0)])
@@ -103,17 +115,34 @@ def test_ignored_tokens_of_a_large_problem_are_packed_away(N, H, V, ignored, dty
     reach a result."""
     from linear_cross_entropy_loss_amd import _lib
 
-    wd, ld = w_dtype or dtype, H if layout else V + (-V) % 8
-    prob = _lib.make_problem(N, H, V, H, ld, H, ld, dtype, wd, dtype, wd, -1, 0.7, 1e-3, 4096, False, 0, _lib.PACK_AUTO, 0, layout)
-    assert 8 * N * H * V >= 1 << 41 and _lib.backward_plan(prob)[1] > V + 255
-    g = torch.Generator(device="cuda").manual_seed(N)
-    x = torch.randn((N, H), generator=g, device="cuda").to(dtype)
-    w = torch.randn((H, V), generator=g, device="cuda").mul_(H ** -0.5).to(wd)
-    y = torch.randint(0, V, (N,), generator=g, device="cuda")
-    y[torch.rand(N, generator=g, device="cuda") < ignored] = -1
-    run, xr, y, out, lse, dx, dw = _check(N, H, V, 0, False, 1e-3, dtype, w_dtype, layout, 4096, _lib.PACK_AUTO, (x, y, w))
+    assert 8 * N * H * V >= 1 << 41
+    run, xr, y, out, lse, dx, dw = _check(N, H, V, 0, False, 1e-3, dtype, w_dtype, layout, 4096, _lib.PACK_AUTO,
+                                          _on_device(N, H, V, dtype, w_dtype, ignored))
     if 0 < ignored < 1:
         xr[y == -1] = float("inf")
         again = run(0)
         for a, b in zip((out[:2], lse, dx, dw), (again[0][:2],) + again[1:]):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.float16, torch.float32, 1)])
+@pytest.mark.parametrize("N,H,V", [(1000, 72, 1300), (129, 24, 5001), (20000, 64, 300)])
+def test_forward_of_packed_rows(N, H, V, dtype, w_dtype, layout):
+    """The forward on the rows that are left; the last case in two chunks of tokens."""
+    from linear_cross_entropy_loss_amd import _lib
+
+    _check(N, H, V, 0, False, 1e-3, dtype, w_dtype, layout, 4096, _lib.PACK_ALWAYS)
+
+
+@pytest.mark.parametrize("mon", [False, True])
+@pytest.mark.parametrize("N", [16385, 40000])
+def test_several_chunks_of_tokens(N, mon):
+    """The forward goes through 16384 tokens at a time."""
+    _check(N, 40, 260, 0, mon, 0.0, torch.bfloat16, None, 0, 65536 // 8)
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+def test_forward_on_slabs_of_an_fp32_weight(layout):
+    """Its copies of an fp32 weight are 256 MiB at most: here two, the second one 300 columns wide."""
+    _check(300, 128, (1 << 20) + 300, 0, False, 1e-3, torch.bfloat16, torch.float32, layout,
+           inputs=_on_device(300, 128, (1 << 20) + 300, torch.bfloat16, torch.float32, 0.1))

@@ -3,7 +3,9 @@ limits its workgroups, on the same staged dz.
 
 The two add the same products in another order: fp32 sums that differ by rounding, which moves a 16-bit result by at most one
 unit in the last place (2^-7 of a bf16 number, 2^-10 of an fp16 one) and only where a sum lies next to a boundary.  In the 2-norm
-that stays below a quarter of such a unit; fp32 results (sums of up to 5000 products) stay within 5000^0.5 * 2^-24 * 2, 1e-5."""
+that stays below a quarter of such a unit; fp32 results (sums of up to n products) stay within n^0.5 * 2^-24 * 2, 1e-5 up to 7000.
+
+(Hidden sizes up to 128 in 16 bits have kernels of their own, lce_narrow.hip: test_gradients_on_small_tiles holds those to the same.)"""
 import ctypes
 
 import pytest
@@ -27,12 +29,9 @@ def _rows(t):
     return pad[:, :t.shape[1]]
 
 
-@pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.bfloat16, None, 1), (torch.float16, None, 0),
-                                                  (torch.float16, torch.float32, 0), (torch.bfloat16, torch.float32, 1),
-                                                  (torch.float32, None, 0)])
-@pytest.mark.parametrize("N,H,V,n_chunk", [(1, 8, 8, 4096), (127, 128, 128, 4096), (129, 136, 1003, 4096), (300, 1000, 260, 4096),
-                                           (700, 72, 4999, 4096), (2000, 264, 1501, 600), (5000, 64, 640, 2048)])
-def test_gradients_on_small_tiles(N, H, V, n_chunk, dtype, w_dtype, layout):
+def _check(N, H, V, n_chunk, dtype, w_dtype, layout, plan=None):
+    """Both gradients against the persistent kernels, one alone against both.  `plan`: whether there are several slabs, dx is cut along
+    K, dW is."""
     from linear_cross_entropy_loss_amd import _lib
 
     print(f"small tiles N={N} H={H} V={V} n_chunk={n_chunk} {dtype} {w_dtype} layout={layout}", flush=True)
@@ -48,6 +47,9 @@ def test_gradients_on_small_tiles(N, H, V, n_chunk, dtype, w_dtype, layout):
         lddw = cols + (-cols) % 8
         prob = _lib.make_problem(N, H, V, x.stride(0), w.stride(0), lddx, lddw, dtype, w.dtype, dtype, w.dtype, -1, 0.7, 1e-3,
                                  n_chunk, False, 0, _lib.PACK_NEVER, workgroups, layout)
+        if workgroups == 0 and plan is not None:
+            slabs, (kernels, dx_cuts, dw_cuts, _) = _lib.backward_plan(prob)[0], _lib.gradient_kernels(prob)
+            assert kernels == _lib.GRADS_SMALL and (slabs > 1, dx_cuts > 1, dw_cuts > 1) == plan, (slabs, kernels, dx_cuts, dw_cuts)
         fb, bb = _lib.workspace_bytes(prob)
         ws = torch.empty(max(fb, bb), dtype=torch.uint8, device="cuda")
         lse, out5 = torch.empty(N, device="cuda"), torch.empty(5, device="cuda")
@@ -65,7 +67,32 @@ def test_gradients_on_small_tiles(N, H, V, n_chunk, dtype, w_dtype, layout):
     for got, ref in ((dx, dx_p), (dw, dw_p)):
         assert torch.isfinite(got).all()
         if ref.double().norm() > 0:
-            assert rel_errors(got, ref)[1] <= BOUND[got.dtype]
+            longest = max(N, V) ** 0.5 * 2.0 ** -23
+            assert rel_errors(got, ref)[1] <= max(BOUND[got.dtype], longest if got.dtype == torch.float32 else 0)
     assert (dx[y == -1] == 0).all()
     # one gradient alone: the same bits
     assert torch.equal(run(0, want_dw=False)[0], dx) and torch.equal(run(0, want_dx=False)[1], dw)
+
+
+@pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.bfloat16, None, 1), (torch.float16, None, 0),
+                                                  (torch.float16, torch.float32, 0), (torch.bfloat16, torch.float32, 1),
+                                                  (torch.float32, None, 0)])
+@pytest.mark.parametrize("N,H,V,n_chunk", [(1, 8, 8, 4096), (127, 128, 128, 4096), (129, 136, 1003, 4096), (300, 1000, 260, 4096),
+                                           (700, 72, 4999, 4096), (2000, 264, 1501, 600), (5000, 64, 640, 2048)])
+def test_gradients_on_small_tiles(N, H, V, n_chunk, dtype, w_dtype, layout):
+    _check(N, H, V, n_chunk, dtype, w_dtype, layout)
+
+
+@pytest.mark.parametrize("dtype,w_dtype,layout", [(torch.bfloat16, None, 0), (torch.bfloat16, None, 1), (torch.float16, None, 0),
+                                                  (torch.float16, torch.float32, 0), (torch.bfloat16, torch.float32, 1),
+                                                  (torch.float32, None, 0)])
+@pytest.mark.parametrize("N,H,V,n_chunk,plan", [
+    (129, 136, 499, 4096, (False, False, False)),    # nothing cut, the vocabulary's end inside a run of eight columns
+    (700, 136, 4999, 4096, (False, True, False)),    # dx cut, one slab
+    (300, 520, 9001, 4096, (False, True, False)),
+    (5000, 136, 640, 16384, (False, False, True)),    # dW cut
+    (200, 520, 9001, 240, (True, True, False)),      # dx cut, and summed over slabs
+    (587, 296, 10053, 600, (True, True, False)),
+    (6000, 136, 1300, 1024, (True, False, True))])   # dW cut in every slab
+def test_cuts_and_slabs(N, H, V, n_chunk, plan, dtype, w_dtype, layout):
+    _check(N, H, V, n_chunk, dtype, w_dtype, layout, plan)
