@@ -28,7 +28,8 @@ int route_of(const lce_problem* p) { return p->route & ~(LCE_ROUTE_EXACT_SUMS | 
 
 // The last plan of a kind that this thread made.  A call asks for its plan up to three times (whether the route covers the
 // problem, the workspace, the launches), and a training step for the same one as the step before; a plan follows from the
-// problem's numbers alone, all of which are compared, and takes 1 to 4 us of the 30 to 60 that a call costs the host.
+// problem's numbers alone, all of which are compared, and takes 1 to 14 us of the 30 to 60 that a call costs the host (N=2000 in bf16:
+// H=64, V=1000 3, H=500, V=10007 8, H=768, V=50257 13; fp32 N=200, H=2048, V=16384 14).
 template <class Plan> struct LastPlan {
   lce_problem of;
   bool made = false;
@@ -211,7 +212,7 @@ struct BwdPlan {
   bool stage_dx;
   bool pack_on;   // tokens with an ignored label are packed away in this backward
   bool parts_on;  // tail tiles of dx / dW may be split along K (partial-sum blocks exist)
-  bool small;     // dx and dW run on 128 x 128 tiles (small_grads_pay)
+  bool small;     // dx and dW run on 128 x 128 tiles (make_plan_bwd, small_cost)
   bool narrow;    // no stage at all (lce_narrow.hip)
   int64_t small_blocks;  // room for the partial sums of either
   int64_t lddxc;
@@ -451,14 +452,16 @@ bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved)
   const size_t block = (size_t)lce::narrow_block_bytes(p->H);
   constexpr int64_t kWished = 1024;  // blocks: at most 64 MiB
   const int64_t room = (int64_t)((budget - fixed - w16) / block), most = room < kWished ? room : kWished;
-  const lce::SmallGrads g = lce::plan_narrow_grads(p->N, p->H, p->V, most);
+  const lce::SmallGrads wished = lce::plan_narrow_grads(p->N, p->H, p->V, kWished);
+  const bool fits = wished.dx_blocks + wished.dw_blocks <= most;
+  const lce::SmallGrads g = fits ? wished : lce::plan_narrow_grads(p->N, p->H, p->V, most);
   // (the kernel that adds a tile's parts goes through them eight at a time, one such after another: 0.2 us a part, N=10303, H=40, V=24
   // with 81 of them 33 us against 30 with nine)
   auto us = [](const lce::SmallGrads& c) -> double {
     const int parts = c.dx_nseg > c.dw_nseg ? c.dx_nseg : c.dw_nseg;
     return c.us + (parts > 8 ? 0.2 * (double)(parts - 8) : 0.0);
   };
-  *starved = most < kWished && us(g) > 1.1 * us(lce::plan_narrow_grads(p->N, p->H, p->V, kWished));
+  *starved = !fits && us(g) > 1.1 * us(wished);
   memset(b, 0, sizeof(*b));
   b->narrow = true;
   b->slabs = 1;

@@ -28,7 +28,6 @@ struct Abi {
   decltype(&lce_forward_backward_workspace_bytes) forward_backward_workspace_bytes;
   decltype(&lce_forward_backward_plan) forward_backward_plan;
   decltype(&lce_forward_backward) forward_backward;
-  decltype(&lce_scale_gradients) scale_gradients;
   decltype(&lce_stand_in) stand_in;
   decltype(&lce_unit_gradient) unit_gradient;
   decltype(&lce_pad_rows) pad_rows;
@@ -44,7 +43,6 @@ void bind(const py::dict& d) {
   bind_one(d, "lce_forward_backward_workspace_bytes", abi.forward_backward_workspace_bytes);
   bind_one(d, "lce_forward_backward_plan", abi.forward_backward_plan);
   bind_one(d, "lce_forward_backward", abi.forward_backward);
-  bind_one(d, "lce_scale_gradients", abi.scale_gradients);
   bind_one(d, "lce_stand_in", abi.stand_in);
   bind_one(d, "lce_unit_gradient", abi.unit_gradient);
   bind_one(d, "lce_pad_rows", abi.pad_rows);
