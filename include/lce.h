@@ -133,8 +133,10 @@ enum {
  * the front on the device and the tile kernels run on them only, so time
  * scales with the number of labelled tokens; the pre-pass costs a few small
  * launches (13 to 60 us of a forward + backward at 2048 to 16384 tokens, 7 to
- * 15 us of a forward alone), which a small problem does not earn back.  LCE_PACK_AUTO packs when 8*N*H*V >= 2^41 FLOPs; results are
- * the same either way up to the summation order of dW and the loss.  Use the same value in lce_workspace_bytes,
+ * 15 us of a forward alone), which a small problem does not earn back.  LCE_PACK_AUTO packs when 8*N*H*V >= 2^41 FLOPs (in lce_backward
+ * with a hidden size of up to 128 and 16-bit x: and H*V >= 2^21); results are
+ * the same either way up to the summation order of dW and the loss.  (A non-finite number in an ignored row of x stays without effect
+ * where rows are packed; elsewhere it reaches dW and that row's dx.)  Use the same value in lce_workspace_bytes,
  * lce_forward and lce_backward of one problem.
  */
 enum {

@@ -445,7 +445,11 @@ bool plan_narrow(const lce_problem* p, size_t budget, BwdPlan* b, bool* starved)
   if (p->w_dtype == LCE_F32 && p->w_layout == LCE_W_HV && lce::pad_to(p->H, 64) * lce::padded_vocab(p->V) * 2 >= (int64_t)1 << 31)
     return false;
   const size_t w16 = p->w_dtype == LCE_F32 ? align_up((size_t)p->H * (size_t)lce::padded_vocab(p->V) * 2) : 0;
-  const bool pack = packs_rows(p);
+  // Packing costs 0.4 to 0.9 ns a token here, a row being short, and a token's gradients little: where H * V is below 2^21 a few per cent
+  // of ignored tokens do not pay for it.  bf16, H=128, us of a backward, all rows / packed, with 5 % and with 85 % ignored: N=2^20, V=2048
+  // 2291 / 3108, 2050 / 690; N=262144, V=8192 2199 / 2360, 1949 / 498; N=131072, V=16384 2197 / 2243; N=65536, V=32768 2089 / 2078,
+  // 1845 / 739.  (Staged and packed 8983, 2235; 10156, 3113; -; 4052, 1414: all rows are no slower below that line.)
+  const bool pack = packs_rows(p) && p->H * p->V >= (int64_t)1 << 21;
   const PackPlan k = plan_pack(p, 0);
   const size_t fixed = pack ? k.end + align_up((size_t)p->N * 4) : 0;
   if (fixed + w16 > budget) return false;

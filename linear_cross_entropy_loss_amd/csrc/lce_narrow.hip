@@ -13,9 +13,9 @@
 // An accumulator block of S has the streaming index along its registers, in the order that the fragments of the second product
 // want along K once lanes l and l + 32 have exchanged quads: dz goes from one matrix instruction to the next without LDS.
 // dz is rounded once to the compute type, as in the staged kernels, and has their bits.
-// Large problems have their tokens with an ignored label packed away first, as with the staged kernels (packs_rows in lce_api.hip): the
-// number of rows is read from the device, and the cuts of dW follow it.  bf16 N=65536, H=128, V=32768, us of a backward, all rows / packed:
-// none ignored 2088 / 2117, 5 % 2089 / 2078, 85 % 1845 / 739; staged 4206, 4052, 1414.
+// Large problems have their tokens with an ignored label packed away first (plan_narrow in lce_api.hip says where): the number of rows is
+// read from the device, and the cuts of dW follow it.  bf16 N=65536, H=128, V=32768, us of a backward, all rows / packed: none ignored
+// 2088 / 2117, 5 % 2089 / 2078, 85 % 1845 / 739; staged 4206, 4052, 1414.
 //
 // Bound by vector instructions, of which an exponential is four, with the matrix instructions only partly under them: 128 x 128
 // logits take two workgroups of a compute unit 3.3 us for the forward and 3.1 for a gradient at a hidden size of 64 (0.6 of 1.4

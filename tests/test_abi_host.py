@@ -480,6 +480,10 @@ def test_narrow_plan_has_room_for_its_sums_or_is_not_taken():
         staged = plan(N, H, V, nc, max_workgroups=1 << 20)[1]  # (a call that limits its workgroups is staged)
         assert size <= 2 * staged
         assert not narrow or size >= 64 * block, (N, H, V, size)  # 64 stretches of the tokens at least
+    # many tokens of little work each are not packed (no room for a copy of x in the scratch), more work each and they are
+    for N, H, V, packed in ((1 << 20, 128, 2048, False), (262144, 128, 8192, False), (131072, 128, 16384, True), (65536, 128, 32768, True)):
+        narrow, size = plan(N, H, V, 4096)
+        assert narrow and (size >= _pack_bytes(N, H)) == packed, (N, H, V, size)
     # the copy of an fp32 weight alone is more than the bound, slabs of it are not
     for nc in (32, 64):
         narrow, size = plan(4096, 128, 50000, nc, torch.float32)
